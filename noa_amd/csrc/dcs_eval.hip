@@ -9,11 +9,17 @@
 #include "dcs_consts.hh"
 #include "dcs_f32m.hh"
 #include "dcs_f64.hh"
+#include "dcs_small.hh"
 #include "dcs_tile.hh"
 
 namespace noa_hip {
 
-constexpr int EVAL_TILE = 2048;
+// Pairs per workgroup of a map of n pairs; 64 is the small-map kernel
+// (dcs_small.hh), 2048 the tile kernel below, whose 98 workgroups at the line
+// take as long as 1024 would. Measured on MI355X (FP64, us, 64 / 2048):
+// 65,536 pairs 14.4 / 88; 131,072 22 / 91; 262,144 41 / 91; 524,288 77 / 92;
+// the mixed form 14.3 / 68, 22 / 71, 41 / 71, 77 / 72.
+inline int eval_tile(int64_t n) { return n <= 200000 ? 64 : 2048; }
 
 // Waves per SIMD the register allocation targets: the mixed form runs 2-3%
 // faster at 5 (96 VGPRs, a few spills in its set-up code) than at the 4 its
@@ -28,7 +34,7 @@ struct EvalWaves<F32MN<1>> {
     static constexpr int value = 5;
 };
 
-// One workgroup per tile of EVAL_TILE consecutive pairs.
+// One workgroup per tile of TILE consecutive pairs.
 template <class P, int TILE>
 __global__ __launch_bounds__(WG) __attribute__((amdgpu_waves_per_eu(EvalWaves<P>::value))) void dcs_eval_kernel(const double* __restrict__ K, const double* __restrict__ q,
                                                       int64_t n, DcsConsts c, Outs<typename P::out_t> o) {
@@ -42,9 +48,11 @@ __global__ __launch_bounds__(WG) __attribute__((amdgpu_waves_per_eu(EvalWaves<P>
 
 // run_tile reads c in place through kernarg_consts(), which locates it by
 // TileKernelArgs: the kernel's leading parameters must stay (K, q, n, c).
-static_assert(std::is_same<decltype(&dcs_eval_kernel<F64, EVAL_TILE>),
+static_assert(std::is_same<decltype(&dcs_eval_kernel<F64, 2048>),
                            void (*)(const double*, const double*, int64_t, DcsConsts, Outs<double>)>::value,
               "dcs_eval_kernel's parameters must begin as TileKernelArgs lays them out");
+static_assert(std::is_same<decltype(&dcs_small_kernel<double>), decltype(&dcs_eval_kernel<F64, 2048>)>::value,
+              "and dcs_small_kernel's with them");
 static_assert(offsetof(TileKernelArgs, c) == 24, "three 8-byte arguments before the constants");
 
 template <class P>
@@ -55,10 +63,12 @@ int launch_eval(const double* K, const double* q, int64_t n, const noa_dcs_eleme
     if (n == 0) return ok();
     if (!K || !q) return fail(NOA_DCS_EINVAL, "K and q must be non-NULL");
     if (!o.b && !o.p && !o.ph && !o.i) return ok();
-    const int64_t tiles = (n + EVAL_TILE - 1) / EVAL_TILE;
+    const int tile = eval_tile(n);
+    const int64_t tiles = (n + tile - 1) / tile;
     if (tiles > int64_t(0x7fffffff)) return fail(NOA_DCS_ERANGE, "n too large (%lld)", (long long)n);
     const DcsConsts c = make_consts(el->A, el->I, el->Z, mass);
-    hipLaunchKernelGGL((dcs_eval_kernel<P, EVAL_TILE>), dim3(uint32_t(tiles)), dim3(WG), 0, stream, K, q, n, c, o);
+    auto* kernel = tile == 64 ? &dcs_small_kernel<typename P::out_t> : &dcs_eval_kernel<P, 2048>;
+    hipLaunchKernelGGL(kernel, dim3(uint32_t(tiles)), dim3(WG), 0, stream, K, q, n, c, o);
     if (int rc = check_hip(hipGetLastError(), "dcs_eval_kernel launch")) return rc;
     return ok();
 }
