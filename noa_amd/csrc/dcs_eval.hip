@@ -15,11 +15,24 @@
 namespace noa_hip {
 
 // Pairs per workgroup of a map of n pairs; 64 is the small-map kernel
-// (dcs_small.hh), 2048 the tile kernel below, whose 98 workgroups at the line
-// take as long as 1024 would. Measured on MI355X (FP64, us, 64 / 2048):
-// 65,536 pairs 14.4 / 88; 131,072 22 / 91; 262,144 41 / 91; 524,288 77 / 92;
-// the mixed form 14.3 / 68, 22 / 71, 41 / 71, 77 / 72.
-inline int eval_tile(int64_t n) { return n <= 200000 ? 64 : 2048; }
+// (dcs_small.hh), larger ones the tile kernel below. Four workgroups of the
+// tile kernel fit a CU, 1024 the chip: a map takes the largest tile that
+// still gives about one round of them, since a partly filled chip costs more
+// than the smaller tile's partly filled waves. Measured on MI355X (FP64 /
+// mixed, us, at tiles of 64, 256, 512, 1024, 2048):
+//   131,072 pairs    22  30  36  51  91   /   22  33  35  45  71
+//   262,144          41  37  42  51  91   /   41  39  42  45  71
+//   524,288          77  69  59  63  92   /   77  66  56  57  72
+//   1,048,576       152 119 100  95 114   /  152 110  91  82  89
+//   3,000,017         -   -  255 243 254  /    -   -  213 194 192
+//   8,388,608         -   -  670 632 621  /    -   -  553 476 442
+inline int eval_tile(int64_t n, bool f64) {
+    if (n <= 200000) return 64;
+    if (n <= 300000) return 256;
+    if (n <= 700000) return 512;
+    if (n <= (f64 ? 7000000 : 2500000)) return 1024;
+    return 2048;
+}
 
 // Waves per SIMD the register allocation targets: the mixed form runs 2-3%
 // faster at 5 (96 VGPRs, a few spills in its set-up code) than at the 4 its
@@ -63,11 +76,15 @@ int launch_eval(const double* K, const double* q, int64_t n, const noa_dcs_eleme
     if (n == 0) return ok();
     if (!K || !q) return fail(NOA_DCS_EINVAL, "K and q must be non-NULL");
     if (!o.b && !o.p && !o.ph && !o.i) return ok();
-    const int tile = eval_tile(n);
+    const int tile = eval_tile(n, !P::has_redo);
     const int64_t tiles = (n + tile - 1) / tile;
     if (tiles > int64_t(0x7fffffff)) return fail(NOA_DCS_ERANGE, "n too large (%lld)", (long long)n);
     const DcsConsts c = make_consts(el->A, el->I, el->Z, mass);
-    auto* kernel = tile == 64 ? &dcs_small_kernel<typename P::out_t> : &dcs_eval_kernel<P, 2048>;
+    auto* kernel = tile == 64     ? &dcs_small_kernel<typename P::out_t>
+                   : tile == 256  ? &dcs_eval_kernel<P, 256>
+                   : tile == 512  ? &dcs_eval_kernel<P, 512>
+                   : tile == 1024 ? &dcs_eval_kernel<P, 1024>
+                                  : &dcs_eval_kernel<P, 2048>;
     hipLaunchKernelGGL(kernel, dim3(uint32_t(tiles)), dim3(WG), 0, stream, K, q, n, c, o);
     if (int rc = check_hip(hipGetLastError(), "dcs_eval_kernel launch")) return rc;
     return ok();

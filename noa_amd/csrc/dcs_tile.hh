@@ -239,21 +239,26 @@ __device__ __forceinline__ void run_tile(int64_t base, int64_t end, const double
     }
     __syncthreads();
 
-    // phase 2: dense integrals, photonuclear (heavier) first
+    // phase 2: dense integrals, photonuclear (heavier) first. The pair-
+    // production items start at a whole wave, so that no wave runs both
+    // integrals one after the other (without it one wave per tile does: 1% on
+    // 2^24 pairs in tiles of 2048, 13% in tiles of 512)
     const uint32_t nph = s.n_photo;
-    const uint32_t total = nph + s.n_pair;
+    const uint32_t pair0 = (nph + 63u) & ~63u;
+    const uint32_t total = pair0 + s.n_pair;
 #pragma unroll 1
     for (uint32_t v = tid; v < total; v += WG) {
         const DcsConsts& c = item_consts(cp);
         bool redo = false;
         uint32_t tag;
-        if (v < nph) {
+        if (v < pair0) {
+            if (v >= nph) continue;
             tag = s.photo[v];
             const int64_t g = base + tag;
             store_stream(&o.ph[g], P::photo(K[g], q[g], c, redo, t));
             tag |= REDO_PHOTO;
         } else {
-            tag = s.pair[v - nph];
+            tag = s.pair[v - pair0];
             const int64_t g = base + tag;
             if constexpr (P::has_redo)
                 store_stream(&o.p[g], P::pair(K[g], q[g], c, redo, t));
