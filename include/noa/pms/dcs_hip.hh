@@ -221,16 +221,13 @@ inline auto vmap_integral(const RecoilIntegral& cs) {
         detail::check_output(result, kinetic_energies, torch::kFloat64);
         const c10::DeviceGuard guard(kinetic_energies.device());
         const int64_t n = kinetic_energies.numel();
-        const int64_t bytes = noa_dcs_recoil_workspace_bytes(n, min_points);
-        const auto ws = torch::empty({std::max<int64_t>(bytes, 8)},
-                                     torch::TensorOptions().dtype(torch::kUInt8).device(kinetic_energies.device()));
         double* p[4] = {nullptr, nullptr, nullptr, nullptr};
         p[cs.process.id] = result.data_ptr<double>();
         const noa_dcs_outputs_f64 o{p[0], p[1], p[2], p[3]};
         const noa_dcs_element e{element.A, element.I, element.Z};
-        detail::raise(noa_dcs_recoil_integrals_f64(kinetic_energies.data_ptr<double>(), n, xlow, &e, mass, min_points,
-                                                   cs.integrand.cel ? nullptr : &o, cs.integrand.cel ? &o : nullptr,
-                                                   ws.data_ptr(), bytes, detail::stream_of(kinetic_energies)));
+        detail::raise(noa_dcs_recoil_integrals_f64_noalloc(
+            kinetic_energies.data_ptr<double>(), n, xlow, &e, mass, min_points, cs.integrand.cel ? nullptr : &o,
+            cs.integrand.cel ? &o : nullptr, detail::stream_of(kinetic_energies)));
     };
 }
 

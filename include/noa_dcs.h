@@ -152,7 +152,10 @@ int noa_dcs_eval_f32mixed(const double* K, const double* q, int64_t n, const noa
  * integrated over t = ln q (integrand dcs q, resp. dcs q^2) with the 6-node
  * rule on ceil(min_points/6) subintervals.
  * Any output pointer may be NULL (del or cel themselves too). workspace is
- * a device buffer of at least noa_dcs_recoil_workspace_bytes(n, min_points).
+ * a device buffer of at least noa_dcs_recoil_workspace_bytes(n, min_points),
+ * as the interface has always asked for; the kernel keeps its nodes on chip
+ * and does not touch it. A caller who would allocate it for this call alone
+ * takes the entry point below.
  */
 int64_t noa_dcs_recoil_workspace_bytes(int64_t n, int32_t min_points);
 int noa_dcs_recoil_integrals_f64(const double* K, int64_t n, double xlow, const noa_dcs_element* element,
@@ -165,14 +168,10 @@ int noa_dcs_recoil_integrals_f64(const double* K, int64_t n, double xlow, const 
  * No counterpart in the reference: for callers that cannot allocate device
  * memory (code under HIP graph capture, serving loops, harnesses that forbid
  * hipMalloc). It calls no hipMalloc / hipFree and no allocating library
- * routine; its node pairs and DCS planes live in a file-scope device array
- * of noa_dcs_recoil_noalloc_scratch_bytes() (32 MiB) that each GPU holds
- * until the process ends. Any n is processed, in chunks of
- * scratch / (48 ceil(min_points / 6) * 6) kinetic energies (3883 at
- * min_points = 180); a min_points whose single kinetic energy would not fit
- * returns NOA_DCS_ERANGE. Results equal noa_dcs_recoil_integrals_f64's bit
- * for bit. Every call on a GPU shares that GPU's array: calls that overlap
- * on one GPU (two streams, or two host threads) race; serialise them.
+ * routine, and holds no device memory; calls may overlap freely. Any n is
+ * processed. Results equal noa_dcs_recoil_integrals_f64's bit for bit.
+ * noa_dcs_recoil_noalloc_scratch_bytes() still returns the 32 MiB that each
+ * GPU used to hold for it, for callers that budget by it.
  */
 int64_t noa_dcs_recoil_noalloc_scratch_bytes(void);
 int noa_dcs_recoil_integrals_f64_noalloc(const double* K, int64_t n, double xlow, const noa_dcs_element* element,

@@ -6,16 +6,18 @@
 // subintervals of [ln(K xlow), ln K] (numerics.hh:72-108). Ionisation below
 // K = (m - m_e)^2 / (2 m_e) takes the reference's analytic form.
 //
-// The DCS map is the cost (180 evaluations per K and process at the
-// reference's min_points = 180), so the nodes of a chunk of K values are
-// materialised as (K, q) pairs and pushed through the same compacting tile
-// kernel as any (K, q) map, all four processes at once; a per-K pass then
-// sums the nodes in the reference's order.
+// The DCS is the cost (180 evaluations per K and process at the reference's
+// min_points = 180). One kernel does the whole of it: a workgroup takes a
+// group of K values, evaluates their nodes like a map's tile (closed forms
+// and exits per node, the open integrals compacted in LDS and drained by
+// whole waves), keeps the node values in LDS and sums them there, so no
+// (K, q) pair, no DCS value and no scratch goes through memory.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <cstddef>
 #include <cstdint>
-#include <mutex>
+#include <type_traits>
 
 #include "capi_util.hh"
 #include "dcs_consts.hh"
@@ -29,52 +31,14 @@ namespace noa_hip {
 static __constant__ double GL6_X[6] = {0.03376524, 0.16939531, 0.38069041, 0.61930959, 0.83060469, 0.96623476};
 static __constant__ double GL6_W[6] = {0.08566225, 0.18038079, 0.23395697, 0.23395697, 0.18038079, 0.08566225};
 
-constexpr int RECOIL_CHUNK = 65536;  // K values per pass
-
-// Scratch of the no-allocation entry point noa_dcs_recoil_integrals_f64_noalloc:
-// file-scope device memory, one copy per GPU the library runs on, held until
-// the process ends. Host code never uses this name as an address (on the host
-// it is a stand-in for the symbol): it takes the device address once per
-// device from hipGetSymbolAddress.
-constexpr int64_t RECOIL_SCRATCH_BYTES = int64_t(32) << 20;
-static __device__ __align__(256) unsigned char scratch[RECOIL_SCRATCH_BYTES];
+constexpr int RECOIL_CHUNK = 65536;                            // K values the workspace is sized for
+constexpr int64_t RECOIL_SCRATCH_BYTES = int64_t(32) << 20;  // as noa_dcs_recoil_noalloc_scratch_bytes reports
 
 struct RecoilGrid {
     double xlow;
     int32_t n_itv;  // subintervals
     int32_t nodes;  // 6 n_itv
 };
-
-// Node j of K: t = lb + h ((j / 6) + x_{j % 6}), lb = ln(K xlow), h = (ln K - lb) / n_itv.
-__device__ __forceinline__ double node_t(double K, const RecoilGrid& g, int j, const fm::Tab& t, double* h_out) {
-#pragma clang fp contract(off)
-    const double lb = fm::log(K * g.xlow, t);
-    const double ub = fm::log(K, t);
-    const double h = (ub - lb) / double(uint32_t(g.n_itv));
-    *h_out = h;
-    return lb + h * (double(uint32_t(j / 6)) + GL6_X[j % 6]);
-}
-
-__global__ __launch_bounds__(256) void recoil_nodes_kernel(const double* __restrict__ K, int64_t nK, RecoilGrid g,
-                                                           double* __restrict__ Kn, double* __restrict__ qn) {
-    __shared__ __attribute__((aligned(fm::TABLE_LDS_ALIGN))) double fm_block[fm::TABLE_DOUBLES];
-    load_fm_tables(fm_block);
-    __syncthreads();
-    const fm::Tab tab = fm::tab_from_block(fm_block);
-    const int64_t total = nK * g.nodes;
-    // node-major: node j of K index i at j * nK + i, so that the per-K pass
-    // reads each node plane coalesced
-    for (int64_t idx = int64_t(blockIdx.x) * blockDim.x + threadIdx.x; idx < total;
-         idx += int64_t(gridDim.x) * blockDim.x) {
-        const int j = int(idx / nK);
-        const int64_t i = idx - int64_t(j) * nK;
-        const double k = K[i];
-        double h;
-        const double tj = node_t(k, g, j, tab, &h);
-        Kn[idx] = k;
-        qn[idx] = fm::exp(tj, tab);
-    }
-}
 
 // dcs.hh:469-496 with the terms of :446-466.
 __device__ __forceinline__ double analytic_ionisation(double K, double xlow, const DcsConsts& c, bool cel,
@@ -98,47 +62,187 @@ __device__ __forceinline__ double analytic_ionisation(double K, double xlow, con
     return 1.535336E-05 * c.Zd / c.A * term;
 }
 
-// One thread per K: sequential sums over the nodes (the reference's order).
-__global__ __launch_bounds__(256) void recoil_reduce_kernel(const double* __restrict__ K, int64_t nK, RecoilGrid g,
-                                                            const double* __restrict__ qn, Outs<double> dcs,
-                                                            DcsConsts c, Outs<double> del, Outs<double> cel) {
-    __shared__ __attribute__((aligned(fm::TABLE_LDS_ALIGN))) double fm_block[fm::TABLE_DOUBLES];
-    load_fm_tables(fm_block);
-    __syncthreads();
-    const fm::Tab tab = fm::tab_from_block(fm_block);
-    for (int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x; i < nK; i += int64_t(gridDim.x) * blockDim.x) {
+// dcs.hh:955-1001: the ionisation integrals take the analytic form up to here.
+__device__ __forceinline__ bool ion_is_analytic(double K, const DcsConsts& c) {
 #pragma clang fp contract(off)
-        const double k = K[i];
-        double h;
-        (void)node_t(k, g, 0, tab, &h);
-        const double E = k + c.mass;
-        const double* planes[4] = {dcs.b, dcs.p, dcs.ph, dcs.i};
-        double* dst_del[4] = {del.b, del.p, del.ph, del.i};
-        double* dst_cel[4] = {cel.b, cel.p, cel.ph, cel.i};
-        const double m1 = c.mass - ELECTRON_MASS;
-        const bool ion_analytic = k <= 0.5 * m1 * m1 / ELECTRON_MASS;
-        for (int p = 0; p < 4; p++) {
-            if (!dst_del[p] && !dst_cel[p]) continue;
-            if (p == 3 && ion_analytic) {
-                if (dst_del[p]) dst_del[p][i] = analytic_ionisation(k, g.xlow, c, false, tab);
-                if (dst_cel[p]) dst_cel[p][i] = analytic_ionisation(k, g.xlow, c, true, tab);
-                continue;
+    const double m1 = c.mass - ELECTRON_MASS;
+    return K <= 0.5 * m1 * m1 / ELECTRON_MASS;
+}
+
+// A workgroup's nodes in LDS, by item: node j of the group's K slot k at k nb + j.
+template <int TILE>
+struct RecoilLds {
+    double q[TILE];
+    double dcs[4][TILE];                // pair production: argmin until its integral has run
+    double K[TILE / 6], lb[TILE / 6], h[TILE / 6];  // K, ln(K xlow) and the subinterval width, by K slot
+    double part[TILE / 6][8];           // the DEL and CEL sums of a K
+    double acc[8];                      // the sums of the node blocks before this one
+    uint16_t photo_list[TILE], pair_list[TILE];
+    uint32_t n_photo, n_pair;
+};
+
+// The leading arguments of recoil_kernel, as TileKernelArgs lays out a map's.
+struct RecoilKernelArgs {
+    const double* K;
+    int64_t n;
+    DcsConsts c;
+};
+
+// Sum over the wave's lanes, in a fixed order, valid in lane 0.
+__device__ __forceinline__ double wave_sum(double v) {
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) v += __shfl_down(v, off, 64);
+    return v;
+}
+
+// Nodes per tile: two K values at min_points = 180, 360 nodes of 512 (lanes
+// are 94% full whether a tile holds 1, 2 or 4 such K values). At 512 four
+// workgroups fit a CU; tiles of 768 leave three and were as fast at 65,536 K
+// and slower below, tiles of 256 (one K) 15% slower there.
+constexpr int RECOIL_TILE = 512;
+
+// One workgroup per `group` K values; their nodes fit one tile, or (BLOCKS)
+// group = 1 and the nodes go in blocks of TILE.
+//
+// Bound: FP64 VALU issue, as the map's tile kernel (the nodes have q >= K
+// xlow, so nearly all open pair production and ~60% photonuclear: ~5000
+// instructions each against the map's 2351). Passing the nodes through
+// memory instead (a kernel that wrote (K, q) pairs, the map in tiles of 2048,
+// and a sum per thread) took, at min_points 180, 444 us for 146 K values and
+// 1790 us for 65,536, of which 296 and 320 us were the serial sums; this
+// kernel takes 28 and 1567. At 30 points 189 -> 21 and 354 -> 336, at 6
+// points 81 -> 24 and 167 -> 127.
+// The nodes-in-blocks form is an instantiation of its own: its loop carries
+// values that made the common one spill 28 registers.
+template <int TILE, bool BLOCKS>
+__global__ __launch_bounds__(WG) __attribute__((amdgpu_waves_per_eu(4))) void recoil_kernel(
+    const double* __restrict__ K, int64_t n, DcsConsts, RecoilGrid g, int32_t group, Outs<double> del,
+    Outs<double> cel) {
+    __shared__ RecoilLds<TILE> s;
+    __shared__ __attribute__((aligned(fm::TABLE_LDS_ALIGN))) double fm_block[fm::TABLE_DOUBLES];
+    using KArg = const __attribute__((address_space(4))) char*;
+    const ConstsPtr cp = (ConstsPtr)((KArg)__builtin_amdgcn_kernarg_segment_ptr() + offsetof(RecoilKernelArgs, c));
+    const int tid = threadIdx.x;
+    const int lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    load_fm_tables(fm_block);
+    const fm::Tab t = fm::tab_from_block(fm_block);
+    const bool want_b = del.b || cel.b, want_p = del.p || cel.p, want_ph = del.ph || cel.ph, want_i = del.i || cel.i;
+    const int64_t k0 = int64_t(blockIdx.x) * group;
+    const int nk = int(n - k0 < group ? n - k0 : group);
+    __syncthreads();
+    for (int kk = tid; kk < nk; kk += WG) {
+#pragma clang fp contract(off)
+        const double k = K[k0 + kk];
+        const double lb = fm::log(k * g.xlow, t);
+        s.K[kk] = k;
+        s.lb[kk] = lb;
+        s.h[kk] = (fm::log(k, t) - lb) / double(uint32_t(g.n_itv));
+    }
+    for (int j0 = 0; j0 < (BLOCKS ? g.nodes : 1); j0 += TILE) {
+        const int nb = BLOCKS && g.nodes - j0 > TILE ? TILE : g.nodes - j0;
+        const int items = nk * nb;
+        if (tid == 0) {
+            s.n_photo = 0;
+            s.n_pair = 0;
+        }
+        __syncthreads();
+        // the nodes: closed forms, exits, the lists of open integrals
+#pragma unroll 1
+        for (int i0 = 0; i0 < items; i0 += WG) {
+            const DcsConsts& c = item_consts(cp);
+            const int i = i0 + tid;
+            bool pa = false, pha = false;
+            if (i < items) {
+                const int kk = i / nb;
+                const int j = j0 + (i - kk * nb);
+                const double k = s.K[kk];
+                double q, am = 0.;
+                {
+#pragma clang fp contract(off)
+                    q = fm::exp(s.lb[kk] + s.h[kk] * (double(uint32_t(j / 6)) + GL6_X[j % 6]), t);
+                }
+                s.q[i] = q;
+                if (want_b) s.dcs[0][i] = F64::brems(k, q, c, t);
+                if (want_i && !ion_is_analytic(k, c)) s.dcs[3][i] = F64::ion(k, q, c, t);
+                if (want_p) {
+                    pa = F64::pair_active(k, q, c, am);
+                    s.dcs[1][i] = pa ? am : 0.;
+                }
+                if (want_ph) {
+                    pha = F64::photo_active(k, q, c);
+                    s.dcs[2][i] = 0.;
+                }
             }
-            const double* d = planes[p] + i;
-            const double* qq = qn + i;
-            double sd = 0., sc = 0.;
-            for (int j = 0; j < g.nodes; j++) {
-                const double w = GL6_W[j % 6];
-                const double qj = qq[int64_t(j) * nK];
-                const double dq = d[int64_t(j) * nK] * qj;
-                sd += dq * h * w;
-                sc += dq * qj * h * w;
+            if (want_ph) wave_append(pha, &s.n_photo, s.photo_list, uint32_t(i));
+            if (want_p) wave_append(pa, &s.n_pair, s.pair_list, uint32_t(i));
+        }
+        __syncthreads();
+        // the integrals, whole waves of one kind, photonuclear (heavier) first
+        const uint32_t nph = s.n_photo;
+        const uint32_t pair0 = (nph + 63u) & ~63u;
+        const uint32_t total = pair0 + s.n_pair;
+#pragma unroll 1
+        for (uint32_t v = tid; v < total; v += WG) {
+            const DcsConsts& c = item_consts(cp);
+            if (v < pair0) {
+                if (v >= nph) continue;
+                const uint32_t i = s.photo_list[v];
+                s.dcs[2][i] = F64::photo(s.K[i / uint32_t(nb)], s.q[i], c, t);
+            } else {
+                const uint32_t i = s.pair_list[v - pair0];
+                s.dcs[1][i] = F64::pair_at(s.K[i / uint32_t(nb)], s.q[i], s.dcs[1][i], c, t);
             }
-            if (dst_del[p]) dst_del[p][i] = sd / E;
-            if (dst_cel[p]) dst_cel[p][i] = sc / E;
+        }
+        __syncthreads();
+        // sums: a wave takes one K
+        for (int kk = wave; kk < nk; kk += WG / 64) {
+#pragma clang fp contract(off)
+            double sum[8] = {};
+            for (int l = lane; l < nb; l += 64) {
+                const int i = kk * nb + l;
+                const double q = s.q[i];
+                const double hw = s.h[kk] * GL6_W[(j0 + l) % 6];
+#pragma unroll
+                for (int p = 0; p < 4; p++) {
+                    const double dq = s.dcs[p][i] * q;
+                    sum[p] += dq * hw;
+                    sum[4 + p] += dq * q * hw;
+                }
+            }
+#pragma unroll
+            for (int p = 0; p < 8; p++) sum[p] = wave_sum(sum[p]);
+            if (lane == 0)
+#pragma unroll
+                for (int p = 0; p < 8; p++) s.part[kk][p] = sum[p];
+        }
+        __syncthreads();
+        const bool last = !BLOCKS || j0 + TILE >= g.nodes;
+        for (int v = tid; v < nk * 8; v += WG) {
+            const int kk = v / 8, p = v % 8;
+            double acc = s.part[kk][p];
+            if (BLOCKS && j0 > 0) acc += s.acc[p];  // (more than one node block: one K)
+            if (!last) {
+                s.acc[p] = acc;
+            } else {
+                const DcsConsts& c = item_consts(cp);
+                const bool is_cel = p >= 4;
+                const Outs<double>& out = is_cel ? cel : del;
+                double* dst = (p & 3) == 0 ? out.b : (p & 3) == 1 ? out.p : (p & 3) == 2 ? out.ph : out.i;
+                const double k = s.K[kk];
+                double r = acc / (k + c.mass);
+                if ((p & 3) == 3 && ion_is_analytic(k, c)) r = analytic_ionisation(k, g.xlow, c, is_cel, t);
+                if (dst) dst[k0 + kk] = r;
+            }
         }
     }
 }
+
+static_assert(std::is_same<decltype(&recoil_kernel<RECOIL_TILE, false>),
+                           void (*)(const double*, int64_t, DcsConsts, RecoilGrid, int32_t, Outs<double>,
+                                    Outs<double>)>::value,
+              "recoil_kernel's parameters must begin as RecoilKernelArgs lays them out");
+static_assert(offsetof(RecoilKernelArgs, c) == 16, "two 8-byte arguments before the constants");
 
 }  // namespace noa_hip
 
@@ -147,10 +251,6 @@ using namespace noa_hip;
 namespace {
 
 int64_t nodes_of(int32_t min_points) { return int64_t((uint32_t(min_points) + 5u) / 6u) * 6; }
-
-// Bytes of scratch per kinetic energy: the node pairs (K, q) and the four
-// DCS planes, 6 doubles per node.
-int64_t bytes_per_K(int32_t min_points) { return nodes_of(min_points) * int64_t(6 * sizeof(double)); }
 
 int check_recoil_args(const double* K, int64_t n, double xlow, const noa_dcs_element* element, double mass,
                       int32_t min_points) {
@@ -162,54 +262,33 @@ int check_recoil_args(const double* K, int64_t n, double xlow, const noa_dcs_ele
     return NOA_DCS_OK;
 }
 
-// The passes over chunks of at most chunk_cap kinetic energies, with the
-// node pairs and DCS planes in `work` (chunk_cap * bytes_per_K bytes).
+// K values per workgroup: one as long as that fills the chip (1024 workgroups,
+// 4 per CU), then as many as a tile holds; and at least a wave's worth of
+// nodes. Measured (min_points 180, one / two K values per workgroup): 1000 K
+// 43 / 51 us, 2000 K 77 / 76, 65,536 K 1802 / 1569; with 30 nodes each, 2000
+// K 46 / 24.
+int32_t recoil_group(int64_t n, int32_t nodes) {
+    const int64_t want = std::max<int64_t>((n + 1023) / 1024, 64 / nodes);
+    return int32_t(std::max<int64_t>(1, std::min<int64_t>(RECOIL_TILE / nodes, want)));
+}
+
 int recoil_run(const double* K, int64_t n, double xlow, const noa_dcs_element* element, double mass,
-               int32_t min_points, const noa_dcs_outputs_f64& D, const noa_dcs_outputs_f64& C, double* work,
-               int64_t chunk_cap, hipStream_t stream) {
-    const bool want[4] = {D.brems || C.brems, D.pair || C.pair, D.photo || C.photo, D.ion || C.ion};
+               int32_t min_points, const noa_dcs_outputs_f64& D, const noa_dcs_outputs_f64& C, hipStream_t stream) {
     const RecoilGrid g{xlow, int32_t((uint32_t(min_points) + 5u) / 6u), int32_t(nodes_of(min_points))};
-    double* Kn = work;
-    double* qn = Kn + chunk_cap * g.nodes;
-    double* planes = qn + chunk_cap * g.nodes;
     const DcsConsts c = make_consts(element->A, element->I, element->Z, mass);
-    for (int64_t k0 = 0; k0 < n; k0 += chunk_cap) {
-        const int64_t nK = std::min<int64_t>(chunk_cap, n - k0);
-        const int64_t nn = nK * g.nodes;
-        const unsigned grid = unsigned(std::min<int64_t>(65536, (nn + 255) / 256));
-        hipLaunchKernelGGL(recoil_nodes_kernel, dim3(grid), dim3(256), 0, stream, K + k0, nK, g, Kn, qn);
-        if (int rc = check_hip(hipGetLastError(), "recoil_nodes_kernel")) return rc;
-        noa_dcs_outputs_f64 node_out{want[0] ? planes : nullptr, want[1] ? planes + nn : nullptr,
-                                     want[2] ? planes + 2 * nn : nullptr, want[3] ? planes + 3 * nn : nullptr};
-        if (int rc = noa_dcs_eval_f64(Kn, qn, nn, element, mass, &node_out, stream)) return rc;
-        const Outs<double> d_out{node_out.brems, node_out.pair, node_out.photo, node_out.ion};
+    const auto kernel = g.nodes > RECOIL_TILE ? &recoil_kernel<RECOIL_TILE, true> : &recoil_kernel<RECOIL_TILE, false>;
+    constexpr int64_t most = int64_t(1) << 30;  // K values per launch (a grid has at most 2^31 - 1 workgroups)
+    for (int64_t k0 = 0; k0 < n; k0 += most) {
+        const int64_t nK = std::min<int64_t>(most, n - k0);
         auto shift = [k0](double* p) { return p ? p + k0 : nullptr; };
         const Outs<double> od{shift(D.brems), shift(D.pair), shift(D.photo), shift(D.ion)};
         const Outs<double> oc{shift(C.brems), shift(C.pair), shift(C.photo), shift(C.ion)};
-        hipLaunchKernelGGL(recoil_reduce_kernel, dim3(unsigned((nK + 255) / 256)), dim3(256), 0, stream, K + k0, nK, g,
-                           qn, d_out, c, od, oc);
-        if (int rc = check_hip(hipGetLastError(), "recoil_reduce_kernel")) return rc;
+        const int32_t group = recoil_group(nK, g.nodes);
+        hipLaunchKernelGGL(kernel, dim3(unsigned((nK + group - 1) / group)), dim3(WG), 0, stream, K + k0, nK, c, g,
+                           group, od, oc);
+        if (int rc = check_hip(hipGetLastError(), "recoil_kernel")) return rc;
     }
     return ok();
-}
-
-// Device address of `scratch` on the current device, looked up once per
-// device (each GPU holds its own copy of the array at its own address).
-int scratch_address(void** out) {
-    static std::mutex mu;
-    static void* addr[64] = {};
-    int dev = 0;
-    if (int rc = check_hip(hipGetDevice(&dev), "hipGetDevice")) return rc;
-    if (dev < 0 || dev >= 64) return fail(NOA_DCS_ERANGE, "device ordinal %d beyond 63", dev);
-    std::lock_guard<std::mutex> lock(mu);
-    if (!addr[dev]) {
-        void* p = nullptr;
-        if (int rc = check_hip(hipGetSymbolAddress(&p, HIP_SYMBOL(scratch)), "hipGetSymbolAddress(scratch)"))
-            return rc;
-        addr[dev] = p;
-    }
-    *out = addr[dev];
-    return NOA_DCS_OK;
 }
 
 }  // namespace
@@ -232,8 +311,7 @@ int noa_dcs_recoil_integrals_f64(const double* K, int64_t n, double xlow, const 
     if (n == 0 || !(D.brems || D.pair || D.photo || D.ion || C.brems || C.pair || C.photo || C.ion)) return ok();
     if (!workspace || workspace_bytes < noa_dcs_recoil_workspace_bytes(n, min_points))
         return fail(NOA_DCS_EINVAL, "workspace must hold noa_dcs_recoil_workspace_bytes(n, min_points) bytes");
-    return recoil_run(K, n, xlow, element, mass, min_points, D, C, static_cast<double*>(workspace),
-                      std::min<int64_t>(n, RECOIL_CHUNK), stream);
+    return recoil_run(K, n, xlow, element, mass, min_points, D, C, stream);
 }
 
 int64_t noa_dcs_recoil_noalloc_scratch_bytes(void) { return RECOIL_SCRATCH_BYTES; }
@@ -246,13 +324,7 @@ int noa_dcs_recoil_integrals_f64_noalloc(const double* K, int64_t n, double xlow
     const noa_dcs_outputs_f64& D = del ? *del : none;
     const noa_dcs_outputs_f64& C = cel ? *cel : none;
     if (n == 0 || !(D.brems || D.pair || D.photo || D.ion || C.brems || C.pair || C.photo || C.ion)) return ok();
-    const int64_t chunk_cap = std::min<int64_t>(n, RECOIL_SCRATCH_BYTES / bytes_per_K(min_points));
-    if (chunk_cap < 1)
-        return fail(NOA_DCS_ERANGE, "min_points %d needs %lld scratch bytes per kinetic energy, more than the %lld held",
-                    min_points, (long long)bytes_per_K(min_points), (long long)RECOIL_SCRATCH_BYTES);
-    void* work = nullptr;
-    if (int rc = scratch_address(&work)) return rc;
-    return recoil_run(K, n, xlow, element, mass, min_points, D, C, static_cast<double*>(work), chunk_cap, stream);
+    return recoil_run(K, n, xlow, element, mass, min_points, D, C, stream);
 }
 
 }  // extern "C"

@@ -264,7 +264,7 @@ cel_integrand = _Integrand("cel_integrand", True)    # dcs.hh:111-113: dcs * q^2
 
 def recoil_integrals(kinetic_energies: torch.Tensor, xlow: float, element: AtomicElement, mass: float,
                      min_points: int = 180, dels=None, cels=None) -> None:
-    """DEL / CEL recoil integrals of the four processes in one pass (noa_dcs_recoil_integrals_f64):
+    """DEL / CEL recoil integrals of the four processes in one pass (noa_dcs_recoil_integrals_f64_noalloc):
     dels and cels are 4-tuples of float64 tensors like K, or None entries."""
     K = kinetic_energies
     _check_inputs(K, K)
@@ -272,15 +272,13 @@ def recoil_integrals(kinetic_energies: torch.Tensor, xlow: float, element: Atomi
     cels = tuple(cels) if cels is not None else (None,) * 4
     for r in dels + cels:
         _check_output(r, K, torch.float64)
-    nbytes = _lib.lib().noa_dcs_recoil_workspace_bytes(K.numel(), int(min_points))
-    ws = torch.empty(max(nbytes, 8), dtype=torch.uint8, device=K.device)
     d = _lib.OutputsF64(*(_ptr(r) for r in dels))
     c = _lib.OutputsF64(*(_ptr(r) for r in cels))
     el = _element(element)
     with torch.cuda.device(K.device):
-        _lib.check(_lib.lib().noa_dcs_recoil_integrals_f64(_ptr(K), K.numel(), float(xlow), ctypes.byref(el),
-                                                           float(mass), int(min_points), ctypes.byref(d),
-                                                           ctypes.byref(c), _ptr(ws), nbytes, _stream(K)))
+        _lib.check(_lib.lib().noa_dcs_recoil_integrals_f64_noalloc(_ptr(K), K.numel(), float(xlow), ctypes.byref(el),
+                                                                   float(mass), int(min_points), ctypes.byref(d),
+                                                                   ctypes.byref(c), _stream(K)))
 
 
 def recoil_integral(dcs_func: Process, integrand: _Integrand):
