@@ -201,7 +201,8 @@ int noa_dcs_hard_scattering_f64(int64_t nel, int64_t nkin, const double* G, cons
                                 double* lb_h, hipStream_t stream);
 /* Replaces dcs::soft_scattering (dcs.hh:940-950): the first transverse
  * transport coefficient of soft ionisation and photonuclear interactions.
- * workspace is a device buffer of noa_dcs_soft_scattering_workspace_bytes(n). */
+ * workspace is a device buffer of noa_dcs_soft_scattering_workspace_bytes(n),
+ * as the interface has always asked for; the kernel does not touch it. */
 int64_t noa_dcs_soft_scattering_workspace_bytes(int64_t n);
 int noa_dcs_soft_scattering_f64(const double* K, int64_t n, const noa_dcs_element* element, double mass,
                                 double* result, void* workspace, int64_t workspace_bytes, hipStream_t stream);

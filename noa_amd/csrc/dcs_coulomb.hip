@@ -13,11 +13,11 @@
 // with the FP64 log/exp tables in LDS. Per-element values the reference
 // recomputes in every call (pow(A, 1/3), pow(Z, 2/3), cos of the soft
 // angle, the node values nu_j = 0.05 exp(t_j), which are the same for every
-// K) are evaluated once on the host with the host libm. The photonuclear DCS
-// at the soft-scattering nodes goes through the same compacting tile kernel
-// as any (K, q) map; a per-K pass then sums the nodes in the reference's
-// order. Every device function keeps the reference's operation order with
-// FMA contraction off.
+// K) are evaluated once on the host with the host libm. Soft scattering is
+// one kernel too: a workgroup compacts the open photonuclear nodes of its K
+// values in LDS, evaluates them in whole waves and sums them there. Every
+// device function keeps the reference's operation order with FMA contraction
+// off.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -38,7 +38,15 @@ constexpr int NSF = 9;                 // physics.hh:87
 
 constexpr int SOFT_ITV = 17;               // ceil(100 / 6) subintervals (dcs.hh:936, numerics.hh:80)
 constexpr int SOFT_NODES = 6 * SOFT_ITV;   // 102
-constexpr int SOFT_CHUNK = 16384;          // K values per pass
+constexpr int SOFT_CHUNK = 16384;          // K values the workspace is sized for
+
+// Nodes per workgroup (22 and 2 K values of the 23 nodes that can be open),
+// and the number of K values up to which the open integrals are spread over
+// lanes by node. A workgroup takes one K as long as 1024 of them fill the
+// chip. Measured on MI355X (us, spread / not): 176 K 9.4 / 20, 1236 12 / 19,
+// 2000 17 / 19, 4000 26 / 23, 16,384 82 / 48, 65,536 312 / 119.
+constexpr int SOFT_TILE = 512, SOFT_SPLIT_TILE = 64;
+constexpr int64_t SOFT_SPLIT_MAX = 2048;
 
 // Host-evaluated per-element values (bit-identical to the reference's).
 struct CoulombElement {
@@ -342,11 +350,14 @@ __device__ __forceinline__ double photo_ratio(double K, double q, double mass, c
 
 // ---- kernels ----
 
-#define NOA_FM_PROLOGUE()                                                                     \
+// The log/exp tables in LDS as `tab`, visible after the next barrier.
+#define NOA_FM_TABLES()                                                                          \
     __shared__ __attribute__((aligned(fm::TABLE_LDS_ALIGN))) double fm_block[fm::TABLE_DOUBLES]; \
-    load_fm_tables(fm_block);                                                                 \
-    __syncthreads();                                                                          \
+    load_fm_tables(fm_block);                                                                    \
     const fm::Tab tab = fm::tab_from_block(fm_block)
+#define NOA_FM_PROLOGUE() \
+    NOA_FM_TABLES();      \
+    __syncthreads()
 
 #define NOA_GRID_LOOP(i, n) \
     for (int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x; i < (n); i += int64_t(gridDim.x) * blockDim.x)
@@ -397,40 +408,136 @@ __global__ __launch_bounds__(256) void hard_scattering_kernel(Mixture m, double 
 struct SoftNodes {
     double nu[SOFT_NODES];  // X_FRACTION exp(t_j), host libm
     double h;               // subinterval width in t
+    int32_t first;          // the nodes before this one have nu below the photonuclear model's 2e-3
 };
-
-// Node j of K index i at j * nK + i (node-major: the per-K pass reads it
-// coalesced).
-__global__ __launch_bounds__(256) void soft_nodes_kernel(const double* __restrict__ K, int64_t nK, SoftNodes sn,
-                                                         double* __restrict__ Kn, double* __restrict__ qn) {
-    NOA_GRID_LOOP(idx, nK * SOFT_NODES) {
-        const int j = int(idx / nK);
-        const int64_t i = idx - int64_t(j) * nK;
-        const double k = K[i];
-        Kn[idx] = k;
-        qn[idx] = sn.nu[j] * k;
-    }
-}
 
 // numerics.hh:91-108 weights.
 static __constant__ double SOFT_W[6] = {0.08566225, 0.18038079, 0.23395697, 0.23395697, 0.18038079, 0.08566225};
 
-__global__ __launch_bounds__(256) void soft_reduce_kernel(const double* __restrict__ K, int64_t nK, SoftNodes sn,
-                                                          const double* __restrict__ photo, CoulombElement c,
-                                                          double* __restrict__ out) {
-    NOA_FM_PROLOGUE();
-    NOA_GRID_LOOP(i, nK) {
+// Node j's term of the integral, given its photonuclear DCS.
+__device__ __forceinline__ double soft_term(double k, double nu, double dcs, int j, double h, double mass,
+                                            const fm::Tab& t) {
 #pragma clang fp contract(off)
-        const double k = K[i];
-        double acc = 0.;
-        for (int j = 0; j < SOFT_NODES; j++) {
-            const double nu = sn.nu[j];
-            const double q = nu * k;
-            const double ratio = photo_ratio(k, q, c.mass, tab);
-            const double f = photo[int64_t(j) * nK + i] * ratio * nu;
-            acc += f * sn.h * SOFT_W[j % 6];
+    return dcs * photo_ratio(k, nu * k, mass, t) * nu * h * SOFT_W[j % 6];
+}
+
+// A workgroup's nodes in LDS, by item: node first + j of K slot k at k nb + j.
+template <int TILE, bool SPLIT>
+struct SoftLds {
+    double nu[SOFT_NODES];
+    double K[TILE];
+    double term[TILE];
+    uint16_t list[TILE];
+    uint32_t n_open;
+    // (SPLIT) the open integrals' shared values and node terms, by list entry
+    double x9[9];
+    F64::PhotoPre pre[SPLIT ? TILE : 1];
+    double f[SPLIT ? 9 * TILE : 1];
+};
+
+__device__ double soft_all_nodes(double k, const SoftNodes& sn, double mass, const DcsConsts& c, const fm::Tab& t) {
+#pragma clang fp contract(off)
+    double acc = 0.;
+#pragma unroll 1
+    for (int j = 0; j < SOFT_NODES; j++) {
+        const double q = sn.nu[j] * k;
+        acc += soft_term(k, sn.nu[j], F64::photo_active(k, q, c) ? F64::photo(k, q, c, t) : 0., j, sn.h, mass, t);
+    }
+    return acc;
+}
+
+// One workgroup per `group` K values.
+//
+// The photonuclear DCS is zero below nu = 2e-3 (and q = 1 GeV), so of an
+// ordinary K's 102 nodes only the last SOFT_NODES - first (23) can count and
+// the others' transport ratios need not be formed; those of K above ~500 GeV
+// all do. K outside [1e-20, 1e30] GeV and NaN, where a ratio might overflow
+// and carry its NaN into the sum, take all nodes in the reference's order
+// (soft_all_nodes).
+//
+// Bound: FP64 VALU issue, ~4500 instructions per open node. Open nodes are
+// compacted in LDS and drained by whole waves; SPLIT spreads each over 9
+// lanes by quadrature node, for calls with too few K values to fill the chip.
+// Measured for 65,536 K: 119 us, against 733 us when the 102 nodes of each K
+// went through memory as (K, q) pairs of a map and one thread per K formed
+// their 102 ratios (64 workgroups per pass of 16,384 K); 9.4 us for 176 K.
+template <int TILE, bool SPLIT>
+__global__ __launch_bounds__(WG) __attribute__((amdgpu_waves_per_eu(SPLIT ? 3 : 4))) void soft_kernel(
+    const double* __restrict__ K, int64_t n, DcsConsts, CoulombElement ce, SoftNodes sn, int32_t group,
+    double* __restrict__ out) {
+    __shared__ SoftLds<TILE, SPLIT> s;
+    NOA_FM_TABLES();
+    const ConstsPtr cp = vector_kernarg_consts();
+    const int tid = threadIdx.x;
+    const int64_t k0 = int64_t(blockIdx.x) * group;
+    const int nk = int(n - k0 < group ? n - k0 : group);
+    const int first = sn.first, nb = SOFT_NODES - first;
+    for (int j = tid; j < SOFT_NODES; j += WG) s.nu[j] = sn.nu[j];
+    for (int kk = tid; kk < nk; kk += WG) s.K[kk] = K[k0 + kk];
+    if (SPLIT && tid < 9) s.x9[tid] = GL9_X[tid];
+    if (tid == 0) s.n_open = 0;
+    __syncthreads();
+#pragma unroll 1
+    for (int i0 = 0; i0 < nk * nb; i0 += WG) {
+        const DcsConsts& c = item_consts(cp);
+        const int i = i0 + tid;
+        bool open = false;
+        if (i < nk * nb) {
+            const int kk = i / nb;
+            const double k = s.K[kk];
+            open = F64::photo_active(k, s.nu[first + (i - kk * nb)] * k, c);
+            s.term[i] = 0.;
         }
-        out[i] = transverse_ionisation(k, c, tab) + 2. * acc;
+        wave_append(open, &s.n_open, s.list, uint32_t(i));
+    }
+    __syncthreads();
+    const uint32_t n_open = s.n_open;
+    if constexpr (SPLIT) {
+        for (uint32_t e = tid; e < n_open; e += WG) {
+            const DcsConsts& c = item_consts(cp);
+            const uint32_t i = s.list[e], kk = i / uint32_t(nb), j = first + (i - kk * nb);
+            const double k = s.K[kk];
+            s.pre[e] = F64::photo_setup<false, true>(k, s.nu[j] * k, c, tab);
+        }
+        __syncthreads();
+        for (uint32_t v = tid; v < 9 * n_open; v += WG) {
+            const DcsConsts& c = item_consts(cp);
+            const uint32_t e = v / 9;
+            const F64::PhotoPre p = s.pre[e];
+            s.f[v] = F64::photo_node<false, true>(p, s.x9[v - 9 * e], c, tab);
+        }
+        __syncthreads();
+    }
+#pragma unroll 1
+    for (uint32_t e = tid; e < n_open; e += WG) {
+        const DcsConsts& c = item_consts(cp);
+        const uint32_t i = s.list[e], kk = i / uint32_t(nb), j = first + (i - kk * nb);
+        const double k = s.K[kk], nu = s.nu[j];
+        double d;
+        if (!SPLIT || !(c.fast_ok && k + c.mass <= F64::FAST_E_MAX)) {
+            d = F64::photo(k, nu * k, c, tab);
+        } else {
+            d = 0.;
+            for (int m = 0; m < 9; m++) d = F64::photo_add<false>(s.f[9 * e + m], GL9_W[m], d);
+            d = F64::photo_finish<false, true>(k, s.pre[e], d, c);
+        }
+        s.term[i] = soft_term(k, nu, d, int(j), sn.h, ce.mass, tab);
+    }
+    __syncthreads();
+    // 8 lanes per K: strided sums, then a fixed-order tree
+    for (int v = tid; v < nk * 8; v += WG) {
+        const int kk = v >> 3;
+        double acc = 0.;
+        for (int j = v & 7; j < nb; j += 8) acc += s.term[kk * nb + j];
+        acc += __shfl_xor(acc, 4, 8);
+        acc += __shfl_xor(acc, 2, 8);
+        acc += __shfl_xor(acc, 1, 8);
+        if ((v & 7) == 0) {
+            const DcsConsts& c = item_consts(cp);
+            const double k = s.K[kk];
+            if (!(k >= 1e-20 && k <= 1e30)) acc = soft_all_nodes(k, sn, ce.mass, c, tab);
+            out[k0 + kk] = transverse_ionisation(k, ce, tab) + 2. * acc;
+        }
     }
 }
 
@@ -505,21 +612,21 @@ int noa_dcs_soft_scattering_f64(const double* K, int64_t n, const noa_dcs_elemen
     const double x6[6] = {0.03376524, 0.16939531, 0.38069041, 0.61930959, 0.83060469, 0.96623476};
     for (int j = 0; j < SOFT_NODES; j++)
         sn.nu[j] = X_FRACTION * std::exp(lb + sn.h * (double(uint32_t(j / 6)) + x6[j % 6]));
-    const CoulombElement c = make_coulomb_element(element->A, element->I, element->Z, mass);
-    const int64_t cap = std::min<int64_t>(n, SOFT_CHUNK);
-    double* Kn = static_cast<double*>(workspace);
-    double* qn = Kn + cap * SOFT_NODES;
-    double* ph = qn + cap * SOFT_NODES;
-    for (int64_t k0 = 0; k0 < n; k0 += SOFT_CHUNK) {
-        const int64_t nK = std::min<int64_t>(SOFT_CHUNK, n - k0);
-        const int64_t nn = nK * SOFT_NODES;
-        hipLaunchKernelGGL(soft_nodes_kernel, dim3(grid_for(nn)), dim3(256), 0, stream, K + k0, nK, sn, Kn, qn);
-        if (int rc = check_hip(hipGetLastError(), "soft_nodes_kernel")) return rc;
-        const noa_dcs_outputs_f64 po{nullptr, nullptr, ph, nullptr};
-        if (int rc = noa_dcs_eval_f64(Kn, qn, nn, element, mass, &po, stream)) return rc;
-        hipLaunchKernelGGL(soft_reduce_kernel, dim3(grid_for(nK)), dim3(256), 0, stream, K + k0, nK, sn, ph, c,
-                           result + k0);
-        if (int rc = check_hip(hipGetLastError(), "soft_reduce_kernel")) return rc;
+    sn.first = 0;
+    while (sn.first < SOFT_NODES && sn.nu[sn.first] < 2E-03 * (1. - 1E-09)) sn.first++;
+    const CoulombElement ce = make_coulomb_element(element->A, element->I, element->Z, mass);
+    const DcsConsts c = make_consts(element->A, element->I, element->Z, mass);
+    const int nb = SOFT_NODES - sn.first;
+    constexpr int64_t most = int64_t(1) << 30;
+    for (int64_t k0 = 0; k0 < n; k0 += most) {
+        const int64_t nK = std::min<int64_t>(most, n - k0);
+        const bool split = nK <= SOFT_SPLIT_MAX;
+        const int32_t group = int32_t(
+            std::max<int64_t>(1, std::min<int64_t>((split ? SOFT_SPLIT_TILE : SOFT_TILE) / nb, (nK + 1023) / 1024)));
+        const auto kernel = split ? &soft_kernel<SOFT_SPLIT_TILE, true> : &soft_kernel<SOFT_TILE, false>;
+        hipLaunchKernelGGL(kernel, dim3(unsigned((nK + group - 1) / group)), dim3(WG), 0, stream, K + k0, nK, c, ce, sn,
+                           group, result + k0);
+        if (int rc = check_hip(hipGetLastError(), "soft_kernel")) return rc;
     }
     return ok();
 }

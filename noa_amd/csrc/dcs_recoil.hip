@@ -15,7 +15,6 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
-#include <cstddef>
 #include <cstdint>
 #include <type_traits>
 
@@ -81,13 +80,6 @@ struct RecoilLds {
     uint32_t n_photo, n_pair;
 };
 
-// The leading arguments of recoil_kernel, as TileKernelArgs lays out a map's.
-struct RecoilKernelArgs {
-    const double* K;
-    int64_t n;
-    DcsConsts c;
-};
-
 // Sum over the wave's lanes, in a fixed order, valid in lane 0.
 __device__ __forceinline__ double wave_sum(double v) {
 #pragma unroll
@@ -120,8 +112,7 @@ __global__ __launch_bounds__(WG) __attribute__((amdgpu_waves_per_eu(4))) void re
     Outs<double> cel) {
     __shared__ RecoilLds<TILE> s;
     __shared__ __attribute__((aligned(fm::TABLE_LDS_ALIGN))) double fm_block[fm::TABLE_DOUBLES];
-    using KArg = const __attribute__((address_space(4))) char*;
-    const ConstsPtr cp = (ConstsPtr)((KArg)__builtin_amdgcn_kernarg_segment_ptr() + offsetof(RecoilKernelArgs, c));
+    const ConstsPtr cp = vector_kernarg_consts();
     const int tid = threadIdx.x;
     const int lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -241,8 +232,7 @@ __global__ __launch_bounds__(WG) __attribute__((amdgpu_waves_per_eu(4))) void re
 static_assert(std::is_same<decltype(&recoil_kernel<RECOIL_TILE, false>),
                            void (*)(const double*, int64_t, DcsConsts, RecoilGrid, int32_t, Outs<double>,
                                     Outs<double>)>::value,
-              "recoil_kernel's parameters must begin as RecoilKernelArgs lays them out");
-static_assert(offsetof(RecoilKernelArgs, c) == 16, "two 8-byte arguments before the constants");
+              "recoil_kernel's parameters must begin as VectorKernelArgs lays them out");
 
 }  // namespace noa_hip
 

@@ -126,6 +126,20 @@ __device__ __forceinline__ ConstsPtr kernarg_consts() {
     return (ConstsPtr)((KArg)__builtin_amdgcn_kernarg_segment_ptr() + offsetof(TileKernelArgs, c));
 }
 
+// The same for a kernel that takes (K, n, DcsConsts c, ...): a vector of
+// kinetic energies.
+struct VectorKernelArgs {
+    const double* K;
+    int64_t n;
+    DcsConsts c;
+};
+static_assert(offsetof(VectorKernelArgs, c) == 16, "two 8-byte arguments before the constants");
+
+__device__ __forceinline__ ConstsPtr vector_kernarg_consts() {
+    using KArg = const __attribute__((address_space(4))) char*;
+    return (ConstsPtr)((KArg)__builtin_amdgcn_kernarg_segment_ptr() + offsetof(VectorKernelArgs, c));
+}
+
 // Copies the log/exp tables into an LDS block (visible after the next barrier).
 __device__ __forceinline__ void load_fm_tables(double* block) {
     for (int k = threadIdx.x; k < fm::TABLE_DOUBLES; k += WG) block[k] = fm::table_entry(k);
