@@ -412,6 +412,50 @@ __device__ double photo_drss(const ElementConsts& c, const Globals& G, double ml
     return (ds < 0.) ? 0. : ds;
 }
 
+// Node `node` of pair_ssr's rule, with skip set where pair_ssr returns 0.
+__device__ __forceinline__ void pair_term(const ElementConsts& c, const Globals& G, double mass, double K, double q,
+                                          int node, double* term, int* skip) {
+#pragma clang fp contract(off)
+    if ((c.Z <= 0) || (c.A <= 0) || (mass <= 0) || (K <= 0) || (q <= 0)) return;
+    if (q <= 4. * ELECTRON_MASS) return;
+    if (q >= K + c.p_qoff) return;
+    const double gamma = 1. + K / mass;
+    const double x0 = 1. - 4. * ELECTRON_MASS / q;
+    const double x1 = 1. - 6. / (gamma * (gamma - q / mass));
+    if (!((x0 > 0) && (x1 > 0))) return;
+    const double rmax = sqrt(x0) * x1;
+    const double ri = 1. - rmax;
+    if ((ri <= 0.) || (ri >= 1.)) return;
+    const double tmin = log(ri);
+    const PairQ s = pair_setup(c, mass, K, q);
+    const double rho = exp(GQ12_X[node] * tmin);
+    *term = pair_d2_ssr(s, G, rho) * rho * GQ12_W[node] * tmin;
+    *skip = 0;
+}
+
+// Node `node` of photo_drss's rule inside dcs()'s range, with skip set where
+// the DCS is 0 or the node is left out of the sum.
+__device__ __forceinline__ void photo_term(const ElementConsts& c, const Globals& G, double ml, double K, double q,
+                                           int node, double* term, int* skip) {
+#pragma clang fp contract(off)
+    const double M = NUCLEON_MASS;
+    const double mpi = PION_MASS;
+    if ((q < mpi + 0.5 * mpi * mpi / M) || (q > K + ml - 0.5 * (M + ml * ml / M))) return;
+    if ((c.Z <= 0) || (c.A <= 0) || (ml <= 0) || (K <= 0)) return;
+    if ((q <= mpi + 0.5 * mpi * mpi / M) || (q >= K + ml - 0.5 * (M + ml * ml / M))) return;
+    const double E = K + ml;
+    const double ml2 = ml * ml;
+    const double Q2min = ml2 * (q * q - 0.5 * ml2) / (E * (E - q));
+    const double Q2max = 2.0 * M * (q - mpi) - mpi * mpi;
+    if ((Q2max < Q2min) | (Q2min < 0)) return;
+    const double lmin = log(Q2min);
+    const double dx = log(Q2max) - lmin;
+    const double Q2 = exp(lmin + dx * GQ9_X[node]);
+    const double tmp = photo_d2_drss(c, G, ml, K, q, Q2);
+    *skip = tmp <= 0.;
+    *term = tmp * (GQ9_W[node] * (dx * Q2));
+}
+
 // The m^2/kg DCS of process 0 (bremsstrahlung), 1 (pair production) or 2
 // (photonuclear) as dcs_get(process) returns it (pumas.c:11018-11112).
 __device__ double dcs(int process, const ElementConsts& c, const Globals& G, double mass, double K, double q) {
@@ -605,85 +649,86 @@ __global__ __launch_bounds__(64) void pumas_alpha_fill_kernel(float* __restrict_
     for (int row = 0; row < n0; row++) a[2 * row] = alpha;
 }
 
-// The m^2/kg model DCS for a whole wave that evaluates one (K, q): every lane
-// computes the same set-up, the quadrature nodes are spread over the lanes
-// (12 for pair production, 9 for photonuclear), and every lane then sums the
-// gathered node terms in the serial loop's order, so the value is that of
-// dcs() bit for bit. Must be called with the wave's 64 lanes active and the
-// same arguments in every lane.
-__device__ double dcs_wave(int process, const ElementConsts& c, const Globals& G, double mass, double K, double q) {
+// The quadrature nodes of up to this many model evaluations fill one wave:
+// 5 x 12 (pair production), 7 x 9 (photonuclear); bremsstrahlung has no nodes.
+__device__ __forceinline__ int model_batch(int process) { return process == 0 ? 64 : process == 1 ? 5 : 7; }
+
+// The m^2/kg model DCS of one (K, q) per lane, for the lanes with need set (K
+// the same in every lane; the other lanes get 0). A wave takes model_batch
+// evaluations at a time, a group of lanes each: every lane of a group forms
+// the set-up and one quadrature node, and the node terms are summed in the
+// serial loop's order, so the values are those of dcs() bit for bit. Must be
+// called with the wave's 64 lanes active.
+__device__ __attribute__((noinline)) double dcs_wave(int process, const ElementConsts& c, const Globals& G, double mass, double K, double q,
+                           bool need) {
 #pragma clang fp contract(off)
     const int lane = threadIdx.x & 63;
-    double d;
+    double d = 0.;
     if (process == 0) {
-        d = brems_ssr(c, G, mass, K, q);
-    } else if (process == 1) {
-        if ((c.Z <= 0) || (c.A <= 0) || (mass <= 0) || (K <= 0) || (q <= 0)) return 0.;
-        if (q <= 4. * ELECTRON_MASS) return 0.;
-        if (q >= K + c.p_qoff) return 0.;
-        const double gamma = 1. + K / mass;
-        const double x0 = 1. - 4. * ELECTRON_MASS / q;
-        const double x1 = 1. - 6. / (gamma * (gamma - q / mass));
-        if (!((x0 > 0) && (x1 > 0))) return 0.;
-        const double rmax = sqrt(x0) * x1;
-        const double ri = 1. - rmax;
-        if ((ri <= 0.) || (ri >= 1.)) return 0.;
-        const double tmin = log(ri);
-        const PairQ s = pair_setup(c, mass, K, q);
-        double term = 0.;
-        if (lane < 12) {
-            const double rho = exp(GQ12_X[lane] * tmin);
-            term = pair_d2_ssr(s, G, rho) * rho * GQ12_W[lane] * tmin;
-        }
-        double I = 0.;
-        for (int i = 0; i < 12; i++) I -= __shfl(term, i, 64);
-        d = (I < 0) ? 0. : I;
+        if (need) d = brems_ssr(c, G, mass, K, q);
     } else {
-        const double M = NUCLEON_MASS;
-        const double mpi = PION_MASS;
-        const double ml = mass;
-        if ((q < mpi + 0.5 * mpi * mpi / M) || (q > K + ml - 0.5 * (M + ml * ml / M))) return 0.;
-        if ((c.Z <= 0) || (c.A <= 0) || (ml <= 0) || (K <= 0)) return 0.;
-        if ((q <= mpi + 0.5 * mpi * mpi / M) || (q >= K + ml - 0.5 * (M + ml * ml / M))) return 0.;
-        const double E = K + ml;
-        const double ml2 = ml * ml;
-        const double Q2min = ml2 * (q * q - 0.5 * ml2) / (E * (E - q));
-        const double Q2max = 2.0 * M * (q - mpi) - mpi * mpi;
-        if ((Q2max < Q2min) | (Q2min < 0)) return 0.;
-        const double lmin = log(Q2min);
-        const double dx = log(Q2max) - lmin;
-        double term = 0.;
-        int skip = 1;
-        if (lane < 9) {
-            const double Q2 = exp(lmin + dx * GQ9_X[lane]);
-            const double tmp = photo_d2_drss(c, G, ml, K, q, Q2);
-            skip = tmp <= 0.;
-            term = tmp * (GQ9_W[lane] * (dx * Q2));
+        const int nodes = process == 1 ? 12 : 9;
+        const int per = model_batch(process);
+        const int group = lane / nodes, node = lane - group * nodes;
+        unsigned long long todo = __ballot(need);
+        while (todo) {
+            // the group's evaluation is the group-th lane still to do
+            unsigned long long m = todo;
+            int mine = -1, owner_group = -1;
+            for (int i = 0; i < per && m; i++) {
+                const int l = __ffsll((long long)m) - 1;
+                m &= m - 1;
+                if (i == group) mine = l;
+                if (l == lane) owner_group = i;
+            }
+            todo = m;
+            const double qg = __shfl(q, mine < 0 ? 0 : mine, 64);
+            double term = 0.;
+            int skip = 1;
+            if (mine >= 0) {
+                if (process == 1)
+                    pair_term(c, G, mass, K, qg, node, &term, &skip);
+                else
+                    photo_term(c, G, mass, K, qg, node, &term, &skip);
+            }
+            const int first = (owner_group < 0 ? 0 : owner_group) * nodes;
+            double sum = 0.;
+            for (int i = 0; i < nodes; i++) {
+                const double t = __shfl(term, first + i, 64);
+                if (!__shfl(skip, first + i, 64)) sum = process == 1 ? sum - t : sum + t;
+            }
+            if (owner_group >= 0) d = (sum < 0) ? 0. : sum;
         }
-        double ds = 0.;
-        for (int i = 0; i < 9; i++) {
-            const double t = __shfl(term, i, 64);
-            if (!__shfl(skip, i, 64)) ds += t;
-        }
-        d = (ds < 0.) ? 0. : ds;
     }
-    return d * 1E+03 * AVOGADRO_NUMBER * (mass + K) / c.A;
+    return need ? d * 1E+03 * AVOGADRO_NUMBER * (mass + K) / c.A : 0.;
 }
 
 // ---- the envelope maximum (dcs_tabulate_envelope_row, pumas.c:11526-11679) ----
 //
-// One wave per row: the reference's serial search (bisections that find where the DCS
-// becomes positive at the range ends, then two bracketing bisections,
-// math_find_minimum with algo 0, pumas.c:12172-12232 and 12416-12459, and for
-// pair production at K >= 1e7 a logarithmic scan next to the upper end) of
-// the maximum of DCS x^alpha over ln x, where DCS is the table interpolated as
-// dcs_evaluate does without a context (pumas.c:11307-11398) and the model
-// where the table does not apply. The rows read are those of the finished
-// table. The search's control flow is the same in every lane of the wave
-// (same row, same values), and the model evaluations spread their quadrature
-// nodes over the lanes (dcs_wave), so rows do not diverge against each other. The reference's search reads the nodes from physics->table_DCS_x,
-// which compute_dcs_table writes only after element 0 (pumas.c:11775-11783),
-// so element 0's search sees zero nodes and takes the model everywhere; the
+// One wave per row. The reference searches the maximum of DCS x^alpha over ln x
+// serially, 100 to 240 evaluations of one point each: bisections that find
+// where the DCS becomes positive at the range ends, then two bracketing
+// bisections (math_find_minimum with algo 0, pumas.c:12172-12232 and
+// 12416-12459), and for pair production at K >= 1e7 a logarithmic scan next to
+// the upper end. DCS is the table interpolated as dcs_evaluate does without a
+// context (pumas.c:11307-11398) and the model where the table does not apply.
+// The rows read are those of the finished table.
+//
+// Every step of those searches has two outcomes and the next point depends
+// only on the outcomes so far, so the wave evaluates the points of the next d
+// steps at once, all 2^d - 1 of their decision tree, one per lane, and then
+// walks the tree: the same points, values and decisions as the serial search.
+// d is 6 where the table serves the tree, less where points need the model: as
+// many levels as their model evaluations fit one batch of dcs_wave (5 of pair
+// production, 7 of photonuclear).
+//
+// Where the range end is the logarithm of a negative number (K below the
+// kinematic threshold) the reference's search makes 200 evaluations at NaN;
+// they all have the first one's value, so two evaluations settle the row.
+//
+// The reference's search reads the nodes from physics->table_DCS_x, which
+// compute_dcs_table writes only after element 0 (pumas.c:11775-11783), so
+// element 0's search sees zero nodes and takes the model everywhere; the
 // kernel does the same.
 
 struct EnvRow {
@@ -730,11 +775,13 @@ __device__ __forceinline__ int table_index(const double* table, int n_K, double 
     return i1;
 }
 
-__device__ double dcs_interpolated(const EnvRow& a, double K, double q) {
+// The interpolated DCS at q without its factor K / (K + m), or *need set where
+// it is the model's.
+__device__ double dcs_from_table(const EnvRow& a, double K, double q, bool* need) {
 #pragma clang fp contract(off)
-    const double wj = K / (K + a.mass);
     const ElementConsts& c = *a.c;
     double qlow = 0., qmin, qmax;
+    *need = false;
     if (a.process == 2) {
         qmin = PION_MASS + 0.5 * PION_MASS * PION_MASS / NUCLEON_MASS;
         qmax = K + a.mass - 0.5 * (NUCLEON_MASS + a.mass * a.mass / NUCLEON_MASS);
@@ -749,21 +796,23 @@ __device__ double dcs_interpolated(const EnvRow& a, double K, double q) {
             qmin = 0.;
         if ((q < qmin) || (q > qmax)) return 0.;
     }
-    if (q < qlow) return dcs_wave(a.process, c, *a.G, a.mass, K, q) * wj;
+    *need = true;
+    if (q < qlow) return 0.;
     const int nx = a.n;
     const float xmin = a.xt[0], xmax = a.xt[nx - 1];
     const float x = logf((float)(q / K));
-    if ((x < xmin) || (x >= xmax)) return dcs_wave(a.process, c, *a.G, a.mass, K, q) * wj;
+    if ((x < xmin) || (x >= xmax)) return 0.;
     int ix = 0, tmpi = nx - 1;
     bracketf(a.xt, x, &ix, &tmpi);
-    if ((ix < 0) || (ix >= nx - 1)) return dcs_wave(a.process, c, *a.G, a.mass, K, q) * wj;
-    if (a.below) return dcs_wave(a.process, c, *a.G, a.mass, K, q) * wj;
+    if ((ix < 0) || (ix >= nx - 1)) return 0.;
+    if (a.below) return 0.;
     float p00 = a.ra[2 * ix], m00 = a.ra[2 * ix + 1], p01 = a.ra[2 * ix + 2], m01 = a.ra[2 * ix + 3];
     float p10 = a.rb[2 * ix], m10 = a.rb[2 * ix + 1], p11 = a.rb[2 * ix + 2], m11 = a.rb[2 * ix + 3];
     const float h0 = a.h0, h1 = a.h1;
     if (((p00 == 0.f) && (m00 == 0.f)) || ((p01 == 0.f) && (m01 == 0.f)) || ((p10 == 0.f) && (m10 == 0.f)) ||
         ((p11 == 0.f) && (m11 == 0.f)))
-        return dcs_wave(a.process, c, *a.G, a.mass, K, q) * wj;
+        return 0.;
+    *need = false;
     const float x0 = a.xt[ix];
     const float x1 = a.xt[ix + 1];
     const float dx = x1 - x0;
@@ -780,96 +829,182 @@ __device__ double dcs_interpolated(const EnvRow& a, double K, double q) {
         const float c13 = 2 * (p10 - p11) + m10 + m11;
         r += expf(p10 + t * (m10 + t * (c12 + t * c13))) * h1;
     }
-    return r * wj;
+    return r;
 }
 
+constexpr int TREE_DEPTH = 6;  // 2^6 - 1 points, one per lane
+
+// -DCS x^alpha at one ln x per lane. `levels`: in, the levels of the decision
+// tree that the lanes hold (lane i its node i in breadth-first order); out, the
+// levels evaluated. levels = -n: the first n lanes are independent points.
 struct EnvObjective {
     const EnvRow& a;
     double K, alpha;
-    __device__ double operator()(double lnx) const {
+    __device__ double operator()(double lnx, int* levels) const {
 #pragma clang fp contract(off)
+        const int lane = threadIdx.x & 63;
+        const double wj = K / (K + a.mass);
         const double x = exp(lnx);
         const double q = x * K;
-        return -dcs_interpolated(a, K, q) * pow(x, alpha);
+        bool need;
+        double d = dcs_from_table(a, K, q, &need);
+        if (*levels > 0) {
+            // as many levels as one batch of model evaluations covers
+            const unsigned long long m = __ballot(need);
+            int l = *levels;
+            while (l > 1 && __popcll(m & ((1ull << ((1 << l) - 1)) - 1)) > model_batch(a.process)) l--;
+            *levels = l;
+            need = need && lane < (1 << l) - 1;
+        } else {
+            need = need && lane < -*levels;
+        }
+        if (__ballot(need)) {
+            const double md = dcs_wave(a.process, *a.c, *a.G, a.mass, K, q, need);
+            if (need) d = md;
+        }
+        return -(d * wj) * pow(x, alpha);
+    }
+    // the same at one point for the whole wave
+    __device__ double at(double lnx) const {
+        int one = -1;
+        return __shfl((*this)(lnx, &one), 0, 64);
     }
 };
 
-template <class F>
-__device__ int find_minimum_bisection(const F& f, double xa, double xb, double xc, const double* fb_p, double tol,
-                                      int max_iter, double* fopt) {
-#pragma clang fp contract(off)
-    double fb = fb_p ? *fb_p : f(xb);
-    tol *= fabs(xc - xa);
-    int i = 0;
-    while ((xc - xa > tol) && (i < max_iter)) {
+// Runs a search of two-outcome steps from state s until s.done(): s.point() is
+// the next point, s.next(bit) the state after the outcome `bit`, and
+// s.step(v) the true step with the value v there, which returns its outcome,
+// or -1 to stop.
+template <class F, class S>
+__device__ void search(const F& f, S& s) {
+    const int lane = threadIdx.x & 63;
+    while (!s.done()) {
+        // this lane's node: the bits of lane + 1 below its leading one, from the top, are its path
+        S mine = s;
+        const int depth = 31 - __clz(lane + 1);
+        for (int i = depth - 1; i >= 0; i--) mine.next((lane + 1) >> i & 1);
+        int levels = TREE_DEPTH;
+        const double v = f(mine.point(), &levels);
+        int node = 0;
+        for (int l = 0; l < levels && !s.done(); l++) {
+            const int bit = s.step(__shfl(v, node, 64));
+            if (bit < 0) return;
+            node = 2 * node + 1 + bit;
+        }
+    }
+}
+
+// Bisection for the edge of the region where f != 0 between x0 and x1; the
+// nonzero side is x1 (up) or x0.
+struct EdgeSearch {
+    static constexpr double RESOLUTION = 1E-10;
+    double x0, x1, edge, value;
+    bool up;
+    __device__ bool done() const { return !(x1 - x0 > RESOLUTION); }
+    __device__ double point() const { return 0.5 * (x0 + x1); }
+    __device__ void next(int nonzero) {
+        const double x2 = 0.5 * (x0 + x1);
+        if (bool(nonzero) == up)
+            x1 = x2;
+        else
+            x0 = x2;
+    }
+    __device__ int step(double f2) {
+        const int nonzero = f2 != 0;
+        if (nonzero) {
+            edge = point();
+            value = f2;
+        }
+        next(nonzero);
+        return nonzero;
+    }
+};
+
+// find_minimum's bisection around xb (pumas.c:12416-12459).
+struct MinimumBisection {
+    double xa, xb, xc, fb, tol;
+    int i, max_iter;
+    __device__ bool done() const { return !((xc - xa > tol) && (i < max_iter)); }
+    __device__ double point() const { return (xb - xa > xc - xb) ? 0.5 * (xa + xb) : 0.5 * (xb + xc); }
+    __device__ void next(int lower) {
+        const double x = point();
         if (xb - xa > xc - xb) {
-            const double x = 0.5 * (xa + xb);
-            const double fi = f(x);
-            if (fi < fb) {
+            if (lower) {
                 xc = xb;
                 xb = x;
-                fb = fi;
             } else {
                 xa = x;
             }
         } else {
-            const double x = 0.5 * (xb + xc);
-            const double fi = f(x);
-            if (fi < fb) {
+            if (lower) {
                 xa = xb;
                 xb = x;
-                fb = fi;
             } else {
                 xc = x;
             }
         }
         i++;
     }
-    *fopt = fb;
-    return (i <= max_iter) ? i : -1;
-}
+    __device__ int step(double fi) {
+        const int lower = fi < fb;
+        if (lower) fb = fi;
+        next(lower);
+        return lower;
+    }
+};
 
-template <class F>
-__device__ int find_minimum(const F& f, double xa, double xc, const double* fa_p, const double* fc_p, double tol,
-                            int max_iter, double* fopt) {
-#pragma clang fp contract(off)
-    double fa = fa_p ? *fa_p : f(xa);
-    double fc = fc_p ? *fc_p : f(xc);
-    const double atol = tol * fabs(xc - xa);
-    double xb = 0, fb = 0;
-    int i;
-    for (i = 0; i < max_iter; i++) {
-        xb = 0.5 * (xa + xc);
-        fb = f(xb);
-        if ((fb < fa) && (fb < fc)) break;
-        if (fabs(xc - xa) <= atol) {
-            *fopt = fb;
-            return i;
+// find_minimum's first stage: halves [xa, xc] towards the lower end until the
+// midpoint lies below both ends (found), or the interval is spent (flat).
+struct MinimumBracket {
+    double xa, xb, xc, fa, fb, fc, atol;
+    int i, max_iter;
+    bool found, flat;
+    __device__ bool done() const { return found || flat || i >= max_iter; }
+    __device__ double point() const { return 0.5 * (xa + xc); }
+    __device__ void next(int right) {
+        if (right)
+            xa = point();
+        else
+            xc = point();
+    }
+    __device__ int step(double f) {
+        xb = point();
+        fb = f;
+        if ((fb < fa) && (fb < fc)) {
+            found = true;
+            return -1;
         }
+        if (fabs(xc - xa) <= atol) {
+            flat = true;
+            return -1;
+        }
+        i++;
         if (fb < fc) {
             xc = xb;
             fc = fb;
-        } else {
-            xa = xb;
-            fa = fb;
+            return 0;
         }
+        xa = xb;
+        fa = fb;
+        return 1;
     }
-    if (i == max_iter) {
-        if (fa < fb) {
-            fb = fa;
-        } else if (fc < fb) {
-            fb = fc;
-        }
-        *fopt = fb;
-        return -1;
-    }
-    const int status = find_minimum_bisection(f, xa, xb, xc, &fb, tol, max_iter - i, fopt);
-    return (status < 0) ? -2 : status + i;
+};
+
+template <class F>
+__device__ double find_minimum(const F& f, double xa, double xc, double fa, double fc, double tol, int max_iter) {
+    MinimumBracket b{xa, 0., xc, fa, 0., fc, tol * fabs(xc - xa), 0, max_iter, false, false};
+    search(f, b);
+    if (b.flat) return b.fb;
+    if (!b.found) return (b.fa < b.fb) ? b.fa : (b.fc < b.fb) ? b.fc : b.fb;
+    MinimumBisection m{b.xa, b.xb, b.xc, b.fb, tol * fabs(b.xc - b.xa), 0, max_iter - b.i};
+    search(f, m);
+    return m.fb;
 }
 
 __device__ float envelope_max(const EnvRow& a, double K, double cutoff, float alpha, double cs) {
 #pragma clang fp contract(off)
-    constexpr double RESOLUTION = 1E-10;
+    constexpr double RESOLUTION = EdgeSearch::RESOLUTION;
+    const int lane = threadIdx.x & 63;
     if (cs <= 0.) return 0.f;
     double qmin, qmax;
     if (a.process == 2) {  // dcs_get_range (pumas.c:11047-11056)
@@ -885,33 +1020,39 @@ __device__ float envelope_max(const EnvRow& a, double K, double cutoff, float al
     double xmax = log(qmax / K);
     if (xmin >= xmax) return 0.f;
     const EnvObjective f{a, K, (double)alpha};
-    double f0 = f(xmin);
-    double f1 = f(xmax);
+    int two = -2;
+    const double ends = f(lane == 0 ? xmin : xmax, &two);
+    double f0 = __shfl(ends, 0, 64);
+    double f1 = __shfl(ends, 1, 64);
+    if (xmax != xmax) {  // every further point is at NaN and has f1's value
+        const double fopt = f0 < f1 ? f0 : f1;
+        return (float)(-fopt);
+    }
     if (f0 == 0.) {
-        double x0 = xmin, x1 = xmax;
-        while (x1 - x0 > RESOLUTION) {
-            const double x2 = 0.5 * (x0 + x1);
-            const double f2 = f(x2);
-            if (f2 != 0) {
-                x1 = xmin = x2;
-                f0 = f2;
-            } else {
-                x0 = x2;
-            }
-        }
+        EdgeSearch s{xmin, xmax, xmin, f0, true};
+        search(f, s);
+        xmin = s.edge;
+        f0 = s.value;
     }
     if (f1 == 0.) {
         double x0, x1;
         if (K >= 1E+01) {
+            // the first of xm - delta, delta = 1e-10 2^i, with f != 0
             const double xm = exp(xmax);
             double delta = RESOLUTION, x = xmax, fx = f1;
-            while (xm > delta) {
-                x = log(xm - delta);
-                fx = f(x);
-                if (fx != 0.)
-                    break;
-                else
-                    delta += delta;
+            bool hit = false;
+            while (xm > delta && !hit) {
+                const int some = model_batch(a.process);
+                const double dl = ldexp(delta, lane < some ? lane : 0);
+                const double xl = log(xm - dl);
+                int points = -some;
+                const double v = f(xl, &points);
+                const unsigned long long in = __ballot(lane < some && xm > dl), nz = __ballot(v != 0.) & in;
+                const int at = nz ? __ffsll((long long)nz) - 1 : 63 - __clzll((long long)in);
+                hit = nz != 0;
+                x = __shfl(xl, at, 64);
+                fx = __shfl(v, at, 64);
+                delta = ldexp(delta, hit ? at : at + 1);
             }
             f1 = fx;
             x0 = xmax = x;
@@ -920,38 +1061,34 @@ __device__ float envelope_max(const EnvRow& a, double K, double cutoff, float al
             x0 = xmin;
             x1 = xmax;
         }
-        while (x1 - x0 > RESOLUTION) {
-            const double x2 = 0.5 * (x0 + x1);
-            const double f2 = f(x2);
-            if (f2 != 0) {
-                x0 = xmax = x2;
-                f1 = f2;
-            } else {
-                x1 = x2;
-            }
-        }
+        EdgeSearch s{x0, x1, xmax, f1, false};
+        search(f, s);
+        xmax = s.edge;
+        f1 = s.value;
     }
     const double xm = 0.5 * (xmin + xmax);
-    const double fm = f(xm);
-    double fopt0 = 0., fopt1 = 0.;
-    find_minimum(f, xmin, xm, &f0, &fm, RESOLUTION, 100, &fopt0);
-    find_minimum(f, xm, xmax, &fm, &f1, RESOLUTION, 100, &fopt1);
+    const double fm = f.at(xm);
+    const double fopt0 = find_minimum(f, xmin, xm, f0, fm, RESOLUTION, 100);
+    double fopt1 = find_minimum(f, xm, xmax, fm, f1, RESOLUTION, 100);
     if ((a.process == 1) && (K >= 1E+07)) {  // a sharp peak next to xmax: a logarithmic scan
         constexpr int N_SCAN = 7;
-        double xs[N_SCAN], fs[N_SCAN], fmin = 0.;
+        const double xl = xmax + log(1. - pow(10., double(-((lane < N_SCAN ? lane : 0) + 1))));
+        int points = -N_SCAN;
+        const double fl = f(xl, &points);
+        double fmin = 0.;
         int imin = -1;
         for (int i = 0; i < N_SCAN; i++) {
-            xs[i] = xmax + log(1. - pow(10., double(-(i + 1))));
-            fs[i] = f(xs[i]);
-            if (fs[i] < fmin) {
+            const double fi = __shfl(fl, i, 64);
+            if (fi < fmin) {
                 imin = i;
-                fmin = fs[i];
+                fmin = fi;
             }
         }
         if ((imin > 0) && (imin < N_SCAN - 1)) {
-            double fopt2 = 0.;
-            find_minimum_bisection(f, xs[imin - 1], xs[imin], xs[imin + 1], fs + imin, RESOLUTION, 100, &fopt2);
-            if (fopt2 < fopt1) fopt1 = fopt2;
+            const double xa = __shfl(xl, imin - 1, 64), xb = __shfl(xl, imin, 64), xc = __shfl(xl, imin + 1, 64);
+            MinimumBisection s{xa, xb, xc, fmin, RESOLUTION * fabs(xc - xa), 0, 100};
+            search(f, s);
+            if (s.fb < fopt1) fopt1 = s.fb;
         }
     }
     double fopt = (fopt0 < fopt1) ? fopt0 : fopt1;
