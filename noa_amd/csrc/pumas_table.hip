@@ -17,14 +17,17 @@
 // (pumas.c:11745-11761), and a third the envelope maxima (pumas.c:11526-11679,
 // a search over the interpolated table; see pumas_envelope_kernel).
 //
-// FP64 throughout, with the device libm (log, exp, pow, sqrt, log10); the
-// grid is computed on the host with the reference's operations.
+// FP64 throughout, with the table-driven log and exp of fastmath.hh (powers as
+// exp of a multiple of the log); the grid is computed on the host with the
+// reference's operations.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cmath>
 #include <cstdint>
 
 #include "capi_util.hh"
+#include "fastmath.hh"
 
 namespace noa_hip {
 namespace pumas {
@@ -45,6 +48,7 @@ constexpr double NEUTRON_MASS = 0.939565;
 constexpr double PION_MASS = 0.13957018;
 constexpr double AVOGADRO_NUMBER = 6.02214076E+23;
 constexpr double PI = 3.14159265358979323846;
+constexpr double INV_LN10 = 0.43429448190325182765;
 constexpr double NUCLEON_MASS = 0.5 * (PROTON_MASS + NEUTRON_MASS);
 // MeV-unit constants of the SSR models (pumas.c:13891-13894, 14461-14463)
 constexpr double SSR_SQRTE = 1.648721270700128;
@@ -115,8 +119,29 @@ struct ElementBlock {
     ElementConsts e[MAX_EL];
 };
 
+// The envelope kernel reads the nodes as floats only, which leaves room for
+// more elements per launch.
+constexpr int MAX_ENV_EL = 24;
+
+struct GridF {
+    float x[MAX_X];
+    int32_t n;
+    double cutoff;
+};
+
+struct EnvelopeBlock {
+    ElementConsts e[MAX_ENV_EL];
+};
+
+// The log/exp tables in LDS as `tb` (every thread of the workgroup calls it).
+#define NOA_PUMAS_TABLES()                                                                                    \
+    __shared__ __attribute__((aligned(fm::TABLE_LDS_ALIGN))) double fm_block[fm::TABLE_DOUBLES];             \
+    for (unsigned i = threadIdx.x; i < fm::TABLE_DOUBLES; i += blockDim.x) fm_block[i] = fm::table_entry(int(i)); \
+    __syncthreads();                                                                                          \
+    const fm::Tab tb = fm::tab_from_block(fm_block)
+
 // Li2(x) by the RDILOG reductions onto [0, 1] and the Clenshaw sum.
-__device__ double dilog(double x) {
+__device__ double dilog(double x, const fm::Tab& tb) {
 #pragma clang fp contract(off)
     const double PI3 = PI * PI / 3.;
     const double PI6 = PI * PI / 6.;
@@ -128,22 +153,22 @@ __device__ double dilog(double x) {
     if (T <= -2) {
         Y = -1. / (1. + T);
         S = 1.;
-        const double l1 = log(-T), l2 = log(1. + 1. / T);
+        const double l1 = fm::log(-T, tb), l2 = fm::log(1. + 1. / T, tb);
         A = -PI3 + 0.5 * (l1 * l1 - l2 * l2);
     } else if (T < -1.) {
         Y = -1. - T;
         S = -1.;
-        A = log(-T);
-        A = -PI6 + A * (A + log(1. + 1. / T));
+        A = fm::log(-T, tb);
+        A = -PI6 + A * (A + fm::log(1. + 1. / T, tb));
     } else if (T <= -0.5) {
         Y = -(1. + T) / T;
         S = 1.;
-        A = log(-T);
-        A = -PI6 + A * (-0.5 * A + log(1. + T));
+        A = fm::log(-T, tb);
+        A = -PI6 + A * (-0.5 * A + fm::log(1. + T, tb));
     } else if (T < 0.) {
         Y = -T / (1. + T);
         S = -1.;
-        const double l = log(1 + T);
+        const double l = fm::log(1 + T, tb);
         A = 0.5 * (l * l);
     } else if (T <= 1.) {
         Y = T;
@@ -152,7 +177,7 @@ __device__ double dilog(double x) {
     } else {
         Y = 1. / T;
         S = -1.;
-        const double l = log(T);
+        const double l = fm::log(T, tb);
         A = PI6 + 0.5 * (l * l);
     }
     const double H = Y + Y - 1;
@@ -168,7 +193,7 @@ __device__ double dilog(double x) {
 }
 
 // SSR bremsstrahlung, atomic DCS in m^2 / GeV (pumas.c:13979-14068).
-__device__ double brems_ssr(const ElementConsts& c, const Globals& G, double m, double K, double q) {
+__device__ double brems_ssr(const ElementConsts& c, const Globals& G, double m, double K, double q, const fm::Tab& tb) {
 #pragma clang fp contract(off)
     const double Z = c.Z;
     if ((Z <= 0) || (c.A <= 0) || (m <= 0) || (K <= 0) || (q <= 0)) return 0.;
@@ -180,13 +205,13 @@ __device__ double brems_ssr(const ElementConsts& c, const Globals& G, double m, 
     const double rl_inel = (Z == 1.) ? 446. : 1429.;
     const double delta = m * m * v / (2. * energy * (1. - v));
     const double rz = c.rl * Z13;
-    double phi1 = log(rz * (m / SSR_ME) / (1. + rz * G.e05 * delta / SSR_ME));
-    double phi2 = log(rz * G.e_16 * (m / SSR_ME) / (1. + rz * G.e13 * delta / SSR_ME));
+    double phi1 = fm::log(rz * (m / SSR_ME) / (1. + rz * G.e05 * delta / SSR_ME), tb);
+    double phi2 = fm::log(rz * G.e_16 * (m / SSR_ME) / (1. + rz * G.e13 * delta / SSR_ME), tb);
     const double iz = 1. - 1. / Z;
     phi1 -= c.b_delta1 * iz;
     phi2 -= c.b_delta2 * iz;
-    const double s1 = log(m / delta / (m * delta / (SSR_ME * SSR_ME) + SSR_SQRTE));
-    const double s2 = log(1. + SSR_ME / (delta * rl_inel * Z13 * Z13 * SSR_SQRTE));
+    const double s1 = fm::log(m / delta / (m * delta / (SSR_ME * SSR_ME) + SSR_SQRTE), tb);
+    const double s2 = fm::log(1. + SSR_ME / (delta * rl_inel * Z13 * Z13 * SSR_SQRTE), tb);
     const double s_atomic = (4. / 3. * (1. - v) + v * v) * (s1 - s2);
     double s_rad;
     if (v < .0 || v > 1.) {
@@ -197,12 +222,12 @@ __device__ double brems_ssr(const ElementConsts& c, const Globals& G, double m, 
         s_rad = 0.1642 + 132.573 * v + -585.361 * v * v + 1407.77 * v * v * v;
     } else if (v < 0.9) {
         s_rad = -2.8922 + -19.0156 * v + 57.698 * v * v;
-        const double t = log(1. - v);
-        s_rad += -63.418 * v * log(v) + 14.1166 * t + 1.84206 * t * t;
+        const double t = fm::log(1. - v, tb);
+        s_rad += -63.418 * v * fm::log(v, tb) + 14.1166 * t + 1.84206 * t * t;
     } else {
         s_rad = 2134.19 + 581.823 * v + -2708.85 * v * v;
-        const double t = log(1. - v);
-        s_rad += 4767.05 * v * log(v) + 1.52918 * t + 0.361933 * t * t;
+        const double t = fm::log(1. - v, tb);
+        s_rad += 4767.05 * v * fm::log(v, tb) + 1.52918 * t + 0.361933 * t * t;
     }
     const double result =
         ((2. - 2. * v + v * v) * phi1 - 2. / 3. * (1. - v) * phi2) + 1. / Z * s_atomic + 0.25 * ALPHA_EM * phi1 * s_rad;
@@ -217,7 +242,27 @@ struct PairQ {
     double v, m, energy, ev, rl, Z13, d_n, beta, xi0, pref, me_dn2, me_m2;
 };
 
-__device__ __forceinline__ PairQ pair_setup(const ElementConsts& c, double m_gev, double K, double q) {
+// The atomic-electron factor zeta of pair production (pumas.c:14482-14492),
+// which depends on the element and K only.
+__device__ __forceinline__ double pair_zeta(const ElementConsts& c, double m_gev, double K, const fm::Tab& tb) {
+#pragma clang fp contract(off)
+    const double Z = c.Z;
+    const double energy = (K + m_gev) * 1E+03;
+    const double m = m_gev * 1E+03;
+    double g1, g2;
+    if (Z == 1.) {
+        g1 = 4.4E-05;
+        g2 = 4.8E-05;
+    } else {
+        g1 = 1.95E-05;
+        g2 = 5.3E-05;
+    }
+    const double zeta1 = (0.073 * fm::log(energy / m / (1. + g1 * c.Z23 * energy / m), tb) - 0.26);
+    const double zeta2 = (0.058 * fm::log(energy / m / (1 + g2 / c.Z13m * energy / m), tb) - 0.14);
+    return ((zeta1 > 0.) && (zeta2 > 0.)) ? zeta1 / zeta2 : 0.;
+}
+
+__device__ __forceinline__ PairQ pair_setup(const ElementConsts& c, double m_gev, double K, double q, double zeta) {
 #pragma clang fp contract(off)
     const double Z = c.Z;
     PairQ s;
@@ -230,17 +275,6 @@ __device__ __forceinline__ PairQ pair_setup(const ElementConsts& c, double m_gev
     const double const_prefactor = 4. / (3. * PI) * Z * (are * are);
     s.Z13 = c.Z13m;
     s.d_n = c.dn;
-    double g1, g2;
-    if (Z == 1.) {
-        g1 = 4.4E-05;
-        g2 = 4.8E-05;
-    } else {
-        g1 = 1.95E-05;
-        g2 = 5.3E-05;
-    }
-    const double zeta1 = (0.073 * log(s.energy / s.m / (1. + g1 * c.Z23 * s.energy / s.m)) - 0.26);
-    const double zeta2 = (0.058 * log(s.energy / s.m / (1 + g2 / s.Z13 * s.energy / s.m)) - 0.14);
-    const double zeta = ((zeta1 > 0.) && (zeta2 > 0.)) ? zeta1 / zeta2 : 0.;
     s.pref = const_prefactor * (Z + zeta) * (1. - s.v) / s.v;
     s.beta = s.v * s.v / (2. * (1. - s.v));
     const double mv = s.m * s.v / (2. * SSR_ME);
@@ -253,7 +287,7 @@ __device__ __forceinline__ PairQ pair_setup(const ElementConsts& c, double m_gev
 }
 
 // SSR pair DDCS at the reference's rho (pumas.c:14499-14609).
-__device__ double pair_d2_ssr(const PairQ& s, const Globals& G, double rho) {
+__device__ double pair_d2_ssr(const PairQ& s, const Globals& G, double rho, const fm::Tab& tb) {
 #pragma clang fp contract(off)
     rho = 1 - rho;
     const double rho2 = rho * rho;
@@ -266,49 +300,49 @@ __device__ double pair_d2_ssr(const PairQ& s, const Globals& G, double rho) {
     const double c13 = 2. * SSR_ME * G.e13 * s.rl * s.Z13 * xi1 / w;
 
     // electron diagram
-    const double lxi_i = log(1. + 1. / xi);
+    const double lxi_i = fm::log(1. + 1. / xi, tb);
     const double Pe = (2. + rho2) * (1. + beta) + xi * (3. + rho2);
     const double Be = Pe * lxi_i + (1. - rho2 - beta) / xi1 - (3. + rho2);
     const double Ce2 = (omr * (1. + beta) + xi * (3. - rho2)) * lxi_i + 2. * (1. - beta - rho2) / xi1 - (3. - rho2);
     const double Ce1 = Be - Ce2;
-    const double De = Pe * dilog(1. / xi1) - (2. + rho2) * xi * lxi_i - (xi + rho2 + beta) / xi1;
+    const double De = Pe * dilog(1. / xi1, tb) - (2. + rho2) * xi * lxi_i - (xi + rho2 + beta) / xi1;
     const double sx = s.rl * s.Z13 * sqrt(xi1);
     const double sx6 = s.rl * s.Z13 * G.e_16 * sqrt(xi1);
     const double re = De / Be;
     double Le1, Le2;
     if (re > 0.) {
-        const double Xe = (re < 100) ? exp(-re) : 0.;
-        Le1 = log(sx / (Xe + c05)) - re - 0.5 * log(Xe + s.me_dn2 * xi1);
-        Le2 = log(sx6 / (Xe + c13)) - re - 0.5 * log(Xe + s.me_dn2 * G.e_13 * xi1);
+        const double Xe = (re < 100) ? fm::exp(-re, tb) : 0.;
+        Le1 = fm::log(sx / (Xe + c05), tb) - re - 0.5 * fm::log(Xe + s.me_dn2 * xi1, tb);
+        Le2 = fm::log(sx6 / (Xe + c13), tb) - re - 0.5 * fm::log(Xe + s.me_dn2 * G.e_13 * xi1, tb);
     } else {
-        const double Xi = (re > -100) ? exp(re) : 0.;
-        Le1 = log(sx / (1. + Xi * c05)) - 0.5 * re - 0.5 * log(1. + Xi * s.me_dn2 * xi1);
-        Le2 = log(sx6 / (1. + Xi * c13)) - 0.5 * re - 0.5 * log(1. + Xi * s.me_dn2 * G.e_13 * xi1);
+        const double Xi = (re > -100) ? fm::exp(re, tb) : 0.;
+        Le1 = fm::log(sx / (1. + Xi * c05), tb) - 0.5 * re - 0.5 * fm::log(1. + Xi * s.me_dn2 * xi1, tb);
+        Le2 = fm::log(sx6 / (1. + Xi * c13), tb) - 0.5 * re - 0.5 * fm::log(1. + Xi * s.me_dn2 * G.e_13 * xi1, tb);
     }
     double diagram_e = s.pref * (Ce1 * Le1 + Ce2 * Le2);
     if (diagram_e < 0.) diagram_e = 0.;
 
     // muon diagram
-    const double lxi = log(xi1);
+    const double lxi = fm::log(xi1, tb);
     const double b15 = 1. + (3. * beta) / 2.;
     const double Pm = (1. + rho2) * b15 - 1. / xi * (1. + 2. * beta) * omr;
     const double Bm = Pm * lxi + xi * (1. - rho2 - beta) / xi1 + (1. + 2. * beta) * omr;
     const double Cm2 = ((1. - beta) * omr - xi * (1. + rho2)) * lxi / xi - 2. * (1. - beta - rho2) / xi1 + 1. - beta -
                        (1. + beta) * rho2;
     const double Cm1 = Bm - Cm2;
-    const double Dm = Pm * dilog(xi / xi1) + b15 * omr / xi * lxi +
+    const double Dm = Pm * dilog(xi / xi1, tb) + b15 * omr / xi * lxi +
                       (1. - rho2 - beta / 2. * (1. + rho2) + omr / (2. * xi) * beta) * xi / xi1;
     const double num = s.m / SSR_ME * s.rl * s.Z13 / s.d_n;
     const double rm = Dm / Bm;
     double Lm1, Lm2;
     if (rm > 0.) {
-        const double Xm = (rm < 100) ? exp(-rm) : 0.;
-        Lm1 = log(num / (Xm + c05)) - rm;
-        Lm2 = log(num / (Xm + c13)) - rm;
+        const double Xm = (rm < 100) ? fm::exp(-rm, tb) : 0.;
+        Lm1 = fm::log(num / (Xm + c05), tb) - rm;
+        Lm2 = fm::log(num / (Xm + c13), tb) - rm;
     } else {
-        const double Xv = (rm > -100) ? exp(rm) : 0.;
-        Lm1 = log(num / (1. + c05 * Xv));
-        Lm2 = log(num / (1. + c13 * Xv));
+        const double Xv = (rm > -100) ? fm::exp(rm, tb) : 0.;
+        Lm1 = fm::log(num / (1. + c05 * Xv), tb);
+        Lm2 = fm::log(num / (1. + c13 * Xv), tb);
     }
     double diagram_mu = s.pref * s.me_m2 * (Cm1 * Lm1 + Cm2 * Lm2);
     if (diagram_mu < 0.) diagram_mu = 0.;
@@ -317,7 +351,8 @@ __device__ double pair_d2_ssr(const PairQ& s, const Globals& G, double rho) {
 
 // SSR pair production, atomic DCS in m^2 / GeV (pumas.c:14624-14671): the
 // 12-point rule over t = ln(rho) on [ln(1 - rmax), 0].
-__device__ double pair_ssr(const ElementConsts& c, const Globals& G, double mass, double K, double q) {
+__device__ double pair_ssr(const ElementConsts& c, const Globals& G, double mass, double K, double q,
+                           const fm::Tab& tb) {
 #pragma clang fp contract(off)
     if ((c.Z <= 0) || (c.A <= 0) || (mass <= 0) || (K <= 0) || (q <= 0)) return 0.;
     if (q <= 4. * ELECTRON_MASS) return 0.;
@@ -329,56 +364,60 @@ __device__ double pair_ssr(const ElementConsts& c, const Globals& G, double mass
     const double rmax = sqrt(x0) * x1;
     const double ri = 1. - rmax;
     if ((ri <= 0.) || (ri >= 1.)) return 0.;
-    const double tmin = log(ri);
+    const double tmin = fm::log(ri, tb);
     // the DDCS's own range check (pumas.c:14469-14471) holds at every node:
     // 4 m_e < q < K + p_qoff
-    const PairQ s = pair_setup(c, mass, K, q);
+    const PairQ s = pair_setup(c, mass, K, q, pair_zeta(c, mass, K, tb));
     double I = 0.;
+#pragma unroll 1
     for (int i = 0; i < 12; i++) {
-        const double rho = exp(GQ12_X[i] * tmin);
-        I -= pair_d2_ssr(s, G, rho) * rho * GQ12_W[i] * tmin;
+        const double rho = fm::exp(GQ12_X[i] * tmin, tb);
+        I -= pair_d2_ssr(s, G, rho, tb) * rho * GQ12_W[i] * tmin;
     }
     return (I < 0) ? 0. : I;
 }
 
 // ALLM97 proton structure function F2 (pumas.c:14690-14745); lq0 is
-// log(Q0^2 / Lambda^2).
-__device__ double f2p_allm97(double x, double Q2, double lq0) {
+// fm::log(Q0^2 / Lambda^2, tb).
+__device__ double f2p_allm97(double x, double Q2, double lq0, const fm::Tab& tb) {
 #pragma clang fp contract(off)
     const double m02 = 0.31985, mP2 = 49.457, mR2 = 0.15052, Q02 = 0.52544, Lambda2 = 0.06527;
     const double M2 = NUCLEON_MASS * NUCLEON_MASS;
     const double W2 = M2 + Q2 * (1.0 / x - 1.0);
-    const double t = log(log((Q2 + Q02) / Lambda2) / lq0);
+    const double t = fm::log(fm::log((Q2 + Q02) / Lambda2, tb) / lq0, tb);
+    // t^c as exp(c log t); t is 0 in exact arithmetic as Q2 -> 0, and clamped there
+    const double lnt = fm::log(t < 0. ? 0. : t, tb);
     const double xP = (Q2 + mP2) / (Q2 + mP2 + W2 - M2);
     const double xR = (Q2 + mR2) / (Q2 + mR2 + W2 - M2);
-    const double cP = 0.28067 + (0.28067 - 0.22291) * (1.0 / (1.0 + pow(t, 2.1979)) - 1.0);
-    const double aP = -0.0808 + (-0.0808 - -0.44812) * (1.0 / (1.0 + pow(t, 1.1709)) - 1.0);
-    const double bP = 0.36292 + 1.8917 * pow(t, 1.8439);
-    const double cR = 0.80107 + 0.97307 * pow(t, 3.4942);
-    const double aR = 0.58400 + 0.37888 * pow(t, 2.6063);
-    const double bR = 0.01147 + 3.7582 * pow(t, 0.49338);
-    const double l1x = log(1 - x);
-    const double F2P = cP * exp(aP * log(xP) + bP * l1x);
-    const double F2R = cR * exp(aR * log(xR) + bR * l1x);
+    const double cP = 0.28067 + (0.28067 - 0.22291) * (1.0 / (1.0 + fm::exp(2.1979 * lnt, tb)) - 1.0);
+    const double aP = -0.0808 + (-0.0808 - -0.44812) * (1.0 / (1.0 + fm::exp(1.1709 * lnt, tb)) - 1.0);
+    const double bP = 0.36292 + 1.8917 * fm::exp(1.8439 * lnt, tb);
+    const double cR = 0.80107 + 0.97307 * fm::exp(3.4942 * lnt, tb);
+    const double aR = 0.58400 + 0.37888 * fm::exp(2.6063 * lnt, tb);
+    const double bR = 0.01147 + 3.7582 * fm::exp(0.49338 * lnt, tb);
+    const double l1x = fm::log(1 - x, tb);
+    const double F2P = cP * fm::exp(aP * fm::log(xP, tb) + bP * l1x, tb);
+    const double F2R = cR * fm::exp(aR * fm::log(xR, tb) + bR * l1x, tb);
     return Q2 / (Q2 + m02) * (F2P + F2R);
 }
 
 // DRSS photonuclear DDCS d2S / (dq dQ2) (pumas.c:14752-14785, 14987-15010).
-__device__ double photo_d2_drss(const ElementConsts& c, const Globals& G, double ml, double K, double q, double Q2) {
+__device__ double photo_d2_drss(const ElementConsts& c, const Globals& G, double ml, double K, double q, double Q2,
+                                const fm::Tab& tb) {
 #pragma clang fp contract(off)
     const double Z = c.Z, A = c.A;
     const double cf = 4 * PI * ALPHA_EM * ALPHA_EM * HBAR_C * HBAR_C;
     const double E = K + ml;
     const double y = q / E;
     const double x = 0.5 * Q2 / (NUCLEON_MASS * q);
-    const double F2p = f2p_allm97(x, Q2, G.lq0);
+    const double F2p = f2p_allm97(x, Q2, G.lq0, tb);
     double shadowing;
     if (Z == 1.)
         shadowing = 1.;
     else if (x < 0.0014)
         shadowing = c.shadow_low;
     else if (x < 0.04)
-        shadowing = exp((0.069 * log10(x) + 0.097) * c.lnA);
+        shadowing = fm::exp((0.069 * (fm::log(x, tb) * INV_LN10) + 0.097) * c.lnA, tb);
     else
         shadowing = 1.;
     const double F2A = F2p * shadowing * (Z + (A - Z) * (1.0 + x * (-1.85 + x * (2.45 + x * (-2.35 + x)))));
@@ -389,7 +428,8 @@ __device__ double photo_d2_drss(const ElementConsts& c, const Globals& G, double
 
 // DRSS photonuclear, atomic DCS in m^2 / GeV (pumas.c:15066-15146, mode 0):
 // the 9-point rule on ln Q^2 over [Q2min, Q2max].
-__device__ double photo_drss(const ElementConsts& c, const Globals& G, double ml, double K, double q) {
+__device__ double photo_drss(const ElementConsts& c, const Globals& G, double ml, double K, double q,
+                             const fm::Tab& tb) {
 #pragma clang fp contract(off)
     if ((c.Z <= 0) || (c.A <= 0) || (ml <= 0) || (K <= 0)) return 0.;
     const double M = NUCLEON_MASS;
@@ -400,12 +440,13 @@ __device__ double photo_drss(const ElementConsts& c, const Globals& G, double ml
     const double Q2min = ml2 * (q * q - 0.5 * ml2) / (E * (E - q));
     const double Q2max = 2.0 * M * (q - mpi) - mpi * mpi;
     if ((Q2max < Q2min) | (Q2min < 0)) return 0.;
-    const double lmin = log(Q2min);
-    const double dx = log(Q2max) - lmin;
+    const double lmin = fm::log(Q2min, tb);
+    const double dx = fm::log(Q2max, tb) - lmin;
     double ds = 0.;
+#pragma unroll 1
     for (int i = 0; i < 9; i++) {
-        const double Q2 = exp(lmin + dx * GQ9_X[i]);
-        const double tmp = photo_d2_drss(c, G, ml, K, q, Q2);
+        const double Q2 = fm::exp(lmin + dx * GQ9_X[i], tb);
+        const double tmp = photo_d2_drss(c, G, ml, K, q, Q2, tb);
         if (tmp <= 0.) continue;
         ds += tmp * (GQ9_W[i] * (dx * Q2));
     }
@@ -414,7 +455,7 @@ __device__ double photo_drss(const ElementConsts& c, const Globals& G, double ml
 
 // Node `node` of pair_ssr's rule, with skip set where pair_ssr returns 0.
 __device__ __forceinline__ void pair_term(const ElementConsts& c, const Globals& G, double mass, double K, double q,
-                                          int node, double* term, int* skip) {
+                                          double zeta, int node, double* term, int* skip, const fm::Tab& tb) {
 #pragma clang fp contract(off)
     if ((c.Z <= 0) || (c.A <= 0) || (mass <= 0) || (K <= 0) || (q <= 0)) return;
     if (q <= 4. * ELECTRON_MASS) return;
@@ -426,17 +467,17 @@ __device__ __forceinline__ void pair_term(const ElementConsts& c, const Globals&
     const double rmax = sqrt(x0) * x1;
     const double ri = 1. - rmax;
     if ((ri <= 0.) || (ri >= 1.)) return;
-    const double tmin = log(ri);
-    const PairQ s = pair_setup(c, mass, K, q);
-    const double rho = exp(GQ12_X[node] * tmin);
-    *term = pair_d2_ssr(s, G, rho) * rho * GQ12_W[node] * tmin;
+    const double tmin = fm::log(ri, tb);
+    const PairQ s = pair_setup(c, mass, K, q, zeta);
+    const double rho = fm::exp(GQ12_X[node] * tmin, tb);
+    *term = pair_d2_ssr(s, G, rho, tb) * rho * GQ12_W[node] * tmin;
     *skip = 0;
 }
 
 // Node `node` of photo_drss's rule inside dcs()'s range, with skip set where
 // the DCS is 0 or the node is left out of the sum.
 __device__ __forceinline__ void photo_term(const ElementConsts& c, const Globals& G, double ml, double K, double q,
-                                           int node, double* term, int* skip) {
+                                           int node, double* term, int* skip, const fm::Tab& tb) {
 #pragma clang fp contract(off)
     const double M = NUCLEON_MASS;
     const double mpi = PION_MASS;
@@ -448,28 +489,29 @@ __device__ __forceinline__ void photo_term(const ElementConsts& c, const Globals
     const double Q2min = ml2 * (q * q - 0.5 * ml2) / (E * (E - q));
     const double Q2max = 2.0 * M * (q - mpi) - mpi * mpi;
     if ((Q2max < Q2min) | (Q2min < 0)) return;
-    const double lmin = log(Q2min);
-    const double dx = log(Q2max) - lmin;
-    const double Q2 = exp(lmin + dx * GQ9_X[node]);
-    const double tmp = photo_d2_drss(c, G, ml, K, q, Q2);
+    const double lmin = fm::log(Q2min, tb);
+    const double dx = fm::log(Q2max, tb) - lmin;
+    const double Q2 = fm::exp(lmin + dx * GQ9_X[node], tb);
+    const double tmp = photo_d2_drss(c, G, ml, K, q, Q2, tb);
     *skip = tmp <= 0.;
     *term = tmp * (GQ9_W[node] * (dx * Q2));
 }
 
 // The m^2/kg DCS of process 0 (bremsstrahlung), 1 (pair production) or 2
 // (photonuclear) as dcs_get(process) returns it (pumas.c:11018-11112).
-__device__ double dcs(int process, const ElementConsts& c, const Globals& G, double mass, double K, double q) {
+__device__ double dcs(int process, const ElementConsts& c, const Globals& G, double mass, double K, double q,
+                      const fm::Tab& tb) {
 #pragma clang fp contract(off)
     double d;
     if (process == 0) {
-        d = brems_ssr(c, G, mass, K, q);
+        d = brems_ssr(c, G, mass, K, q, tb);
     } else if (process == 1) {
-        d = pair_ssr(c, G, mass, K, q);
+        d = pair_ssr(c, G, mass, K, q, tb);
     } else {
         const double qmin = PION_MASS + 0.5 * PION_MASS * PION_MASS / NUCLEON_MASS;
         const double qmax = K + mass - 0.5 * (NUCLEON_MASS + mass * mass / NUCLEON_MASS);
         if ((q < qmin) || (q > qmax)) return 0.;
-        d = photo_drss(c, G, mass, K, q);
+        d = photo_drss(c, G, mass, K, q, tb);
     }
     return d * 1E+03 * AVOGADRO_NUMBER * (mass + K) / c.A;
 }
@@ -477,8 +519,9 @@ __device__ double dcs(int process, const ElementConsts& c, const Globals& G, dou
 __global__ __launch_bounds__(256) void pumas_dcs_kernel(int process, ElementConsts c, Globals G, double mass,
                                                         const double* __restrict__ K, const double* __restrict__ q,
                                                         int64_t n, double* __restrict__ out) {
+    NOA_PUMAS_TABLES();
     for (int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x; i < n; i += int64_t(gridDim.x) * blockDim.x)
-        out[i] = dcs(process, c, G, mass, K[i], q[i]);
+        out[i] = dcs(process, c, G, mass, K[i], q[i], tb);
 }
 
 // One 64-lane workgroup per row of the launch's element block: block row
@@ -490,6 +533,7 @@ __global__ __launch_bounds__(64) void pumas_table_kernel(Grid g, ElementBlock bl
                                                          float* __restrict__ x_out, float* __restrict__ env,
                                                          const double* __restrict__ csn) {
 #pragma clang fp contract(off)
+    NOA_PUMAS_TABLES();
     __shared__ double ys[MAX_X];
     __shared__ double ms[MAX_X];
     __shared__ int pos[MAX_X];
@@ -520,10 +564,10 @@ __global__ __launch_bounds__(64) void pumas_table_kernel(Grid g, ElementBlock bl
     }
 
     for (int i = lane; i < n; i += 64) {
-        const double q = K * exp(g.x[i]);
-        const double d = dcs(p, c, G, mass, K, q);
+        const double q = K * fm::exp(g.x[i], tb);
+        const double d = dcs(p, c, G, mass, K, q, tb);
         pos[i] = d > 0;
-        ys[i] = d > 0 ? log(d) : 0.;
+        ys[i] = d > 0 ? fm::log(d, tb) : 0.;
         if (b == 0 && x_out) x_out[i] = float(g.x[i]);
     }
     __syncthreads();
@@ -611,7 +655,7 @@ __global__ __launch_bounds__(64) void pumas_table_kernel(Grid g, ElementBlock bl
         const double qrev = X_REVERSE * K;
         qmax *= 0.5;
         if (qmax > qrev) qmax = qrev;
-        const double xmin = log(qmin / K), xmax = log(qmax / K);
+        const double xmin = fm::log(qmin / K, tb), xmax = fm::log(qmax / K, tb);
         int ia0 = imax, ia1 = imin;
         for (int i = imin; i <= imax && i < n; i++) {
             if ((g.x[i] > xmin) && (g.x[i] < xmax)) {
@@ -659,13 +703,13 @@ __device__ __forceinline__ int model_batch(int process) { return process == 0 ? 
 // the set-up and one quadrature node, and the node terms are summed in the
 // serial loop's order, so the values are those of dcs() bit for bit. Must be
 // called with the wave's 64 lanes active.
-__device__ __attribute__((noinline)) double dcs_wave(int process, const ElementConsts& c, const Globals& G, double mass, double K, double q,
-                           bool need) {
+__device__ __forceinline__ double dcs_wave(int process, const ElementConsts& c, const Globals& G, double mass, double K,
+                                           double zeta, double q, bool need, const fm::Tab& tb) {
 #pragma clang fp contract(off)
     const int lane = threadIdx.x & 63;
     double d = 0.;
     if (process == 0) {
-        if (need) d = brems_ssr(c, G, mass, K, q);
+        if (need) d = brems_ssr(c, G, mass, K, q, tb);
     } else {
         const int nodes = process == 1 ? 12 : 9;
         const int per = model_batch(process);
@@ -687,15 +731,23 @@ __device__ __attribute__((noinline)) double dcs_wave(int process, const ElementC
             int skip = 1;
             if (mine >= 0) {
                 if (process == 1)
-                    pair_term(c, G, mass, K, qg, node, &term, &skip);
+                    pair_term(c, G, mass, K, qg, zeta, node, &term, &skip, tb);
                 else
-                    photo_term(c, G, mass, K, qg, node, &term, &skip);
+                    photo_term(c, G, mass, K, qg, node, &term, &skip, tb);
             }
             const int first = (owner_group < 0 ? 0 : owner_group) * nodes;
             double sum = 0.;
-            for (int i = 0; i < nodes; i++) {
-                const double t = __shfl(term, first + i, 64);
-                if (!__shfl(skip, first + i, 64)) sum = process == 1 ? sum - t : sum + t;
+            if (process == 1) {
+                const int skipped = __shfl(skip, first, 64);  // a whole evaluation at once
+#pragma unroll
+                for (int i = 0; i < 12; i++) sum -= __shfl(term, first + i, 64);
+                if (skipped) sum = 0.;
+            } else {
+#pragma unroll
+                for (int i = 0; i < 9; i++) {
+                    const double t = __shfl(term, first + i, 64);
+                    if (!__shfl(skip, first + i, 64)) sum += t;
+                }
             }
             if (owner_group >= 0) d = (sum < 0) ? 0. : sum;
         }
@@ -708,19 +760,20 @@ __device__ __attribute__((noinline)) double dcs_wave(int process, const ElementC
 // One wave per row. The reference searches the maximum of DCS x^alpha over ln x
 // serially, 100 to 240 evaluations of one point each: bisections that find
 // where the DCS becomes positive at the range ends, then two bracketing
-// bisections (math_find_minimum with algo 0, pumas.c:12172-12232 and
-// 12416-12459), and for pair production at K >= 1e7 a logarithmic scan next to
-// the upper end. DCS is the table interpolated as dcs_evaluate does without a
-// context (pumas.c:11307-11398) and the model where the table does not apply.
-// The rows read are those of the finished table.
+// bisections, one in each half of the range (math_find_minimum with algo 0,
+// pumas.c:12172-12232 and 12416-12459), and for pair production at K >= 1e7 a
+// logarithmic scan next to the upper end. DCS is the table interpolated as
+// dcs_evaluate does without a context (pumas.c:11307-11398) and the model
+// where the table does not apply. The rows read are those of the finished
+// table.
 //
 // Every step of those searches has two outcomes and the next point depends
-// only on the outcomes so far, so the wave evaluates the points of the next d
-// steps at once, all 2^d - 1 of their decision tree, one per lane, and then
-// walks the tree: the same points, values and decisions as the serial search.
-// d is 6 where the table serves the tree, less where points need the model: as
-// many levels as their model evaluations fit one batch of dcs_wave (5 of pair
-// production, 7 of photonuclear).
+// only on the outcomes so far, so half a wave evaluates the points of a
+// search's next 5 steps at once, all 31 of their decision tree, one per lane,
+// and then walks the tree: the points and decisions of the serial search. The
+// two halves run the two bracketing searches side by side. Where points need
+// the model, fewer steps: as many as their model evaluations fit one batch of
+// dcs_wave (5 of pair production, 7 of photonuclear).
 //
 // Where the range end is the logarithm of a negative number (K below the
 // kinematic threshold) the reference's search makes 200 evaluations at NaN;
@@ -730,10 +783,17 @@ __device__ __attribute__((noinline)) double dcs_wave(int process, const ElementC
 // compute_dcs_table writes only after element 0 (pumas.c:11775-11783), so
 // element 0's search sees zero nodes and takes the model everywhere; the
 // kernel does the same.
+//
+// What bounds it is the length of a row's chain of rounds (about 30, up to 60
+// where every point needs the model, of ~1000 to 2500 dependent instructions
+// each), with two or three waves per SIMD to overlap. Measured for 48 elements
+// x 146 energies, the whole table call: one point per step for the whole wave
+// 10,600 us; trees of one search per wave 4113; two searches side by side with
+// the table log / exp 2810; the rows' constants and the searches kept out of
+// the registers, 24 elements per launch and pair production's rows, the
+// longest, first: 1980 us, of which the two envelope launches are 1650.
 
 struct EnvRow {
-    const ElementConsts* c;
-    const Globals* G;
     int process;
     double mass;
     const float* xt;    // the nodes as the search sees them (LDS)
@@ -777,9 +837,8 @@ __device__ __forceinline__ int table_index(const double* table, int n_K, double 
 
 // The interpolated DCS at q without its factor K / (K + m), or *need set where
 // it is the model's.
-__device__ double dcs_from_table(const EnvRow& a, double K, double q, bool* need) {
+__device__ __forceinline__ double dcs_from_table(const EnvRow& a, const ElementConsts& c, double K, double q, bool* need) {
 #pragma clang fp contract(off)
-    const ElementConsts& c = *a.c;
     double qlow = 0., qmin, qmax;
     *need = false;
     if (a.process == 2) {
@@ -832,264 +891,363 @@ __device__ double dcs_from_table(const EnvRow& a, double K, double q, bool* need
     return r;
 }
 
-constexpr int TREE_DEPTH = 6;  // 2^6 - 1 points, one per lane
+// One search of a half-wave (the same state in its 32 lanes).
+enum SearchKind { SEARCH_NONE, SEARCH_EDGE, SEARCH_BRACKET, SEARCH_BISECT };
+constexpr double RESOLUTION = 1E-10;
 
-// -DCS x^alpha at one ln x per lane. `levels`: in, the levels of the decision
-// tree that the lanes hold (lane i its node i in breadth-first order); out, the
-// levels evaluated. levels = -n: the first n lanes are independent points.
-struct EnvObjective {
-    const EnvRow& a;
-    double K, alpha;
-    __device__ double operator()(double lnx, int* levels) const {
-#pragma clang fp contract(off)
-        const int lane = threadIdx.x & 63;
-        const double wj = K / (K + a.mass);
-        const double x = exp(lnx);
-        const double q = x * K;
-        bool need;
-        double d = dcs_from_table(a, K, q, &need);
-        if (*levels > 0) {
-            // as many levels as one batch of model evaluations covers
-            const unsigned long long m = __ballot(need);
-            int l = *levels;
-            while (l > 1 && __popcll(m & ((1ull << ((1 << l) - 1)) - 1)) > model_batch(a.process)) l--;
-            *levels = l;
-            need = need && lane < (1 << l) - 1;
-        } else {
-            need = need && lane < -*levels;
-        }
-        if (__ballot(need)) {
-            const double md = dcs_wave(a.process, *a.c, *a.G, a.mass, K, q, need);
-            if (need) d = md;
-        }
-        return -(d * wj) * pow(x, alpha);
-    }
-    // the same at one point for the whole wave
-    __device__ double at(double lnx) const {
-        int one = -1;
-        return __shfl((*this)(lnx, &one), 0, 64);
-    }
-};
+struct Search {
+    int kind;
+    // EDGE: bisection of [xa, xc] for the edge of the region where f != 0; the
+    //   nonzero side is xc (up) or xa; xb, fb the last nonzero point and value
+    // BRACKET: find_minimum's first stage, halving [xa, xc] towards the lower
+    //   end until the midpoint lies below both ends
+    // BISECT: find_minimum's bisection around xb; fb is the result
+    double xa, xb, xc, fa, fb, fc, tol;
+    int i, max_iter, up;
 
-// Runs a search of two-outcome steps from state s until s.done(): s.point() is
-// the next point, s.next(bit) the state after the outcome `bit`, and
-// s.step(v) the true step with the value v there, which returns its outcome,
-// or -1 to stop.
-template <class F, class S>
-__device__ void search(const F& f, S& s) {
-    const int lane = threadIdx.x & 63;
-    while (!s.done()) {
-        // this lane's node: the bits of lane + 1 below its leading one, from the top, are its path
-        S mine = s;
-        const int depth = 31 - __clz(lane + 1);
-        for (int i = depth - 1; i >= 0; i--) mine.next((lane + 1) >> i & 1);
-        int levels = TREE_DEPTH;
-        const double v = f(mine.point(), &levels);
-        int node = 0;
-        for (int l = 0; l < levels && !s.done(); l++) {
-            const int bit = s.step(__shfl(v, node, 64));
-            if (bit < 0) return;
-            node = 2 * node + 1 + bit;
-        }
+    __device__ __forceinline__ bool done() const {
+        if (kind == SEARCH_EDGE) return !(xc - xa > RESOLUTION);
+        if (kind == SEARCH_BISECT) return !((xc - xa > tol) && (i < max_iter));
+        return kind == SEARCH_NONE;
     }
-}
-
-// Bisection for the edge of the region where f != 0 between x0 and x1; the
-// nonzero side is x1 (up) or x0.
-struct EdgeSearch {
-    static constexpr double RESOLUTION = 1E-10;
-    double x0, x1, edge, value;
-    bool up;
-    __device__ bool done() const { return !(x1 - x0 > RESOLUTION); }
-    __device__ double point() const { return 0.5 * (x0 + x1); }
-    __device__ void next(int nonzero) {
-        const double x2 = 0.5 * (x0 + x1);
-        if (bool(nonzero) == up)
-            x1 = x2;
-        else
-            x0 = x2;
+    __device__ __forceinline__ double point() const {
+        const bool low = kind != SEARCH_BISECT || xb - xa > xc - xb;
+        const double u = (kind == SEARCH_BISECT && !low) ? xb : xa;
+        const double v = (kind == SEARCH_BISECT && low) ? xb : xc;
+        return 0.5 * (u + v);
     }
-    __device__ int step(double f2) {
-        const int nonzero = f2 != 0;
-        if (nonzero) {
-            edge = point();
-            value = f2;
-        }
-        next(nonzero);
-        return nonzero;
-    }
-};
-
-// find_minimum's bisection around xb (pumas.c:12416-12459).
-struct MinimumBisection {
-    double xa, xb, xc, fb, tol;
-    int i, max_iter;
-    __device__ bool done() const { return !((xc - xa > tol) && (i < max_iter)); }
-    __device__ double point() const { return (xb - xa > xc - xb) ? 0.5 * (xa + xb) : 0.5 * (xb + xc); }
-    __device__ void next(int lower) {
+    // The state's points after outcome `bit` of the next step. EDGE: 1 =
+    // nonzero; BRACKET: 1 = the minimum is right; BISECT: 1 = lower than xb.
+    __device__ __forceinline__ void next(int bit) {
         const double x = point();
-        if (xb - xa > xc - xb) {
-            if (lower) {
-                xc = xb;
-                xb = x;
-            } else {
-                xa = x;
-            }
+        if (kind == SEARCH_BISECT) {
+            const bool low = xb - xa > xc - xb;
+            const double b = xb;
+            if (bit) xb = x;
+            // lower on the low side: xc = old xb; on the high side: xa = old
+            // xb; not lower: the bracket's end on that side moves to x
+            if (low == bool(bit))
+                xc = bit ? b : x;
+            else
+                xa = bit ? b : x;
         } else {
-            if (lower) {
-                xa = xb;
-                xb = x;
-            } else {
+            const bool to_c = kind == SEARCH_EDGE ? bit == up : !bit;
+            if (to_c)
                 xc = x;
+            else
+                xa = x;
+        }
+    }
+    // The true step with value v at point(): its outcome.
+    __device__ __forceinline__ int step(double v) {
+        int bit;
+        if (kind == SEARCH_EDGE) {
+            bit = v != 0;
+            if (bit) {
+                xb = point();
+                fb = v;
             }
+        } else if (kind == SEARCH_BISECT) {
+            bit = v < fb;
+            if (bit) fb = v;
+            i++;
+        } else {  // BRACKET
+            xb = point();
+            fb = v;
+            if ((fb < fa) && (fb < fc)) {  // bracketed: on to the bisection, with the iterations left
+                kind = SEARCH_BISECT;
+                tol = RESOLUTION * fabs(xc - xa);
+                max_iter -= i;
+                i = 0;
+                return -1;
+            }
+            i++;
+            if (fabs(xc - xa) <= tol) {  // spent
+                kind = SEARCH_NONE;
+                return -1;
+            }
+            bit = !(fb < fc);
+            if (bit)
+                fa = fb;
+            else
+                fc = fb;
+            next(bit);
+            if (i >= max_iter) {
+                kind = SEARCH_NONE;
+                if (fa < fb)
+                    fb = fa;
+                else if (fc < fb)
+                    fb = fc;
+            }
+            return bit;
         }
-        i++;
-    }
-    __device__ int step(double fi) {
-        const int lower = fi < fb;
-        if (lower) fb = fi;
-        next(lower);
-        return lower;
-    }
-};
-
-// find_minimum's first stage: halves [xa, xc] towards the lower end until the
-// midpoint lies below both ends (found), or the interval is spent (flat).
-struct MinimumBracket {
-    double xa, xb, xc, fa, fb, fc, atol;
-    int i, max_iter;
-    bool found, flat;
-    __device__ bool done() const { return found || flat || i >= max_iter; }
-    __device__ double point() const { return 0.5 * (xa + xc); }
-    __device__ void next(int right) {
-        if (right)
-            xa = point();
-        else
-            xc = point();
-    }
-    __device__ int step(double f) {
-        xb = point();
-        fb = f;
-        if ((fb < fa) && (fb < fc)) {
-            found = true;
-            return -1;
-        }
-        if (fabs(xc - xa) <= atol) {
-            flat = true;
-            return -1;
-        }
-        i++;
-        if (fb < fc) {
-            xc = xb;
-            fc = fb;
-            return 0;
-        }
-        xa = xb;
-        fa = fb;
-        return 1;
+        next(bit);
+        return bit;
     }
 };
 
-template <class F>
-__device__ double find_minimum(const F& f, double xa, double xc, double fa, double fc, double tol, int max_iter) {
-    MinimumBracket b{xa, 0., xc, fa, 0., fc, tol * fabs(xc - xa), 0, max_iter, false, false};
-    search(f, b);
-    if (b.flat) return b.fb;
-    if (!b.found) return (b.fa < b.fb) ? b.fa : (b.fc < b.fb) ? b.fc : b.fb;
-    MinimumBisection m{b.xa, b.xb, b.xc, b.fb, tol * fabs(b.xc - b.xa), 0, max_iter - b.i};
-    search(f, m);
-    return m.fb;
+__device__ __forceinline__ Search new_search(int kind, double xa, double xc, double fa, double fc, double tol, int up,
+                                             double xb, double fb) {
+    Search s;
+    s.kind = kind;
+    s.xa = xa;
+    s.xb = xb;
+    s.xc = xc;
+    s.fa = fa;
+    s.fb = fb;
+    s.fc = fc;
+    s.tol = tol;
+    s.i = 0;
+    s.max_iter = 100;
+    s.up = up;
+    return s;
 }
 
-__device__ float envelope_max(const EnvRow& a, double K, double cutoff, float alpha, double cs) {
+// Orders the wave's LDS accesses before and after it.
+__device__ __forceinline__ void wave_lds_order() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// Stores a half's search (its 32 lanes hold the same values).
+__device__ __forceinline__ void put(Search& to, const Search& s) {
+    wave_lds_order();
+    to = s;
+    wave_lds_order();
+}
+
+// v of one lane, as a wave-uniform (scalar) value.
+__device__ __forceinline__ double from_lane(double v, int lane) {
+    const uint64_t u = __builtin_bit_cast(uint64_t, v);
+    const int l = __builtin_amdgcn_readfirstlane(lane);
+    const uint32_t lo = uint32_t(__builtin_amdgcn_readlane(int(uint32_t(u)), l));
+    const uint32_t hi = uint32_t(__builtin_amdgcn_readlane(int(uint32_t(u >> 32)), l));
+    return __builtin_bit_cast(double, (uint64_t(hi) << 32) | lo);
+}
+
+// The row's constants in the kernel-argument segment, re-read where they are
+// used: an empty asm hides the pointer, and hide() a value, so that what
+// follows from them alone is not formed before the search and held in
+// registers throughout (it took 250 VGPRs, two waves per SIMD).
+using ElementPtr = const __attribute__((address_space(4))) ElementConsts*;
+__device__ __forceinline__ const ElementConsts& row_consts(ElementPtr p) {
+    asm volatile("" : "+s"(p));
+    return *(const ElementConsts*)p;
+}
+__device__ __forceinline__ double hide(double v) {
+    asm volatile("" : "+s"(v));
+    return v;
+}
+
+__device__ __forceinline__ float envelope_max(const EnvRow& a, ElementPtr cp, const Globals& G, double K, double cutoff,
+                                               float alpha_f, double cs, Search* searches, const fm::Tab& tb) {
 #pragma clang fp contract(off)
-    constexpr double RESOLUTION = EdgeSearch::RESOLUTION;
+    const ElementConsts& c0 = *(const ElementConsts*)cp;
     const int lane = threadIdx.x & 63;
+    const int half = lane >> 5, node = lane & 31;
     if (cs <= 0.) return 0.f;
+    const double alpha = (double)alpha_f;
     double qmin, qmax;
     if (a.process == 2) {  // dcs_get_range (pumas.c:11047-11056)
         qmin = PION_MASS + 0.5 * PION_MASS * PION_MASS / NUCLEON_MASS;
         qmax = K + a.mass - 0.5 * (NUCLEON_MASS + a.mass * a.mass / NUCLEON_MASS);
     } else {
         qmin = (a.process == 0) ? 0. : 4. * ELECTRON_MASS;
-        qmax = K + a.c->p_qoff;
+        qmax = K + c0.p_qoff;
     }
     double xmin = qmin / K;
     if (xmin < cutoff) xmin = cutoff;
-    xmin = log(xmin);
-    double xmax = log(qmax / K);
+    xmin = fm::log(xmin, tb);
+    double xmax = fm::log(qmax / K, tb);
     if (xmin >= xmax) return 0.f;
-    const EnvObjective f{a, K, (double)alpha};
-    int two = -2;
-    const double ends = f(lane == 0 ? xmin : xmax, &two);
-    double f0 = __shfl(ends, 0, 64);
-    double f1 = __shfl(ends, 1, 64);
-    if (xmax != xmax) {  // every further point is at NaN and has f1's value
-        const double fopt = f0 < f1 ? f0 : f1;
-        return (float)(-fopt);
-    }
-    if (f0 == 0.) {
-        EdgeSearch s{xmin, xmax, xmin, f0, true};
-        search(f, s);
-        xmin = s.edge;
-        f0 = s.value;
-    }
-    if (f1 == 0.) {
-        double x0, x1;
-        if (K >= 1E+01) {
-            // the first of xm - delta, delta = 1e-10 2^i, with f != 0
-            const double xm = exp(xmax);
-            double delta = RESOLUTION, x = xmax, fx = f1;
-            bool hit = false;
-            while (xm > delta && !hit) {
-                const int some = model_batch(a.process);
-                const double dl = ldexp(delta, lane < some ? lane : 0);
-                const double xl = log(xm - dl);
-                int points = -some;
-                const double v = f(xl, &points);
-                const unsigned long long in = __ballot(lane < some && xm > dl), nz = __ballot(v != 0.) & in;
-                const int at = nz ? __ffsll((long long)nz) - 1 : 63 - __clzll((long long)in);
-                hit = nz != 0;
-                x = __shfl(xl, at, 64);
-                fx = __shfl(v, at, 64);
-                delta = ldexp(delta, hit ? at : at + 1);
-            }
-            f1 = fx;
-            x0 = xmax = x;
-            x1 = log(xm - delta / 2);
+    const double wj = K / (K + a.mass);
+    const int batch = model_batch(a.process);
+    const double zeta = a.process == 1 ? pair_zeta(c0, a.mass, K, tb) : 0.;
+
+    // ENDS: the range ends and the midpoint; EDGE_LOW, BACKOFF, EDGE_HIGH: the
+    // ends' searches; MID: the midpoint between moved ends; PAIR: the two
+    // bracketing searches; SCAN and PEAK: the scan next to the upper end
+    enum { ENDS, EDGE_LOW, BACKOFF, EDGE_HIGH, MID, PAIR, SCAN, PEAK } phase = ENDS;
+    constexpr int N_SCAN = 7;
+    // the halves' searches live in LDS: not in registers across an evaluation
+    Search& s = searches[half];
+    double f0 = 0., f1 = 0., fmid = 0., fopt0 = 0., fopt1 = 0.;
+    double delta = RESOLUTION, exm = 0.;
+    bool moved = false;
+#pragma unroll 1
+    for (;;) {
+        const ElementConsts& c = row_consts(cp);
+        const double mass = hide(a.mass);
+        // this lane's point, and whether it is part of a tree or one of n points
+        double lnx;
+        int points = 0;
+        if (phase == ENDS) {
+            points = 3;
+            lnx = lane == 0 ? xmin : lane == 1 ? xmax : 0.5 * (xmin + xmax);
+        } else if (phase == MID) {
+            points = 1;
+            lnx = 0.5 * (xmin + xmax);
+        } else if (phase == BACKOFF) {
+            points = batch;
+            lnx = fm::log(exm - ldexp(delta, lane < points ? lane : 0), tb);
+        } else if (phase == SCAN) {
+            points = N_SCAN;
+            // xmax + log(1 - 10^-(i + 1))
+            lnx = xmax + fm::log(1. - pow(10., double(-((lane < N_SCAN ? lane : 0) + 1))), tb);
         } else {
-            x0 = xmin;
-            x1 = xmax;
+            // node + 1 in binary: below its leading one, the path to this lane's node
+            wave_lds_order();
+            Search mine = s;
+            const int depth = 31 - __clz(node + 1);
+#pragma unroll 1
+            for (int l = 4; l >= 0; l--)
+                if (l < depth) mine.next((node + 1) >> l & 1);
+            lnx = mine.point();
         }
-        EdgeSearch s{x0, x1, xmax, f1, false};
-        search(f, s);
-        xmax = s.edge;
-        f1 = s.value;
-    }
-    const double xm = 0.5 * (xmin + xmax);
-    const double fm = f.at(xm);
-    const double fopt0 = find_minimum(f, xmin, xm, f0, fm, RESOLUTION, 100);
-    double fopt1 = find_minimum(f, xm, xmax, fm, f1, RESOLUTION, 100);
-    if ((a.process == 1) && (K >= 1E+07)) {  // a sharp peak next to xmax: a logarithmic scan
-        constexpr int N_SCAN = 7;
-        const double xl = xmax + log(1. - pow(10., double(-((lane < N_SCAN ? lane : 0) + 1))));
-        int points = -N_SCAN;
-        const double fl = f(xl, &points);
-        double fmin = 0.;
-        int imin = -1;
-        for (int i = 0; i < N_SCAN; i++) {
-            const double fi = __shfl(fl, i, 64);
-            if (fi < fmin) {
-                imin = i;
-                fmin = fi;
+        // -DCS x^alpha there
+        const double x = fm::exp(lnx, tb);
+        const double q = x * K;
+        bool need;
+        double d = dcs_from_table(a, c, K, q, &need);
+        const bool asked = need;
+        if (points) {
+            need = need && lane < points;
+        } else {
+            need = need && !s.done() && node < 31;
+            const unsigned long long m = __ballot(need);
+            const uint32_t m0 = uint32_t(m), m1 = uint32_t(m >> 32);
+            // the model's points of as many levels (of each half's tree) as one batch takes
+            int l0 = 5, l1 = 5;
+            while (__popc(m0 & ((1u << ((1 << l0) - 1)) - 1)) + __popc(m1 & ((1u << ((1 << l1) - 1)) - 1)) > batch) {
+                if (m1 && (l1 > l0 || !m0))
+                    l1--;
+                else
+                    l0--;
+            }
+            need = need && node < (1 << (half ? l1 : l0)) - 1;
+        }
+        if (__ballot(need)) {
+            const double md = dcs_wave(a.process, c, G, mass, K, zeta, q, need, tb);
+            if (need) d = md;
+        }
+        const double v = -(d * wj) * (alpha == 0. ? 1. : fm::exp(alpha * lnx, tb));
+
+        if (!points) {  // walk the trees as far as their points have values
+            const int known = need || !asked;
+            int at = 0;
+            Search walk = s;
+#pragma unroll 1
+            for (int l = 0; l < 5; l++) {
+                const int from = 32 * half + at;
+                const double w = __shfl(v, from, 64);
+                const bool go = __shfl(known, from, 64) && at < 31 && !walk.done();
+                int bit = -1;
+                if (go) bit = walk.step(w);
+                at = bit < 0 ? 31 : 2 * at + 1 + bit;
+                at = at < 31 ? at : 31;
+            }
+            put(s, walk);
+        }
+
+        // what comes next (the same in every lane): `settled` counts the
+        // parts that are complete, the lower end, the upper end, the midpoint
+        // and the two searches
+        int settled = 0;
+        if (phase == ENDS) {
+            f0 = from_lane(v, 0);
+            f1 = from_lane(v, 1);
+            fmid = from_lane(v, 2);
+            if (xmax != xmax) {
+                const double fopt = f0 < f1 ? f0 : f1;
+                return (float)(-fopt);
+            }
+            if (f0 == 0.) {
+                moved = true;
+                put(s, new_search(half ? SEARCH_NONE : SEARCH_EDGE, xmin, xmax, 0., 0., 0., 1, xmin, f0));
+                phase = EDGE_LOW;
+            } else {
+                settled = 1;
+            }
+        } else if (phase == BACKOFF) {
+            // the first of exm - delta, delta = 1e-10 2^i, with f != 0
+            const unsigned long long in = __ballot(lane < points && exm > ldexp(delta, lane < points ? lane : 0));
+            const unsigned long long nz = __ballot(v != 0.) & in;
+            const int i = nz ? __ffsll((long long)nz) - 1 : 63 - __clzll((long long)in);
+            xmax = from_lane(lnx, i);
+            f1 = from_lane(v, i);
+            delta = ldexp(delta, nz ? i : i + 1);
+            if (!nz && exm > delta) continue;
+            put(s, new_search(half ? SEARCH_NONE : SEARCH_EDGE, xmax, fm::log(exm - delta / 2, tb), 0., 0., 0., 0, xmax, f1));
+            phase = EDGE_HIGH;
+        } else if (phase == MID) {
+            fmid = from_lane(v, 0);
+            settled = 3;
+        } else if (phase == SCAN) {
+            double fmin = 0.;
+            int imin = -1;
+            for (int i = 0; i < N_SCAN; i++) {
+                const double fi = from_lane(v, i);
+                if (fi < fmin) {
+                    imin = i;
+                    fmin = fi;
+                }
+            }
+            if (!((imin > 0) && (imin < N_SCAN - 1))) break;
+            const double xa = from_lane(lnx, imin - 1), xc = from_lane(lnx, imin + 1);
+            put(s, new_search(half ? SEARCH_NONE : SEARCH_BISECT, xa, xc, 0., 0., RESOLUTION * fabs(xc - xa), 0, from_lane(lnx, imin), fmin));
+            phase = PEAK;
+        }
+        if (settled == 0) {  // a search is under way
+            if (__ballot(!s.done())) continue;
+            const double xs = from_lane(s.xb, 0), fs = from_lane(s.fb, 0);
+            if (phase == EDGE_LOW) {
+                xmin = xs;
+                f0 = fs;
+                settled = 1;
+            } else if (phase == EDGE_HIGH) {
+                xmax = xs;
+                f1 = fs;
+                settled = 2;
+            } else if (phase == PAIR) {
+                fopt0 = fs;
+                fopt1 = from_lane(s.fb, 32);
+                settled = 4;
+            } else {  // PEAK
+                if (fs < fopt1) fopt1 = fs;
+                break;
             }
         }
-        if ((imin > 0) && (imin < N_SCAN - 1)) {
-            const double xa = __shfl(xl, imin - 1, 64), xb = __shfl(xl, imin, 64), xc = __shfl(xl, imin + 1, 64);
-            MinimumBisection s{xa, xb, xc, fmin, RESOLUTION * fabs(xc - xa), 0, 100};
-            search(f, s);
-            if (s.fb < fopt1) fopt1 = s.fb;
+        if (settled == 1) {
+            if (f1 == 0.) {
+                moved = true;
+                if (K >= 1E+01) {
+                    exm = fm::exp(xmax, tb);
+                    phase = BACKOFF;
+                    if (exm > delta) continue;
+                }
+                put(s, new_search(half ? SEARCH_NONE : SEARCH_EDGE, K >= 1E+01 ? xmax : xmin, K >= 1E+01 ? fm::log(exm - delta / 2, tb) : xmax, 0., 0.,
+                        0., 0, xmax, f1));
+                phase = EDGE_HIGH;
+                if (__ballot(!s.done())) continue;
+            }
+            settled = 2;
         }
+        if (settled == 2) {
+            phase = MID;
+            if (moved) continue;
+            settled = 3;
+        }
+        if (settled == 3) {
+            const double xm = 0.5 * (xmin + xmax);
+            const double lo = half ? xm : xmin, hi = half ? xmax : xm;
+            put(s, new_search(SEARCH_BRACKET, lo, hi, half ? fmid : f0, half ? f1 : fmid, RESOLUTION * fabs(hi - lo), 0, xm,
+                              fmid));
+            phase = PAIR;
+            continue;
+        }
+        if (!((a.process == 1) && (K >= 1E+07))) break;
+        phase = SCAN;
     }
     double fopt = (fopt0 < fopt1) ? fopt0 : fopt1;
     if (f0 < fopt) fopt = f0;
@@ -1097,29 +1255,34 @@ __device__ float envelope_max(const EnvRow& a, double K, double cutoff, float al
     return (float)(-fopt);
 }
 
+// The leading arguments of pumas_envelope_kernel, as the kernel-argument
+// segment holds them.
+struct EnvelopeArgs {
+    GridF g;
+    EnvelopeBlock blk;
+};
+
 // One 64-lane workgroup per (process, block element j, kinetic energy k) row
 // of the launch's element block; env[2 r + 1] of table row r.
-__global__ __launch_bounds__(64) void pumas_envelope_kernel(Grid g, ElementBlock blk, Globals G, int32_t e0,
+template <int WAVES>
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(WAVES))) void pumas_envelope_kernel(GridF g, EnvelopeBlock blk, Globals G, int32_t e0,
                                                             int32_t n_blk, int32_t n_el, double mass,
                                                             const double* __restrict__ Ks, int32_t n_K,
                                                             const float* __restrict__ table,
                                                             const double* __restrict__ csn, float* __restrict__ env) {
     __shared__ float xt[MAX_X];
     __shared__ float ra[2 * MAX_X], rb[2 * MAX_X];
-    __shared__ ElementConsts sc;  // the row's element and the globals, in LDS for the search's calls
-    __shared__ Globals sg;
+    __shared__ Search searches[2];
+    NOA_PUMAS_TABLES();
+    // pair production's rows first: they have the longest searches
     const int64_t b = blockIdx.x;
-    const int p = int(b / (int64_t(n_blk) * n_K));
+    const int p = (1 + int(b / (int64_t(n_blk) * n_K))) % 3;
     const int j = int((b / n_K) % n_blk);
     const int k = int(b % n_K);
     const int e = e0 + j;
     const int64_t pe = int64_t(p) * n_el + e;
     const int64_t r = pe * n_K + k;
-    for (int i = threadIdx.x; i < g.n; i += 64) xt[i] = (e == 0) ? 0.f : (float)g.x[i];
-    if (threadIdx.x == 0) {
-        sc = blk.e[j];
-        sg = G;
-    }
+    for (int i = threadIdx.x; i < g.n; i += 64) xt[i] = (e == 0) ? 0.f : g.x[i];
     // dcs_evaluate's energy bracket of the row's own energy (pumas.c:11352-11381)
     const double K = Ks[k];
     const float* rows = table + pe * n_K * 2 * g.n;
@@ -1140,8 +1303,6 @@ __global__ __launch_bounds__(64) void pumas_envelope_kernel(Grid g, ElementBlock
     }
     __syncthreads();
     EnvRow a;
-    a.c = &sc;
-    a.G = &sg;
     a.process = p;
     a.mass = mass;
     a.n = g.n;
@@ -1151,7 +1312,9 @@ __global__ __launch_bounds__(64) void pumas_envelope_kernel(Grid g, ElementBlock
     a.h0 = h0;
     a.h1 = h1;
     a.below = i0 < 0;
-    const float v = envelope_max(a, K, g.cutoff, env[2 * r], csn ? csn[r] : 1.);
+    const auto args = (const __attribute__((address_space(4))) EnvelopeArgs*)__builtin_amdgcn_kernarg_segment_ptr();
+    const ElementPtr cp = &args->blk.e[j];
+    const float v = envelope_max(a, cp, G, K, g.cutoff, env[2 * r], csn ? csn[r] : 1., searches, tb);
     if (threadIdx.x == 0) env[2 * r + 1] = v;
 }
 
@@ -1300,13 +1463,23 @@ int noa_pumas_dcs_table(const double* Z, const double* A, int32_t n_elements, do
                            envelope, n_pe, n_K);
         if (int rc = check_hip(hipGetLastError(), "pumas_alpha_fill_kernel")) return rc;
         // the envelope maxima, over the finished rows and exponents
-        for (int e0 = 0; e0 < n_elements; e0 += pumas::MAX_EL) {
-            const int n_blk = n_elements - e0 < pumas::MAX_EL ? n_elements - e0 : pumas::MAX_EL;
-            pumas::ElementBlock blk{};
+        pumas::GridF gf{};
+        gf.n = g.n;
+        gf.cutoff = g.cutoff;
+        for (int i = 0; i < g.n; i++) gf.x[i] = (float)g.x[i];
+        // (a grid has at most 2^31 - 1 workgroups)
+        const int per = int(std::min<int64_t>(pumas::MAX_ENV_EL, int64_t(0x7fffffff) / (int64_t(3) * n_K)));
+        for (int e0 = 0; e0 < n_elements; e0 += per) {
+            const int n_blk = std::min(n_elements - e0, per);
+            pumas::EnvelopeBlock blk{};
             for (int j = 0; j < n_blk; j++) blk.e[j] = pumas::make_element(Z[e0 + j], A[e0 + j], mass, G);
             const unsigned rows = unsigned(3 * n_blk * n_K);
-            hipLaunchKernelGGL(pumas::pumas_envelope_kernel, dim3(rows), dim3(64), 0, stream, g, blk, G, e0, n_blk,
-                               n_elements, mass, K, n_K, table, csn, envelope);
+            // three waves per SIMD (a few registers spilled) where the rows
+            // exceed the 2048 that two hold: 1963 against 2115 us for 48
+            // elements x 146 energies, 766 against 718 for 1 x 30
+            hipLaunchKernelGGL((rows > 2048 ? &pumas::pumas_envelope_kernel<3> : &pumas::pumas_envelope_kernel<2>),
+                               dim3(rows), dim3(64), 0, stream, gf, blk, G, e0, n_blk, n_elements, mass, K, n_K, table,
+                               csn, envelope);
             if (int rc = check_hip(hipGetLastError(), "pumas_envelope_kernel")) return rc;
         }
     }

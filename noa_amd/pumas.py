@@ -10,8 +10,8 @@ photonuclear (pumas.c:190-198).
 
 Z and A are sequences of floats (or host arrays), K a float64 GPU tensor; table is [3, n_el, n_K, n_x, 2] float32
 (ln DCS and PCHIP slope per node, PUMAS's table_DCS layout), x the n_x nodes
-ln(q / K), envelope [3, n_el, n_K, 2] (the exponent; entry 1, the envelope
-maximum, is 0: not computed).
+ln(q / K), envelope [3, n_el, n_K, 2] (the exponent and the envelope
+maximum).
 """
 from __future__ import annotations
 
