@@ -2,6 +2,7 @@
 // workload generator, and their C entry points (include/noa_dcs.h).
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cstdint>
 #include <type_traits>
 
@@ -59,6 +60,58 @@ __global__ __launch_bounds__(WG) __attribute__((amdgpu_waves_per_eu(EvalWaves<P>
     run_tile<P, TILE>(base, end, K, q, kernarg_consts(), o, s, fm::tab_from_block(fm_block));
 }
 
+// Maps that ask for closed forms only (bremsstrahlung, ionisation): one pair
+// per thread and step, no tile, 44 registers and 8 waves per SIMD. Bound: HBM
+// and VALU issue together. Measured on 2^24 pairs, FP64: bremsstrahlung 94 us
+// (4.3 TB/s; 107 by the tile kernel), ionisation 74 (94), both 155 (167); mixed
+// 57 (78), 59 (79), 83 (104).
+inline int64_t closed_grid(int64_t n) {
+    // four pairs per thread, up to 4096 workgroups, but at least one per CU
+    // and SIMD slot while there are pairs: 2^20 pairs 8.7 us with 1024
+    // workgroups, 10.1 with 4096; 2^24 94 with 4096, 99 with 1024
+    return std::min<int64_t>(4096, std::max((n + 4 * WG - 1) / (4 * WG), std::min<int64_t>(1024, (n + WG - 1) / WG)));
+}
+
+template <class P>
+__global__ __launch_bounds__(WG) void dcs_closed_kernel(const double* __restrict__ K, const double* __restrict__ q,
+                                                        int64_t n, DcsConsts, Outs<typename P::out_t> o) {
+    using out_t = typename P::out_t;
+    __shared__ __attribute__((aligned(fm::TABLE_LDS_ALIGN))) double fm_block[fm::TABLE_DOUBLES];
+    const ConstsPtr cp = kernarg_consts();
+    const int64_t stride = int64_t(gridDim.x) * WG;
+    int64_t g = int64_t(blockIdx.x) * WG + threadIdx.x;
+    double k = 1., qq = 0.;
+    if (g < n) {
+        k = K[g];
+        qq = q[g];
+    }
+    load_fm_tables(fm_block);
+    __syncthreads();
+    const fm::Tab t = fm::tab_from_block(fm_block);
+#pragma unroll 1
+    while (g < n) {
+        const DcsConsts& c = item_consts(cp);
+        const int64_t next = g + stride;
+        double k1 = 1., q1 = 0.;
+        if (next < n) {
+            k1 = K[next];
+            q1 = q[next];
+        }
+        bool in = true;
+        if constexpr (P::has_redo) in = P::in_range(k, qq, c);
+        if (o.b) store_stream(&o.b[g], in ? P::brems(k, qq, c, t) : out_t(F64::brems(k, qq, c, t)));
+        if (o.i) {
+            if constexpr (P::has_redo)
+                store_stream(&o.i[g], in ? P::ion(k, qq, c, t) : out_t(F64::ion_redo(k, qq, c, t)));
+            else
+                store_stream(&o.i[g], P::ion(k, qq, c, t));
+        }
+        g = next;
+        k = k1;
+        qq = q1;
+    }
+}
+
 // run_tile reads c in place through kernarg_consts(), which locates it by
 // TileKernelArgs: the kernel's leading parameters must stay (K, q, n, c).
 static_assert(std::is_same<decltype(&dcs_eval_kernel<F64, 2048>),
@@ -85,7 +138,12 @@ int launch_eval(const double* K, const double* q, int64_t n, const noa_dcs_eleme
                    : tile == 512  ? &dcs_eval_kernel<P, 512>
                    : tile == 1024 ? &dcs_eval_kernel<P, 1024>
                                   : &dcs_eval_kernel<P, 2048>;
-    hipLaunchKernelGGL(kernel, dim3(uint32_t(tiles)), dim3(WG), 0, stream, K, q, n, c, o);
+    int64_t grid = tiles;
+    if (!o.p && !o.ph) {
+        kernel = &dcs_closed_kernel<P>;
+        grid = closed_grid(n);
+    }
+    hipLaunchKernelGGL(kernel, dim3(uint32_t(grid)), dim3(WG), 0, stream, K, q, n, c, o);
     if (int rc = check_hip(hipGetLastError(), "dcs_eval_kernel launch")) return rc;
     return ok();
 }

@@ -81,6 +81,24 @@ def test_one_output_requested(big, n, p):
     assert _same(got, full[p][:n])
 
 
+@pytest.mark.parametrize("n", [1, 257, 262145, 5_000_001])
+def test_closed_forms_only(big, n):
+    """Bremsstrahlung and ionisation without the integrals, together and alone,
+    as in the full map; the mixed form within its 1e-5 of FP64 there (these two
+    have no branch on an FP32 value)."""
+    K, q, _ = big
+    full = _full(big, STANDARD_ROCK, MUON_MASS)
+    K, q = K[:n].contiguous(), q[:n].contiguous()
+    b, i = (torch.full((n,), -3.0, dtype=torch.float64, device=K.device) for _ in range(2))
+    dcs.eval_f64(K, q, STANDARD_ROCK, MUON_MASS, brems=b, ion=i)
+    assert _same(b, full[0][:n]) and _same(i, full[3][:n])
+    for p in (0, 3):
+        alone = [None] * 4
+        alone[p] = torch.full((n,), -3.0, dtype=torch.float32, device=K.device)
+        dcs.eval_f32mixed(K, q, STANDARD_ROCK, MUON_MASS, *alone)
+        assert_parity(alone[p].cpu().numpy(), full[p][:n].float().cpu().numpy(), 1e-5, f"process {p}")
+
+
 @pytest.fixture(scope="module")
 def mixed_full(big):
     K, q, _ = big
