@@ -163,7 +163,7 @@ inline auto vmap_threads(const Process& dcs_func, int threads) {
 inline auto map_threads(const Process& dcs_func, int threads) {
     return [dcs_func, threads](const Energies& kinetic_energies, const Energies& recoil_energies,
                                const AtomicElement& element, const ParticleMass& mass) {
-        const auto result = torch::zeros_like(kinetic_energies);
+        const auto result = torch::empty_like(kinetic_energies);
         vmap_threads(dcs_func, threads)(result, kinetic_energies, recoil_energies, element, mass);
         return result;
     };
@@ -355,8 +355,8 @@ inline void vmap_all(const std::array<Calculation, 4>& results, const Energies& 
 
 inline std::array<Calculation, 4> map_all(const Energies& kinetic_energies, const Energies& recoil_energies,
                                           const AtomicElement& element, const ParticleMass& mass) {
-    std::array<Calculation, 4> r{torch::zeros_like(kinetic_energies), torch::zeros_like(kinetic_energies),
-                                 torch::zeros_like(kinetic_energies), torch::zeros_like(kinetic_energies)};
+    std::array<Calculation, 4> r{torch::empty_like(kinetic_energies), torch::empty_like(kinetic_energies),
+                                 torch::empty_like(kinetic_energies), torch::empty_like(kinetic_energies)};
     vmap_all(r, kinetic_energies, recoil_energies, element, mass);
     return r;
 }
@@ -365,8 +365,8 @@ inline std::array<Calculation, 4> map_all(const Energies& kinetic_energies, cons
 inline std::array<Calculation, 4> map_all_f32mixed(const Energies& kinetic_energies, const Energies& recoil_energies,
                                                    const AtomicElement& element, const ParticleMass& mass) {
     const auto opts = kinetic_energies.options().dtype(torch::kFloat32);
-    std::array<Calculation, 4> r{torch::zeros(kinetic_energies.sizes(), opts), torch::zeros(kinetic_energies.sizes(), opts),
-                                 torch::zeros(kinetic_energies.sizes(), opts), torch::zeros(kinetic_energies.sizes(), opts)};
+    std::array<Calculation, 4> r{torch::empty(kinetic_energies.sizes(), opts), torch::empty(kinetic_energies.sizes(), opts),
+                                 torch::empty(kinetic_energies.sizes(), opts), torch::empty(kinetic_energies.sizes(), opts)};
     detail::eval_f32mixed(kinetic_energies, recoil_energies, element, mass, {&r[0], &r[1], &r[2], &r[3]});
     return r;
 }

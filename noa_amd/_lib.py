@@ -146,6 +146,31 @@ def last_error() -> str:
     return lib().noa_dcs_last_error().decode()
 
 
+def launch(fn, device_index: int, *args) -> None:
+    """Calls the C entry point fn(*args, stream) on the device, with torch's
+    current stream there, and raises on a non-zero status. Arguments are
+    plain values (addresses as integers): ctypes converts them by the
+    declared types. The device is switched only if it is not the current one."""
+    import torch
+    if torch.cuda.current_device() == device_index:
+        rc = fn(*args, raw_stream(device_index))
+    else:
+        with torch.cuda.device(device_index):
+            rc = fn(*args, raw_stream(device_index))
+    if rc != NOA_DCS_OK:
+        raise NoaDcsError(rc, last_error())
+
+
+def raw_stream(device_index: int) -> int:
+    """The handle of torch's current stream on a device (0.1 us through torch's
+    own accessor, 1.9 us through a torch.cuda.Stream object)."""
+    import torch
+    get = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+    if get is not None:
+        return get(device_index)
+    return torch.cuda.current_stream(device_index).cuda_stream
+
+
 def check(rc: int) -> None:
     if rc != NOA_DCS_OK:
         raise NoaDcsError(rc, last_error())

@@ -61,9 +61,7 @@ class BatchPlan:
     def launch(self) -> None:
         if self._handle is None:
             raise RuntimeError("plan was closed")
-        with torch.cuda.device(self.device):
-            stream = ctypes.c_void_p(torch.cuda.current_stream(self.device).cuda_stream)
-            _lib.check(_lib.lib().noa_dcs_batch_launch(self._handle, stream))
+        _lib.launch(_lib.lib().noa_dcs_batch_launch, self.K.get_device(), self._handle)
 
     def info(self) -> dict:
         t, w, u, n = ctypes.c_int32(), ctypes.c_int32(), ctypes.c_int32(), ctypes.c_int64()

@@ -51,7 +51,7 @@ torch::Tensor recoil_integral(int process, bool cel, torch::Tensor kinetic_energ
                               int Z, double mass, int min_points) {
     TORCH_CHECK(process >= 0 && process < 4, "process must be 0..3");
     const dcs::Process procs[4] = {dcs::bremsstrahlung, dcs::pair_production, dcs::photonuclear, dcs::ionisation};
-    auto result = torch::zeros_like(kinetic_energies);
+    auto result = torch::empty_like(kinetic_energies);
     dcs::vmap_integral(dcs::recoil_integral(procs[process], cel ? dcs::cel_integrand : dcs::del_integrand))(
         result, kinetic_energies, xlow, AtomicElement{A, I, Z}, mass, min_points);
     return result;
@@ -63,9 +63,9 @@ torch::Tensor recoil_integral(int process, bool cel, torch::Tensor kinetic_energ
 std::vector<torch::Tensor> coulomb_chain(torch::Tensor kinetic_energies, double A, double I, int Z, double mass) {
     const int64_t n = kinetic_energies.numel();
     const auto opt = kinetic_energies.options();
-    auto fCM = torch::zeros({n, 2}, opt), screen = torch::zeros({n, 9}, opt);
-    auto fspin = torch::zeros({n}, opt), invlambda = torch::zeros({n}, opt), G = torch::zeros({n, 2}, opt);
-    auto mu0 = torch::zeros({n}, opt), lb_h = torch::zeros({n}, opt);
+    auto fCM = torch::empty({n, 2}, opt), screen = torch::empty({n, 9}, opt);
+    auto fspin = torch::empty({n}, opt), invlambda = torch::empty({n}, opt), G = torch::empty({n, 2}, opt);
+    auto mu0 = torch::empty({n}, opt), lb_h = torch::empty({n}, opt);
     dcs::coulomb_data(fCM, screen, fspin, invlambda, kinetic_energies, AtomicElement{A, I, Z}, mass);
     dcs::coulomb_transport(G, screen, fspin, torch::tensor(1.0, torch::dtype(torch::kDouble)));  // as the reference test
     dcs::hard_scattering(mu0, lb_h, G.view({1, n, 2}), fCM.view({1, n, 2}), screen.view({1, n, 9}),
@@ -75,7 +75,7 @@ std::vector<torch::Tensor> coulomb_chain(torch::Tensor kinetic_energies, double 
 
 // dcs::soft_scattering.
 torch::Tensor soft_scattering(torch::Tensor kinetic_energies, double A, double I, int Z, double mass) {
-    auto result = torch::zeros_like(kinetic_energies);
+    auto result = torch::empty_like(kinetic_energies);
     dcs::soft_scattering(result, kinetic_energies, AtomicElement{A, I, Z}, mass);
     return result;
 }

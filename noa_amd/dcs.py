@@ -26,9 +26,9 @@ takes GPU tensors only.
 from __future__ import annotations
 
 import ctypes
+import math
 from types import SimpleNamespace
 
-import numpy as np
 import torch
 
 from . import _lib
@@ -113,11 +113,31 @@ def _check_output(r: torch.Tensor | None, K: torch.Tensor, dtype: torch.dtype) -
 
 
 def _ptr(t: torch.Tensor | None):
-    return None if t is None else ctypes.c_void_p(t.data_ptr())
+    return None if t is None else t.data_ptr()
 
 
-def _stream(K: torch.Tensor):
-    return ctypes.c_void_p(torch.cuda.current_stream(K.device).cuda_stream)
+def _launch(fn, t: torch.Tensor, *args) -> None:
+    """The C call fn(*args, stream) on t's device."""
+    _lib.launch(fn, t.get_device(), *args)
+
+
+def _eval_f64(K, q, element, mass, outs, threads: int = 0) -> None:
+    """The FP64 call with checked tensors; outs the four outputs or None."""
+    out = _lib.OutputsF64(*[None if r is None else r.data_ptr() for r in outs])
+    el = _element(element)
+    if K.is_cuda:
+        _launch(_lib.lib().noa_dcs_eval_f64, K, K.data_ptr(), q.data_ptr(), K.numel(), ctypes.byref(el), float(mass),
+                ctypes.byref(out))
+        return
+    _lib.check(_lib.lib().noa_dcs_eval_f64_host(K.data_ptr(), q.data_ptr(), K.numel(), ctypes.byref(el), float(mass),
+                                                ctypes.byref(out), int(threads)))
+
+
+def _eval_f32mixed(K, q, element, mass, outs) -> None:
+    out = _lib.OutputsF32(*[None if r is None else r.data_ptr() for r in outs])
+    el = _element(element)
+    _launch(_lib.lib().noa_dcs_eval_f32mixed, K, K.data_ptr(), q.data_ptr(), K.numel(), ctypes.byref(el), float(mass),
+            ctypes.byref(out))
 
 
 def eval_f64(K: torch.Tensor, q: torch.Tensor, element: AtomicElement, mass: float,
@@ -126,30 +146,20 @@ def eval_f64(K: torch.Tensor, q: torch.Tensor, element: AtomicElement, mass: flo
     GPU tensors; for CPU tensors the host build, serial for threads == 1,
     the OpenMP default team for 0, k threads for k > 1."""
     _check_inputs(K, q, allow_cpu=True)
-    for r in (brems, pair, photo, ion):
+    outs = (brems, pair, photo, ion)
+    for r in outs:
         _check_output(r, K, torch.float64)
-    out = _lib.OutputsF64(*(_ptr(r) for r in (brems, pair, photo, ion)))
-    el = _element(element)
-    if K.device.type == "cpu":
-        _lib.check(_lib.lib().noa_dcs_eval_f64_host(_ptr(K), _ptr(q), K.numel(), ctypes.byref(el), float(mass),
-                                                    ctypes.byref(out), int(threads)))
-        return
-    with torch.cuda.device(K.device):
-        _lib.check(_lib.lib().noa_dcs_eval_f64(_ptr(K), _ptr(q), K.numel(), ctypes.byref(el), float(mass),
-                                               ctypes.byref(out), _stream(K)))
+    _eval_f64(K, q, element, mass, outs, threads)
 
 
 def eval_f32mixed(K: torch.Tensor, q: torch.Tensor, element: AtomicElement, mass: float,
                   brems=None, pair=None, photo=None, ion=None) -> None:
     """Mixed-precision form: float64 inputs, float32 outputs."""
     _check_inputs(K, q)
-    for r in (brems, pair, photo, ion):
+    outs = (brems, pair, photo, ion)
+    for r in outs:
         _check_output(r, K, torch.float32)
-    out = _lib.OutputsF32(*(_ptr(r) for r in (brems, pair, photo, ion)))
-    el = _element(element)
-    with torch.cuda.device(K.device):
-        _lib.check(_lib.lib().noa_dcs_eval_f32mixed(_ptr(K), _ptr(q), K.numel(), ctypes.byref(el), float(mass),
-                                                    ctypes.byref(out), _stream(K)))
+    _eval_f32mixed(K, q, element, mass, outs)
 
 
 def _process(f) -> Process:
@@ -175,8 +185,11 @@ def _map(dcs_func: Process, threads: int):
 
     def run(kinetic_energies: torch.Tensor, recoil_energies: torch.Tensor, element: AtomicElement,
             mass: float) -> torch.Tensor:
-        result = torch.zeros_like(kinetic_energies)
-        _vmap(p, threads)(result, kinetic_energies, recoil_energies, element, mass)
+        _check_inputs(kinetic_energies, recoil_energies, allow_cpu=True)
+        result = torch.empty_like(kinetic_energies)  # written in full by the call
+        outs = [None] * 4
+        outs[p.id] = result
+        _eval_f64(kinetic_energies, recoil_energies, element, mass, outs, threads)
         return result
     return run
 
@@ -216,9 +229,11 @@ def _hip_namespace() -> SimpleNamespace:
         return run
 
     def gpu_map(p):
+        f = map(p)
+
         def run(kinetic_energies, recoil_energies, element, mass):
             _check_inputs(kinetic_energies, recoil_energies)
-            return map(p)(kinetic_energies, recoil_energies, element, mass)
+            return f(kinetic_energies, recoil_energies, element, mass)
         return run
 
     for p in PROCESSES:
@@ -231,14 +246,15 @@ def _hip_namespace() -> SimpleNamespace:
         eval_f64(kinetic_energies, recoil_energies, element, mass, *results)
 
     def map_all(kinetic_energies, recoil_energies, element, mass):
-        res = tuple(torch.zeros_like(kinetic_energies) for _ in range(4))
-        vmap_all(res, kinetic_energies, recoil_energies, element, mass)
+        _check_inputs(kinetic_energies, recoil_energies)
+        res = tuple(torch.empty_like(kinetic_energies) for _ in range(4))
+        _eval_f64(kinetic_energies, recoil_energies, element, mass, res)
         return res
 
     def map_all_f32mixed(kinetic_energies, recoil_energies, element, mass):
-        res = tuple(torch.zeros(kinetic_energies.shape, dtype=torch.float32, device=kinetic_energies.device)
-                    for _ in range(4))
-        eval_f32mixed(kinetic_energies, recoil_energies, element, mass, *res)
+        _check_inputs(kinetic_energies, recoil_energies)
+        res = tuple(torch.empty_like(kinetic_energies, dtype=torch.float32) for _ in range(4))
+        _eval_f32mixed(kinetic_energies, recoil_energies, element, mass, res)
         return res
 
     ns.update(vmap_all=vmap_all, map_all=map_all, map_all_f32mixed=map_all_f32mixed)
@@ -275,10 +291,8 @@ def recoil_integrals(kinetic_energies: torch.Tensor, xlow: float, element: Atomi
     d = _lib.OutputsF64(*(_ptr(r) for r in dels))
     c = _lib.OutputsF64(*(_ptr(r) for r in cels))
     el = _element(element)
-    with torch.cuda.device(K.device):
-        _lib.check(_lib.lib().noa_dcs_recoil_integrals_f64_noalloc(_ptr(K), K.numel(), float(xlow), ctypes.byref(el),
-                                                                   float(mass), int(min_points), ctypes.byref(d),
-                                                                   ctypes.byref(c), _stream(K)))
+    _launch(_lib.lib().noa_dcs_recoil_integrals_f64_noalloc, K, _ptr(K), K.numel(), float(xlow), ctypes.byref(el),
+            float(mass), int(min_points), ctypes.byref(d), ctypes.byref(c))
 
 
 def recoil_integral(dcs_func: Process, integrand: _Integrand):
@@ -314,8 +328,8 @@ def _check_f64(name: str, t, shape, device) -> None:
         raise ValueError(f"{name} must be on {device} (got {t.device}); there is no CPU path")
     if not t.is_contiguous():
         raise ValueError(f"{name} must be contiguous")
-    if shape is not None and t.numel() != int(np.prod(shape)):
-        raise ValueError(f"{name} must hold {int(np.prod(shape))} values as {tuple(shape)} (got {tuple(t.shape)})")
+    if shape is not None and t.numel() != math.prod(shape):
+        raise ValueError(f"{name} must hold {math.prod(shape)} values as {tuple(shape)} (got {tuple(t.shape)})")
 
 
 def coulomb_data(fCM: torch.Tensor, screening: torch.Tensor, fspin: torch.Tensor, invlambda: torch.Tensor,
@@ -329,9 +343,8 @@ def coulomb_data(fCM: torch.Tensor, screening: torch.Tensor, fspin: torch.Tensor
                            ("invlambda", invlambda, (n,))):
         _check_f64(name, t, shape, K.device)
     el = _element(element)
-    with torch.cuda.device(K.device):
-        _lib.check(_lib.lib().noa_dcs_coulomb_data_f64(_ptr(K), n, ctypes.byref(el), float(mass), _ptr(fCM),
-                                                       _ptr(screening), _ptr(fspin), _ptr(invlambda), _stream(K)))
+    _launch(_lib.lib().noa_dcs_coulomb_data_f64, K, _ptr(K), n, ctypes.byref(el), float(mass), _ptr(fCM),
+            _ptr(screening), _ptr(fspin), _ptr(invlambda))
 
 
 def coulomb_transport(coefficients: torch.Tensor, screening: torch.Tensor, fspin: torch.Tensor,
@@ -348,9 +361,8 @@ def coulomb_transport(coefficients: torch.Tensor, screening: torch.Tensor, fspin
     _check_f64("mu", mu, None, dev)
     if mu.numel() not in (1, n):
         raise ValueError(f"mu must hold 1 or {n} values (got {mu.numel()})")
-    with torch.cuda.device(dev):
-        _lib.check(_lib.lib().noa_dcs_coulomb_transport_f64(_ptr(screening), _ptr(fspin), _ptr(mu), mu.numel(), n,
-                                                            _ptr(coefficients), _stream(fspin)))
+    _launch(_lib.lib().noa_dcs_coulomb_transport_f64, fspin, _ptr(screening), _ptr(fspin), _ptr(mu), mu.numel(), n,
+            _ptr(coefficients))
 
 
 def hard_scattering(mu0: torch.Tensor, lb_h: torch.Tensor, coefficients: torch.Tensor, transform: torch.Tensor,
@@ -371,10 +383,8 @@ def hard_scattering(mu0: torch.Tensor, lb_h: torch.Tensor, coefficients: torch.T
                            ("transform", transform, (nel, nkin, 2)), ("screening", screening, (nel, nkin, 9)),
                            ("invlambdas", invlambdas, (nel, nkin)), ("fspins", fspins, (nel, nkin))):
         _check_f64(name, t, shape, dev)
-    with torch.cuda.device(dev):
-        _lib.check(_lib.lib().noa_dcs_hard_scattering_f64(nel, nkin, _ptr(coefficients), _ptr(transform),
-                                                          _ptr(screening), _ptr(invlambdas), _ptr(fspins),
-                                                          _ptr(mu0), _ptr(lb_h), _stream(invlambdas)))
+    _launch(_lib.lib().noa_dcs_hard_scattering_f64, invlambdas, nel, nkin, _ptr(coefficients), _ptr(transform),
+            _ptr(screening), _ptr(invlambdas), _ptr(fspins), _ptr(mu0), _ptr(lb_h))
 
 
 def soft_scattering(ms1: torch.Tensor, kinetic_energies: torch.Tensor, element: AtomicElement,
@@ -387,9 +397,8 @@ def soft_scattering(ms1: torch.Tensor, kinetic_energies: torch.Tensor, element: 
     nbytes = _lib.lib().noa_dcs_soft_scattering_workspace_bytes(K.numel())
     ws = torch.empty(max(nbytes, 8), dtype=torch.uint8, device=K.device)
     el = _element(element)
-    with torch.cuda.device(K.device):
-        _lib.check(_lib.lib().noa_dcs_soft_scattering_f64(_ptr(K), K.numel(), ctypes.byref(el), float(mass),
-                                                          _ptr(ms1), _ptr(ws), nbytes, _stream(K)))
+    _launch(_lib.lib().noa_dcs_soft_scattering_f64, K, _ptr(K), K.numel(), ctypes.byref(el), float(mass), _ptr(ms1),
+            _ptr(ws), nbytes)
 
 
 def relative_error(computed: torch.Tensor, expected: torch.Tensor) -> torch.Tensor:

@@ -24,11 +24,7 @@ from . import _lib
 
 
 def _ptr(t):
-    return None if t is None else ctypes.c_void_p(t.data_ptr())
-
-
-def _stream(t: torch.Tensor):
-    return ctypes.c_void_p(torch.cuda.current_stream(t.device).cuda_stream)
+    return None if t is None else t.data_ptr()
 
 
 def _check(name: str, t: torch.Tensor, device=None) -> None:
@@ -54,9 +50,8 @@ def dcs(process: int, Z: float, A: float, mass: float, K: torch.Tensor, q: torch
     if q.numel() != K.numel():
         raise ValueError("K and q must have equal numel")
     out = torch.empty_like(K)
-    with torch.cuda.device(K.device):
-        _lib.check(_lib.lib().noa_pumas_dcs_f64(int(process), float(Z), float(A), float(mass), _ptr(K), _ptr(q),
-                                                K.numel(), _ptr(out), _stream(K)))
+    _lib.launch(_lib.lib().noa_pumas_dcs_f64, K.get_device(), int(process), float(Z), float(A), float(mass), _ptr(K),
+                _ptr(q), K.numel(), _ptr(out))
     return out
 
 
@@ -81,9 +76,6 @@ def dcs_table(Z, A, mass: float, cutoff: float, K: torch.Tensor, fp64: bool = Fa
     x = torch.empty(n, dtype=torch.float32, device=K.device)
     env = torch.empty(3, n_el, n_K, 2, dtype=torch.float32, device=K.device)
     t64 = torch.empty(3, n_el, n_K, n, 2, dtype=torch.float64, device=K.device) if fp64 else None
-    with torch.cuda.device(K.device):
-        _lib.check(_lib.lib().noa_pumas_dcs_table(Zh.ctypes.data_as(ctypes.c_void_p), Ah.ctypes.data_as(ctypes.c_void_p),
-                                                  n_el, float(mass), float(cutoff), _ptr(K), n_K,
-                                                  _ptr(table), _ptr(x), _ptr(env), _ptr(t64),
-                                                  _ptr(csn) if csn is not None else None, _stream(K)))
+    _lib.launch(_lib.lib().noa_pumas_dcs_table, K.get_device(), Zh.ctypes.data, Ah.ctypes.data, n_el, float(mass),
+                float(cutoff), _ptr(K), n_K, _ptr(table), _ptr(x), _ptr(env), _ptr(t64), _ptr(csn))
     return (table, x, env, t64) if fp64 else (table, x, env)

@@ -273,7 +273,9 @@ class Surrogate:
         n = K.numel()
         dev = K.device
         if outputs is None:
-            outputs = tuple(torch.zeros(n, dtype=torch.float32, device=dev) for _ in range(NPROC))
+            # (every query of the offsets' range is written)
+            new = torch.empty if int(offsets[0]) == 0 and int(offsets[-1]) == n else torch.zeros
+            outputs = tuple(new(n, dtype=torch.float32, device=dev) for _ in range(NPROC))
         counters = self.workspace(n, dev) if workspace is None else workspace
         els = (_lib.Element * len(self.elements))(*[_lib.Element(e.A, e.I, e.Z) for e in self.elements])
         offs = (ctypes.c_int64 * len(offsets))(*[int(x) for x in offsets])
