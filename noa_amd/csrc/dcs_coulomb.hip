@@ -176,14 +176,35 @@ __device__ __forceinline__ void transport_one(const double* s, double fspin, dou
     G[1] = g1 * (2. * k);
 }
 
+// Screening parameters for which the quotients and logarithms of
+// restricted_cs have positive normal operands and results at any 0 <= mu < 1
+// (NaN fails): there a division is fm::div_rn by the correctly rounded
+// reciprocal and the logarithm fm::log_pos, the same values without the IEEE
+// sequence (whose VCC use serialises the poles) and without special arguments.
+__device__ __forceinline__ bool screening_ordinary(const double* s) {
+    return s[0] >= 1e-100 && s[0] <= 1e100 && s[1] >= 1e-100 && s[1] <= 1e100 && s[2] >= 1e-100 && s[2] <= 1e100;
+}
+
+template <bool Fast>
+__device__ __forceinline__ double cs_div(double a, double b) {
+    if constexpr (Fast) return fm::div_rn(a, b, fm::recip_pos(b));
+    else return a / b;
+}
+template <bool Fast>
+__device__ __forceinline__ double cs_log(double x, const fm::Tab& t) {
+    if constexpr (Fast) return fm::log_pos(x, t);
+    else return fm::log(x, t);
+}
+
 // dcs.hh:697-735.
+template <bool Fast>
 __device__ __forceinline__ double restricted_cs(double mu, double fspin, const double* s, const fm::Tab& t) {
 #pragma clang fp contract(off)
     if (mu >= 1.) return 0.;
     const double nuc = (s[1] < s[2]) ? s[1] : s[2];
     if (mu < 1E-08 * nuc) {
-        const double L = fm::log((s[0] + 1.) / (s[0] + mu), t);
-        const double r = (1. - mu) / ((s[0] + mu) * (s[0] + 1.));
+        const double L = cs_log<Fast>(cs_div<Fast>(s[0] + 1., s[0] + mu), t);
+        const double r = cs_div<Fast>(1. - mu, (s[0] + mu) * (s[0] + 1.));
         const double k = s[0] * (1. + s[0]);
         return k * (r - fspin * (L - s[0] * r));
     }
@@ -191,8 +212,8 @@ __device__ __forceinline__ double restricted_cs(double mu, double fspin, const d
 #pragma unroll
     for (int i = 0; i < 3; i++) {
         const double si = s[i];
-        const double L = fm::log((si + 1.) / (si + mu), t);
-        const double r = (1. - mu) / ((si + mu) * (si + 1.));
+        const double L = cs_log<Fast>(cs_div<Fast>(si + 1., si + mu), t);
+        const double r = cs_div<Fast>(1. - mu, (si + mu) * (si + 1.));
         const double I1 = L - si * r;
         const double J1 = mu - si * L;
         cs += s[3 + i] * (L - fspin * J1) + s[6 + i] * (r - fspin * I1);
@@ -210,21 +231,77 @@ struct Mixture {
     int64_t nel, nkin;
 };
 
-// dcs.hh:737-751 at kinetic-energy index i.
-__device__ __forceinline__ double objective(double cs_h, double mu, const Mixture& m, int64_t i, const fm::Tab& t) {
-#pragma clang fp contract(off)
-    double cs = 0.;
-    for (int64_t e = 0; e < m.nel; e++) {
-        const int64_t o = e * m.nkin + i;
-        cs += m.invlambda[o] * restricted_cs(mu, m.fspin[o], m.screen + NSF * o, t);
+// One kinetic energy of a mixture, shared by a group of L lanes (a power of
+// two): lane l of the group holds the values of elements l, L + l, ..., (E - 1)
+// L + l and evaluates those elements' terms; every sum over the elements is
+// then taken in element order from the group's lanes, so that all of them hold
+// the serial loop's value. Elements from L E on are read as they are needed.
+template <int L, int E>
+struct MixtureK {
+    const Mixture& m;
+    int64_t i;
+    int lane;            // this lane's place in the group
+    double s[E][NSF];    // its elements' screening parameters
+    double fspin[E], invlambda[E];
+    bool ordinary;       // screening_ordinary for all of them
+
+    __device__ __forceinline__ MixtureK(const Mixture& mix, int64_t idx, int l) : m(mix), i(idx), lane(l) {
+#pragma unroll
+        for (int k = 0; k < E; k++) load(k * L + l, s[k], &fspin[k], &invlambda[k]);
+        ordinary = true;
+#pragma unroll
+        for (int k = 0; k < E; k++) ordinary = ordinary && screening_ordinary(s[k]);
     }
-    return cs - cs_h;
-}
+
+    // (an element beyond the mixture reads the first one's values, unused)
+    __device__ __forceinline__ void load(int64_t e, double* sc, double* sp, double* il) const {
+        const int64_t o = (e < m.nel ? e : 0) * m.nkin + i;
+#pragma unroll
+        for (int k = 0; k < NSF; k++) sc[k] = m.screen[NSF * o + k];
+        *sp = m.fspin[o];
+        *il = m.invlambda[o];
+    }
+
+    // acc + the terms of elements first, first + 1, ... of the group's lanes
+    __device__ __forceinline__ double add_in_order(double acc, double term, int64_t first) const {
+#pragma clang fp contract(off)
+        if constexpr (L == 1) return first < m.nel ? acc + term : acc;
+#pragma unroll
+        for (int l = 0; l < L; l++) {
+            const double t = __shfl(term, l, L);
+            if (first + l < m.nel) acc += t;
+        }
+        return acc;
+    }
+
+    // dcs.hh:737-751
+    __device__ __forceinline__ double objective(double cs_h, double mu, const fm::Tab& t) const {
+#pragma clang fp contract(off)
+        double term[E];
+        if (ordinary && mu >= 0.) {
+#pragma unroll
+            for (int k = 0; k < E; k++) term[k] = invlambda[k] * restricted_cs<true>(mu, fspin[k], s[k], t);
+        } else {
+#pragma unroll
+            for (int k = 0; k < E; k++) term[k] = invlambda[k] * restricted_cs<false>(mu, fspin[k], s[k], t);
+        }
+        double cs = 0.;
+#pragma unroll
+        for (int k = 0; k < E; k++) cs = add_in_order(cs, term[k], k * L);
+        for (int64_t e0 = L * E; e0 < m.nel; e0 += L) {
+            double sc[NSF], sp, il;
+            load(e0 + lane, sc, &sp, &il);
+            cs = add_in_order(cs, il * restricted_cs<false>(mu, sp, sc, t), e0);
+        }
+        return cs - cs_h;
+    }
+};
 
 // numerics.hh:154-214, with the end values given; false where the
 // reference returns std::nullopt.
-__device__ bool ridders(double xa, double xb, double fa, double fb, double xtol, double rtol, uint32_t max_iter,
-                        double cs_h, const Mixture& m, int64_t i, const fm::Tab& t, double* root) {
+template <class M>
+__device__ __forceinline__ bool ridders(double xa, double xb, double fa, double fb, double xtol, double rtol,
+                                        uint32_t max_iter, double cs_h, const M& m, const fm::Tab& t, double* root) {
 #pragma clang fp contract(off)
     if (fa * fb > 0) return false;
     if (fa == 0) { *root = xa; return true; }
@@ -233,7 +310,7 @@ __device__ bool ridders(double xa, double xb, double fa, double fb, double xtol,
     for (uint32_t it = 0; it < max_iter; it++) {
         double dm = 0.5 * (xb - xa);
         const double xm = xa + dm;
-        const double fm_ = objective(cs_h, xm, m, i, t);
+        const double fm_ = m.objective(cs_h, xm, t);
         double sgn = (fb > fa) ? 1. : -1.;
         double dn = sgn * dm * fm_ / sqrt(fm_ * fm_ - fa * fb);
         sgn = (dn > 0.) ? 1. : -1.;
@@ -241,7 +318,7 @@ __device__ bool ridders(double xa, double xb, double fa, double fb, double xtol,
         dm = fabs(dm) - 0.5 * tol;
         if (dn < dm) dm = dn;
         const double xn = xm - sgn * dm;
-        const double fn = objective(cs_h, xn, m, i, t);
+        const double fn = m.objective(cs_h, xn, t);
         if (fn * fm_ < 0.0) {
             xa = xn; fa = fn; xb = xm; fb = fm_;
         } else if (fn * fa < 0.0) {
@@ -254,20 +331,22 @@ __device__ bool ridders(double xa, double xb, double fa, double fb, double xtol,
     return false;
 }
 
-// dcs.hh:753-838.
-__device__ void hard_one(const Mixture& m, int64_t i, double max_mu0, double* mu0_out, double* lb_h_out,
-                         const fm::Tab& t) {
+// dcs.hh:753-838. All lanes of the group get the result.
+template <int L, int E>
+__device__ __forceinline__ void hard_one(const Mixture& mix, int64_t i, int lane, double max_mu0, double* mu0_out,
+                                         double* lb_h_out, const fm::Tab& t) {
 #pragma clang fp contract(off)
+    const MixtureK<L, E> m(mix, i, lane);
     double invlb_m = 0., invlb1_m = 0., s_m_l = 0., s_m_h = 0.;
-    for (int64_t e = 0; e < m.nel; e++) {
-        const int64_t o = e * m.nkin + i;
-        const double invlb = m.invlambda[o];
-        const double scr = m.screen[NSF * o];
-        invlb_m += invlb * m.G[2 * o];
-        s_m_h += scr * invlb;
-        s_m_l += invlb / scr;
-        const double d = 1. / (m.fCM[2 * o] * (1. + m.fCM[1 + 2 * o]));
-        invlb1_m += invlb * m.G[1 + 2 * o] * d * d;
+    for (int64_t e0 = 0; e0 < mix.nel; e0 += L) {
+        const int64_t o = (e0 + lane < mix.nel ? e0 + lane : 0) * mix.nkin + i;
+        const double invlb = mix.invlambda[o];
+        const double scr = mix.screen[NSF * o];
+        const double d = 1. / (mix.fCM[2 * o] * (1. + mix.fCM[1 + 2 * o]));
+        invlb_m = m.add_in_order(invlb_m, invlb * mix.G[2 * o], e0);
+        s_m_h = m.add_in_order(s_m_h, scr * invlb, e0);
+        s_m_l = m.add_in_order(s_m_l, invlb / scr, e0);
+        invlb1_m = m.add_in_order(invlb1_m, invlb * mix.G[1 + 2 * o] * d * d, e0);
     }
     const double lb_m = 1. / invlb_m;
     double lb_h = fmin(EHS_OVER_MSC / invlb1_m, EHS_PATH_MAX);
@@ -278,24 +357,24 @@ __device__ void hard_one(const Mixture& m, int64_t i, double max_mu0, double* mu
         const double cs_h = 1. / lb_h;
         double mu_max = fmin(4. * mu0, 1.);
         double mu_min = 0.25 * mu0;
-        double fmax = objective(cs_h, mu_max, m, i, t), fmin_;
+        double fmax = m.objective(cs_h, mu_max, t), fmin_;
         if (fmax > 0.) {
             // as in the reference, mu0 and lb_h keep their estimates here
         } else {
-            fmin_ = objective(cs_h, mu_min, m, i, t);
+            fmin_ = m.objective(cs_h, mu_min, t);
             if (fmin_ < 0.) {
                 mu_max = mu_min;
                 fmax = fmin_;
                 mu_min = 0.;
-                fmin_ = objective(cs_h, mu_min, m, i, t);
+                fmin_ = m.objective(cs_h, mu_min, t);
             }
             if (mu_min < max_mu0) {
                 mu_max = fmin(mu_max, max_mu0);
                 double root;
-                if (ridders(mu_min, mu_max, fmin_, fmax, 1E-6 * mu0, 1E-6, 100, cs_h, m, i, t, &root)) mu0 = root;
+                if (ridders(mu_min, mu_max, fmin_, fmax, 1E-6 * mu0, 1E-6, 100, cs_h, m, t, &root)) mu0 = root;
             }
             mu0 = fmin(mu0, max_mu0);
-            lb_h = objective(cs_h, mu0, m, i, t) + cs_h;
+            lb_h = m.objective(cs_h, mu0, t) + cs_h;
             lb_h = (lb_h <= 1. / EHS_PATH_MAX) ? EHS_PATH_MAX : 1. / lb_h;
         }
     } else {
@@ -394,14 +473,26 @@ __global__ __launch_bounds__(256) void coulomb_transport_kernel(const double* __
     }
 }
 
+// What bounds it is the length of a K's chain of ~17 evaluations of the
+// objective, one after the other, each three poles per element. One thread per
+// K that read its elements' 11 values from memory in each evaluation took 96
+// us for 65,536 K of three elements (74 with the first element's values in
+// registers); held in registers, with the divisions and logarithms that
+// restricted_cs needs no special cases for, 44 us.
+template <int L, int E>
 __global__ __launch_bounds__(256) void hard_scattering_kernel(Mixture m, double max_mu0, double* __restrict__ mu0,
                                                               double* __restrict__ lb_h) {
     NOA_FM_PROLOGUE();
-    NOA_GRID_LOOP(i, m.nkin) {
+    const int lane = threadIdx.x % L;
+    // (the lanes of a group share i, so they leave the loop together)
+    NOA_GRID_LOOP(v, m.nkin * L) {
+        const int64_t i = v / L;
         double a, b;
-        hard_one(m, i, max_mu0, &a, &b, tab);
-        mu0[i] = a;
-        lb_h[i] = b;
+        hard_one<L, E>(m, i, lane, max_mu0, &a, &b, tab);
+        if (lane == 0) {
+            mu0[i] = a;
+            lb_h[i] = b;
+        }
     }
 }
 
@@ -541,6 +632,24 @@ __global__ __launch_bounds__(WG) __attribute__((amdgpu_waves_per_eu(SPLIT ? 3 : 
     }
 }
 
+// Lanes per K and elements per lane of the hard-scattering kernel for nel
+// elements at n energies. Few energies: one element per lane (up to 8 lanes),
+// the shortest chain. Once its waves exceed two per SIMD, as few lanes as hold
+// the mixture in registers (3 elements each), since every lane of a group
+// repeats the root search around its elements' terms. Measured (us, spread /
+// held): 3 elements 64 K 22 / 43, 65,536 K 54 / 44, 262,144 K 188 / 132; 5
+// elements 64 K 22 / 42, 65,536 K 90 / 63; 1 element 65,536 K 20.5.
+struct HardShape {
+    int lanes, elements;
+};
+inline HardShape hard_shape(int64_t nel, int64_t n) {
+    const int spread = nel <= 1 ? 1 : nel <= 2 ? 2 : nel <= 4 ? 4 : 8;
+    if (n * spread <= 131072 || nel > 12) return {spread, 1};
+    if (nel <= 3) return {1, int(nel)};
+    if (nel <= 6) return {2, nel == 4 ? 2 : 3};
+    return {4, nel <= 8 ? 2 : 3};
+}
+
 unsigned grid_for(int64_t n) { return unsigned(std::max<int64_t>(1, std::min<int64_t>(65536, (n + 255) / 256))); }
 
 }  // namespace noa_hip
@@ -587,7 +696,24 @@ int noa_dcs_hard_scattering_f64(int64_t nel, int64_t nkin, const double* G, cons
     // physics.hh:81-84, with the host libm as in the reference
     const double max_mu0 = 0.5 * (1. - std::cos(1E+00 * M_PI / 180.));
     const Mixture m{G, fCM, screening, invlambda, fspin, nel, nkin};
-    hipLaunchKernelGGL(hard_scattering_kernel, dim3(grid_for(nkin)), dim3(256), 0, stream, m, max_mu0, mu0, lb_h);
+    const HardShape shape = hard_shape(nel, nkin);
+    const int lanes = shape.lanes;
+    auto* kernel = &hard_scattering_kernel<1, 1>;
+    if (lanes == 1) {
+        if (shape.elements == 2) kernel = &hard_scattering_kernel<1, 2>;
+        if (shape.elements == 3) kernel = &hard_scattering_kernel<1, 3>;
+    } else if (lanes == 2) {
+        kernel = shape.elements == 1   ? &hard_scattering_kernel<2, 1>
+                 : shape.elements == 2 ? &hard_scattering_kernel<2, 2>
+                                       : &hard_scattering_kernel<2, 3>;
+    } else if (lanes == 4) {
+        kernel = shape.elements == 1   ? &hard_scattering_kernel<4, 1>
+                 : shape.elements == 2 ? &hard_scattering_kernel<4, 2>
+                                       : &hard_scattering_kernel<4, 3>;
+    } else {
+        kernel = &hard_scattering_kernel<8, 1>;
+    }
+    hipLaunchKernelGGL(kernel, dim3(grid_for(nkin * lanes)), dim3(256), 0, stream, m, max_mu0, mu0, lb_h);
     if (int rc = check_hip(hipGetLastError(), "hard_scattering_kernel")) return rc;
     return ok();
 }
