@@ -41,9 +41,11 @@ constexpr int IWG = 512;              // 8 waves
 constexpr int QW = 64;                // queries per wave pass (two 32-column N-tiles)
 constexpr int QWG = QW * (IWG / 64);  // 512 queries per workgroup pass
 
+// (16-byte aligned: a fragment is one ds_read_b128; at the arrays' natural
+// alignment the compiler split every one into four-byte pairs)
 struct MlpLds {
-    uint16_t frag[FRAG_TOTAL];
-    float bh[3][H];
+    alignas(16) uint16_t frag[FRAG_TOTAL];
+    alignas(16) float bh[3][H];
     float b5[OUT];
     float w1[H * IN];
     float b1[H];
