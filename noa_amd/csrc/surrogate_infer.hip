@@ -21,6 +21,7 @@
 #include <cmath>
 #include <cstdint>
 #include <cstring>
+#include <functional>
 #include <vector>
 
 #include "capi_util.hh"
@@ -420,6 +421,63 @@ int n_cus() {
     return std::max(1, n);
 }
 
+// Items shorter than SUR_ITEM are cut only while this many per CU hold the
+// call: so the list's reserved length does not fall as calls grow.
+constexpr int64_t SHORT_ITEMS_PER_CU = 4;
+
+// Queries per work item. One workgroup per CU takes items in turn, so a call
+// lasts as long as its busiest CU: with items of 4096 a call of 2^18 queries
+// keeps 96 of 256 CUs busy and one of 2^21 lasts three rounds for two and a
+// half. Each candidate's longest queue is added up as the kernel will form it
+// (whole items in rounds, then the remainders, longest first, to the emptiest
+// queue), with ITEM_COST queries' time for an item's start and its partly
+// filled last exact waves; the shortest one is taken, the longer item on a
+// tie. Measured, 48 elements, tolerance 3e-2, items of 4096 in element order
+// against this rule (us): 2^16 queries 127 / 83 (items of 512), 2^18 266 / 138
+// (1536), 2^20 367 / 325 (4096, remainders last), 2^21 638 / 562 (3072),
+// 2^22 1042 / 999 (4096). An ITEM_COST below 256 picks items of 256, which
+// leave half the waves of a pass idle (2^16: 112 us); above 400 nothing moves.
+constexpr int64_t ITEM_COST = 400;
+
+int64_t item_length(const int64_t* offsets, int n_elements, int64_t cus) {
+    constexpr int64_t lengths[] = {4096, 3584, 3072, 2560, 2048, 1536, 1024, 512, 256};
+    static_assert(lengths[0] == SUR_ITEM, "the longest item fills the lists");
+    int64_t best = SUR_ITEM, best_cost = INT64_MAX;
+    std::vector<int64_t> rest, queue;
+    for (const int64_t len : lengths) {
+        int64_t whole = 0;
+        rest.clear();
+        for (int e = 0; e < n_elements; e++) {
+            const int64_t n = offsets[e + 1] - offsets[e];
+            whole += n / len;
+            if (n % len) rest.push_back(n % len);
+        }
+        if (whole + int64_t(rest.size()) > SHORT_ITEMS_PER_CU * cus) break;
+        const int64_t item = len + ITEM_COST, low = whole / cus * item, busier = whole % cus;
+        int64_t cost = busier ? low + item : low;
+        if (!rest.empty() && int64_t(rest.size()) <= cus - busier) {
+            cost = std::max(cost, low + *std::max_element(rest.begin(), rest.end()) + ITEM_COST);
+        } else if (!rest.empty()) {
+            std::sort(rest.begin(), rest.end(), std::greater<int64_t>());
+            queue.assign(size_t(cus), low);
+            std::fill_n(queue.begin(), busier, low + item);
+            // a heap whose front is the emptiest queue
+            std::make_heap(queue.begin(), queue.end(), std::greater<int64_t>());
+            for (const int64_t r : rest) {
+                std::pop_heap(queue.begin(), queue.end(), std::greater<int64_t>());
+                queue.back() += r + ITEM_COST;
+                std::push_heap(queue.begin(), queue.end(), std::greater<int64_t>());
+            }
+            cost = *std::max_element(queue.begin(), queue.end());
+        }
+        if (cost < best_cost) {
+            best = len;
+            best_cost = cost;
+        }
+    }
+    return best;
+}
+
 }  // namespace
 
 extern "C" {
@@ -461,11 +519,22 @@ int noa_dcs_surrogate_eval(noa_dcs_mlp* net, const noa_dcs_element* elements, co
         els[e].c = make_consts(elements[e].A, elements[e].I, elements[e].Z, mass);
         els[e].ln_a = float(std::log(elements[e].A));
     }
-    std::vector<SurItem> items;
-    for (int e = 0; e < n_elements; e++)
-        for (int64_t a = offsets[e]; a < offsets[e + 1]; a += SUR_ITEM)
-            items.push_back(SurItem{a, int32_t(std::min<int64_t>(SUR_ITEM, offsets[e + 1] - a)), e});
-    const size_t need = els.size() * sizeof(SurElem) + items.size() * sizeof(SurItem) + 256;
+    // whole items first, the elements' remainders after them, longest first:
+    // the workgroups take them in this order
+    const int64_t per = item_length(offsets, n_elements, n_cus());
+    std::vector<SurItem> items, rest;
+    for (int e = 0; e < n_elements; e++) {
+        int64_t a = offsets[e];
+        for (; offsets[e + 1] - a >= per; a += per) items.push_back(SurItem{a, int32_t(per), e});
+        if (a < offsets[e + 1]) rest.push_back(SurItem{a, int32_t(offsets[e + 1] - a), e});
+    }
+    std::stable_sort(rest.begin(), rest.end(), [](const SurItem& x, const SurItem& y) { return x.len > y.len; });
+    items.insert(items.end(), rest.begin(), rest.end());
+    // room that grows with the call, whatever the item length: a smaller call
+    // after a larger one finds the scratch large enough
+    const int64_t most_items =
+        std::max(total / SUR_ITEM, SHORT_ITEMS_PER_CU * int64_t(n_cus())) + n_elements;
+    const size_t need = els.size() * sizeof(SurElem) + size_t(most_items) * sizeof(SurItem) + 256;
     if (need > net->scratch_bytes) {
         if (net->scratch) (void)hipFree(net->scratch);
         net->scratch = nullptr;
