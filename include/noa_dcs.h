@@ -207,7 +207,7 @@ int64_t noa_dcs_soft_scattering_workspace_bytes(int64_t n);
 int noa_dcs_soft_scattering_f64(const double* K, int64_t n, const noa_dcs_element* element, double mass,
                                 double* result, void* workspace, int64_t workspace_bytes, hipStream_t stream);
 
-/* ---- batched uneven elements: one persistent launch, captured in a hipGraph ----
+/* ---- batched uneven elements: one launch, captured in a hipGraph ----
  * Element e owns pairs [offsets[e], offsets[e+1]) of the concatenated K, q
  * and output arrays. The reference has no batched form: a caller loops
  * dcs::vmap over elements (src/noa/pms/dcs.hh:35-48). The plan binds the
@@ -220,8 +220,8 @@ typedef struct noa_dcs_batch noa_dcs_batch;
 
 typedef struct noa_dcs_batch_config {
     int32_t precision;      /* NOA_DCS_PREC_F64 or NOA_DCS_PREC_F32MIXED */
-    int32_t tile;           /* pairs per work item; 0 = autotuned */
-    int32_t waves_per_cu;   /* persistent workgroups per CU; 0 = autotuned */
+    int32_t tile;           /* most pairs per work item; 0 = autotuned */
+    int32_t waves_per_cu;   /* most workgroups resident per CU; 0 = what the kernel's registers and LDS allow */
     int32_t use_graph;      /* 1 = capture the launch in a hipGraph */
     const char* tune_cache; /* autotune cache file, NULL = none */
     int32_t unroll;         /* unroll of the integrals' node loops, 1 or 2; 0 = autotuned */

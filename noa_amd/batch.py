@@ -1,4 +1,4 @@
-"""Batched multi-element evaluation: one persistent launch replayed from a hipGraph.
+"""Batched multi-element evaluation: one launch replayed from a hipGraph.
 
     plan = BatchPlan(elements, offsets, K, q, MUON_MASS, precision="f64")
     plan.launch()                 # replays the captured graph on the current stream

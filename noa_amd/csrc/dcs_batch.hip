@@ -1,18 +1,24 @@
 // Batched DCS evaluation over many elements with uneven pair counts, as one
-// persistent launch replayed from a hipGraph.
+// launch replayed from a hipGraph.
 //
 // The reference evaluates one element per adaptor call (src/noa/pms/dcs.hh:35-48);
 // a material table of 48 elements with 2^10..2^20 pairs each would be 48
 // launches, most of them far too small to fill 256 CUs. Here the pairs of all
 // elements are cut into work items (element, begin, len <= TILE), ordered
-// longest first (LPT), and a persistent grid of (CUs x workgroups per CU)
-// drains them through one global atomic counter. Each item's element
+// longest first, one workgroup each: the hardware hands the workgroups out in
+// this order as slots come free, which is list scheduling. An item's element
 // constants are read with scalar loads from a read-only table; the tile
 // itself runs the same phased, compacting evaluation as the single-element
-// kernel. The counter is reset by
-// a one-thread kernel inside the same graph (no memset node), so a replay is
-// self-contained. Tile size and workgroups per CU are picked by timing the
-// candidates on the actual batch, cached per (device, precision, shape).
+// kernel. Tile size and node-loop unroll are picked by timing the candidates
+// on the actual batch, cached per (device, precision, shape).
+//
+// Measured on MI355X (us; a persistent grid that took equal items from an
+// atomic counter, reset by a second kernel, against this), 48 elements of
+// 2^10..2^20 pairs, 6.8e6 in all: FP64 545 / 508, mixed 429 / 365; 20 of
+// 2^10..2^17, 4.1e5: 94 / 61, 93 / 55; 12 of 2^10..2^14, 6.6e4, in groups of
+// 64 pairs: see SMALL_BATCH. The persistent loop held more constants across
+// items than the SGPRs take (93 to 143 spills) and the mixed form could not
+// run at the 5 waves per SIMD that it runs at here.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -21,12 +27,14 @@
 #include <cstring>
 #include <mutex>
 #include <string>
+#include <type_traits>
 #include <vector>
 
 #include "capi_util.hh"
 #include "dcs_consts.hh"
 #include "dcs_f32m.hh"
 #include "dcs_f64.hh"
+#include "dcs_small.hh"
 #include "dcs_tile.hh"
 
 namespace noa_hip {
@@ -37,44 +45,45 @@ struct WorkItem {
     int32_t element;
 };
 
-__global__ void reset_counter_kernel(uint32_t* counter) { *counter = 0u; }
+// The item list and the element table are read-only for the whole launch:
+// addressed through the constant address space their fields are scalar loads.
+using ItemPtr = const __attribute__((address_space(4))) WorkItem*;
 
-// Minimum resident waves per SIMD asked of the compiler. Left free, the
-// item loop pushes the mixed form to 136 VGPRs (3 waves/SIMD); bounded to
-// 4 it fits 128 with no scratch. The unrolled FP64 form outgrows 256 VGPRs
+// Minimum resident waves per SIMD asked of the compiler, as for the
+// single-element kernel. The unrolled FP64 form outgrows 256 VGPRs
 // (1 wave/SIMD, spilling into the accumulator registers); bounded to 2 or 4
 // it spills 1.1-1.6 KB per lane to scratch instead, so it stays unbounded.
-template <class P>
+template <class P, int TILE>
 struct BatchMinWaves {
-    static constexpr int value = 4;
-};
-template <>
-struct BatchMinWaves<F64N<2>> {
-    static constexpr int value = 1;
+    static constexpr int value = std::is_same<P, F64N<2>>::value ? 1
+                                 : TILE == 4096                  ? (P::has_redo ? 3 : 2)  // what the tile's LDS allows
+                                 : std::is_same<P, F32MN<1>>::value ? 5
+                                                                    : 4;
 };
 
 template <class P, int TILE>
-__global__ __launch_bounds__(WG) __attribute__((amdgpu_waves_per_eu(BatchMinWaves<P>::value))) void dcs_batch_kernel(
+__global__ __launch_bounds__(WG) __attribute__((amdgpu_waves_per_eu(BatchMinWaves<P, TILE>::value))) void dcs_batch_kernel(
     const double* __restrict__ K, const double* __restrict__ q, const DcsConsts* __restrict__ consts,
-    const WorkItem* __restrict__ items, uint32_t n_items, uint32_t* counter, Outs<typename P::out_t> o) {
+    const WorkItem* __restrict__ items, Outs<typename P::out_t> o) {
     __shared__ TileLists<TILE, P::has_redo> s;
-    __shared__ uint32_t s_item;
     __shared__ __attribute__((aligned(fm::TABLE_LDS_ALIGN))) double fm_block[fm::TABLE_DOUBLES];
-    load_fm_tables(fm_block);  // published by the barrier below
-    const fm::Tab tab = fm::tab_from_block(fm_block);
-    for (;;) {
-        if (threadIdx.x == 0) s_item = atomicAdd(counter, 1u);
-        __syncthreads();
-        // wave-uniform item index: the item and its element constants are
-        // then read with scalar loads into SGPRs, as kernel arguments are
-        const uint32_t it = __builtin_amdgcn_readfirstlane(s_item);
-        if (it >= n_items) break;  // workgroup-uniform exit, reached by every workgroup
-        const WorkItem w = items[it];
-        // the element table is read-only for the whole launch: address it
-        // through the constant address space so its fields stay scalar loads
-        run_tile<P, TILE>(w.begin, w.begin + w.len, K, q, (ConstsPtr)(consts + w.element), o, s,
-                          tab);  // ends with a barrier
-    }
+    load_fm_tables(fm_block);  // published by run_tile's first barrier
+    const WorkItem& w = *(const WorkItem*)((ItemPtr)items + blockIdx.x);
+    run_tile<P, TILE>(w.begin, w.begin + w.len, K, q, (ConstsPtr)(consts + w.element), o, s,
+                      fm::tab_from_block(fm_block));
+}
+
+// Small batches: items of at most SMALL_TILE pairs, spread over lanes by
+// quadrature node (dcs_small.hh).
+template <class OutT>
+__global__ __launch_bounds__(WG) void dcs_small_batch_kernel(const double* __restrict__ K,
+                                                             const double* __restrict__ q,
+                                                             const DcsConsts* __restrict__ consts,
+                                                             const WorkItem* __restrict__ items, Outs<OutT> o) {
+    __shared__ SmallLds s;
+    __shared__ __attribute__((aligned(fm::TABLE_LDS_ALIGN))) double fm_block[fm::TABLE_DOUBLES];
+    const WorkItem& w = *(const WorkItem*)((ItemPtr)items + blockIdx.x);
+    run_small<OutT>(w.begin, w.begin + w.len, K, q, (ConstsPtr)(consts + w.element), o, s, fm_block);
 }
 
 }  // namespace noa_hip
@@ -84,8 +93,12 @@ using namespace noa_hip;
 struct noa_dcs_batch {
     int precision = 0;
     int tile = 0;
-    int wpc = 0;
+    int wpc = 0;             // workgroups resident per CU
+    bool limit_wpc = false;  // at most wpc, as asked for; otherwise what registers and LDS allow
     int unroll = 1;
+    bool small = false;  // items of SMALL_TILE pairs, dcs_small_batch_kernel
+    const void* kernel = nullptr;
+    size_t lds_pad = 0;
     int use_graph = 1;
     int n_cu = 0;
     int device = 0;
@@ -98,7 +111,6 @@ struct noa_dcs_batch {
     DcsConsts* d_consts = nullptr;
     WorkItem* d_items = nullptr;
     uint32_t n_items = 0;
-    uint32_t* d_counter = nullptr;
     hipGraph_t graph = nullptr;
     hipGraphExec_t exec = nullptr;
 };
@@ -107,41 +119,87 @@ namespace {
 
 std::mutex g_tune_mutex;
 
-template <class P, int TILE>
-hipError_t launch_batch(noa_dcs_batch* b, hipStream_t stream) {
-    using out_t = typename P::out_t;
-    Outs<out_t> o{static_cast<out_t*>(b->outs[0]), static_cast<out_t*>(b->outs[1]), static_cast<out_t*>(b->outs[2]),
-                  static_cast<out_t*>(b->outs[3])};
-    hipLaunchKernelGGL(reset_counter_kernel, dim3(1), dim3(1), 0, stream, b->d_counter);
-    const uint32_t grid = uint32_t(b->n_cu) * uint32_t(b->wpc);
-    hipLaunchKernelGGL((dcs_batch_kernel<P, TILE>), dim3(grid), dim3(WG), 0, stream, b->K, b->q, b->d_consts,
-                       b->d_items, b->n_items, b->d_counter, o);
-    return hipGetLastError();
-}
+// A batch of up to this many pairs runs in items of 64, as maps of these
+// sizes do (dcs_eval.hip, eval_tile): 6.6e4 pairs of 12 elements take 20 us, a
+// replay's 5 included (32 in items of 512, 72 in tiles of 1024).
+constexpr int64_t SMALL_BATCH = 200000;
 
 template <class P>
-hipError_t launch_tile(noa_dcs_batch* b, hipStream_t stream) {
-    switch (b->tile) {
-        case 1024: return launch_batch<P, 1024>(b, stream);
-        case 2048: return launch_batch<P, 2048>(b, stream);
-        default: return launch_batch<P, 4096>(b, stream);
-    }
+const void* tile_kernel(int tile) {
+    return tile == 1024   ? reinterpret_cast<const void*>(&dcs_batch_kernel<P, 1024>)
+           : tile == 2048 ? reinterpret_cast<const void*>(&dcs_batch_kernel<P, 2048>)
+                          : reinterpret_cast<const void*>(&dcs_batch_kernel<P, 4096>);
 }
+
+// The plan's kernel for its tile and unroll, and how many of its workgroups a
+// CU holds. A limit asked for is kept by LDS that the kernel does not use.
+int choose_kernel(noa_dcs_batch* b) {
+    if (b->precision == NOA_DCS_PREC_F64)
+        b->kernel = b->small         ? reinterpret_cast<const void*>(&dcs_small_batch_kernel<double>)
+                    : b->unroll == 2 ? tile_kernel<F64N<2>>(b->tile)
+                                     : tile_kernel<F64N<1>>(b->tile);
+    else
+        b->kernel = b->small         ? reinterpret_cast<const void*>(&dcs_small_batch_kernel<float>)
+                    : b->unroll == 2 ? tile_kernel<F32MN<2>>(b->tile)
+                                     : tile_kernel<F32MN<1>>(b->tile);
+    b->lds_pad = 0;
+    if (b->limit_wpc) {
+        int per_block = 0, per_cu = 0;
+        hipFuncAttributes attr;
+        if (int rc = check_hip(hipFuncGetAttributes(&attr, b->kernel), "hipFuncGetAttributes")) return rc;
+        if (int rc = check_hip(hipDeviceGetAttribute(&per_block, hipDeviceAttributeMaxSharedMemoryPerBlock, b->device),
+                               "hipDeviceGetAttribute"))
+            return rc;
+        if (int rc = check_hip(hipDeviceGetAttribute(
+                                   &per_cu, hipDeviceAttributeMaxSharedMemoryPerMultiprocessor, b->device),
+                               "hipDeviceGetAttribute"))
+            return rc;
+        const int64_t want = std::min<int64_t>(per_block, per_cu / (b->wpc + 1) + 1024);
+        b->lds_pad = size_t(std::max<int64_t>(0, want - int64_t(attr.sharedSizeBytes)));
+        return NOA_DCS_OK;
+    }
+    if (int rc = check_hip(hipOccupancyMaxActiveBlocksPerMultiprocessor(&b->wpc, b->kernel, WG, 0),
+                           "hipOccupancyMaxActiveBlocksPerMultiprocessor"))
+        return rc;
+    b->wpc = std::max(1, b->wpc);
+    return NOA_DCS_OK;
+}
+
+// (both output types: four pointers)
+static_assert(sizeof(Outs<double>) == sizeof(Outs<float>) && sizeof(Outs<double>) == 4 * sizeof(void*),
+              "noa_dcs_batch::outs stands for either");
 
 hipError_t launch_direct(noa_dcs_batch* b, hipStream_t stream) {
-    if (b->precision == NOA_DCS_PREC_F64)
-        return b->unroll == 2 ? launch_tile<F64N<2>>(b, stream) : launch_tile<F64N<1>>(b, stream);
-    return b->unroll == 2 ? launch_tile<F32MN<2>>(b, stream) : launch_tile<F32MN<1>>(b, stream);
+    if (b->n_items == 0) return hipSuccess;
+    void* args[] = {&b->K, &b->q, &b->d_consts, &b->d_items, &b->outs};
+    return hipLaunchKernel(b->kernel, dim3(b->n_items), dim3(WG), args, b->lds_pad, stream);
 }
 
-// Work items of `tile` pairs (the last of each element shorter), longest first.
-std::vector<WorkItem> make_items(const std::vector<int64_t>& offsets, int tile) {
-    std::vector<WorkItem> items;
+// Work items, longest first. Tiles are `tile` pairs while much is left, then
+// shorten with what is left, to two even shares of the 4 slots per CU and no
+// less than `least`, so that the last ones end together. Measured (us;
+// equal tiles against this): 4.1e5 pairs 69 / 61, 3.8e6 326 / 301, 1.2e7 903 /
+// 895, mixed 636 / 618; `least` of 256 is slower from 4e5 pairs on, as the
+// tiles of a map are (dcs_eval.hip, eval_tile).
+std::vector<WorkItem> make_items(const noa_dcs_batch* b) {
+    const std::vector<int64_t>& offsets = b->offsets;
     const int n_el = int(offsets.size()) - 1;
-    for (int e = 0; e < n_el; e++) {
-        for (int64_t a = offsets[e]; a < offsets[e + 1]; a += tile) {
-            const int64_t len = std::min<int64_t>(tile, offsets[e + 1] - a);
+    int64_t left = offsets.back() - offsets.front();
+    const int64_t least = left <= 300000 ? 256 : 512, slots = 4 * int64_t(b->n_cu);
+    std::vector<int32_t> order(n_el);
+    for (int e = 0; e < n_el; e++) order[e] = e;
+    std::stable_sort(order.begin(), order.end(), [&](int32_t x, int32_t y) {
+        return offsets[x + 1] - offsets[x] > offsets[y + 1] - offsets[y];
+    });
+    std::vector<WorkItem> items;
+    for (const int32_t e : order) {
+        for (int64_t a = offsets[e]; a < offsets[e + 1];) {
+            const int64_t share = (2 * left / slots + 63) / 64 * 64;
+            const int64_t most = b->small ? SMALL_TILE : std::min<int64_t>(b->tile, std::max(least, share));
+            const int64_t len = std::min(most, offsets[e + 1] - a);
             items.push_back(WorkItem{a, int32_t(len), e});
+            a += len;
+            left -= len;
         }
     }
     std::stable_sort(items.begin(), items.end(), [](const WorkItem& x, const WorkItem& y) { return x.len > y.len; });
@@ -149,8 +207,9 @@ std::vector<WorkItem> make_items(const std::vector<int64_t>& offsets, int tile) 
 }
 
 int upload_items(noa_dcs_batch* b) {
-    const std::vector<WorkItem> items = make_items(b->offsets, b->tile);
-    if (items.size() > 0xffffffffull) return fail(NOA_DCS_ERANGE, "too many work items");
+    if (int rc = choose_kernel(b)) return rc;
+    const std::vector<WorkItem> items = make_items(b);
+    if (items.size() > 0x7fffffffull) return fail(NOA_DCS_ERANGE, "too many work items");
     if (b->d_items) (void)hipFree(b->d_items);
     b->d_items = nullptr;
     b->n_items = uint32_t(items.size());
@@ -167,7 +226,7 @@ std::string tune_key(const noa_dcs_batch* b) {
     int lg = 0;
     while ((int64_t(1) << (lg + 1)) <= total) lg++;
     char buf[256];
-    snprintf(buf, sizeof(buf), "%s|cu%d|prec%d|el%zu|log2n%d|tile-wpc-unroll", prop.gcnArchName, b->n_cu,
+    snprintf(buf, sizeof(buf), "%s|cu%d|prec%d|el%zu|log2n%d|item-grid|tile-wpc-unroll", prop.gcnArchName, b->n_cu,
              b->precision, b->elements.size(), lg);
     for (char* p = buf; *p; p++)
         if (*p == ' ') *p = '_';
@@ -202,62 +261,45 @@ void cache_store(const char* path, const std::string& key, int tile, int wpc, in
     fclose(f);
 }
 
-// Times every (tile, workgroups per CU, node-loop unroll) candidate on the
-// real batch and keeps the fastest. The outputs are overwritten with correct
-// values by each run.
-int autotune(noa_dcs_batch* b, hipStream_t stream, bool tune_tile, bool tune_wpc, bool tune_unroll) {
-    const int tiles[3] = {1024, 2048, 4096};
-    const int wpcs[4] = {2, 3, 4, 8};
-    const int unrolls[2] = {1, 2};
-    const int fixed_tile = b->tile, fixed_wpc = b->wpc, fixed_unroll = b->unroll;
-    hipEvent_t e0, e1;
-    if (int rc = check_hip(hipEventCreate(&e0), "hipEventCreate")) return rc;
-    if (int rc = check_hip(hipEventCreate(&e1), "hipEventCreate")) {
-        (void)hipEventDestroy(e0);
-        return rc;
-    }
-    float best = 1e30f;
-    int best_tile = tune_tile ? 2048 : fixed_tile, best_wpc = tune_wpc ? 4 : fixed_wpc;
-    int best_unroll = tune_unroll ? 1 : fixed_unroll;
-    int rc = NOA_DCS_OK;
-    for (int ti = 0; ti < 3 && rc == NOA_DCS_OK; ti++) {
-        const int t = tiles[ti];
-        if (!tune_tile && t != fixed_tile) continue;
-        b->tile = t;
-        if ((rc = upload_items(b))) break;
-        for (int wu = 0; wu < 8 && rc == NOA_DCS_OK; wu++) {
-            const int w = wpcs[wu % 4], u = unrolls[wu / 4];
-            if (!tune_wpc && w != fixed_wpc) continue;
-            if (!tune_unroll && u != fixed_unroll) continue;
-            b->wpc = w;
-            b->unroll = u;
-            if ((rc = check_hip(launch_direct(b, stream), "batch warm-up launch"))) break;
-            float ms_min = 1e30f;
-            for (int r = 0; r < 3; r++) {
-                (void)hipEventRecord(e0, stream);
-                (void)launch_direct(b, stream);
-                (void)hipEventRecord(e1, stream);
-                if ((rc = check_hip(hipEventSynchronize(e1), "autotune sync"))) break;
-                float ms = 0;
-                (void)hipEventElapsedTime(&ms, e0, e1);
-                ms_min = std::min(ms_min, ms);
-            }
-            if (rc) break;
-            if (ms_min < best) {
-                best = ms_min;
-                best_tile = t;
-                best_wpc = w;
-                best_unroll = u;
-            }
+// Times the candidate tiles and node-loop unrolls on the real batch and keeps
+// the fastest. The outputs are overwritten with correct values by each run.
+// Candidates are timed in turn, since the clock falls over the first
+// milliseconds of load: one after the other, the first looked up to 6% faster
+// than it was. Not among them, as never the fastest: tiles of 4096 (their LDS
+// leaves 2 or 3 workgroups per CU: 6.8e6 pairs FP64 648 us against 492 in
+// 2048) and the unrolled FP64 form (its registers leave one: 1111 us).
+int autotune(noa_dcs_batch* b, hipStream_t stream, bool tune_unroll) {
+    std::vector<noa_dcs_batch> cand;
+    for (const int t : {1024, 2048})
+        for (const int u : {1, 2}) {
+            if (tune_unroll ? u == 2 && b->precision == NOA_DCS_PREC_F64 : u != b->unroll) continue;
+            cand.push_back(*b);
+            cand.back().tile = t;
+            cand.back().unroll = u;
+        }
+    hipEvent_t e0 = nullptr, e1 = nullptr;
+    int rc = check_hip(hipEventCreate(&e0), "hipEventCreate");
+    if (!rc) rc = check_hip(hipEventCreate(&e1), "hipEventCreate");
+    for (size_t k = 0; k < cand.size() && !rc; k++) rc = upload_items(&cand[k]);
+    std::vector<float> best(cand.size(), 1e30f);
+    for (int r = 0; r < 5 && !rc; r++) {  // (the first round warms up)
+        for (size_t k = 0; k < cand.size() && !rc; k++) {
+            (void)hipEventRecord(e0, stream);
+            rc = check_hip(launch_direct(&cand[k], stream), "autotune launch");
+            (void)hipEventRecord(e1, stream);
+            if (!rc) rc = check_hip(hipEventSynchronize(e1), "autotune sync");
+            float ms = 0;
+            if (!rc) rc = check_hip(hipEventElapsedTime(&ms, e0, e1), "hipEventElapsedTime");
+            if (r > 0) best[k] = std::min(best[k], ms);
         }
     }
-    (void)hipEventDestroy(e0);
-    (void)hipEventDestroy(e1);
-    if (rc) return rc;
-    b->tile = best_tile;
-    b->wpc = best_wpc;
-    b->unroll = best_unroll;
-    return upload_items(b);
+    if (e0) (void)hipEventDestroy(e0);
+    if (e1) (void)hipEventDestroy(e1);
+    const size_t win = size_t(std::min_element(best.begin(), best.end()) - best.begin());
+    for (size_t k = 0; k < cand.size(); k++)
+        if ((rc || k != win) && cand[k].d_items) (void)hipFree(cand[k].d_items);
+    if (!rc) *b = cand[win];
+    return rc;
 }
 
 int capture_graph(noa_dcs_batch* b, hipStream_t stream) {
@@ -284,7 +326,6 @@ void release(noa_dcs_batch* b) {
     if (b->graph) (void)hipGraphDestroy(b->graph);
     if (b->d_consts) (void)hipFree(b->d_consts);
     if (b->d_items) (void)hipFree(b->d_items);
-    if (b->d_counter) (void)hipFree(b->d_counter);
     delete b;
 }
 
@@ -338,32 +379,26 @@ int noa_dcs_batch_create(const noa_dcs_element* elements, const int64_t* offsets
     if (!rc)
         rc = check_hip(hipMemcpy(b->d_consts, consts.data(), consts.size() * sizeof(DcsConsts), hipMemcpyHostToDevice),
                        "hipMemcpy(consts)");
-    if (!rc) rc = check_hip(hipMalloc(&b->d_counter, sizeof(uint32_t)), "hipMalloc(counter)");
     if (!rc) {
         b->tile = cfg.tile ? cfg.tile : 2048;
-        b->wpc = cfg.waves_per_cu ? cfg.waves_per_cu : 4;
+        b->wpc = cfg.waves_per_cu;
+        b->limit_wpc = cfg.waves_per_cu != 0;
         b->unroll = cfg.unroll ? cfg.unroll : 1;
-        const bool tune_tile = cfg.tile == 0, tune_wpc = cfg.waves_per_cu == 0, tune_unroll = cfg.unroll == 0;
-        if (tune_tile || tune_wpc || tune_unroll) {
-            std::lock_guard<std::mutex> lock(g_tune_mutex);
-            const std::string key = tune_key(b);
-            const bool all = tune_tile && tune_wpc && tune_unroll;
-            int t = 0, w = 0, u = 0;
-            if (all && cache_lookup(cfg.tune_cache, key, &t, &w, &u) && (t == 1024 || t == 2048 || t == 4096) &&
-                w >= 1 && w <= 32 && (u == 1 || u == 2)) {
-                b->tile = t;
-                b->wpc = w;
-                b->unroll = u;
-                rc = upload_items(b);
-            } else {
-                rc = autotune(b, stream, tune_tile, tune_wpc, tune_unroll);
-                if (!rc && all) cache_store(cfg.tune_cache, key, b->tile, b->wpc, b->unroll);
-            }
-        } else {
-            rc = upload_items(b);
+        const bool all = cfg.tile == 0 && cfg.waves_per_cu == 0 && cfg.unroll == 0;
+        std::lock_guard<std::mutex> lock(g_tune_mutex);
+        const std::string key = tune_key(b);
+        int t = 0, w = 0, u = 0;
+        const bool cached = all && cache_lookup(cfg.tune_cache, key, &t, &w, &u) &&
+                            (t == 1024 || t == 2048 || t == 4096) && w >= 1 && w <= 32 && (u == 1 || u == 2);
+        if (cached) {
+            b->tile = t;
+            b->unroll = u;
         }
+        b->small = all && offsets[n_elements] - offsets[0] <= SMALL_BATCH;
+        rc = cfg.tile == 0 && !cached && !b->small ? autotune(b, stream, cfg.unroll == 0) : upload_items(b);
+        if (!rc && all && !cached) cache_store(cfg.tune_cache, key, b->tile, b->wpc, b->unroll);
     }
-    if (!rc && b->use_graph) rc = capture_graph(b, stream);
+    if (!rc && b->use_graph && b->n_items) rc = capture_graph(b, stream);
     if (rc) {
         release(b);
         return rc;

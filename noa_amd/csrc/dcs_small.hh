@@ -57,20 +57,18 @@ __device__ __forceinline__ uint32_t wave_rank(bool pred, uint32_t* count) {
     return __builtin_amdgcn_mbcnt_hi(uint32_t(m >> 32), __builtin_amdgcn_mbcnt_lo(uint32_t(m), 0u));
 }
 
-// FP64 physics for both output types: the mixed-precision form at these sizes
-// is no faster in FP32, and its results are then the rounded FP64 values.
+// Pairs [base, end), at most SMALL_TILE of them, by one workgroup. FP64
+// physics for both output types: the mixed-precision form at these sizes is
+// no faster in FP32, and its results are then the rounded FP64 values.
 template <class OutT>
-__global__ __launch_bounds__(WG) void dcs_small_kernel(const double* __restrict__ K, const double* __restrict__ q,
-                                                       int64_t n, DcsConsts, Outs<OutT> o) {
-    __shared__ SmallLds s;
-    __shared__ __attribute__((aligned(fm::TABLE_LDS_ALIGN))) double fm_block[fm::TABLE_DOUBLES];
+__device__ __forceinline__ void run_small(int64_t base, int64_t end, const double* __restrict__ K,
+                                          const double* __restrict__ q, ConstsPtr cp, const Outs<OutT>& o,
+                                          SmallLds& s, double* fm_block) {
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(int(threadIdx.x >> 6));
-    const ConstsPtr cp = kernarg_consts();
     const fm::Tab t = fm::tab_from_block(fm_block);
-    const int64_t base = int64_t(blockIdx.x) * SMALL_TILE;
     const int64_t g = base + lane;
-    const bool valid = g < n;
+    const bool valid = g < end;
     const double k = valid ? K[g] : 1., qq = valid ? q[g] : 0.;
     load_fm_tables(fm_block);
     if (threadIdx.x < 9) {  // the node tables in LDS: the node index varies by lane
@@ -161,6 +159,14 @@ __global__ __launch_bounds__(WG) void dcs_small_kernel(const double* __restrict_
         o.ph[base + s.photo_at[lane]] =
             OutT(F64::photo_finish<false, true>(s.photo_K[lane], s.photo[lane], ds, c));
     }
+}
+
+template <class OutT>
+__global__ __launch_bounds__(WG) void dcs_small_kernel(const double* __restrict__ K, const double* __restrict__ q,
+                                                       int64_t n, DcsConsts, Outs<OutT> o) {
+    __shared__ SmallLds s;
+    __shared__ __attribute__((aligned(fm::TABLE_LDS_ALIGN))) double fm_block[fm::TABLE_DOUBLES];
+    run_small<OutT>(int64_t(blockIdx.x) * SMALL_TILE, n, K, q, kernarg_consts(), o, s, fm_block);
 }
 
 }  // namespace noa_hip

@@ -221,7 +221,7 @@ __device__ __forceinline__ void phase1(int64_t base, int64_t end, const double* 
 
 // Evaluates pairs [base, end) (end - base <= TILE) of one element with the
 // log/exp tables `t` in LDS. Must be called by all WG threads of the
-// workgroup.
+// workgroup, once: no barrier follows the last use of the lists.
 template <class P, int TILE>
 __device__ __forceinline__ void run_tile(int64_t base, int64_t end, const double* __restrict__ K,
                                          const double* __restrict__ q, ConstsPtr cp,
@@ -312,7 +312,6 @@ __device__ __forceinline__ void run_tile(int64_t base, int64_t end, const double
             }
         }
     }
-    __syncthreads();  // the lists are reused by the next tile of a persistent workgroup
 }
 
 }  // namespace noa_hip

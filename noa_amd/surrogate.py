@@ -113,7 +113,7 @@ def features(K: torch.Tensor, q: torch.Tensor, offsets, elements) -> torch.Tenso
 
 
 def exact_dcs(K, q, offsets, elements, mass=MUON_MASS):
-    """Exact FP64 DCS of a batch (the persistent batched kernel)."""
+    """Exact FP64 DCS of a batch (the batched kernel)."""
     plan = BatchPlan(elements, offsets, K, q, mass, precision="f64", tile=2048, waves_per_cu=4, use_graph=False)
     plan.launch()
     out = plan.outputs
