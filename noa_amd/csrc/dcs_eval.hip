@@ -15,24 +15,62 @@
 
 namespace noa_hip {
 
-// Pairs per workgroup of a map of n pairs; 64 is the small-map kernel
-// (dcs_small.hh), larger ones the tile kernel below. Four workgroups of the
-// tile kernel fit a CU, 1024 the chip: a map takes the largest tile that
-// still gives about one round of them, since a partly filled chip costs more
-// than the smaller tile's partly filled waves. Measured on MI355X (FP64 /
-// mixed, us, at tiles of 64, 256, 512, 1024, 2048):
-//   131,072 pairs    22  30  36  51  91   /   22  33  35  45  71
-//   262,144          41  37  42  51  91   /   41  39  42  45  71
-//   524,288          77  69  59  63  92   /   77  66  56  57  72
-//   1,048,576       152 119 100  95 114   /  152 110  91  82  89
-//   3,000,017         -   -  255 243 254  /    -   -  213 194 192
-//   8,388,608         -   -  670 632 621  /    -   -  553 476 442
-inline int eval_tile(int64_t n, bool f64) {
+// Pairs per workgroup of a map of n pairs: 64 is the small-map kernel
+// (dcs_small.hh), larger ones the tile kernel below, whose tiles shorten from
+// this towards the end of the map (TileCut). Four workgroups of the tile
+// kernel fit a CU, 1024 the chip, and a tile of 2048 pairs among four lasts
+// 150 us: below 1.5e6 pairs it would outlast the rest. Measured on MI355X
+// (FP64 / mixed, us, at tiles of 64, 256, 1024, 2048):
+//   131,072 pairs    22  30   -   -   /   22  33   -   -
+//   250,000          41  38  43  42   /   41  39  43  43
+//   414,000           -  59  59  60   /    -  55  55  55
+//   600,000           -  76  64  64   /    -  68  58  58
+//   1,240,000         - 137 115 118   /    - 119  97  95
+//   3,000,017         -   - 234 233   /    -   - 188 181
+//   8,000,000         -   - 583 565   /    -   - 450 419
+//   16,777,216        -   - 1196 1168 /    -   - 912 844
+inline int eval_tile(int64_t n) {
     if (n <= 200000) return 64;
     if (n <= 300000) return 256;
-    if (n <= 700000) return 512;
-    if (n <= (f64 ? 7000000 : 2500000)) return 1024;
+    if (n <= 1500000) return 1024;
     return 2048;
+}
+
+// Where the tiles of a map shorten: workgroups up to end[l] run tiles of
+// cut_tile(l) pairs. A length is kept while two even shares of what is left,
+// over the 1024 slots, are as long, so the workgroups end together and not
+// with a last round of whole tiles (us, equal tiles / this: 600,000 pairs FP64
+// 71 / 64, 3,000,017 mixed 191 / 181, 8,000,000 FP64 598 / 565 and mixed 439 /
+// 419, 2^24 1171 / 1168). Tiles below 512 cost more in partly filled waves than
+// they even out.
+constexpr int CUT_LEVELS = 5;
+struct TileCut {
+    uint32_t end[CUT_LEVELS];
+};
+
+template <int TILE>
+__host__ __device__ constexpr int cut_tile(int level) {
+    constexpr int eighths[CUT_LEVELS] = {8, 6, 4, 3, 2};
+    return TILE / 8 * eighths[level];
+}
+
+template <int TILE>
+TileCut cut_tiles(int64_t n) {
+    constexpr int64_t least = TILE < 512 ? TILE : 512, slots = 1024;
+    TileCut c{};
+    int64_t left = n, items = 0;
+    for (int l = 0; l < CUT_LEVELS; l++) {
+        const int64_t len = cut_tile<TILE>(l);
+        const bool last = l + 1 == CUT_LEVELS || cut_tile<TILE>(l + 1) < least;
+        const int64_t keep = last ? 0 : len * slots / 2;
+        if (len >= least && left > keep) {
+            const int64_t k = (left - keep + len - 1) / len;
+            items += k;
+            left -= k * len;
+        }
+        c.end[l] = uint32_t(items);
+    }
+    return c;
 }
 
 // Waves per SIMD the register allocation targets: the mixed form runs 2-3%
@@ -48,15 +86,23 @@ struct EvalWaves<F32MN<1>> {
     static constexpr int value = 5;
 };
 
-// One workgroup per tile of TILE consecutive pairs.
+// One workgroup per tile of up to TILE consecutive pairs.
 template <class P, int TILE>
 __global__ __launch_bounds__(WG) __attribute__((amdgpu_waves_per_eu(EvalWaves<P>::value))) void dcs_eval_kernel(const double* __restrict__ K, const double* __restrict__ q,
-                                                      int64_t n, DcsConsts c, Outs<typename P::out_t> o) {
+                                                      int64_t n, DcsConsts c, Outs<typename P::out_t> o, TileCut cut) {
     __shared__ TileLists<TILE, P::has_redo> s;
     __shared__ __attribute__((aligned(fm::TABLE_LDS_ALIGN))) double fm_block[fm::TABLE_DOUBLES];
     load_fm_tables(fm_block);  // published by run_tile's first barrier
-    const int64_t base = int64_t(blockIdx.x) * TILE;
-    const int64_t end = (base + TILE < n) ? base + TILE : n;
+    int64_t base = 0;
+    uint32_t first = 0;  // of the level's workgroups
+    int level = 0;
+    for (; level + 1 < CUT_LEVELS && blockIdx.x >= cut.end[level]; level++) {
+        base += int64_t(cut.end[level] - first) * cut_tile<TILE>(level);
+        first = cut.end[level];
+    }
+    const int64_t len = cut_tile<TILE>(level);
+    base += int64_t(blockIdx.x - first) * len;
+    const int64_t end = (base + len < n) ? base + len : n;
     run_tile<P, TILE>(base, end, K, q, kernarg_consts(), o, s, fm::tab_from_block(fm_block));
 }
 
@@ -115,10 +161,12 @@ __global__ __launch_bounds__(WG) void dcs_closed_kernel(const double* __restrict
 // run_tile reads c in place through kernarg_consts(), which locates it by
 // TileKernelArgs: the kernel's leading parameters must stay (K, q, n, c).
 static_assert(std::is_same<decltype(&dcs_eval_kernel<F64, 2048>),
-                           void (*)(const double*, const double*, int64_t, DcsConsts, Outs<double>)>::value,
+                           void (*)(const double*, const double*, int64_t, DcsConsts, Outs<double>, TileCut)>::value,
               "dcs_eval_kernel's parameters must begin as TileKernelArgs lays them out");
-static_assert(std::is_same<decltype(&dcs_small_kernel<double>), decltype(&dcs_eval_kernel<F64, 2048>)>::value,
-              "and dcs_small_kernel's with them");
+static_assert(std::is_same<decltype(&dcs_small_kernel<double>),
+                           void (*)(const double*, const double*, int64_t, DcsConsts, Outs<double>)>::value &&
+                  std::is_same<decltype(&dcs_small_kernel<double>), decltype(&dcs_closed_kernel<F64>)>::value,
+              "and dcs_small_kernel's and dcs_closed_kernel's with them");
 static_assert(offsetof(TileKernelArgs, c) == 24, "three 8-byte arguments before the constants");
 
 template <class P>
@@ -129,21 +177,21 @@ int launch_eval(const double* K, const double* q, int64_t n, const noa_dcs_eleme
     if (n == 0) return ok();
     if (!K || !q) return fail(NOA_DCS_EINVAL, "K and q must be non-NULL");
     if (!o.b && !o.p && !o.ph && !o.i) return ok();
-    const int tile = eval_tile(n, !P::has_redo);
-    const int64_t tiles = (n + tile - 1) / tile;
-    if (tiles > int64_t(0x7fffffff)) return fail(NOA_DCS_ERANGE, "n too large (%lld)", (long long)n);
+    const int tile = eval_tile(n);
+    if (n / tile > int64_t(0x7fffffff) - 4096) return fail(NOA_DCS_ERANGE, "n too large (%lld)", (long long)n);
     const DcsConsts c = make_consts(el->A, el->I, el->Z, mass);
-    auto* kernel = tile == 64     ? &dcs_small_kernel<typename P::out_t>
-                   : tile == 256  ? &dcs_eval_kernel<P, 256>
-                   : tile == 512  ? &dcs_eval_kernel<P, 512>
-                   : tile == 1024 ? &dcs_eval_kernel<P, 1024>
-                                  : &dcs_eval_kernel<P, 2048>;
-    int64_t grid = tiles;
     if (!o.p && !o.ph) {
-        kernel = &dcs_closed_kernel<P>;
-        grid = closed_grid(n);
+        hipLaunchKernelGGL(dcs_closed_kernel<P>, dim3(uint32_t(closed_grid(n))), dim3(WG), 0, stream, K, q, n, c, o);
+    } else if (tile == SMALL_TILE) {
+        hipLaunchKernelGGL(dcs_small_kernel<typename P::out_t>, dim3(uint32_t((n + SMALL_TILE - 1) / SMALL_TILE)),
+                           dim3(WG), 0, stream, K, q, n, c, o);
+    } else {
+        const TileCut cut = tile == 256 ? cut_tiles<256>(n) : tile == 1024 ? cut_tiles<1024>(n) : cut_tiles<2048>(n);
+        auto* kernel = tile == 256    ? &dcs_eval_kernel<P, 256>
+                       : tile == 1024 ? &dcs_eval_kernel<P, 1024>
+                                      : &dcs_eval_kernel<P, 2048>;
+        hipLaunchKernelGGL(kernel, dim3(cut.end[CUT_LEVELS - 1]), dim3(WG), 0, stream, K, q, n, c, o, cut);
     }
-    hipLaunchKernelGGL(kernel, dim3(uint32_t(grid)), dim3(WG), 0, stream, K, q, n, c, o);
     if (int rc = check_hip(hipGetLastError(), "dcs_eval_kernel launch")) return rc;
     return ok();
 }

@@ -19,7 +19,7 @@
 // pairs (25-88 us in tiles of 2048), 14.4 us for 65,536 (88), 22 us for
 // 131,072 (91; 30 in tiles of 256). A chain per node spends more on set-up
 // (constants, LDS reads, partly filled waves), so per pair it is at ~65% of
-// the tile kernel's speed once the chip is full: see eval_path for the line.
+// the tile kernel's speed once the chip is full: see eval_tile for the line.
 // Larger groups (128 pairs) and 128 instead of 159 registers were 10% slower
 // at 10,000 and 65,536 pairs.
 #pragma once

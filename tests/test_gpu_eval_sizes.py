@@ -14,8 +14,8 @@ from tests.parity import assert_parity
 
 pytestmark = pytest.mark.gpu
 
-BIG = 7_000_003  # tiles of 2048
-SIZES = [1, 63, 64, 65, 127, 10007, 200000, 200001, 300001, 700001, 2500001]
+BIG = 7_000_003  # tiles of 2048, shortening
+SIZES = [1, 63, 64, 65, 127, 10007, 200000, 200001, 300000, 300001, 700001, 1500000, 1500001, 2500001]
 HYDROGEN = AtomicElement(A=1.00794, I=19.2e-9, Z=1)
 
 
@@ -105,7 +105,7 @@ def mixed_full(big):
     return dcs.hip.map_all_f32mixed(K, q, STANDARD_ROCK, MUON_MASS)
 
 
-@pytest.mark.parametrize("n", [1, 65, 10007, 200000, 200001, 300001, 700001, 2500000])
+@pytest.mark.parametrize("n", [1, 65, 10007, 200000, 200001, 300001, 700001, 1500001, 2500000])
 def test_mixed_at_the_same_sizes(big, mixed_full, n):
     """The small-map kernel's mixed results are the rounded FP64 ones, every
     tile's the same as in tiles of 2048."""
