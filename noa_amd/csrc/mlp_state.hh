@@ -87,6 +87,8 @@ struct MlpWork {
     float* loss_partial = nullptr;  // one per 32 rows
     float* ws = nullptr;  // STEP_SPLITS partial gradients [STEP_SPLITS x NPARAM], then STEP_SPLITS losses
     double* loss = nullptr;  // the last step's loss
+    double* epoch_loss = nullptr;  // the sum of each epoch's losses
+    int64_t epoch_room = 0;
 };
 
 }  // namespace mlp
@@ -144,7 +146,7 @@ inline int mlp_alloc(noa_dcs_mlp* net, int max_rows) {
 inline void mlp_free(noa_dcs_mlp* net) {
     void* ptrs[] = {net->params,       net->grads,        net->adam_m, net->adam_v,  net->work.Y,
                     net->work.small,   net->work.loss_partial, net->work.ws, net->work.loss, net->packed,
-                    net->packedT,      net->scratch};
+                    net->packedT,      net->scratch,      net->work.epoch_loss};
     for (void* p : ptrs)
         if (p) (void)hipFree(p);
     for (int l = 0; l < 4; l++) {
@@ -166,11 +168,12 @@ int ensure_packed(noa_dcs_mlp* net, hipStream_t s);
 // M: row r of the batch is dataset row row_of(order, base + r). Forward,
 // masked squared error, back-propagation and the parameter gradient into
 // net->grads, the loss into net->work.loss (and added to *loss_acc, a device
-// double, when not NULL); with `update`, one Adam step (learning rate lr,
-// bias corrections bc1, bc2) that also re-packs the fragments
-// (surrogate_step.hip).
+// double, when not NULL, or with loss_first stored there); with `update`, one
+// Adam step (learning rate lr, bias corrections bc1, bc2) that also re-packs
+// the fragments (surrogate_step.hip).
 int train_step(noa_dcs_mlp* net, const float* X, const float* T, const float* Mk, const RowOrder& order, int64_t base,
-               int rows, bool update, float lr, float bc1, float bc2, double* loss_acc, hipStream_t s);
+               int rows, bool update, float lr, float bc1, float bc2, double* loss_acc, bool loss_first,
+               hipStream_t s);
 
 // The last step's loss (synchronises the stream).
 double step_loss(noa_dcs_mlp* net, hipStream_t s);

@@ -246,7 +246,7 @@ int noa_dcs_mlp_forward_backward(noa_dcs_mlp* net, const float* X, const float* 
                                  double* loss, float* grads_host, hipStream_t s) {
     if (!net || !X || !T || !Mk) return fail(NOA_DCS_EINVAL, "NULL argument");
     if (rows < 1 || rows > net->max_rows) return fail(NOA_DCS_ERANGE, "rows must be in [1, max_rows]");
-    if (int rc = train_step(net, X, T, Mk, RowOrder{}, 0, rows, false, 0.f, 1.f, 1.f, nullptr, s)) return rc;
+    if (int rc = train_step(net, X, T, Mk, RowOrder{}, 0, rows, false, 0.f, 1.f, 1.f, nullptr, false, s)) return rc;
     if (loss) *loss = step_loss(net, s);
     if (grads_host)
         if (int rc = check_hip(hipMemcpy(grads_host, net->grads, NPARAM * sizeof(float), hipMemcpyDeviceToHost),
@@ -270,9 +270,18 @@ int noa_dcs_mlp_train(noa_dcs_mlp* net, const float* X, const float* T, const fl
     const int64_t steps_per_epoch = n / batch;
     const int64_t total_steps = steps_per_epoch * epochs;
     const float b1 = 0.9f, b2 = 0.999f;
-    double* d_loss = nullptr;
-    if (int rc = check_hip(hipMalloc(&d_loss, size_t(epochs) * sizeof(double)), "hipMalloc(loss)")) return rc;
-    int rc = check_hip(hipMemsetAsync(d_loss, 0, size_t(epochs) * sizeof(double), s), "hipMemsetAsync(loss)");
+    // kept with the network: allocated, filled and released around every call
+    // it cost a 16-step call 15 of 472 us
+    if (net->work.epoch_room < epochs) {
+        if (net->work.epoch_loss) (void)hipFree(net->work.epoch_loss);
+        net->work.epoch_loss = nullptr;
+        net->work.epoch_room = 0;
+        if (int rc = check_hip(hipMalloc(&net->work.epoch_loss, size_t(epochs) * sizeof(double)), "hipMalloc(loss)"))
+            return rc;
+        net->work.epoch_room = epochs;
+    }
+    double* d_loss = net->work.epoch_loss;
+    int rc = NOA_DCS_OK;
     for (int ep = 0; ep < epochs && !rc; ep++) {
         const RowOrder order = epoch_order(seed, ep, n);
         for (int64_t st = 0; st < steps_per_epoch && !rc; st++) {
@@ -282,7 +291,7 @@ int noa_dcs_mlp_train(noa_dcs_mlp* net, const float* X, const float* T, const fl
             net->adam_t++;
             const float bc1 = 1.f - std::pow(b1, float(net->adam_t));
             const float bc2 = 1.f - std::pow(b2, float(net->adam_t));
-            rc = train_step(net, X, T, Mk, order, st * batch, batch, true, lr, bc1, bc2, d_loss + ep, s);
+            rc = train_step(net, X, T, Mk, order, st * batch, batch, true, lr, bc1, bc2, d_loss + ep, st == 0, s);
         }
     }
     std::vector<double> ep_loss(epochs, 0.);
@@ -290,7 +299,6 @@ int noa_dcs_mlp_train(noa_dcs_mlp* net, const float* X, const float* T, const fl
         rc = check_hip(hipMemcpyAsync(ep_loss.data(), d_loss, size_t(epochs) * sizeof(double), hipMemcpyDeviceToHost, s),
                        "hipMemcpy(loss)");
     if (!rc) rc = check_hip(hipStreamSynchronize(s), "hipStreamSynchronize");
-    (void)hipFree(d_loss);
     if (!rc && loss_per_epoch)
         for (int ep = 0; ep < epochs; ep++) loss_per_epoch[ep] = float(ep_loss[ep] / double(steps_per_epoch));
     return rc ? rc : ok();
