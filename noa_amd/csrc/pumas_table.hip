@@ -100,33 +100,58 @@ struct Globals {
 
 struct ElementConsts {
     double Z, A;
-    double rl;          // radiation_logarithm(Z)
     double z13;         // Z^(1/3)
     double Z13m;        // Z^(-1/3)
     double Z23;         // Z^(2/3)
     double dn;          // 1.54 A^0.27
     double lnA;         // ln A
     double shadow_low;  // exp(-0.1 ln A)
-    double b_qoff;      // m (1 - 0.75 sqrt(e) Z^(1/3)), bremsstrahlung's sqrt(e)
-    double p_qoff;      // the same with pair production's sqrt(e)
     double b_delta1;    // the bremsstrahlung nuclear-size terms (pumas.c:14009-14016)
     double b_delta2;
 };
 
-constexpr int MAX_EL = 16;  // elements per table launch (kernel-argument budget)
+// What is left of the launch invariants is computed where it is used, from
+// these, with the host's operations: the kernel arguments have 4096 bytes.
+
+// m (1 - 0.75 sqrt(e) Z^(1/3)): the highest energy loss is K plus this, with
+// bremsstrahlung's sqrt(e) or pair production's.
+__device__ __forceinline__ double q_offset(double mass, double sqrte, const ElementConsts& c) {
+#pragma clang fp contract(off)
+    return mass * (1. - 0.75 * sqrte * c.z13);
+}
+
+// Radiation logarithms by Z (pumas.c:13773-13802); 0 = use 182.7.
+static __constant__ double RAD_LOG[92] = {
+    202.4, 151.9, 159.9, 172.3, 177.9, 178.3, 176.6, 173.4, 170.0, 165.8, 165.8, 167.1, 169.1, 170.8, 172.2,
+    173.4, 174.3, 174.8, 175.1, 175.6, 176.2, 176.8, 0.0,   0.0,   0.0,   175.8, 0.0,   0.0,   173.1, 0.0,
+    0.0,   173.0, 0.0,   0.0,   173.5, 0.0,   0.0,   0.0,   0.0,   0.0,   0.0,   175.9, 0.0,   0.0,   0.0,
+    0.0,   0.0,   0.0,   0.0,   177.4, 0.0,   0.0,   178.6, 0.0,   0.0,   0.0,   0.0,   0.0,   0.0,   0.0,
+    0.0,   0.0,   0.0,   0.0,   0.0,   0.0,   0.0,   0.0,   0.0,   0.0,   0.0,   0.0,   0.0,   177.6, 0.0,
+    0.0,   0.0,   0.0,   0.0,   0.0,   0.0,   178.0, 0.0,   0.0,   0.0,   0.0,   0.0,   0.0,   0.0,   0.0,
+    0.0,   179.8};
+
+// (Z is the same for the whole workgroup: a scalar load)
+__device__ __forceinline__ double rad_log(double Z) {
+    const int i = __builtin_amdgcn_readfirstlane((Z >= 1. && Z < 93.) ? int(Z) : 0);
+    const double v = i ? RAD_LOG[i - 1] : 0.;
+    return v > 0. ? v : 182.7;
+}
+
+constexpr int MAX_KERNARG = 4096;
+constexpr int MAX_EL = 30;  // elements per table launch (kernel-argument budget)
 
 struct ElementBlock {
     ElementConsts e[MAX_EL];
 };
 
-// The envelope kernel reads the nodes as floats only, which leaves room for
-// more elements per launch.
-constexpr int MAX_ENV_EL = 24;
+// The grid for the envelope kernel, which reads the nodes as floats only: the
+// m evenly spaced ones are recomputed, which leaves room for more elements.
+constexpr int MAX_ENV_EL = 48;
 
-struct GridF {
-    float x[MAX_X];
-    int32_t n;
-    double cutoff;
+struct EnvelopeGrid {
+    float tail[N_REVERSE];
+    int32_t m;
+    double x0, dx;
 };
 
 struct EnvelopeBlock {
@@ -193,18 +218,19 @@ __device__ double dilog(double x, const fm::Tab& tb) {
 }
 
 // SSR bremsstrahlung, atomic DCS in m^2 / GeV (pumas.c:13979-14068).
-__device__ double brems_ssr(const ElementConsts& c, const Globals& G, double m, double K, double q, const fm::Tab& tb) {
+__device__ double brems_ssr(const ElementConsts& c, double rl, const Globals& G, double m, double K, double q,
+                            const fm::Tab& tb) {
 #pragma clang fp contract(off)
     const double Z = c.Z;
     if ((Z <= 0) || (c.A <= 0) || (m <= 0) || (K <= 0) || (q <= 0)) return 0.;
-    if (q >= K + c.b_qoff) return 0.;
+    if (q >= K + q_offset(m, SSR_SQRTE, c)) return 0.;
     const double energy = (K + m) * 1E+03;
     const double v = q * 1E+03 / energy;
     m *= 1E+03;
     const double Z13 = 1. / c.z13;
     const double rl_inel = (Z == 1.) ? 446. : 1429.;
     const double delta = m * m * v / (2. * energy * (1. - v));
-    const double rz = c.rl * Z13;
+    const double rz = rl * Z13;
     double phi1 = fm::log(rz * (m / SSR_ME) / (1. + rz * G.e05 * delta / SSR_ME), tb);
     double phi2 = fm::log(rz * G.e_16 * (m / SSR_ME) / (1. + rz * G.e13 * delta / SSR_ME), tb);
     const double iz = 1. - 1. / Z;
@@ -262,7 +288,8 @@ __device__ __forceinline__ double pair_zeta(const ElementConsts& c, double m_gev
     return ((zeta1 > 0.) && (zeta2 > 0.)) ? zeta1 / zeta2 : 0.;
 }
 
-__device__ __forceinline__ PairQ pair_setup(const ElementConsts& c, double m_gev, double K, double q, double zeta) {
+__device__ __forceinline__ PairQ pair_setup(const ElementConsts& c, double rl, double m_gev, double K, double q,
+                                            double zeta) {
 #pragma clang fp contract(off)
     const double Z = c.Z;
     PairQ s;
@@ -270,7 +297,7 @@ __device__ __forceinline__ PairQ pair_setup(const ElementConsts& c, double m_gev
     s.v = q / (K + m_gev);
     s.m = m_gev * 1E+03;
     s.ev = s.energy * s.v;
-    s.rl = c.rl;
+    s.rl = rl;
     const double are = ALPHA_EM * SSR_RE;
     const double const_prefactor = 4. / (3. * PI) * Z * (are * are);
     s.Z13 = c.Z13m;
@@ -351,12 +378,12 @@ __device__ double pair_d2_ssr(const PairQ& s, const Globals& G, double rho, cons
 
 // SSR pair production, atomic DCS in m^2 / GeV (pumas.c:14624-14671): the
 // 12-point rule over t = ln(rho) on [ln(1 - rmax), 0].
-__device__ double pair_ssr(const ElementConsts& c, const Globals& G, double mass, double K, double q,
+__device__ double pair_ssr(const ElementConsts& c, double rl, const Globals& G, double mass, double K, double q,
                            const fm::Tab& tb) {
 #pragma clang fp contract(off)
     if ((c.Z <= 0) || (c.A <= 0) || (mass <= 0) || (K <= 0) || (q <= 0)) return 0.;
     if (q <= 4. * ELECTRON_MASS) return 0.;
-    if (q >= K + c.p_qoff) return 0.;
+    if (q >= K + q_offset(mass, PAIR_SQRTE, c)) return 0.;
     const double gamma = 1. + K / mass;
     const double x0 = 1. - 4. * ELECTRON_MASS / q;
     const double x1 = 1. - 6. / (gamma * (gamma - q / mass));
@@ -366,8 +393,8 @@ __device__ double pair_ssr(const ElementConsts& c, const Globals& G, double mass
     if ((ri <= 0.) || (ri >= 1.)) return 0.;
     const double tmin = fm::log(ri, tb);
     // the DDCS's own range check (pumas.c:14469-14471) holds at every node:
-    // 4 m_e < q < K + p_qoff
-    const PairQ s = pair_setup(c, mass, K, q, pair_zeta(c, mass, K, tb));
+    // 4 m_e < q < K + the offset
+    const PairQ s = pair_setup(c, rl, mass, K, q, pair_zeta(c, mass, K, tb));
     double I = 0.;
 #pragma unroll 1
     for (int i = 0; i < 12; i++) {
@@ -454,12 +481,12 @@ __device__ double photo_drss(const ElementConsts& c, const Globals& G, double ml
 }
 
 // Node `node` of pair_ssr's rule, with skip set where pair_ssr returns 0.
-__device__ __forceinline__ void pair_term(const ElementConsts& c, const Globals& G, double mass, double K, double q,
-                                          double zeta, int node, double* term, int* skip, const fm::Tab& tb) {
+__device__ __forceinline__ void pair_term(const ElementConsts& c, double rl, const Globals& G, double mass, double K,
+                                          double q, double zeta, int node, double* term, int* skip, const fm::Tab& tb) {
 #pragma clang fp contract(off)
     if ((c.Z <= 0) || (c.A <= 0) || (mass <= 0) || (K <= 0) || (q <= 0)) return;
     if (q <= 4. * ELECTRON_MASS) return;
-    if (q >= K + c.p_qoff) return;
+    if (q >= K + q_offset(mass, PAIR_SQRTE, c)) return;
     const double gamma = 1. + K / mass;
     const double x0 = 1. - 4. * ELECTRON_MASS / q;
     const double x1 = 1. - 6. / (gamma * (gamma - q / mass));
@@ -468,7 +495,7 @@ __device__ __forceinline__ void pair_term(const ElementConsts& c, const Globals&
     const double ri = 1. - rmax;
     if ((ri <= 0.) || (ri >= 1.)) return;
     const double tmin = fm::log(ri, tb);
-    const PairQ s = pair_setup(c, mass, K, q, zeta);
+    const PairQ s = pair_setup(c, rl, mass, K, q, zeta);
     const double rho = fm::exp(GQ12_X[node] * tmin, tb);
     *term = pair_d2_ssr(s, G, rho, tb) * rho * GQ12_W[node] * tmin;
     *skip = 0;
@@ -504,9 +531,9 @@ __device__ double dcs(int process, const ElementConsts& c, const Globals& G, dou
 #pragma clang fp contract(off)
     double d;
     if (process == 0) {
-        d = brems_ssr(c, G, mass, K, q, tb);
+        d = brems_ssr(c, rad_log(c.Z), G, mass, K, q, tb);
     } else if (process == 1) {
-        d = pair_ssr(c, G, mass, K, q, tb);
+        d = pair_ssr(c, rad_log(c.Z), G, mass, K, q, tb);
     } else {
         const double qmin = PION_MASS + 0.5 * PION_MASS * PION_MASS / NUCLEON_MASS;
         const double qmax = K + mass - 0.5 * (NUCLEON_MASS + mass * mass / NUCLEON_MASS);
@@ -524,69 +551,72 @@ __global__ __launch_bounds__(256) void pumas_dcs_kernel(int process, ElementCons
         out[i] = dcs(process, c, G, mass, K[i], q[i], tb);
 }
 
-// One 64-lane workgroup per row of the launch's element block: block row
-// b = (p n_blk + j) n_K + k is table row r = (p n_el + e0 + j) n_K + k.
-__global__ __launch_bounds__(64) void pumas_table_kernel(Grid g, ElementBlock blk, Globals G, int32_t e0,
-                                                         int32_t n_blk, int32_t n_el, double mass,
-                                                         const double* __restrict__ Ks, int32_t n_K,
-                                                         float* __restrict__ table, double* __restrict__ table64,
-                                                         float* __restrict__ x_out, float* __restrict__ env,
-                                                         const double* __restrict__ csn) {
+// Table row r = (p n_el + e0 + j) n_K + k: process, block element, energy. One
+// workgroup holds as many rows of one (p, j) as its lanes have room for, a
+// lane per node: the 36 nodes of a cutoff of 0.05 alone leave 28 of a wave's
+// lanes idle. Bound: FP64 VALU, the nodes' quadratures run lane by lane.
+// Measured for 48 elements x 146 energies: 158 us, a wave per row 290.
+// Pair production's rows, the longest, start first.
+constexpr int TABLE_WG = 256;
+constexpr int TABLE_ROWS = TABLE_WG / N_REVERSE;  // a grid has at least N_REVERSE nodes
+
+__global__ __launch_bounds__(TABLE_WG) void pumas_table_kernel(Grid g, ElementBlock blk, Globals G, int32_t e0,
+                                                               int32_t n_blk, int32_t n_el, double mass,
+                                                               const double* __restrict__ Ks, int32_t n_K,
+                                                               float* __restrict__ table, double* __restrict__ table64,
+                                                               float* __restrict__ x_out, float* __restrict__ env,
+                                                               const double* __restrict__ csn) {
 #pragma clang fp contract(off)
     NOA_PUMAS_TABLES();
-    __shared__ double ys[MAX_X];
-    __shared__ double ms[MAX_X];
-    __shared__ int pos[MAX_X];
-    const int64_t b = blockIdx.x;
-    const int p = int(b / (int64_t(n_blk) * n_K));
-    const int j = int((b / n_K) % n_blk);
-    const int k = int(b % n_K);
-    const int64_t r = (int64_t(p) * n_el + e0 + j) * n_K + k;
+    __shared__ double xs[MAX_X];
+    __shared__ double ys_all[TABLE_WG], ms_all[TABLE_WG];
+    __shared__ int first[TABLE_ROWS], end[TABLE_ROWS], low[TABLE_ROWS], high[TABLE_ROWS];
     const int n = g.n;
+    const int room = TABLE_WG / n;
+    const int groups = (n_K + room - 1) / room;
+    const int64_t b = blockIdx.x;
+    const int p = int(b / (int64_t(n_blk) * groups) + 1) % 3;
+    const int j = int((b / groups) % n_blk);
+    const int row = int(threadIdx.x) / n, i = int(threadIdx.x) % n;
+    const int k = int(b % groups) * room + row;
+    const bool live = row < room && k < n_K;
+    const int64_t r = (int64_t(p) * n_el + e0 + j) * n_K + k;
     const ElementConsts& c = blk.e[j];
-    const double K = Ks[k];
-    const int lane = threadIdx.x;
-    if (csn && !(csn[r] > 0.)) {  // no cross section: an empty row (pumas.c:11427-11434)
-        for (int i = lane; i < n; i += 64) {
-            table[r * 2 * n + 2 * i] = 0.f;
-            table[r * 2 * n + 2 * i + 1] = 0.f;
-            if (table64) {
-                table64[r * 2 * n + 2 * i] = 0.;
-                table64[r * 2 * n + 2 * i + 1] = 0.;
-            }
-            if (b == 0 && x_out) x_out[i] = float(g.x[i]);
-        }
-        if (lane == 0 && env) {  // the reference leaves the pair as it was; here 0
-            env[2 * r] = 0.f;
-            env[2 * r + 1] = 0.f;
-        }
-        return;
+    if (threadIdx.x < unsigned(n)) {
+        xs[threadIdx.x] = g.x[threadIdx.x];
+        if (b == 0 && x_out) x_out[threadIdx.x] = float(g.x[threadIdx.x]);
     }
-
-    for (int i = lane; i < n; i += 64) {
-        const double q = K * fm::exp(g.x[i], tb);
-        const double d = dcs(p, c, G, mass, K, q, tb);
-        pos[i] = d > 0;
-        ys[i] = d > 0 ? fm::log(d, tb) : 0.;
-        if (b == 0 && x_out) x_out[i] = float(g.x[i]);
+    if (threadIdx.x < TABLE_ROWS) {
+        first[threadIdx.x] = end[threadIdx.x] = n;
+        low[threadIdx.x] = n;
+        high[threadIdx.x] = -1;
     }
     __syncthreads();
-    // the first run of positive values (every lane scans the same LDS)
-    int imin = n, imax = n - 1;
-    for (int i = 0; i < n; i++) {
-        if (pos[i]) {
-            if (i < imin) imin = i;
-        } else if (imin < n) {
-            imax = i - 1;
-            break;
-        }
+    // no cross section: an empty row (pumas.c:11427-11434)
+    const bool some = live && !(csn && !(csn[r] > 0.));
+    double* ys = ys_all + (live ? row * n : 0);
+    double* ms = ms_all + (live ? row * n : 0);
+    const double K = live ? Ks[k] : 1.;
+    bool positive = false;
+    if (some) {
+        const double q = K * fm::exp(xs[i], tb);
+        const double d = dcs(p, c, G, mass, K, q, tb);
+        positive = d > 0;
+        ys[i] = positive ? fm::log(d, tb) : 0.;
+        if (positive) atomicMin(&first[row], i);
     }
+    __syncthreads();
+    // the first run of positive values
+    const int imin = some ? first[row] : n;
+    if (some && !positive && i > imin) atomicMin(&end[row], i);
+    __syncthreads();
+    const int imax = (some ? end[row] : n) - 1;
     // PCHIP slopes over [imin, imax] (math_pchip_initialise with der = 0)
     const int N = imax - imin + 1;
-    for (int i = lane; i < n; i += 64) {
+    if (some) {
         double m = 0.;
         if (N >= 1 && i >= imin && i <= imax) {
-            const double* x = g.x + imin;
+            const double* x = xs + imin;
             const double* y = ys + imin;
             int j = i - imin;
             int nn = N;
@@ -631,44 +661,52 @@ __global__ __launch_bounds__(64) void pumas_table_kernel(Grid g, ElementBlock bl
     done:
         ms[i] = m;
         const bool in = i >= imin && i <= imax;
-        float* row = table + r * 2 * n;
-        row[2 * i] = in ? float(ys[i]) : 0.f;
-        row[2 * i + 1] = in ? float(m) : 0.f;
+        float* out = table + r * 2 * n;
+        out[2 * i] = in ? float(ys[i]) : 0.f;
+        out[2 * i + 1] = in ? float(m) : 0.f;
         if (table64) {
-            double* row64 = table64 + r * 2 * n;
-            row64[2 * i] = in ? ys[i] : 0.;
-            row64[2 * i + 1] = in ? m : 0.;
+            double* out64 = table64 + r * 2 * n;
+            out64[2 * i] = in ? ys[i] : 0.;
+            out64[2 * i + 1] = in ? m : 0.;
+        }
+        if (env && in) {
+            // the nodes of the envelope exponent's range (pumas.c:11462-11507)
+            double qmin, qmax;
+            if (p == 2) {
+                qmin = PION_MASS + 0.5 * PION_MASS * PION_MASS / NUCLEON_MASS;
+                qmax = K + mass - 0.5 * (NUCLEON_MASS + mass * mass / NUCLEON_MASS);
+                qmin += qmin;
+            } else {
+                qmax = K + q_offset(mass, PAIR_SQRTE, c);
+                qmin = (p == 0) ? 0.5 * g.cutoff * K : 4. * ELECTRON_MASS * 4;
+            }
+            const double qrev = X_REVERSE * K;
+            qmax *= 0.5;
+            if (qmax > qrev) qmax = qrev;
+            if ((xs[i] > fm::log(qmin / K, tb)) && (xs[i] < fm::log(qmax / K, tb))) {
+                atomicMin(&low[row], i);
+                atomicMax(&high[row], i);
+            }
+        }
+    } else if (live) {
+        float* out = table + r * 2 * n;
+        out[2 * i] = out[2 * i + 1] = 0.f;
+        if (table64) {
+            double* out64 = table64 + r * 2 * n;
+            out64[2 * i] = out64[2 * i + 1] = 0.;
         }
     }
     __syncthreads();
-    if (lane == 0 && env) {
-        // envelope exponent (pumas.c:11462-11507)
-        double qmin, qmax;
-        if (p == 2) {
-            qmin = PION_MASS + 0.5 * PION_MASS * PION_MASS / NUCLEON_MASS;
-            qmax = K + mass - 0.5 * (NUCLEON_MASS + mass * mass / NUCLEON_MASS);
-            qmin += qmin;
-        } else {
-            qmax = K + c.p_qoff;
-            qmin = (p == 0) ? 0.5 * g.cutoff * K : 4. * ELECTRON_MASS * 4;
-        }
-        const double qrev = X_REVERSE * K;
-        qmax *= 0.5;
-        if (qmax > qrev) qmax = qrev;
-        const double xmin = fm::log(qmin / K, tb), xmax = fm::log(qmax / K, tb);
-        int ia0 = imax, ia1 = imin;
-        for (int i = imin; i <= imax && i < n; i++) {
-            if ((g.x[i] > xmin) && (g.x[i] < xmax)) {
-                if (ia0 > i) ia0 = i;
-                if (ia1 < i) ia1 = i;
+    if (live && i == 0 && env) {
+        float alpha = 0.f;  // an empty row: the reference leaves the pair as it was; here 0
+        if (some) {
+            const int ia0 = min(imax, low[row]), ia1 = max(imin, high[row]);
+            if ((ia0 < ia1) && (ia0 < n - 1)) {
+                const int ia = (3 * ia0 + ia1) / 4;
+                double a = -ms[ia];
+                if (fabs(a - 1.) <= 0.1) a = 1.;
+                alpha = float(a);
             }
-        }
-        float alpha = 0.f;
-        if ((ia0 < ia1) && (ia0 < n - 1)) {
-            const int ia = (3 * ia0 + ia1) / 4;
-            double a = -ms[ia];
-            if (fabs(a - 1.) <= 0.1) a = 1.;
-            alpha = float(a);
         }
         env[2 * r] = alpha;
         env[2 * r + 1] = 0.f;
@@ -676,21 +714,19 @@ __global__ __launch_bounds__(64) void pumas_table_kernel(Grid g, ElementBlock bl
 }
 
 // Rows below the first positive envelope exponent of a (process, element)
-// take that exponent (pumas.c:11745-11761). One thread per (process, element).
-__global__ __launch_bounds__(64) void pumas_alpha_fill_kernel(float* __restrict__ env, int32_t n_pe, int32_t n_K) {
-    const int pe = blockIdx.x * blockDim.x + threadIdx.x;
-    if (pe >= n_pe) return;
-    float* a = env + 2 * int64_t(pe) * n_K;
-    int n0 = 0;
-    float alpha = 0.f;
-    for (int row = 0; row < n_K; row++) {
-        if (a[2 * row] > 0.f) {
-            n0 = row;
-            alpha = a[2 * row];
-            break;
-        }
+// take that exponent (pumas.c:11745-11761). One wave per (process, element).
+__global__ __launch_bounds__(64) void pumas_alpha_fill_kernel(float* __restrict__ env, int32_t n_K) {
+    float* a = env + 2 * int64_t(blockIdx.x) * n_K;
+    const int lane = threadIdx.x;
+    for (int row = 0; row < n_K; row += 64) {
+        const float v = row + lane < n_K ? a[2 * int64_t(row + lane)] : 0.f;
+        const unsigned long long positive = __ballot(v > 0.f);
+        if (!positive) continue;
+        const int at = __ffsll((long long)positive) - 1;
+        const float alpha = __shfl(v, at, 64);
+        for (int below = lane; below < row + at; below += 64) a[2 * int64_t(below)] = alpha;
+        return;
     }
-    for (int row = 0; row < n0; row++) a[2 * row] = alpha;
 }
 
 // The quadrature nodes of up to this many model evaluations fill one wave:
@@ -703,13 +739,13 @@ __device__ __forceinline__ int model_batch(int process) { return process == 0 ? 
 // the set-up and one quadrature node, and the node terms are summed in the
 // serial loop's order, so the values are those of dcs() bit for bit. Must be
 // called with the wave's 64 lanes active.
-__device__ __forceinline__ double dcs_wave(int process, const ElementConsts& c, const Globals& G, double mass, double K,
-                                           double zeta, double q, bool need, const fm::Tab& tb) {
+__device__ __forceinline__ double dcs_wave(int process, const ElementConsts& c, double rl, const Globals& G, double mass,
+                                           double K, double zeta, double q, bool need, const fm::Tab& tb) {
 #pragma clang fp contract(off)
     const int lane = threadIdx.x & 63;
     double d = 0.;
     if (process == 0) {
-        if (need) d = brems_ssr(c, G, mass, K, q, tb);
+        if (need) d = brems_ssr(c, rl, G, mass, K, q, tb);
     } else {
         const int nodes = process == 1 ? 12 : 9;
         const int per = model_batch(process);
@@ -731,7 +767,7 @@ __device__ __forceinline__ double dcs_wave(int process, const ElementConsts& c, 
             int skip = 1;
             if (mine >= 0) {
                 if (process == 1)
-                    pair_term(c, G, mass, K, qg, zeta, node, &term, &skip, tb);
+                    pair_term(c, rl, G, mass, K, qg, zeta, node, &term, &skip, tb);
                 else
                     photo_term(c, G, mass, K, qg, node, &term, &skip, tb);
             }
@@ -796,6 +832,7 @@ __device__ __forceinline__ double dcs_wave(int process, const ElementConsts& c, 
 struct EnvRow {
     int process;
     double mass;
+    double rl;          // rad_log(Z)
     const float* xt;    // the nodes as the search sees them (LDS)
     int n;
     // dcs_evaluate's energy bracket: K is the row's own energy at every
@@ -848,7 +885,7 @@ __device__ __forceinline__ double dcs_from_table(const EnvRow& a, const ElementC
         qlow = 2 * qmin;
     } else {
         qmin = 4. * ELECTRON_MASS;
-        qmax = K + c.p_qoff;
+        qmax = K + q_offset(a.mass, PAIR_SQRTE, c);
         if (a.process == 1)
             qlow = 4 * qmin;
         else
@@ -1054,7 +1091,7 @@ __device__ __forceinline__ float envelope_max(const EnvRow& a, ElementPtr cp, co
         qmax = K + a.mass - 0.5 * (NUCLEON_MASS + a.mass * a.mass / NUCLEON_MASS);
     } else {
         qmin = (a.process == 0) ? 0. : 4. * ELECTRON_MASS;
-        qmax = K + c0.p_qoff;
+        qmax = K + q_offset(a.mass, PAIR_SQRTE, c0);
     }
     double xmin = qmin / K;
     if (xmin < cutoff) xmin = cutoff;
@@ -1128,7 +1165,7 @@ __device__ __forceinline__ float envelope_max(const EnvRow& a, ElementPtr cp, co
             need = need && node < (1 << (half ? l1 : l0)) - 1;
         }
         if (__ballot(need)) {
-            const double md = dcs_wave(a.process, c, G, mass, K, zeta, q, need, tb);
+            const double md = dcs_wave(a.process, c, a.rl, G, mass, K, zeta, q, need, tb);
             if (need) d = md;
         }
         const double v = -(d * wj) * (alpha == 0. ? 1. : fm::exp(alpha * lnx, tb));
@@ -1258,34 +1295,64 @@ __device__ __forceinline__ float envelope_max(const EnvRow& a, ElementPtr cp, co
 // The leading arguments of pumas_envelope_kernel, as the kernel-argument
 // segment holds them.
 struct EnvelopeArgs {
-    GridF g;
+    EnvelopeGrid g;
     EnvelopeBlock blk;
+    Globals G;
+    int32_t n_x, e0, n_blk, n_el;
+    double mass, cutoff;
+    const double* Ks;
+    const float* table;
+    const double* csn;
+    float* env;
+    int32_t n_K;
 };
+static_assert(sizeof(EnvelopeArgs) <= MAX_KERNARG, "48 elements and the grid in one launch");
 
 // One 64-lane workgroup per (process, block element j, kinetic energy k) row
-// of the launch's element block; env[2 r + 1] of table row r.
+// of the launch's element block; env[2 r + 1] of table row r. Rows start
+// longest first: the first element's (element 0 takes the model at every
+// point), then pair production's, and the highest energies (which scan) first.
 template <int WAVES>
-__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(WAVES))) void pumas_envelope_kernel(GridF g, EnvelopeBlock blk, Globals G, int32_t e0,
-                                                            int32_t n_blk, int32_t n_el, double mass,
-                                                            const double* __restrict__ Ks, int32_t n_K,
-                                                            const float* __restrict__ table,
-                                                            const double* __restrict__ csn, float* __restrict__ env) {
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(WAVES))) void pumas_envelope_kernel(EnvelopeArgs by_value) {
     __shared__ float xt[MAX_X];
     __shared__ float ra[2 * MAX_X], rb[2 * MAX_X];
     __shared__ Search searches[2];
     NOA_PUMAS_TABLES();
-    // pair production's rows first: they have the longest searches
-    const int64_t b = blockIdx.x;
-    const int p = (1 + int(b / (int64_t(n_blk) * n_K))) % 3;
-    const int j = int((b / n_K) % n_blk);
-    const int k = int(b % n_K);
+    const auto args = (const __attribute__((address_space(4))) EnvelopeArgs*)__builtin_amdgcn_kernarg_segment_ptr();
+    const Globals G = *(const Globals*)&args->G;
+    const int32_t n_K = args->n_K, n_el = args->n_el, n_blk = args->n_blk, e0 = args->e0, n_x = args->n_x;
+    const double mass = args->mass;
+    const double* __restrict__ Ks = args->Ks;
+    const float* __restrict__ table = args->table;
+    const double* __restrict__ csn = args->csn;
+    float* __restrict__ env = args->env;
+    int64_t b = blockIdx.x;
+    int p = 1, j = 0;
+    if (b < int64_t(3) * n_K) {
+        p += int(b / n_K);
+        b %= n_K;
+    } else {
+        b -= int64_t(3) * n_K;
+        const int64_t rest = int64_t(n_blk - 1) * n_K;
+        p += int(b / rest);
+        b %= rest;
+        j = 1 + int(b % (n_blk - 1));
+        b /= n_blk - 1;
+    }
+    p %= 3;
+    const int k = n_K - 1 - int(b);
     const int e = e0 + j;
     const int64_t pe = int64_t(p) * n_el + e;
     const int64_t r = pe * n_K + k;
-    for (int i = threadIdx.x; i < g.n; i += 64) xt[i] = (e == 0) ? 0.f : g.x[i];
+    for (int i = threadIdx.x; i < n_x; i += 64) {
+#pragma clang fp contract(off)
+        const int m = args->g.m;
+        const float x = i < m ? float(args->g.x0 + i * args->g.dx) : args->g.tail[i - m];
+        xt[i] = (e == 0) ? 0.f : x;
+    }
     // dcs_evaluate's energy bracket of the row's own energy (pumas.c:11352-11381)
     const double K = Ks[k];
-    const float* rows = table + pe * n_K * 2 * g.n;
+    const float* rows = table + pe * n_K * 2 * n_x;
     const int imax = n_K - 1;
     int i0 = 0, ia = imax, ib = imax;
     float h0 = 1.f, h1 = 0.f;
@@ -1297,24 +1364,24 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(WAVES))) voi
         h1 = logf(((float)K) / K0) / logf(K1 / K0);
         h0 = 1.f - h1;
     }
-    for (int i = threadIdx.x; i < 2 * g.n; i += 64) {
-        ra[i] = rows[int64_t(ia) * 2 * g.n + i];
-        rb[i] = rows[int64_t(ib) * 2 * g.n + i];
+    for (int i = threadIdx.x; i < 2 * n_x; i += 64) {
+        ra[i] = rows[int64_t(ia) * 2 * n_x + i];
+        rb[i] = rows[int64_t(ib) * 2 * n_x + i];
     }
     __syncthreads();
     EnvRow a;
     a.process = p;
     a.mass = mass;
-    a.n = g.n;
+    a.n = n_x;
     a.xt = xt;
     a.ra = ra;
     a.rb = rb;
     a.h0 = h0;
     a.h1 = h1;
     a.below = i0 < 0;
-    const auto args = (const __attribute__((address_space(4))) EnvelopeArgs*)__builtin_amdgcn_kernarg_segment_ptr();
     const ElementPtr cp = &args->blk.e[j];
-    const float v = envelope_max(a, cp, G, K, g.cutoff, env[2 * r], csn ? csn[r] : 1., searches, tb);
+    a.rl = rad_log(cp->Z);
+    const float v = envelope_max(a, cp, G, K, args->cutoff, env[2 * r], csn ? csn[r] : 1., searches, tb);
     if (threadIdx.x == 0) env[2 * r + 1] = v;
 }
 
@@ -1341,21 +1408,6 @@ inline Globals make_globals() {
     return G;
 }
 
-// Radiation logarithms by Z (pumas.c:13773-13802); 0 = use 182.7.
-inline double host_rad_log(double Z) {
-    static const double Lz[92] = {
-        202.4, 151.9, 159.9, 172.3, 177.9, 178.3, 176.6, 173.4, 170.0, 165.8, 165.8, 167.1, 169.1, 170.8, 172.2,
-        173.4, 174.3, 174.8, 175.1, 175.6, 176.2, 176.8, 0.0,   0.0,   0.0,   175.8, 0.0,   0.0,   173.1, 0.0,
-        0.0,   173.0, 0.0,   0.0,   173.5, 0.0,   0.0,   0.0,   0.0,   0.0,   0.0,   175.9, 0.0,   0.0,   0.0,
-        0.0,   0.0,   0.0,   0.0,   177.4, 0.0,   0.0,   178.6, 0.0,   0.0,   0.0,   0.0,   0.0,   0.0,   0.0,
-        0.0,   0.0,   0.0,   0.0,   0.0,   0.0,   0.0,   0.0,   0.0,   0.0,   0.0,   0.0,   0.0,   177.6, 0.0,
-        0.0,   0.0,   0.0,   0.0,   0.0,   0.0,   178.0, 0.0,   0.0,   0.0,   0.0,   0.0,   0.0,   0.0,   0.0,
-        0.0,   179.8};
-    const int i = int(Z);
-    if (i >= 1 && i <= 92 && Lz[i - 1] > 0) return Lz[i - 1];
-    return 182.7;
-}
-
 // The element's launch invariants, each in the reference's expression and
 // order (pumas.c:13985-14016, 14301, 14478-14481, 14760, 14632-14634).
 inline ElementConsts make_element(double Z, double A, double mass, const Globals& G) {
@@ -1363,15 +1415,12 @@ inline ElementConsts make_element(double Z, double A, double mass, const Globals
     ElementConsts c;
     c.Z = Z;
     c.A = A;
-    c.rl = host_rad_log(Z);
     c.z13 = std::pow(Z, 1. / 3.);
     c.Z13m = std::pow(Z, -1. / 3.);
     c.Z23 = std::pow(Z, 2. / 3.);
     c.dn = 1.54 * std::pow(A, 0.27);
     c.lnA = std::log(A);
     c.shadow_low = std::exp(-0.1 * c.lnA);
-    c.b_qoff = mass * (1. - 0.75 * SSR_SQRTE * c.z13);
-    c.p_qoff = mass * (1. - 0.75 * PAIR_SQRTE * c.z13);
     const double m = mass * 1E+03;
     const double mu_qc = m / (SSR_MMU * G.e1 / c.dn);
     const double rho = std::sqrt(1. + 4. * mu_qc * mu_qc);
@@ -1381,7 +1430,7 @@ inline ElementConsts make_element(double Z, double A, double mass, const Globals
     return c;
 }
 
-inline void make_grid(double cutoff, Grid& g) {
+inline void make_grid(double cutoff, Grid& g, EnvelopeGrid& eg) {
 #pragma clang fp contract(off)
     const int n = n_table(cutoff);
     g.n = n;
@@ -1394,11 +1443,15 @@ inline void make_grid(double cutoff, Grid& g) {
         const double x0 = std::log(cutoff);
         const double dx = std::log(xrev / cutoff) / (m - 1);
         for (int i = 0; i < m; i++) g.x[i] = x0 + i * dx;
+        eg.x0 = x0;
+        eg.dx = dx;
     } else {
         xrev = cutoff;
     }
     const double dx = std::log((MAX_FRACTION - xrev) / DXMIN) / ((m > 0) ? p : p - 1);
     for (int i = 0; i < p; i++) g.x[n - 1 - i] = std::log(MAX_FRACTION - DXMIN * std::exp(i * dx));
+    eg.m = m;
+    for (int i = 0; i < p; i++) eg.tail[i] = float(g.x[m + i]);
 }
 
 }  // namespace pumas
@@ -1440,46 +1493,59 @@ int noa_pumas_dcs_table(const double* Z, const double* A, int32_t n_elements, do
     if (n_elements < 0 || n_K < 0) return fail(NOA_DCS_EINVAL, "n_elements and n_K must be >= 0");
     if (!(mass > 0.0)) return fail(NOA_DCS_EINVAL, "mass must be > 0 (got %g)", mass);
     if (int64_t(3) * n_elements * n_K == 0) return ok();
-    if (int64_t(3) * pumas::MAX_EL * n_K > int64_t(0x7fffffff)) return fail(NOA_DCS_ERANGE, "n_K too large (%d)", n_K);
+    if (int64_t(3) * 16 * n_K > int64_t(0x7fffffff)) return fail(NOA_DCS_ERANGE, "n_K too large (%d)", n_K);
     if (!Z || !A || !K || !table) return fail(NOA_DCS_EINVAL, "Z, A, K and table must be non-NULL");
     for (int e = 0; e < n_elements; e++)
         if (!(Z[e] >= 1.0) || !(A[e] > 0.0))
             return fail(NOA_DCS_EINVAL, "element %d: Z >= 1 and A > 0 required (got %g, %g)", e, Z[e], A[e]);
     pumas::Grid g;
-    pumas::make_grid(cutoff, g);
+    pumas::EnvelopeGrid eg{};
+    pumas::make_grid(cutoff, g, eg);
     const pumas::Globals G = pumas::make_globals();
-    for (int e0 = 0; e0 < n_elements; e0 += pumas::MAX_EL) {
-        const int n_blk = n_elements - e0 < pumas::MAX_EL ? n_elements - e0 : pumas::MAX_EL;
+    // launches of equal numbers of elements (a grid has at most 2^31 - 1 workgroups)
+    const int64_t most = int64_t(0x7fffffff) / (int64_t(3) * n_K);
+    const auto per_launch = [&](int64_t room) {
+        room = std::min(room, most);
+        const int64_t launches = (n_elements + room - 1) / room;
+        return int((n_elements + launches - 1) / launches);
+    };
+    for (int e0 = 0, per = per_launch(pumas::MAX_EL); e0 < n_elements; e0 += per) {
+        const int n_blk = std::min(n_elements - e0, per);
         pumas::ElementBlock blk{};
         for (int j = 0; j < n_blk; j++) blk.e[j] = pumas::make_element(Z[e0 + j], A[e0 + j], mass, G);
-        const unsigned rows = unsigned(3 * n_blk * n_K);
-        hipLaunchKernelGGL(pumas::pumas_table_kernel, dim3(rows), dim3(64), 0, stream, g, blk, G, e0, n_blk,
+        const int room = pumas::TABLE_WG / g.n;
+        const unsigned grid = unsigned(3 * n_blk * ((n_K + room - 1) / room));
+        hipLaunchKernelGGL(pumas::pumas_table_kernel, dim3(grid), dim3(pumas::TABLE_WG), 0, stream, g, blk, G, e0, n_blk,
                            n_elements, mass, K, n_K, table, table_f64, e0 == 0 ? x : nullptr, envelope, csn);
         if (int rc = check_hip(hipGetLastError(), "pumas_table_kernel")) return rc;
     }
     if (envelope) {
-        const int n_pe = 3 * n_elements;
-        hipLaunchKernelGGL(pumas::pumas_alpha_fill_kernel, dim3(unsigned((n_pe + 63) / 64)), dim3(64), 0, stream,
-                           envelope, n_pe, n_K);
+        hipLaunchKernelGGL(pumas::pumas_alpha_fill_kernel, dim3(unsigned(3 * n_elements)), dim3(64), 0, stream,
+                           envelope, n_K);
         if (int rc = check_hip(hipGetLastError(), "pumas_alpha_fill_kernel")) return rc;
         // the envelope maxima, over the finished rows and exponents
-        pumas::GridF gf{};
-        gf.n = g.n;
-        gf.cutoff = g.cutoff;
-        for (int i = 0; i < g.n; i++) gf.x[i] = (float)g.x[i];
-        // (a grid has at most 2^31 - 1 workgroups)
-        const int per = int(std::min<int64_t>(pumas::MAX_ENV_EL, int64_t(0x7fffffff) / (int64_t(3) * n_K)));
-        for (int e0 = 0; e0 < n_elements; e0 += per) {
-            const int n_blk = std::min(n_elements - e0, per);
-            pumas::EnvelopeBlock blk{};
-            for (int j = 0; j < n_blk; j++) blk.e[j] = pumas::make_element(Z[e0 + j], A[e0 + j], mass, G);
-            const unsigned rows = unsigned(3 * n_blk * n_K);
+        pumas::EnvelopeArgs args{};
+        args.g = eg;
+        args.G = G;
+        args.n_x = g.n;
+        args.n_el = n_elements;
+        args.mass = mass;
+        args.cutoff = cutoff;
+        args.Ks = K;
+        args.table = table;
+        args.csn = csn;
+        args.env = envelope;
+        args.n_K = n_K;
+        for (int per = per_launch(pumas::MAX_ENV_EL); args.e0 < n_elements; args.e0 += per) {
+            args.n_blk = std::min(n_elements - args.e0, per);
+            for (int j = 0; j < args.n_blk; j++)
+                args.blk.e[j] = pumas::make_element(Z[args.e0 + j], A[args.e0 + j], mass, G);
+            const unsigned rows = unsigned(3 * args.n_blk * n_K);
             // three waves per SIMD (a few registers spilled) where the rows
             // exceed the 2048 that two hold: 1963 against 2115 us for 48
             // elements x 146 energies, 766 against 718 for 1 x 30
             hipLaunchKernelGGL((rows > 2048 ? &pumas::pumas_envelope_kernel<3> : &pumas::pumas_envelope_kernel<2>),
-                               dim3(rows), dim3(64), 0, stream, gf, blk, G, e0, n_blk, n_elements, mass, K, n_K, table,
-                               csn, envelope);
+                               dim3(rows), dim3(64), 0, stream, args);
             if (int rc = check_hip(hipGetLastError(), "pumas_envelope_kernel")) return rc;
         }
     }
