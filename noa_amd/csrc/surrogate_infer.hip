@@ -38,9 +38,9 @@ namespace mlp {
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 
-constexpr int IWG = 512;              // 8 waves
+constexpr int IWG = 1024;             // 16 waves
 constexpr int QW = 64;                // queries per wave pass (two 32-column N-tiles)
-constexpr int QWG = QW * (IWG / 64);  // 512 queries per workgroup pass
+constexpr int QWG = QW * (IWG / 64);  // 1024 queries per workgroup pass
 
 // (16-byte aligned: a fragment is one ds_read_b128; at the arrays' natural
 // alignment the compiler split every one into four-byte pairs)
@@ -75,89 +75,74 @@ __device__ __forceinline__ bf16x8 pack8(const float* f) {
     return r;
 }
 
-// The network on this wave's 64 queries: x[nt] are the features of query
-// column lane%32 of N-tile nt; out[nt][p] is valid on lanes < 32.
-__device__ __forceinline__ void mlp_wave(const MlpLds& L, const float (&x)[2][IN], float (&out)[2][OUT]) {
+// The network on 32 queries: x are the features of this lane's column lane %
+// 32; out[p] is valid on lanes < 32.
+__device__ __forceinline__ void mlp_tile(const MlpLds& L, const float (&x)[IN], float (&out)[OUT]) {
     const int lane = threadIdx.x & 63;
-    bf16x8 B[2][8];
-    // layer 1, FP32: each weight row serves both query tiles as it is read
+    bf16x8 B[8];
 #pragma unroll
-    for (int m = 0; m < 4; m++) {
-        float a[2][16];
+    for (int m = 0; m < 4; m++) {  // layer 1, FP32
+        float a[16];
 #pragma unroll
         for (int v = 0; v < 16; v++) {
             const int f = 32 * m + d_row(lane, v);
-            const float w0 = L.w1[f * IN], w1 = L.w1[f * IN + 1], w2 = L.w1[f * IN + 2], b = L.b1[f];
-#pragma unroll
-            for (int nt = 0; nt < 2; nt++)
-                a[nt][v] = silu_fast(fmaf(w2, x[nt][2], fmaf(w1, x[nt][1], fmaf(w0, x[nt][0], b))));
+            a[v] = silu_fast(
+                fmaf(L.w1[f * IN + 2], x[2], fmaf(L.w1[f * IN + 1], x[1], fmaf(L.w1[f * IN], x[0], L.b1[f]))));
         }
-#pragma unroll
-        for (int nt = 0; nt < 2; nt++) {
-            B[nt][2 * m] = pack8(a[nt]);
-            B[nt][2 * m + 1] = pack8(a[nt] + 8);
-        }
+        B[2 * m] = pack8(a);
+        B[2 * m + 1] = pack8(a + 8);
     }
-    // Hidden layers, two M-tiles at a time: 4 accumulator tiles (2 M x 2 N)
-    // plus this layer's and the next layer's B operands stay in registers.
 #pragma unroll 1
-    for (int li = 0; li < 3; li++) {
-        bf16x8 Bn[2][8];
+    for (int li = 0; li < 3; li++) {  // hidden layers
+        bf16x8 Bn[8];
 #pragma unroll
-        for (int mp = 0; mp < 2; mp++) {
-            f32x16 acc[2][2];
+        for (int m = 0; m < 4; m++) {
+            f32x16 acc;
 #pragma unroll
-            for (int mi = 0; mi < 2; mi++)
-#pragma unroll
-                for (int v = 0; v < 16; v++) {
-                    const float bv = L.bh[li][32 * (2 * mp + mi) + d_row(lane, v)];
-                    acc[0][mi][v] = bv;
-                    acc[1][mi][v] = bv;
-                }
+            for (int v = 0; v < 16; v++) acc[v] = L.bh[li][32 * m + d_row(lane, v)];
 #pragma unroll
             for (int b = 0; b < 8; b++)
+                acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
+                    *reinterpret_cast<const bf16x8*>(L.frag + (((li * 4 + m) * 8 + b) * 64 + lane) * 8), B[b], acc, 0,
+                    0, 0);
+            float t[16];
 #pragma unroll
-                for (int mi = 0; mi < 2; mi++) {
-                    const int m = 2 * mp + mi;
-                    const bf16x8 a =
-                        *reinterpret_cast<const bf16x8*>(L.frag + (((li * 4 + m) * 8 + b) * 64 + lane) * 8);
-                    acc[0][mi] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, B[0][b], acc[0][mi], 0, 0, 0);
-                    acc[1][mi] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, B[1][b], acc[1][mi], 0, 0, 0);
-                }
-#pragma unroll
-            for (int nt = 0; nt < 2; nt++)
-#pragma unroll
-                for (int mi = 0; mi < 2; mi++) {
-                    const int m = 2 * mp + mi;
-                    float t[16];
-#pragma unroll
-                    for (int v = 0; v < 16; v++) t[v] = silu_fast(acc[nt][mi][v]);
-                    Bn[nt][2 * m] = pack8(t);
-                    Bn[nt][2 * m + 1] = pack8(t + 8);
-                }
+            for (int v = 0; v < 16; v++) t[v] = silu_fast(acc[v]);
+            Bn[2 * m] = pack8(t);
+            Bn[2 * m + 1] = pack8(t + 8);
         }
 #pragma unroll
-        for (int nt = 0; nt < 2; nt++)
-#pragma unroll
-            for (int b = 0; b < 8; b++) B[nt][b] = Bn[nt][b];
+        for (int b = 0; b < 8; b++) B[b] = Bn[b];
     }
-    f32x16 o[2];
+    f32x16 o;
 #pragma unroll
-    for (int v = 0; v < 16; v++) {
-        const float bv = (lane < 32 && v < OUT) ? L.b5[v] : 0.f;
-        o[0][v] = bv;
-        o[1][v] = bv;
-    }
+    for (int v = 0; v < 16; v++) o[v] = (lane < 32 && v < OUT) ? L.b5[v] : 0.f;
 #pragma unroll
-    for (int b = 0; b < 8; b++) {
-        const bf16x8 a = *reinterpret_cast<const bf16x8*>(L.frag + FRAG_HIDDEN + (b * 64 + lane) * 8);
-        o[0] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, B[0][b], o[0], 0, 0, 0);
-        o[1] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, B[1][b], o[1], 0, 0, 0);
-    }
+    for (int b = 0; b < 8; b++)
+        o = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
+            *reinterpret_cast<const bf16x8*>(L.frag + FRAG_HIDDEN + (b * 64 + lane) * 8), B[b], o, 0, 0, 0);
 #pragma unroll
-    for (int p = 0; p < OUT; p++) {
-        out[0][p] = o[0][p];
-        out[1][p] = o[1][p];
+    for (int p = 0; p < OUT; p++) out[p] = o[p];
+}
+
+// The network on the wave's 64 queries, one per lane: xs its features, t its
+// outputs.
+__device__ __forceinline__ void mlp_wave(const MlpLds& L, const float (&xs)[IN], float (&t)[OUT]) {
+    const int lane = threadIdx.x & 63;
+#pragma unroll 1
+    for (int nt = 0; nt < 2; nt++) {
+        // compiler-only fence: the weights are re-read from LDS each time
+        // instead of being hoisted out of the loop into (spilled) registers
+        asm volatile("" ::: "memory");
+        float x[IN], out[OUT];
+#pragma unroll
+        for (int j = 0; j < IN; j++) x[j] = __shfl(xs[j], 32 * nt | (lane & 31));
+        mlp_tile(L, x, out);
+#pragma unroll
+        for (int p = 0; p < OUT; p++) {
+            const float o = __shfl(out[p], lane & 31);
+            if ((lane >> 5) == nt) t[p] = o;
+        }
     }
 }
 
@@ -170,30 +155,14 @@ __global__ __launch_bounds__(IWG) void mlp_fused_kernel(const float* __restrict_
     const int wave = threadIdx.x / 64, lane = threadIdx.x % 64;
     for (int64_t base = (int64_t(blockIdx.x) * (IWG / 64) + wave) * QW; base < n;
          base += int64_t(gridDim.x) * QWG) {  // wave-uniform trip count
-        // compiler-only fence: the weight fragments are re-read from LDS each
-        // pass instead of being hoisted out of the loop into (spilled) registers
-        asm volatile("" ::: "memory");
-        float x[2][IN];
+        const int64_t g = base + lane;
+        float x[IN], y[OUT] = {};
 #pragma unroll
-        for (int nt = 0; nt < 2; nt++) {
-            const int64_t g = base + 32 * nt + lane % 32;
+        for (int j = 0; j < IN; j++) x[j] = g < n ? X[g * IN + j] : 0.f;
+        mlp_wave(L, x, y);
+        if (g < n)
 #pragma unroll
-            for (int j = 0; j < IN; j++) x[nt][j] = g < n ? X[g * IN + j] : 0.f;
-        }
-        // lane l's own query qb + l is N-tile l/32's column l%32
-        float xs[IN];
-#pragma unroll
-        for (int j = 0; j < IN; j++) xs[j] = lane < 32 ? x[0][j] : x[1][j];
-        float out[2][OUT];
-        mlp_wave(L, x, out);
-        if (lane < 32)
-#pragma unroll
-            for (int nt = 0; nt < 2; nt++) {
-                const int64_t g = base + 32 * nt + lane;
-                if (g < n)
-#pragma unroll
-                    for (int p = 0; p < OUT; p++) Y[g * OUT + p] = out[nt][p];
-            }
+            for (int p = 0; p < OUT; p++) Y[g * OUT + p] = y[p];
     }
 }
 
@@ -221,7 +190,7 @@ struct SurCfg {
     uint64_t seed;
 };
 
-constexpr int SUR_ITEM = 4096;             // queries per work item: 8 passes of QWG
+constexpr int SUR_ITEM = 4096;             // queries per work item, at most
 constexpr uint32_t SUR_RECHECK = 0x8000u;  // list tag: compare the network's value before the overwrite
 
 // Per-item lists of the queries whose pair production / photonuclear DCS is
@@ -229,10 +198,21 @@ constexpr uint32_t SUR_RECHECK = 0x8000u;  // list tag: compare the network's va
 struct SurLists {
     uint16_t pair[SUR_ITEM];
     uint16_t photo[SUR_ITEM];
-    uint32_t n_pair;
-    uint32_t n_photo;
 };
-static_assert(SUR_ITEM <= 0x8000 && SUR_ITEM % QWG == 0, "15-bit item offsets, whole passes");
+static_assert(SUR_ITEM <= 0x8000, "15-bit item offsets");
+
+// Per item: what its lists hold, and the next 64 queries (phase A) or 64 list
+// entries (phase B) that no wave has taken.
+struct SurControl {
+    uint32_t item, n_pair, n_photo, next_query, next_entry;
+};
+
+// The wave's next 64 of a counter in LDS.
+__device__ __forceinline__ uint32_t wave_take(uint32_t* next) {
+    uint32_t v = 0;
+    if ((threadIdx.x & 63) == 0) v = atomicAdd(next, 64u);
+    return __builtin_amdgcn_readfirstlane(v);
+}
 
 __device__ __forceinline__ uint64_t mix64(uint64_t z) {
     z = (z ^ (z >> 30)) * 0xBF58476D1CE4E5B9ull;
@@ -253,6 +233,20 @@ __device__ __forceinline__ bool ion_active(double K, double q, const DcsConsts& 
 // DCS evaluated exactly, [2]: largest relative error of the network over the
 // recheck sample (float bits).
 //
+// The leading arguments of surrogate_dcs_kernel, as the kernel-argument
+// segment holds them.
+struct SurKernelArgs {
+    SurCfg cfg;
+};
+
+// The configuration, re-read where it is used (as item_consts does for an
+// element's constants): its 60 numbers alone would fill the scalar registers.
+__device__ __forceinline__ const SurCfg& sur_cfg() {
+    auto p = (const __attribute__((address_space(4))) SurKernelArgs*)__builtin_amdgcn_kernarg_segment_ptr();
+    asm volatile("" : "+s"(p));
+    return ((const SurKernelArgs*)p)->cfg;
+}
+
 // A workgroup takes items of up to SUR_ITEM queries of one element. Phase A,
 // in passes of 64 queries per wave: lane l owns one query, whose routing
 // comes first (out-of-domain queries and the seeded recheck sample take every
@@ -263,46 +257,59 @@ __device__ __forceinline__ bool ion_active(double K, double q, const DcsConsts& 
 // production and photonuclear queries are appended to the item's lists in
 // LDS. Phase B drains the lists densely (photonuclear, the heavier, first),
 // so the FP64 integrals run in full waves.
+//
+// The weights leave room for one workgroup per CU, so nothing else fills the
+// time its waves wait for each other: they take 64 queries or list entries at
+// a time from the item's counters, and a wave that finds phase B's list taken
+// goes on to the next item (lists in two copies, counters in three), one
+// barrier per item. Bound: VALU issue, most of it the network's 512 SiLU per
+// query (an exponential and a reciprocal at a quarter of the rate each), and
+// the FP64 integrals where they run, so 16 waves of 128 registers, with the
+// network on 32 queries and one M-tile at a time; on 64 queries and two
+// M-tiles it took 256 registers and left two waves per SIMD. Measured, 2^22
+// queries of 48 elements (us): tolerance 3e-2 1002 -> 829, 1e-3 (all exact)
+// 577 -> 426; 12 waves 870 and 442, 16 waves with a barrier after each phase
+// 915 and 460. The constants and the configuration are re-read where they are used:
+// held, they were 150 spilled scalar registers and 20 to 40 us.
 __global__ __launch_bounds__(IWG) void surrogate_dcs_kernel(
-    const double* __restrict__ K, const double* __restrict__ q, const SurElem* __restrict__ els,
-    const SurItem* __restrict__ items, uint32_t n_items, uint32_t* counters, Outs<float> o, SurCfg cfg,
+    SurCfg, const double* __restrict__ K, const double* __restrict__ q, const SurElem* __restrict__ els,
+    const SurItem* __restrict__ items, uint32_t n_items, uint32_t* counters, Outs<float> o,
     const uint16_t* __restrict__ frag, const float* __restrict__ P) {
     __shared__ MlpLds L;
     __shared__ __attribute__((aligned(fm::TABLE_LDS_ALIGN))) double fm_block[fm::TABLE_DOUBLES];
-    __shared__ SurLists S;
-    __shared__ uint32_t s_item;
+    __shared__ SurLists lists[2];
+    __shared__ SurControl control[3];
     load_lds(L, frag, P);
     for (int k = threadIdx.x; k < fm::TABLE_DOUBLES; k += IWG) fm_block[k] = fm::table_entry(k);
     const fm::Tab tab = fm::tab_from_block(fm_block);
-    const int wave = threadIdx.x / 64, lane = threadIdx.x % 64;
+    const int lane = threadIdx.x % 64;
     float worst = 0.f;
-    for (;;) {
-        if (threadIdx.x == 0) {
-            s_item = atomicAdd(&counters[0], 1u);
-            S.n_pair = 0;
-            S.n_photo = 0;
-        }
-        __syncthreads();  // also publishes the LDS contents on the first pass
-        const uint32_t it = __builtin_amdgcn_readfirstlane(s_item);
+    if (threadIdx.x == 0) control[0] = SurControl{atomicAdd(&counters[0], 1u), 0, 0, 0, 0};
+    __syncthreads();  // also publishes the LDS contents
+    for (int turn = 0;; turn++) {
+        SurControl& now = control[turn % 3];
+        SurLists& S = lists[turn % 2];
+        const uint32_t it = __builtin_amdgcn_readfirstlane(now.item);
         if (it >= n_items) break;  // workgroup-uniform exit
         const SurItem w = items[it];
         using ConstPtr = const __attribute__((address_space(4))) SurElem*;
         const SurElem& E = *(const SurElem*)((ConstPtr)(els + w.element));
+        const ConstsPtr cp = &((ConstPtr)(els + w.element))->c;
         const int64_t end = w.begin + w.len;
         // phase A
 #pragma unroll 1
-        for (int pass = 0; pass < SUR_ITEM / QWG; pass++) {
-            const int64_t qb = w.begin + int64_t(pass) * QWG + int64_t(wave) * QW;
-            if (qb >= end) break;  // wave-uniform: the later passes start further on
+        for (;;) {
+            const uint32_t first = wave_take(&now.next_query);
+            if (first >= uint32_t(w.len)) break;
+            const int64_t qb = w.begin + first;
             const int64_t g = qb + lane;
             const bool live = g < end;
-            double k = 1., qq = 0.5;
+            const SurCfg& cfg = sur_cfg();
             uint32_t cellmask = 0, mask = 0;
             bool sample = false;
             float xs[IN] = {0.f, 0.f, 0.f};
             if (live) {
-                k = K[g];
-                qq = q[g];
+                const double k = K[g], qq = q[g];
                 const double nu = qq / k;
                 if (!(k >= 1e-3 && k <= 1e6 && nu >= 1e-6 && nu < 1.0)) {
                     mask = 0xFu;  // out of the trained domain
@@ -323,28 +330,16 @@ __global__ __launch_bounds__(IWG) void surrogate_dcs_kernel(
             }
             const bool need_net = live && (mask != 0xFu || sample) && (mask != 0xFu || cellmask != 0xFu);
             float t[OUT] = {0.f, 0.f, 0.f, 0.f};
-            if (__ballot(need_net)) {  // wave-uniform
-                // MFMA layout: column lane%32 of N-tile nt is query qb + 32 nt + lane%32
-                float x[2][IN];
-#pragma unroll
-                for (int j = 0; j < IN; j++) {
-                    x[0][j] = __shfl(xs[j], lane & 31);
-                    x[1][j] = __shfl(xs[j], 32 | (lane & 31));
-                }
-                float out[2][OUT];
-                mlp_wave(L, x, out);
-                // lane l takes query qb + l: N-tile 1's outputs move from lane l-32
-#pragma unroll
-                for (int p = 0; p < OUT; p++) {
-                    const float o1 = __shfl(out[1][p], lane & 31);
-                    t[p] = lane < 32 ? out[0][p] : o1;
-                }
-            }
+            if (__ballot(need_net)) mlp_wave(L, xs, t);  // wave-uniform
             bool to_pair = false, to_photo = false;
             uint32_t tag_pair = uint32_t(g - w.begin), tag_photo = tag_pair;
+            const DcsConsts& c = item_consts(cp);
+            const SurCfg& scale = sur_cfg();
             if (live) {
-                const bool act[OUT] = {true, F64::pair_active(k, qq, E.c), F64::photo_active(k, qq, E.c),
-                                       ion_active(k, qq, E.c)};
+                // (read again rather than held across the network)
+                const double k = K[g], qq = q[g];
+                const bool act[OUT] = {true, F64::pair_active(k, qq, c), F64::photo_active(k, qq, c),
+                                       ion_active(k, qq, c)};
                 const float a = xs[0], b = xs[1], z = xs[2];
                 const float phi[NTREND] = {a,         b,         a * a, b * b, a * b, a * a * a, b * b * b,
                                            a * a * b, a * b * b, z,     z * a, z * b, z * z};
@@ -352,9 +347,9 @@ __global__ __launch_bounds__(IWG) void surrogate_dcs_kernel(
 #pragma unroll
                 for (int p = 0; p < OUT; p++) {
                     if (!dst[p]) continue;
-                    float lnad = fmaf(cfg.stdv[p], t[p], cfg.mean[p]);
+                    float lnad = fmaf(scale.stdv[p], t[p], scale.mean[p]);
 #pragma unroll
-                    for (int j = 0; j < NTREND; j++) lnad = fmaf(cfg.trend[p][j], phi[j], lnad);
+                    for (int j = 0; j < NTREND; j++) lnad = fmaf(scale.trend[p][j], phi[j], lnad);
                     const float net = __expf(lnad - E.ln_a);
                     const bool exact = (mask >> p) & 1u;
                     const bool recheck = sample && !((cellmask >> p) & 1u);
@@ -362,7 +357,7 @@ __global__ __launch_bounds__(IWG) void surrogate_dcs_kernel(
                     if (!act[p]) {
                         v = 0.f;
                     } else if (exact && (p == 0 || p == 3)) {
-                        const double ex = (p == 0) ? F64::brems(k, qq, E.c, tab) : F64::ion(k, qq, E.c, tab);
+                        const double ex = (p == 0) ? F64::brems(k, qq, c, tab) : F64::ion(k, qq, c, tab);
                         if (recheck && ex > 0.) worst = fmaxf(worst, float(fabs(double(net) / ex - 1.)));
                         v = float(ex);
                     } else if (exact && p == 1) {
@@ -375,28 +370,38 @@ __global__ __launch_bounds__(IWG) void surrogate_dcs_kernel(
                     dst[p][g] = v;
                 }
             }
-            wave_append(to_pair, &S.n_pair, S.pair, tag_pair);
-            wave_append(to_photo, &S.n_photo, S.photo, tag_photo);
+            wave_append(to_pair, &now.n_pair, S.pair, tag_pair);
+            wave_append(to_photo, &now.n_photo, S.photo, tag_photo);
         }
-        __syncthreads();  // the lists, and phase A's outputs for the recheck, are complete
+        if (threadIdx.x == 0) control[(turn + 1) % 3] = SurControl{atomicAdd(&counters[0], 1u), 0, 0, 0, 0};
+        // the lists, and phase A's outputs for the recheck, are complete; so is
+        // phase B of the turn before, whose lists the next turn overwrites
+        __syncthreads();
         // phase B: the item's exact integrals, densely
-        const uint32_t nph = S.n_photo, npa = S.n_pair;
+        // (whole waves of one kind)
+        const uint32_t nph = now.n_photo, npa = now.n_pair;
+        const uint32_t pair0 = (nph + 63u) & ~63u;
 #pragma unroll 1
-        for (uint32_t v = threadIdx.x; v < nph + npa; v += IWG) {
-            const bool photo = v < nph;
-            const uint32_t tag = photo ? S.photo[v] : S.pair[v - nph];
-            const int64_t g = w.begin + (tag & (SUR_RECHECK - 1u));
-            const double k = K[g], qq = q[g];
-            const double val = photo ? F64::photo(k, qq, E.c, tab) : F64::pair(k, qq, E.c, tab);
-            float* dst = photo ? o.ph : o.p;
-            if ((tag & SUR_RECHECK) && val > 0.) worst = fmaxf(worst, float(fabs(double(dst[g]) / val - 1.)));
-            dst[g] = float(val);
+        for (;;) {
+            const uint32_t first = wave_take(&now.next_entry);
+            if (first >= pair0 + npa) break;
+            const uint32_t v = first + lane;
+            const bool photo = v < pair0;
+            if (v < (photo ? nph : pair0 + npa)) {
+                const DcsConsts& c = item_consts(cp);
+                const uint32_t tag = photo ? S.photo[v] : S.pair[v - pair0];
+                const int64_t g = w.begin + (tag & (SUR_RECHECK - 1u));
+                const double k = K[g], qq = q[g];
+                const double val = photo ? F64::photo(k, qq, c, tab) : F64::pair(k, qq, c, tab);
+                float* dst = photo ? o.ph : o.p;
+                if ((tag & SUR_RECHECK) && val > 0.) worst = fmaxf(worst, float(fabs(double(dst[g]) / val - 1.)));
+                dst[g] = float(val);
+            }
         }
         if (threadIdx.x == 0) {
             if (npa) atomicAdd(&counters[1], npa);
             if (nph) atomicAdd(&counters[3], nph);
         }
-        __syncthreads();  // the lists and s_item are rewritten by the next item
     }
     // non-negative floats order like their bit patterns
     if (worst > 0.f) atomicMax(&counters[2], __float_as_uint(worst));
@@ -427,16 +432,14 @@ constexpr int64_t SHORT_ITEMS_PER_CU = 4;
 
 // Queries per work item. One workgroup per CU takes items in turn, so a call
 // lasts as long as its busiest CU: with items of 4096 a call of 2^18 queries
-// keeps 96 of 256 CUs busy and one of 2^21 lasts three rounds for two and a
-// half. Each candidate's longest queue is added up as the kernel will form it
-// (whole items in rounds, then the remainders, longest first, to the emptiest
-// queue), with ITEM_COST queries' time for an item's start and its partly
-// filled last exact waves; the shortest one is taken, the longer item on a
-// tie. Measured, 48 elements, tolerance 3e-2, items of 4096 in element order
-// against this rule (us): 2^16 queries 127 / 83 (items of 512), 2^18 266 / 138
-// (1536), 2^20 367 / 325 (4096, remainders last), 2^21 638 / 562 (3072),
-// 2^22 1042 / 999 (4096). An ITEM_COST below 256 picks items of 256, which
-// leave half the waves of a pass idle (2^16: 112 us); above 400 nothing moves.
+// keeps 96 of 256 CUs busy. Each candidate's longest queue is added up as the
+// kernel will form it (whole items in rounds, then the remainders, longest
+// first, to the emptiest queue), with ITEM_COST queries' time for an item's
+// start; the shortest one is taken, the longer item on a
+// tie. Measured, 48 elements, tolerance 3e-2, items of 4096 against this rule
+// (us): 2^16 queries 115 / 79 (items of 512), 2^18 222 / 130 (1536), 5e5 223 /
+// 165 (2048), 2^20 and 2^22 the same (4096, remainders last). An ITEM_COST
+// below 256 picks items of 256 (2^16: 100 us); above 400 nothing moves.
 constexpr int64_t ITEM_COST = 400;
 
 int64_t item_length(const int64_t* offsets, int n_elements, int64_t cus) {
@@ -568,8 +571,8 @@ int noa_dcs_surrogate_eval(noa_dcs_mlp* net, const noa_dcs_element* elements, co
     hipLaunchKernelGGL(reset_counters_kernel, dim3(1), dim3(64), 0, s, counters);
     if (!items.empty()) {
         const unsigned grid = unsigned(std::min<int64_t>(int64_t(items.size()), int64_t(n_cus())));
-        hipLaunchKernelGGL(surrogate_dcs_kernel, dim3(grid), dim3(IWG), 0, s, K, q, d_els, d_items,
-                           uint32_t(items.size()), counters, o, c, net->packed, net->params);
+        hipLaunchKernelGGL(surrogate_dcs_kernel, dim3(grid), dim3(IWG), 0, s, c, K, q, d_els, d_items,
+                           uint32_t(items.size()), counters, o, net->packed, net->params);
     }
     if (int rc = check_hip(hipGetLastError(), "surrogate launch")) return rc;
     return ok();
