@@ -928,7 +928,7 @@ __device__ __forceinline__ double dcs_from_table(const EnvRow& a, const ElementC
     return r;
 }
 
-// One search of a half-wave (the same state in its 32 lanes).
+// One search of a half-wave, or its state at one node of the decision tree.
 enum SearchKind { SEARCH_NONE, SEARCH_EDGE, SEARCH_BRACKET, SEARCH_BISECT };
 constexpr double RESOLUTION = 1E-10;
 
@@ -969,21 +969,20 @@ struct Search {
                 xa = bit ? b : x;
         } else {
             const bool to_c = kind == SEARCH_EDGE ? bit == up : !bit;
+            if (kind == SEARCH_EDGE && bit) xb = x;
             if (to_c)
                 xc = x;
             else
                 xa = x;
         }
     }
-    // The true step with value v at point(): its outcome.
+    // The true step with value v at point(): its outcome, or -1 where the
+    // tree ends with it.
     __device__ __forceinline__ int step(double v) {
         int bit;
         if (kind == SEARCH_EDGE) {
             bit = v != 0;
-            if (bit) {
-                xb = point();
-                fb = v;
-            }
+            if (bit) fb = v;
         } else if (kind == SEARCH_BISECT) {
             bit = v < fb;
             if (bit) fb = v;
@@ -1015,6 +1014,7 @@ struct Search {
                     fb = fa;
                 else if (fc < fb)
                     fb = fc;
+                return -1;
             }
             return bit;
         }
@@ -1078,11 +1078,18 @@ __device__ __forceinline__ double hide(double v) {
 }
 
 __device__ __forceinline__ float envelope_max(const EnvRow& a, ElementPtr cp, const Globals& G, double K, double cutoff,
-                                               float alpha_f, double cs, Search* searches, const fm::Tab& tb) {
+                                               float alpha_f, double cs, Search* searches, double (*tree)[64],
+                                               const fm::Tab& tb) {
 #pragma clang fp contract(off)
     const ElementConsts& c0 = *(const ElementConsts*)cp;
     const int lane = threadIdx.x & 63;
     const int half = lane >> 5, node = lane & 31;
+    // the tree's nodes are numbered by level (children 2 node + 1 + outcome):
+    // node + 1 in binary is a one and the outcomes on the path to the node.
+    // last1, last0: the last node on that path with outcome 1 and 0, or -1
+    const int depth = 31 - __clz(node + 1);
+    const int last1 = ((node + 1) >> __ffs(node + 1)) - 1;
+    const int last0 = ((node + 1) >> __ffs(~(node + 1))) - 1;
     if (cs <= 0.) return 0.f;
     const double alpha = (double)alpha_f;
     double qmin, qmax;
@@ -1133,14 +1140,16 @@ __device__ __forceinline__ float envelope_max(const EnvRow& a, ElementPtr cp, co
             // xmax + log(1 - 10^-(i + 1))
             lnx = xmax + fm::log(1. - pow(10., double(-((lane < N_SCAN ? lane : 0) + 1))), tb);
         } else {
-            // node + 1 in binary: below its leading one, the path to this lane's node
+            // the search's state at this lane's node
             wave_lds_order();
             Search mine = s;
-            const int depth = 31 - __clz(node + 1);
 #pragma unroll 1
-            for (int l = 4; l >= 0; l--)
-                if (l < depth) mine.next((node + 1) >> l & 1);
+            for (int l = 3; l >= 0; l--)
+                if (l < depth && node < 31) mine.next((node + 1) >> l & 1);
             lnx = mine.point();
+            tree[0][lane] = mine.xa;
+            tree[1][lane] = mine.xb;
+            tree[2][lane] = mine.xc;
         }
         // -DCS x^alpha there
         const double x = fm::exp(lnx, tb);
@@ -1170,21 +1179,39 @@ __device__ __forceinline__ float envelope_max(const EnvRow& a, ElementPtr cp, co
         }
         const double v = -(d * wj) * (alpha == 0. ? 1. : fm::exp(alpha * lnx, tb));
 
-        if (!points) {  // walk the trees as far as their points have values
-            const int known = need || !asked;
-            int at = 0;
-            Search walk = s;
-#pragma unroll 1
-            for (int l = 0; l < 5; l++) {
-                const int from = 32 * half + at;
-                const double w = __shfl(v, from, 64);
-                const bool go = __shfl(known, from, 64) && at < 31 && !walk.done();
-                int bit = -1;
-                if (go) bit = walk.step(w);
-                at = bit < 0 ? 31 : 2 * at + 1 + bit;
-                at = at < 31 ? at : 31;
+        if (!points) {
+            // every node's own step, then the path through the outcomes; the
+            // last node on it holds the search's new state
+            const double up = __shfl(v, 32 * half + (last1 < 0 ? 0 : last1), 64);
+            const double down = __shfl(v, 32 * half + (last0 < 0 ? 0 : last0), 64);
+            Search mine = s;
+            mine.xa = tree[0][lane];
+            mine.xb = tree[1][lane];
+            mine.xc = tree[2][lane];
+            mine.i += depth;
+            if (last1 >= 0) {
+                mine.fa = up;
+                if (mine.kind != SEARCH_BRACKET) mine.fb = up;
             }
-            put(s, walk);
+            if (last0 >= 0) mine.fc = down;
+            const bool go = (need || !asked) && node < 31 && !mine.done();
+            const int bit = go ? mine.step(v) : -1;
+            const uint32_t goes = uint32_t(__ballot(go) >> (32 * half));
+            const uint32_t ends = uint32_t(__ballot(bit < 0) >> (32 * half));
+            const uint32_t ones = uint32_t(__ballot(bit > 0) >> (32 * half));
+            int at = 0, last = -1;
+#pragma unroll
+            for (int l = 0; l < 5; l++) {
+                if (at < 31 && (goes >> at & 1)) {
+                    last = at;
+                    at = (ends >> at & 1) ? 31 : 2 * at + 1 + int(ones >> at & 1);
+                } else {
+                    at = 31;
+                }
+            }
+            wave_lds_order();
+            if (node == last) s = mine;
+            wave_lds_order();
         }
 
         // what comes next (the same in every lane): `settled` counts the
@@ -1308,19 +1335,27 @@ struct EnvelopeArgs {
 };
 static_assert(sizeof(EnvelopeArgs) <= MAX_KERNARG, "48 elements and the grid in one launch");
 
+// The row's nodes and the two table rows it reads. (Sized by the grid, not by
+// MAX_X: the LDS then holds 12 workgroups per CU, three waves per SIMD, up to
+// ~145 nodes.)
+constexpr int ENVELOPE_LDS = 5;
+
 // One 64-lane workgroup per (process, block element j, kinetic energy k) row
 // of the launch's element block; env[2 r + 1] of table row r. Rows start
 // longest first: the first element's (element 0 takes the model at every
 // point), then pair production's, and the highest energies (which scan) first.
 template <int WAVES>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(WAVES))) void pumas_envelope_kernel(EnvelopeArgs by_value) {
-    __shared__ float xt[MAX_X];
-    __shared__ float ra[2 * MAX_X], rb[2 * MAX_X];
+    extern __shared__ float row_lds[];  // ENVELOPE_LDS floats per grid node
     __shared__ Search searches[2];
+    __shared__ double tree[3][64];
     NOA_PUMAS_TABLES();
     const auto args = (const __attribute__((address_space(4))) EnvelopeArgs*)__builtin_amdgcn_kernarg_segment_ptr();
     const Globals G = *(const Globals*)&args->G;
     const int32_t n_K = args->n_K, n_el = args->n_el, n_blk = args->n_blk, e0 = args->e0, n_x = args->n_x;
+    float* const xt = row_lds;
+    float* const ra = xt + n_x;
+    float* const rb = ra + 2 * n_x;
     const double mass = args->mass;
     const double* __restrict__ Ks = args->Ks;
     const float* __restrict__ table = args->table;
@@ -1381,7 +1416,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(WAVES))) voi
     a.below = i0 < 0;
     const ElementPtr cp = &args->blk.e[j];
     a.rl = rad_log(cp->Z);
-    const float v = envelope_max(a, cp, G, K, args->cutoff, env[2 * r], csn ? csn[r] : 1., searches, tb);
+    const float v = envelope_max(a, cp, G, K, args->cutoff, env[2 * r], csn ? csn[r] : 1., searches, tree, tb);
     if (threadIdx.x == 0) env[2 * r + 1] = v;
 }
 
@@ -1545,7 +1580,7 @@ int noa_pumas_dcs_table(const double* Z, const double* A, int32_t n_elements, do
             // exceed the 2048 that two hold: 1963 against 2115 us for 48
             // elements x 146 energies, 766 against 718 for 1 x 30
             hipLaunchKernelGGL((rows > 2048 ? &pumas::pumas_envelope_kernel<3> : &pumas::pumas_envelope_kernel<2>),
-                               dim3(rows), dim3(64), 0, stream, args);
+                               dim3(rows), dim3(64), size_t(pumas::ENVELOPE_LDS) * g.n * sizeof(float), stream, args);
             if (int rc = check_hip(hipGetLastError(), "pumas_envelope_kernel")) return rc;
         }
     }
