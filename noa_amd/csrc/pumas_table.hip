@@ -175,7 +175,16 @@ __device__ double dilog(double x, const fm::Tab& tb) {
     if ((x == -1.) || (1. - x == 0.)) return -PI12;
     const double T = -x;
     double A, S, Y;
-    if (T <= -2) {
+    if (T > -1. && T < 0.) {
+        // the range of both of pair production's arguments: the reductions on
+        // either side of -0.5 as one, since the lanes of a wave take both
+        const bool big = T <= -0.5;
+        const double T1 = 1. + T;
+        Y = (big ? -T1 : -T) / (big ? T : T1);
+        S = big ? 1. : -1.;
+        const double l = fm::log(-T, tb), l1 = fm::log(T1, tb);
+        A = big ? -PI6 + l * (-0.5 * l + l1) : 0.5 * (l1 * l1);
+    } else if (T <= -2) {
         Y = -1. / (1. + T);
         S = 1.;
         const double l1 = fm::log(-T, tb), l2 = fm::log(1. + 1. / T, tb);
@@ -185,16 +194,6 @@ __device__ double dilog(double x, const fm::Tab& tb) {
         S = -1.;
         A = fm::log(-T, tb);
         A = -PI6 + A * (A + fm::log(1. + 1. / T, tb));
-    } else if (T <= -0.5) {
-        Y = -(1. + T) / T;
-        S = 1.;
-        A = fm::log(-T, tb);
-        A = -PI6 + A * (-0.5 * A + fm::log(1. + T, tb));
-    } else if (T < 0.) {
-        Y = -T / (1. + T);
-        S = -1.;
-        const double l = fm::log(1 + T, tb);
-        A = 0.5 * (l * l);
     } else if (T <= 1.) {
         Y = T;
         S = 1.;
@@ -336,16 +335,15 @@ __device__ double pair_d2_ssr(const PairQ& s, const Globals& G, double rho, cons
     const double sx = s.rl * s.Z13 * sqrt(xi1);
     const double sx6 = s.rl * s.Z13 * G.e_16 * sqrt(xi1);
     const double re = De / Be;
-    double Le1, Le2;
-    if (re > 0.) {
-        const double Xe = (re < 100) ? fm::exp(-re, tb) : 0.;
-        Le1 = fm::log(sx / (Xe + c05), tb) - re - 0.5 * fm::log(Xe + s.me_dn2 * xi1, tb);
-        Le2 = fm::log(sx6 / (Xe + c13), tb) - re - 0.5 * fm::log(Xe + s.me_dn2 * G.e_13 * xi1, tb);
-    } else {
-        const double Xi = (re > -100) ? fm::exp(re, tb) : 0.;
-        Le1 = fm::log(sx / (1. + Xi * c05), tb) - 0.5 * re - 0.5 * fm::log(1. + Xi * s.me_dn2 * xi1, tb);
-        Le2 = fm::log(sx6 / (1. + Xi * c13), tb) - 0.5 * re - 0.5 * fm::log(1. + Xi * s.me_dn2 * G.e_13 * xi1, tb);
-    }
+    // the forms for re > 0 and re <= 0 share their logarithms (and the muon
+    // diagram's): nodes of one wave take both
+    const bool pe = re > 0.;
+    const double Xe = (fabs(re) < 100) ? fm::exp(-fabs(re), tb) : 0.;
+    const double be = pe ? Xe : 1.;
+    const double fe = pe ? s.me_dn2 : Xe * s.me_dn2;
+    const double ree = pe ? re : 0.5 * re;
+    const double Le1 = fm::log(sx / (be + (pe ? c05 : Xe * c05)), tb) - ree - 0.5 * fm::log(be + fe * xi1, tb);
+    const double Le2 = fm::log(sx6 / (be + (pe ? c13 : Xe * c13)), tb) - ree - 0.5 * fm::log(be + fe * G.e_13 * xi1, tb);
     double diagram_e = s.pref * (Ce1 * Le1 + Ce2 * Le2);
     if (diagram_e < 0.) diagram_e = 0.;
 
@@ -361,16 +359,12 @@ __device__ double pair_d2_ssr(const PairQ& s, const Globals& G, double rho, cons
                       (1. - rho2 - beta / 2. * (1. + rho2) + omr / (2. * xi) * beta) * xi / xi1;
     const double num = s.m / SSR_ME * s.rl * s.Z13 / s.d_n;
     const double rm = Dm / Bm;
-    double Lm1, Lm2;
-    if (rm > 0.) {
-        const double Xm = (rm < 100) ? fm::exp(-rm, tb) : 0.;
-        Lm1 = fm::log(num / (Xm + c05), tb) - rm;
-        Lm2 = fm::log(num / (Xm + c13), tb) - rm;
-    } else {
-        const double Xv = (rm > -100) ? fm::exp(rm, tb) : 0.;
-        Lm1 = fm::log(num / (1. + c05 * Xv), tb);
-        Lm2 = fm::log(num / (1. + c13 * Xv), tb);
-    }
+    const bool pm = rm > 0.;
+    const double Xm = (fabs(rm) < 100) ? fm::exp(-fabs(rm), tb) : 0.;
+    const double bm = pm ? Xm : 1.;
+    const double rmm = pm ? rm : 0.;
+    const double Lm1 = fm::log(num / (bm + (pm ? c05 : c05 * Xm)), tb) - rmm;
+    const double Lm2 = fm::log(num / (bm + (pm ? c13 : c13 * Xm)), tb) - rmm;
     double diagram_mu = s.pref * s.me_m2 * (Cm1 * Lm1 + Cm2 * Lm2);
     if (diagram_mu < 0.) diagram_mu = 0.;
     return (diagram_e + diagram_mu) * 1E-01 / s.energy;
@@ -733,6 +727,14 @@ __global__ __launch_bounds__(64) void pumas_alpha_fill_kernel(float* __restrict_
 // 5 x 12 (pair production), 7 x 9 (photonuclear); bremsstrahlung has no nodes.
 __device__ __forceinline__ int model_batch(int process) { return process == 0 ? 64 : process == 1 ? 5 : 7; }
 
+// What a lane pushed to this one (several to one lane: one of them; none: 0).
+__device__ __forceinline__ double push_to(double v, int lane) {
+    const uint64_t u = __builtin_bit_cast(uint64_t, v);
+    const uint32_t lo = uint32_t(__builtin_amdgcn_ds_permute(4 * lane, int(uint32_t(u))));
+    const uint32_t hi = uint32_t(__builtin_amdgcn_ds_permute(4 * lane, int(uint32_t(u >> 32))));
+    return __builtin_bit_cast(double, (uint64_t(hi) << 32) | lo);
+}
+
 // The m^2/kg model DCS of one (K, q) per lane, for the lanes with need set (K
 // the same in every lane; the other lanes get 0). A wave takes model_batch
 // evaluations at a time, a group of lanes each: every lane of a group forms
@@ -750,22 +752,18 @@ __device__ __forceinline__ double dcs_wave(int process, const ElementConsts& c, 
         const int nodes = process == 1 ? 12 : 9;
         const int per = model_batch(process);
         const int group = lane / nodes, node = lane - group * nodes;
-        unsigned long long todo = __ballot(need);
-        while (todo) {
-            // the group's evaluation is the group-th lane still to do
-            unsigned long long m = todo;
-            int mine = -1, owner_group = -1;
-            for (int i = 0; i < per && m; i++) {
-                const int l = __ffsll((long long)m) - 1;
-                m &= m - 1;
-                if (i == group) mine = l;
-                if (l == lane) owner_group = i;
-            }
-            todo = m;
-            const double qg = __shfl(q, mine < 0 ? 0 : mine, 64);
+        const unsigned long long todo = __ballot(need);
+        const int total = __popcll(todo);
+        const int rank = __popcll(todo & ((1ull << lane) - 1));
+        for (int base = 0; base < total; base += per) {
+            // the group's evaluation is that of the group-th lane still to do,
+            // which hands its q to lane `group`
+            const int mine = rank - base;
+            const int owner_group = need && mine >= 0 && mine < per ? mine : -1;
+            const double qg = __shfl(push_to(q, owner_group < 0 ? 63 : owner_group), group, 64);
             double term = 0.;
             int skip = 1;
-            if (mine >= 0) {
+            if (group < min(per, total - base)) {
                 if (process == 1)
                     pair_term(c, rl, G, mass, K, qg, zeta, node, &term, &skip, tb);
                 else
@@ -779,11 +777,9 @@ __device__ __forceinline__ double dcs_wave(int process, const ElementConsts& c, 
                 for (int i = 0; i < 12; i++) sum -= __shfl(term, first + i, 64);
                 if (skipped) sum = 0.;
             } else {
+                if (skip) term = 0.;
 #pragma unroll
-                for (int i = 0; i < 9; i++) {
-                    const double t = __shfl(term, first + i, 64);
-                    if (!__shfl(skip, first + i, 64)) sum += t;
-                }
+                for (int i = 0; i < 9; i++) sum += __shfl(term, first + i, 64);
             }
             if (owner_group >= 0) d = (sum < 0) ? 0. : sum;
         }
@@ -829,6 +825,15 @@ __device__ __forceinline__ double dcs_wave(int process, const ElementConsts& c, 
 // the registers, 24 elements per launch and pair production's rows, the
 // longest, first: 1980 us, of which the two envelope launches are 1650.
 
+// v of one lane, as a wave-uniform (scalar) value.
+__device__ __forceinline__ double from_lane(double v, int lane) {
+    const uint64_t u = __builtin_bit_cast(uint64_t, v);
+    const int l = __builtin_amdgcn_readfirstlane(lane);
+    const uint32_t lo = uint32_t(__builtin_amdgcn_readlane(int(uint32_t(u)), l));
+    const uint32_t hi = uint32_t(__builtin_amdgcn_readlane(int(uint32_t(u >> 32)), l));
+    return __builtin_bit_cast(double, (uint64_t(hi) << 32) | lo);
+}
+
 struct EnvRow {
     int process;
     double mass;
@@ -841,18 +846,20 @@ struct EnvRow {
     const float* ra;  // row i0 (or the last row)
     const float* rb;  // row i0 + 1 (or the last row again)
     float h0, h1;
+    double qmin, qlow, qmax;  // table_range
     bool below;  // K below the grid (never the case for a row's own energy)
 };
 
-__device__ __forceinline__ void bracketf(const float* table, float value, int* p1, int* p2) {
-    while (true) {
-        const int i3 = (*p1 + *p2) / 2;
-        if (value >= table[i3])
-            *p1 = i3;
-        else
-            *p2 = i3;
-        if (*p2 - *p1 < 2) break;
+// The cell of the nodes t[0..n-1] that holds x (t[0] <= x < t[n - 1]), or 0 for
+// NaN: four parts a step, so that three loads are in flight.
+__device__ __forceinline__ int cell(const float* t, int n, float x) {
+    int i = 0;
+    for (int d = n - 1; d > 1;) {
+        d = (d + 3) / 4;
+        const float a = t[min(i + d, n - 1)], b = t[min(i + 2 * d, n - 1)], c = t[min(i + 3 * d, n - 1)];
+        i += d * (int(x >= a) + int(x >= b) + int(x >= c));
     }
+    return i;
 }
 
 // table_index without a context (pumas.c:4249-4290, 4299-4306).
@@ -872,60 +879,57 @@ __device__ __forceinline__ int table_index(const double* table, int n_K, double 
     return i1;
 }
 
-// The interpolated DCS at q without its factor K / (K + m), or *need set where
-// it is the model's.
-__device__ __forceinline__ double dcs_from_table(const EnvRow& a, const ElementConsts& c, double K, double q, bool* need) {
+// The range of dcs_evaluate (pumas.c:11319-11349): 0 outside [qmin, qmax], the
+// model below qlow.
+__device__ __forceinline__ void table_range(EnvRow& a, const ElementConsts& c, double K) {
 #pragma clang fp contract(off)
-    double qlow = 0., qmin, qmax;
-    *need = false;
     if (a.process == 2) {
-        qmin = PION_MASS + 0.5 * PION_MASS * PION_MASS / NUCLEON_MASS;
-        qmax = K + a.mass - 0.5 * (NUCLEON_MASS + a.mass * a.mass / NUCLEON_MASS);
-        if ((q < qmin) || (q > qmax)) return 0.;
-        qlow = 2 * qmin;
+        a.qmin = PION_MASS + 0.5 * PION_MASS * PION_MASS / NUCLEON_MASS;
+        a.qmax = K + a.mass - 0.5 * (NUCLEON_MASS + a.mass * a.mass / NUCLEON_MASS);
+        a.qlow = 2 * a.qmin;
     } else {
-        qmin = 4. * ELECTRON_MASS;
-        qmax = K + q_offset(a.mass, PAIR_SQRTE, c);
-        if (a.process == 1)
-            qlow = 4 * qmin;
-        else
-            qmin = 0.;
-        if ((q < qmin) || (q > qmax)) return 0.;
+        a.qmin = a.process == 1 ? 4. * ELECTRON_MASS : 0.;
+        a.qmax = K + q_offset(a.mass, PAIR_SQRTE, c);
+        a.qlow = 4 * a.qmin;
     }
-    *need = true;
-    if (q < qlow) return 0.;
+    a.qmax = from_lane(a.qmax, 0);
+}
+
+// The interpolated DCS at q without its factor K / (K + m), or *need set where
+// it is the model's. Without early returns: a wave's lanes rarely differ in
+// them, and each cost a branch.
+__device__ __forceinline__ double dcs_from_table(const EnvRow& a, double K, double q, bool* need) {
+#pragma clang fp contract(off)
+    const bool in = !((q < a.qmin) || (q > a.qmax));
     const int nx = a.n;
-    const float xmin = a.xt[0], xmax = a.xt[nx - 1];
     const float x = logf((float)(q / K));
-    if ((x < xmin) || (x >= xmax)) return 0.;
-    int ix = 0, tmpi = nx - 1;
-    bracketf(a.xt, x, &ix, &tmpi);
-    if ((ix < 0) || (ix >= nx - 1)) return 0.;
-    if (a.below) return 0.;
-    float p00 = a.ra[2 * ix], m00 = a.ra[2 * ix + 1], p01 = a.ra[2 * ix + 2], m01 = a.ra[2 * ix + 3];
-    float p10 = a.rb[2 * ix], m10 = a.rb[2 * ix + 1], p11 = a.rb[2 * ix + 2], m11 = a.rb[2 * ix + 3];
-    const float h0 = a.h0, h1 = a.h1;
-    if (((p00 == 0.f) && (m00 == 0.f)) || ((p01 == 0.f) && (m01 == 0.f)) || ((p10 == 0.f) && (m10 == 0.f)) ||
-        ((p11 == 0.f) && (m11 == 0.f)))
-        return 0.;
-    *need = false;
-    const float x0 = a.xt[ix];
-    const float x1 = a.xt[ix + 1];
-    const float dx = x1 - x0;
-    m00 *= dx;
-    m01 *= dx;
-    const float t = (x - x0) / dx;
-    const float c02 = -3 * (p00 - p01) - 2 * m00 - m01;
-    const float c03 = 2 * (p00 - p01) + m00 + m01;
-    float r = expf(p00 + t * (m00 + t * (c02 + t * c03))) * h0;
-    if (h1 > 0.f) {
-        m10 *= dx;
-        m11 *= dx;
-        const float c12 = -3 * (p10 - p11) - 2 * m10 - m11;
-        const float c13 = 2 * (p10 - p11) + m10 + m11;
-        r += expf(p10 + t * (m10 + t * (c12 + t * c13))) * h1;
+    bool ok = in && !(q < a.qlow) && !((x < a.xt[0]) || (x >= a.xt[nx - 1])) && !a.below;
+    float r = 0.f;
+    if (__ballot(ok)) {
+        const int ix = cell(a.xt, nx, ok ? x : a.xt[0]);
+        const float p00 = a.ra[2 * ix], p01 = a.ra[2 * ix + 2], p10 = a.rb[2 * ix], p11 = a.rb[2 * ix + 2];
+        float m00 = a.ra[2 * ix + 1], m01 = a.ra[2 * ix + 3], m10 = a.rb[2 * ix + 1], m11 = a.rb[2 * ix + 3];
+        ok = ok & !(((p00 == 0.f) & (m00 == 0.f)) | ((p01 == 0.f) & (m01 == 0.f)) | ((p10 == 0.f) & (m10 == 0.f)) |
+                    ((p11 == 0.f) & (m11 == 0.f)));
+        const float x0 = a.xt[ix];
+        const float x1 = a.xt[ix + 1];
+        const float dx = x1 - x0;
+        m00 *= dx;
+        m01 *= dx;
+        const float t = (x - x0) / dx;
+        const float c02 = -3 * (p00 - p01) - 2 * m00 - m01;
+        const float c03 = 2 * (p00 - p01) + m00 + m01;
+        r = expf(p00 + t * (m00 + t * (c02 + t * c03))) * a.h0;
+        if (a.h1 > 0.f) {
+            m10 *= dx;
+            m11 *= dx;
+            const float c12 = -3 * (p10 - p11) - 2 * m10 - m11;
+            const float c13 = 2 * (p10 - p11) + m10 + m11;
+            r += expf(p10 + t * (m10 + t * (c12 + t * c13))) * a.h1;
+        }
     }
-    return r;
+    *need = in && !ok;
+    return ok ? r : 0.f;
 }
 
 // One search of a half-wave, or its state at one node of the decision tree.
@@ -1054,15 +1058,6 @@ __device__ __forceinline__ void put(Search& to, const Search& s) {
     wave_lds_order();
 }
 
-// v of one lane, as a wave-uniform (scalar) value.
-__device__ __forceinline__ double from_lane(double v, int lane) {
-    const uint64_t u = __builtin_bit_cast(uint64_t, v);
-    const int l = __builtin_amdgcn_readfirstlane(lane);
-    const uint32_t lo = uint32_t(__builtin_amdgcn_readlane(int(uint32_t(u)), l));
-    const uint32_t hi = uint32_t(__builtin_amdgcn_readlane(int(uint32_t(u >> 32)), l));
-    return __builtin_bit_cast(double, (uint64_t(hi) << 32) | lo);
-}
-
 // The row's constants in the kernel-argument segment, re-read where they are
 // used: an empty asm hides the pointer, and hide() a value, so that what
 // follows from them alone is not formed before the search and held in
@@ -1155,23 +1150,21 @@ __device__ __forceinline__ float envelope_max(const EnvRow& a, ElementPtr cp, co
         const double x = fm::exp(lnx, tb);
         const double q = x * K;
         bool need;
-        double d = dcs_from_table(a, c, K, q, &need);
+        double d = dcs_from_table(a, K, q, &need);
         const bool asked = need;
         if (points) {
             need = need && lane < points;
         } else {
             need = need && !s.done() && node < 31;
             const unsigned long long m = __ballot(need);
-            const uint32_t m0 = uint32_t(m), m1 = uint32_t(m >> 32);
-            // the model's points of as many levels (of each half's tree) as one batch takes
-            int l0 = 5, l1 = 5;
-            while (__popc(m0 & ((1u << ((1 << l0) - 1)) - 1)) + __popc(m1 & ((1u << ((1 << l1) - 1)) - 1)) > batch) {
-                if (m1 && (l1 > l0 || !m0))
-                    l1--;
-                else
-                    l0--;
+            if (m) {
+                // the model's points in the order of their levels, half 1 before
+                // half 0, as many as one batch takes
+                const auto levels = [](int l) { return (1u << ((1 << l) - 1)) - 1; };
+                const uint32_t own = uint32_t(m >> (32 * half)), other = uint32_t(m >> (32 * (half ^ 1)));
+                const int before = __popc(own & ((1u << node) - 1)) + __popc(other & levels(depth + 1 - half));
+                need = need && before < batch;
             }
-            need = need && node < (1 << (half ? l1 : l0)) - 1;
         }
         if (__ballot(need)) {
             const double md = dcs_wave(a.process, c, a.rl, G, mass, K, zeta, q, need, tb);
@@ -1416,6 +1409,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(WAVES))) voi
     a.below = i0 < 0;
     const ElementPtr cp = &args->blk.e[j];
     a.rl = rad_log(cp->Z);
+    table_range(a, *(const ElementConsts*)cp, K);
     const float v = envelope_max(a, cp, G, K, args->cutoff, env[2 * r], csn ? csn[r] : 1., searches, tree, tb);
     if (threadIdx.x == 0) env[2 * r + 1] = v;
 }
