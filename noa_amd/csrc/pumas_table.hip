@@ -816,14 +816,16 @@ __device__ __forceinline__ double dcs_wave(int process, const ElementConsts& c, 
 // element 0's search sees zero nodes and takes the model everywhere; the
 // kernel does the same.
 //
-// What bounds it is the length of a row's chain of rounds (about 30, up to 60
-// where every point needs the model, of ~1000 to 2500 dependent instructions
-// each), with two or three waves per SIMD to overlap. Measured for 48 elements
-// x 146 energies, the whole table call: one point per step for the whole wave
-// 10,600 us; trees of one search per wave 4113; two searches side by side with
-// the table log / exp 2810; the rows' constants and the searches kept out of
-// the registers, 24 elements per launch and pair production's rows, the
-// longest, first: 1980 us, of which the two envelope launches are 1650.
+// What bounds it is the instructions of a row's chain of rounds (about 20, up
+// to 60 where every point needs the model, of ~500 to 2000 vector instructions
+// each), with three waves per SIMD to overlap: the vector units are busy 72% of
+// the launch. Measured for 48 elements x 146 energies, the whole table call:
+// one point per step for the whole wave 10,600 us; trees of one search per wave
+// 4113; two searches side by side with the table log / exp 2810; the rows'
+// constants and the searches kept out of the registers 1980; one launch for 48
+// elements 1334; a tree's nodes taking their steps at once 1217; selections for
+// branches 1177; model batches filled point by point 1105; a copy of the search
+// per process and the longest rows first 960.
 
 // v of one lane, as a wave-uniform (scalar) value.
 __device__ __forceinline__ double from_lane(double v, int lane) {
@@ -1072,6 +1074,7 @@ __device__ __forceinline__ double hide(double v) {
     return v;
 }
 
+template <int Process>
 __device__ __forceinline__ float envelope_max(const EnvRow& a, ElementPtr cp, const Globals& G, double K, double cutoff,
                                                float alpha_f, double cs, Search* searches, double (*tree)[64],
                                                const fm::Tab& tb) {
@@ -1088,11 +1091,11 @@ __device__ __forceinline__ float envelope_max(const EnvRow& a, ElementPtr cp, co
     if (cs <= 0.) return 0.f;
     const double alpha = (double)alpha_f;
     double qmin, qmax;
-    if (a.process == 2) {  // dcs_get_range (pumas.c:11047-11056)
+    if (Process == 2) {  // dcs_get_range (pumas.c:11047-11056)
         qmin = PION_MASS + 0.5 * PION_MASS * PION_MASS / NUCLEON_MASS;
         qmax = K + a.mass - 0.5 * (NUCLEON_MASS + a.mass * a.mass / NUCLEON_MASS);
     } else {
-        qmin = (a.process == 0) ? 0. : 4. * ELECTRON_MASS;
+        qmin = (Process == 0) ? 0. : 4. * ELECTRON_MASS;
         qmax = K + q_offset(a.mass, PAIR_SQRTE, c0);
     }
     double xmin = qmin / K;
@@ -1101,8 +1104,8 @@ __device__ __forceinline__ float envelope_max(const EnvRow& a, ElementPtr cp, co
     double xmax = fm::log(qmax / K, tb);
     if (xmin >= xmax) return 0.f;
     const double wj = K / (K + a.mass);
-    const int batch = model_batch(a.process);
-    const double zeta = a.process == 1 ? pair_zeta(c0, a.mass, K, tb) : 0.;
+    const int batch = model_batch(Process);
+    const double zeta = Process == 1 ? pair_zeta(c0, a.mass, K, tb) : 0.;
 
     // ENDS: the range ends and the midpoint; EDGE_LOW, BACKOFF, EDGE_HIGH: the
     // ends' searches; MID: the midpoint between moved ends; PAIR: the two
@@ -1167,7 +1170,7 @@ __device__ __forceinline__ float envelope_max(const EnvRow& a, ElementPtr cp, co
             }
         }
         if (__ballot(need)) {
-            const double md = dcs_wave(a.process, c, a.rl, G, mass, K, zeta, q, need, tb);
+            const double md = dcs_wave(Process, c, a.rl, G, mass, K, zeta, q, need, tb);
             if (need) d = md;
         }
         const double v = -(d * wj) * (alpha == 0. ? 1. : fm::exp(alpha * lnx, tb));
@@ -1303,7 +1306,7 @@ __device__ __forceinline__ float envelope_max(const EnvRow& a, ElementPtr cp, co
             phase = PAIR;
             continue;
         }
-        if (!((a.process == 1) && (K >= 1E+07))) break;
+        if (!((Process == 1) && (K >= 1E+07))) break;
         phase = SCAN;
     }
     double fopt = (fopt0 < fopt1) ? fopt0 : fopt1;
@@ -1336,7 +1339,11 @@ constexpr int ENVELOPE_LDS = 5;
 // One 64-lane workgroup per (process, block element j, kinetic energy k) row
 // of the launch's element block; env[2 r + 1] of table row r. Rows start
 // longest first: the first element's (element 0 takes the model at every
-// point), then pair production's, and the highest energies (which scan) first.
+// point), then pair production's, and of each the lowest energies first: those
+// just above the threshold, with few valid table nodes, take 2 to 3 times as
+// long as the highest. The launch's length over its rows' sum is 1.20 with the
+// highest energies first and 1.10 so (1095 against 1020 us for 48 elements x
+// 146 energies).
 template <int WAVES>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(WAVES))) void pumas_envelope_kernel(EnvelopeArgs by_value) {
     extern __shared__ float row_lds[];  // ENVELOPE_LDS floats per grid node
@@ -1368,7 +1375,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(WAVES))) voi
         b /= n_blk - 1;
     }
     p %= 3;
-    const int k = n_K - 1 - int(b);
+    const int k = int(b);
     const int e = e0 + j;
     const int64_t pe = int64_t(p) * n_el + e;
     const int64_t r = pe * n_K + k;
@@ -1410,7 +1417,11 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(WAVES))) voi
     const ElementPtr cp = &args->blk.e[j];
     a.rl = rad_log(cp->Z);
     table_range(a, *(const ElementConsts*)cp, K);
-    const float v = envelope_max(a, cp, G, K, args->cutoff, env[2 * r], csn ? csn[r] : 1., searches, tree, tb);
+    const float alpha = env[2 * r];
+    const double cs = csn ? csn[r] : 1.;
+    const float v = p == 0   ? envelope_max<0>(a, cp, G, K, args->cutoff, alpha, cs, searches, tree, tb)
+                    : p == 1 ? envelope_max<1>(a, cp, G, K, args->cutoff, alpha, cs, searches, tree, tb)
+                             : envelope_max<2>(a, cp, G, K, args->cutoff, alpha, cs, searches, tree, tb);
     if (threadIdx.x == 0) env[2 * r + 1] = v;
 }
 
