@@ -182,18 +182,18 @@ __device__ double dilog(double x, const fm::Tab& tb) {
         const double T1 = 1. + T;
         Y = (big ? -T1 : -T) / (big ? T : T1);
         S = big ? 1. : -1.;
-        const double l = fm::log(-T, tb), l1 = fm::log(T1, tb);
+        const double l = fm::log_sel(-T, tb), l1 = fm::log_sel(T1, tb);
         A = big ? -PI6 + l * (-0.5 * l + l1) : 0.5 * (l1 * l1);
     } else if (T <= -2) {
         Y = -1. / (1. + T);
         S = 1.;
-        const double l1 = fm::log(-T, tb), l2 = fm::log(1. + 1. / T, tb);
+        const double l1 = fm::log_sel(-T, tb), l2 = fm::log_sel(1. + 1. / T, tb);
         A = -PI3 + 0.5 * (l1 * l1 - l2 * l2);
     } else if (T < -1.) {
         Y = -1. - T;
         S = -1.;
-        A = fm::log(-T, tb);
-        A = -PI6 + A * (A + fm::log(1. + 1. / T, tb));
+        A = fm::log_sel(-T, tb);
+        A = -PI6 + A * (A + fm::log_sel(1. + 1. / T, tb));
     } else if (T <= 1.) {
         Y = T;
         S = 1.;
@@ -201,7 +201,7 @@ __device__ double dilog(double x, const fm::Tab& tb) {
     } else {
         Y = 1. / T;
         S = -1.;
-        const double l = fm::log(T, tb);
+        const double l = fm::log_sel(T, tb);
         A = PI6 + 0.5 * (l * l);
     }
     const double H = Y + Y - 1;
@@ -230,13 +230,13 @@ __device__ double brems_ssr(const ElementConsts& c, double rl, const Globals& G,
     const double rl_inel = (Z == 1.) ? 446. : 1429.;
     const double delta = m * m * v / (2. * energy * (1. - v));
     const double rz = rl * Z13;
-    double phi1 = fm::log(rz * (m / SSR_ME) / (1. + rz * G.e05 * delta / SSR_ME), tb);
-    double phi2 = fm::log(rz * G.e_16 * (m / SSR_ME) / (1. + rz * G.e13 * delta / SSR_ME), tb);
+    double phi1 = fm::log_sel(rz * (m / SSR_ME) / (1. + rz * G.e05 * delta / SSR_ME), tb);
+    double phi2 = fm::log_sel(rz * G.e_16 * (m / SSR_ME) / (1. + rz * G.e13 * delta / SSR_ME), tb);
     const double iz = 1. - 1. / Z;
     phi1 -= c.b_delta1 * iz;
     phi2 -= c.b_delta2 * iz;
-    const double s1 = fm::log(m / delta / (m * delta / (SSR_ME * SSR_ME) + SSR_SQRTE), tb);
-    const double s2 = fm::log(1. + SSR_ME / (delta * rl_inel * Z13 * Z13 * SSR_SQRTE), tb);
+    const double s1 = fm::log_sel(m / delta / (m * delta / (SSR_ME * SSR_ME) + SSR_SQRTE), tb);
+    const double s2 = fm::log_sel(1. + SSR_ME / (delta * rl_inel * Z13 * Z13 * SSR_SQRTE), tb);
     const double s_atomic = (4. / 3. * (1. - v) + v * v) * (s1 - s2);
     double s_rad;
     if (v < .0 || v > 1.) {
@@ -247,12 +247,12 @@ __device__ double brems_ssr(const ElementConsts& c, double rl, const Globals& G,
         s_rad = 0.1642 + 132.573 * v + -585.361 * v * v + 1407.77 * v * v * v;
     } else if (v < 0.9) {
         s_rad = -2.8922 + -19.0156 * v + 57.698 * v * v;
-        const double t = fm::log(1. - v, tb);
-        s_rad += -63.418 * v * fm::log(v, tb) + 14.1166 * t + 1.84206 * t * t;
+        const double t = fm::log_sel(1. - v, tb);
+        s_rad += -63.418 * v * fm::log_sel(v, tb) + 14.1166 * t + 1.84206 * t * t;
     } else {
         s_rad = 2134.19 + 581.823 * v + -2708.85 * v * v;
-        const double t = fm::log(1. - v, tb);
-        s_rad += 4767.05 * v * fm::log(v, tb) + 1.52918 * t + 0.361933 * t * t;
+        const double t = fm::log_sel(1. - v, tb);
+        s_rad += 4767.05 * v * fm::log_sel(v, tb) + 1.52918 * t + 0.361933 * t * t;
     }
     const double result =
         ((2. - 2. * v + v * v) * phi1 - 2. / 3. * (1. - v) * phi2) + 1. / Z * s_atomic + 0.25 * ALPHA_EM * phi1 * s_rad;
@@ -282,8 +282,8 @@ __device__ __forceinline__ double pair_zeta(const ElementConsts& c, double m_gev
         g1 = 1.95E-05;
         g2 = 5.3E-05;
     }
-    const double zeta1 = (0.073 * fm::log(energy / m / (1. + g1 * c.Z23 * energy / m), tb) - 0.26);
-    const double zeta2 = (0.058 * fm::log(energy / m / (1 + g2 / c.Z13m * energy / m), tb) - 0.14);
+    const double zeta1 = (0.073 * fm::log_sel(energy / m / (1. + g1 * c.Z23 * energy / m), tb) - 0.26);
+    const double zeta2 = (0.058 * fm::log_sel(energy / m / (1 + g2 / c.Z13m * energy / m), tb) - 0.14);
     return ((zeta1 > 0.) && (zeta2 > 0.)) ? zeta1 / zeta2 : 0.;
 }
 
@@ -326,7 +326,7 @@ __device__ double pair_d2_ssr(const PairQ& s, const Globals& G, double rho, cons
     const double c13 = 2. * SSR_ME * G.e13 * s.rl * s.Z13 * xi1 / w;
 
     // electron diagram
-    const double lxi_i = fm::log(1. + 1. / xi, tb);
+    const double lxi_i = fm::log_sel(1. + 1. / xi, tb);
     const double Pe = (2. + rho2) * (1. + beta) + xi * (3. + rho2);
     const double Be = Pe * lxi_i + (1. - rho2 - beta) / xi1 - (3. + rho2);
     const double Ce2 = (omr * (1. + beta) + xi * (3. - rho2)) * lxi_i + 2. * (1. - beta - rho2) / xi1 - (3. - rho2);
@@ -342,13 +342,13 @@ __device__ double pair_d2_ssr(const PairQ& s, const Globals& G, double rho, cons
     const double be = pe ? Xe : 1.;
     const double fe = pe ? s.me_dn2 : Xe * s.me_dn2;
     const double ree = pe ? re : 0.5 * re;
-    const double Le1 = fm::log(sx / (be + (pe ? c05 : Xe * c05)), tb) - ree - 0.5 * fm::log(be + fe * xi1, tb);
-    const double Le2 = fm::log(sx6 / (be + (pe ? c13 : Xe * c13)), tb) - ree - 0.5 * fm::log(be + fe * G.e_13 * xi1, tb);
+    const double Le1 = fm::log_sel(sx / (be + (pe ? c05 : Xe * c05)), tb) - ree - 0.5 * fm::log_sel(be + fe * xi1, tb);
+    const double Le2 = fm::log_sel(sx6 / (be + (pe ? c13 : Xe * c13)), tb) - ree - 0.5 * fm::log_sel(be + fe * G.e_13 * xi1, tb);
     double diagram_e = s.pref * (Ce1 * Le1 + Ce2 * Le2);
     if (diagram_e < 0.) diagram_e = 0.;
 
     // muon diagram
-    const double lxi = fm::log(xi1, tb);
+    const double lxi = fm::log_sel(xi1, tb);
     const double b15 = 1. + (3. * beta) / 2.;
     const double Pm = (1. + rho2) * b15 - 1. / xi * (1. + 2. * beta) * omr;
     const double Bm = Pm * lxi + xi * (1. - rho2 - beta) / xi1 + (1. + 2. * beta) * omr;
@@ -363,8 +363,8 @@ __device__ double pair_d2_ssr(const PairQ& s, const Globals& G, double rho, cons
     const double Xm = (fabs(rm) < 100) ? fm::exp(-fabs(rm), tb) : 0.;
     const double bm = pm ? Xm : 1.;
     const double rmm = pm ? rm : 0.;
-    const double Lm1 = fm::log(num / (bm + (pm ? c05 : c05 * Xm)), tb) - rmm;
-    const double Lm2 = fm::log(num / (bm + (pm ? c13 : c13 * Xm)), tb) - rmm;
+    const double Lm1 = fm::log_sel(num / (bm + (pm ? c05 : c05 * Xm)), tb) - rmm;
+    const double Lm2 = fm::log_sel(num / (bm + (pm ? c13 : c13 * Xm)), tb) - rmm;
     double diagram_mu = s.pref * s.me_m2 * (Cm1 * Lm1 + Cm2 * Lm2);
     if (diagram_mu < 0.) diagram_mu = 0.;
     return (diagram_e + diagram_mu) * 1E-01 / s.energy;
@@ -385,7 +385,7 @@ __device__ double pair_ssr(const ElementConsts& c, double rl, const Globals& G, 
     const double rmax = sqrt(x0) * x1;
     const double ri = 1. - rmax;
     if ((ri <= 0.) || (ri >= 1.)) return 0.;
-    const double tmin = fm::log(ri, tb);
+    const double tmin = fm::log_sel(ri, tb);
     // the DDCS's own range check (pumas.c:14469-14471) holds at every node:
     // 4 m_e < q < K + the offset
     const PairQ s = pair_setup(c, rl, mass, K, q, pair_zeta(c, mass, K, tb));
@@ -399,15 +399,15 @@ __device__ double pair_ssr(const ElementConsts& c, double rl, const Globals& G, 
 }
 
 // ALLM97 proton structure function F2 (pumas.c:14690-14745); lq0 is
-// fm::log(Q0^2 / Lambda^2, tb).
+// fm::log_sel(Q0^2 / Lambda^2, tb).
 __device__ double f2p_allm97(double x, double Q2, double lq0, const fm::Tab& tb) {
 #pragma clang fp contract(off)
     const double m02 = 0.31985, mP2 = 49.457, mR2 = 0.15052, Q02 = 0.52544, Lambda2 = 0.06527;
     const double M2 = NUCLEON_MASS * NUCLEON_MASS;
     const double W2 = M2 + Q2 * (1.0 / x - 1.0);
-    const double t = fm::log(fm::log((Q2 + Q02) / Lambda2, tb) / lq0, tb);
+    const double t = fm::log_sel(fm::log_sel((Q2 + Q02) / Lambda2, tb) / lq0, tb);
     // t^c as exp(c log t); t is 0 in exact arithmetic as Q2 -> 0, and clamped there
-    const double lnt = fm::log(t < 0. ? 0. : t, tb);
+    const double lnt = fm::log_sel(t < 0. ? 0. : t, tb);
     const double xP = (Q2 + mP2) / (Q2 + mP2 + W2 - M2);
     const double xR = (Q2 + mR2) / (Q2 + mR2 + W2 - M2);
     const double cP = 0.28067 + (0.28067 - 0.22291) * (1.0 / (1.0 + fm::exp(2.1979 * lnt, tb)) - 1.0);
@@ -416,9 +416,9 @@ __device__ double f2p_allm97(double x, double Q2, double lq0, const fm::Tab& tb)
     const double cR = 0.80107 + 0.97307 * fm::exp(3.4942 * lnt, tb);
     const double aR = 0.58400 + 0.37888 * fm::exp(2.6063 * lnt, tb);
     const double bR = 0.01147 + 3.7582 * fm::exp(0.49338 * lnt, tb);
-    const double l1x = fm::log(1 - x, tb);
-    const double F2P = cP * fm::exp(aP * fm::log(xP, tb) + bP * l1x, tb);
-    const double F2R = cR * fm::exp(aR * fm::log(xR, tb) + bR * l1x, tb);
+    const double l1x = fm::log_sel(1 - x, tb);
+    const double F2P = cP * fm::exp(aP * fm::log_sel(xP, tb) + bP * l1x, tb);
+    const double F2R = cR * fm::exp(aR * fm::log_sel(xR, tb) + bR * l1x, tb);
     return Q2 / (Q2 + m02) * (F2P + F2R);
 }
 
@@ -438,7 +438,7 @@ __device__ double photo_d2_drss(const ElementConsts& c, const Globals& G, double
     else if (x < 0.0014)
         shadowing = c.shadow_low;
     else if (x < 0.04)
-        shadowing = fm::exp((0.069 * (fm::log(x, tb) * INV_LN10) + 0.097) * c.lnA, tb);
+        shadowing = fm::exp((0.069 * (fm::log_sel(x, tb) * INV_LN10) + 0.097) * c.lnA, tb);
     else
         shadowing = 1.;
     const double F2A = F2p * shadowing * (Z + (A - Z) * (1.0 + x * (-1.85 + x * (2.45 + x * (-2.35 + x)))));
@@ -461,8 +461,8 @@ __device__ double photo_drss(const ElementConsts& c, const Globals& G, double ml
     const double Q2min = ml2 * (q * q - 0.5 * ml2) / (E * (E - q));
     const double Q2max = 2.0 * M * (q - mpi) - mpi * mpi;
     if ((Q2max < Q2min) | (Q2min < 0)) return 0.;
-    const double lmin = fm::log(Q2min, tb);
-    const double dx = fm::log(Q2max, tb) - lmin;
+    const double lmin = fm::log_sel(Q2min, tb);
+    const double dx = fm::log_sel(Q2max, tb) - lmin;
     double ds = 0.;
 #pragma unroll 1
     for (int i = 0; i < 9; i++) {
@@ -488,7 +488,7 @@ __device__ __forceinline__ void pair_term(const ElementConsts& c, double rl, con
     const double rmax = sqrt(x0) * x1;
     const double ri = 1. - rmax;
     if ((ri <= 0.) || (ri >= 1.)) return;
-    const double tmin = fm::log(ri, tb);
+    const double tmin = fm::log_sel(ri, tb);
     const PairQ s = pair_setup(c, rl, mass, K, q, zeta);
     const double rho = fm::exp(GQ12_X[node] * tmin, tb);
     *term = pair_d2_ssr(s, G, rho, tb) * rho * GQ12_W[node] * tmin;
@@ -510,8 +510,8 @@ __device__ __forceinline__ void photo_term(const ElementConsts& c, const Globals
     const double Q2min = ml2 * (q * q - 0.5 * ml2) / (E * (E - q));
     const double Q2max = 2.0 * M * (q - mpi) - mpi * mpi;
     if ((Q2max < Q2min) | (Q2min < 0)) return;
-    const double lmin = fm::log(Q2min, tb);
-    const double dx = fm::log(Q2max, tb) - lmin;
+    const double lmin = fm::log_sel(Q2min, tb);
+    const double dx = fm::log_sel(Q2max, tb) - lmin;
     const double Q2 = fm::exp(lmin + dx * GQ9_X[node], tb);
     const double tmp = photo_d2_drss(c, G, ml, K, q, Q2, tb);
     *skip = tmp <= 0.;
@@ -596,7 +596,7 @@ __global__ __launch_bounds__(TABLE_WG) void pumas_table_kernel(Grid g, ElementBl
         const double q = K * fm::exp(xs[i], tb);
         const double d = dcs(p, c, G, mass, K, q, tb);
         positive = d > 0;
-        ys[i] = positive ? fm::log(d, tb) : 0.;
+        ys[i] = positive ? fm::log_sel(d, tb) : 0.;
         if (positive) atomicMin(&first[row], i);
     }
     __syncthreads();
@@ -677,7 +677,7 @@ __global__ __launch_bounds__(TABLE_WG) void pumas_table_kernel(Grid g, ElementBl
             const double qrev = X_REVERSE * K;
             qmax *= 0.5;
             if (qmax > qrev) qmax = qrev;
-            if ((xs[i] > fm::log(qmin / K, tb)) && (xs[i] < fm::log(qmax / K, tb))) {
+            if ((xs[i] > fm::log_sel(qmin / K, tb)) && (xs[i] < fm::log_sel(qmax / K, tb))) {
                 atomicMin(&low[row], i);
                 atomicMax(&high[row], i);
             }
@@ -825,7 +825,7 @@ __device__ __forceinline__ double dcs_wave(int process, const ElementConsts& c, 
 // constants and the searches kept out of the registers 1980; one launch for 48
 // elements 1334; a tree's nodes taking their steps at once 1217; selections for
 // branches 1177; model batches filled point by point 1105; a copy of the search
-// per process and the longest rows first 960.
+// per process, the longest rows first and the logarithms without branches 953.
 
 // v of one lane, as a wave-uniform (scalar) value.
 __device__ __forceinline__ double from_lane(double v, int lane) {
@@ -1100,8 +1100,8 @@ __device__ __forceinline__ float envelope_max(const EnvRow& a, ElementPtr cp, co
     }
     double xmin = qmin / K;
     if (xmin < cutoff) xmin = cutoff;
-    xmin = fm::log(xmin, tb);
-    double xmax = fm::log(qmax / K, tb);
+    xmin = fm::log_sel(xmin, tb);
+    double xmax = fm::log_sel(qmax / K, tb);
     if (xmin >= xmax) return 0.f;
     const double wj = K / (K + a.mass);
     const int batch = model_batch(Process);
@@ -1132,11 +1132,11 @@ __device__ __forceinline__ float envelope_max(const EnvRow& a, ElementPtr cp, co
             lnx = 0.5 * (xmin + xmax);
         } else if (phase == BACKOFF) {
             points = batch;
-            lnx = fm::log(exm - ldexp(delta, lane < points ? lane : 0), tb);
+            lnx = fm::log_sel(exm - ldexp(delta, lane < points ? lane : 0), tb);
         } else if (phase == SCAN) {
             points = N_SCAN;
             // xmax + log(1 - 10^-(i + 1))
-            lnx = xmax + fm::log(1. - pow(10., double(-((lane < N_SCAN ? lane : 0) + 1))), tb);
+            lnx = xmax + fm::log_sel(1. - pow(10., double(-((lane < N_SCAN ? lane : 0) + 1))), tb);
         } else {
             // the search's state at this lane's node
             wave_lds_order();
@@ -1238,7 +1238,7 @@ __device__ __forceinline__ float envelope_max(const EnvRow& a, ElementPtr cp, co
             f1 = from_lane(v, i);
             delta = ldexp(delta, nz ? i : i + 1);
             if (!nz && exm > delta) continue;
-            put(s, new_search(half ? SEARCH_NONE : SEARCH_EDGE, xmax, fm::log(exm - delta / 2, tb), 0., 0., 0., 0, xmax, f1));
+            put(s, new_search(half ? SEARCH_NONE : SEARCH_EDGE, xmax, fm::log_sel(exm - delta / 2, tb), 0., 0., 0., 0, xmax, f1));
             phase = EDGE_HIGH;
         } else if (phase == MID) {
             fmid = from_lane(v, 0);
@@ -1286,7 +1286,7 @@ __device__ __forceinline__ float envelope_max(const EnvRow& a, ElementPtr cp, co
                     phase = BACKOFF;
                     if (exm > delta) continue;
                 }
-                put(s, new_search(half ? SEARCH_NONE : SEARCH_EDGE, K >= 1E+01 ? xmax : xmin, K >= 1E+01 ? fm::log(exm - delta / 2, tb) : xmax, 0., 0.,
+                put(s, new_search(half ? SEARCH_NONE : SEARCH_EDGE, K >= 1E+01 ? xmax : xmin, K >= 1E+01 ? fm::log_sel(exm - delta / 2, tb) : xmax, 0., 0.,
                         0., 0, xmax, f1));
                 phase = EDGE_HIGH;
                 if (__ballot(!s.done())) continue;
