@@ -40,12 +40,12 @@ constexpr int SOFT_ITV = 17;               // ceil(100 / 6) subintervals (dcs.hh
 constexpr int SOFT_NODES = 6 * SOFT_ITV;   // 102
 constexpr int SOFT_CHUNK = 16384;          // K values the workspace is sized for
 
-// Nodes per workgroup (22 and 2 K values of the 23 nodes that can be open),
+// Nodes per workgroup (66 and 2 K values of the 23 nodes that can be open),
 // and the number of K values up to which the open integrals are spread over
 // lanes by node. A workgroup takes one K as long as 1024 of them fill the
 // chip. Measured on MI355X (us, spread / not): 176 K 9.4 / 20, 1236 12 / 19,
-// 2000 17 / 19, 4000 26 / 23, 16,384 82 / 48, 65,536 312 / 119.
-constexpr int SOFT_TILE = 512, SOFT_SPLIT_TILE = 64;
+// 2000 17 / 19, 4000 26 / 23, 16,384 82 / 48, 65,536 312 / 111.
+constexpr int SOFT_TILE = 1536, SOFT_SPLIT_TILE = 64;
 constexpr int64_t SOFT_SPLIT_MAX = 2048;
 
 // Host-evaluated per-element values (bit-identical to the reference's).
@@ -549,7 +549,7 @@ __device__ double soft_all_nodes(double k, const SoftNodes& sn, double mass, con
 // Bound: FP64 VALU issue, ~4500 instructions per open node. Open nodes are
 // compacted in LDS and drained by whole waves; SPLIT spreads each over 9
 // lanes by quadrature node, for calls with too few K values to fill the chip.
-// Measured for 65,536 K: 119 us, against 733 us when the 102 nodes of each K
+// Measured for 65,536 K: 111 us, against 733 us when the 102 nodes of each K
 // went through memory as (K, q) pairs of a map and one thread per K formed
 // their 102 ratios (64 workgroups per pass of 16,384 K); 9.4 us for 176 K.
 template <int TILE, bool SPLIT>
@@ -650,6 +650,19 @@ inline HardShape hard_shape(int64_t nel, int64_t n) {
     return {4, nel <= 8 ? 2 : 3};
 }
 
+// K values per workgroup of the soft-scattering kernel, of which a tile holds
+// `room`: equal shares for the fewest whole rounds of the 1024 workgroups that
+// the chip holds. About half of the nodes are open and a workgroup drains them
+// 256 at a time, so a small group leaves most lanes of its last pass idle.
+// Measured (us; 22 K values per workgroup / up to 66 / up to 66 in equal
+// shares): 65,536 K 119 / 110 / 110, 70,000 125 / 131 / 120, 100,000 168 / 171 /
+// 163, 2^20 1509 / 1279 / 1273.
+int32_t soft_group(int64_t n, int64_t room) {
+    const int64_t round = 1024 * std::max<int64_t>(1, room);
+    const int64_t slots = 1024 * ((n + round - 1) / round);
+    return int32_t((n + slots - 1) / slots);
+}
+
 unsigned grid_for(int64_t n) { return unsigned(std::max<int64_t>(1, std::min<int64_t>(65536, (n + 255) / 256))); }
 
 }  // namespace noa_hip
@@ -747,8 +760,7 @@ int noa_dcs_soft_scattering_f64(const double* K, int64_t n, const noa_dcs_elemen
     for (int64_t k0 = 0; k0 < n; k0 += most) {
         const int64_t nK = std::min<int64_t>(most, n - k0);
         const bool split = nK <= SOFT_SPLIT_MAX;
-        const int32_t group = int32_t(
-            std::max<int64_t>(1, std::min<int64_t>((split ? SOFT_SPLIT_TILE : SOFT_TILE) / nb, (nK + 1023) / 1024)));
+        const int32_t group = soft_group(nK, (split ? SOFT_SPLIT_TILE : SOFT_TILE) / nb);
         const auto kernel = split ? &soft_kernel<SOFT_SPLIT_TILE, true> : &soft_kernel<SOFT_TILE, false>;
         hipLaunchKernelGGL(kernel, dim3(unsigned((nK + group - 1) / group)), dim3(WG), 0, stream, K + k0, nK, c, ce, sn,
                            group, result + k0);
