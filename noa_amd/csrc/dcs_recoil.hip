@@ -93,7 +93,7 @@ __device__ __forceinline__ double wave_sum(double v) {
 // and slower below, tiles of 256 (one K) 15% slower there.
 constexpr int RECOIL_TILE = 512;
 
-// One workgroup per `group` K values; their nodes fit one tile, or (BLOCKS)
+// One workgroup of LANES lanes per `group` K values; their nodes fit one tile, or (BLOCKS)
 // group = 1 and the nodes go in blocks of TILE.
 //
 // Bound: FP64 VALU issue, as the map's tile kernel (the nodes have q >= K
@@ -102,12 +102,12 @@ constexpr int RECOIL_TILE = 512;
 // memory instead (a kernel that wrote (K, q) pairs, the map in tiles of 2048,
 // and a sum per thread) took, at min_points 180, 444 us for 146 K values and
 // 1790 us for 65,536, of which 296 and 320 us were the serial sums; this
-// kernel takes 28 and 1567. At 30 points 189 -> 21 and 354 -> 336, at 6
+// kernel takes 20 and 1567. At 30 points 189 -> 20 and 354 -> 336, at 6
 // points 81 -> 24 and 167 -> 127.
 // The nodes-in-blocks form is an instantiation of its own: its loop carries
 // values that made the common one spill 28 registers.
-template <int TILE, bool BLOCKS>
-__global__ __launch_bounds__(WG) __attribute__((amdgpu_waves_per_eu(4))) void recoil_kernel(
+template <int TILE, bool BLOCKS, int LANES>
+__global__ __launch_bounds__(LANES) __attribute__((amdgpu_waves_per_eu(4))) void recoil_kernel(
     const double* __restrict__ K, int64_t n, DcsConsts, RecoilGrid g, int32_t group, Outs<double> del,
     Outs<double> cel) {
     __shared__ RecoilLds<TILE> s;
@@ -116,13 +116,13 @@ __global__ __launch_bounds__(WG) __attribute__((amdgpu_waves_per_eu(4))) void re
     const int tid = threadIdx.x;
     const int lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    load_fm_tables(fm_block);
+    for (int i = tid; i < fm::TABLE_DOUBLES; i += LANES) fm_block[i] = fm::table_entry(i);
     const fm::Tab t = fm::tab_from_block(fm_block);
     const bool want_b = del.b || cel.b, want_p = del.p || cel.p, want_ph = del.ph || cel.ph, want_i = del.i || cel.i;
     const int64_t k0 = int64_t(blockIdx.x) * group;
     const int nk = int(n - k0 < group ? n - k0 : group);
     __syncthreads();
-    for (int kk = tid; kk < nk; kk += WG) {
+    for (int kk = tid; kk < nk; kk += LANES) {
 #pragma clang fp contract(off)
         const double k = K[k0 + kk];
         const double lb = fm::log(k * g.xlow, t);
@@ -140,7 +140,7 @@ __global__ __launch_bounds__(WG) __attribute__((amdgpu_waves_per_eu(4))) void re
         __syncthreads();
         // the nodes: closed forms, exits, the lists of open integrals
 #pragma unroll 1
-        for (int i0 = 0; i0 < items; i0 += WG) {
+        for (int i0 = 0; i0 < items; i0 += LANES) {
             const DcsConsts& c = item_consts(cp);
             const int i = i0 + tid;
             bool pa = false, pha = false;
@@ -174,7 +174,7 @@ __global__ __launch_bounds__(WG) __attribute__((amdgpu_waves_per_eu(4))) void re
         const uint32_t pair0 = (nph + 63u) & ~63u;
         const uint32_t total = pair0 + s.n_pair;
 #pragma unroll 1
-        for (uint32_t v = tid; v < total; v += WG) {
+        for (uint32_t v = tid; v < total; v += LANES) {
             const DcsConsts& c = item_consts(cp);
             if (v < pair0) {
                 if (v >= nph) continue;
@@ -187,7 +187,7 @@ __global__ __launch_bounds__(WG) __attribute__((amdgpu_waves_per_eu(4))) void re
         }
         __syncthreads();
         // sums: a wave takes one K
-        for (int kk = wave; kk < nk; kk += WG / 64) {
+        for (int kk = wave; kk < nk; kk += LANES / 64) {
 #pragma clang fp contract(off)
             double sum[8] = {};
             for (int l = lane; l < nb; l += 64) {
@@ -209,7 +209,7 @@ __global__ __launch_bounds__(WG) __attribute__((amdgpu_waves_per_eu(4))) void re
         }
         __syncthreads();
         const bool last = !BLOCKS || j0 + TILE >= g.nodes;
-        for (int v = tid; v < nk * 8; v += WG) {
+        for (int v = tid; v < nk * 8; v += LANES) {
             const int kk = v / 8, p = v % 8;
             double acc = s.part[kk][p];
             if (BLOCKS && j0 > 0) acc += s.acc[p];  // (more than one node block: one K)
@@ -229,7 +229,7 @@ __global__ __launch_bounds__(WG) __attribute__((amdgpu_waves_per_eu(4))) void re
     }
 }
 
-static_assert(std::is_same<decltype(&recoil_kernel<RECOIL_TILE, false>),
+static_assert(std::is_same<decltype(&recoil_kernel<RECOIL_TILE, false, WG>),
                            void (*)(const double*, int64_t, DcsConsts, RecoilGrid, int32_t, Outs<double>,
                                     Outs<double>)>::value,
               "recoil_kernel's parameters must begin as VectorKernelArgs lays them out");
@@ -266,7 +266,6 @@ int recoil_run(const double* K, int64_t n, double xlow, const noa_dcs_element* e
                int32_t min_points, const noa_dcs_outputs_f64& D, const noa_dcs_outputs_f64& C, hipStream_t stream) {
     const RecoilGrid g{xlow, int32_t((uint32_t(min_points) + 5u) / 6u), int32_t(nodes_of(min_points))};
     const DcsConsts c = make_consts(element->A, element->I, element->Z, mass);
-    const auto kernel = g.nodes > RECOIL_TILE ? &recoil_kernel<RECOIL_TILE, true> : &recoil_kernel<RECOIL_TILE, false>;
     constexpr int64_t most = int64_t(1) << 30;  // K values per launch (a grid has at most 2^31 - 1 workgroups)
     for (int64_t k0 = 0; k0 < n; k0 += most) {
         const int64_t nK = std::min<int64_t>(most, n - k0);
@@ -274,8 +273,19 @@ int recoil_run(const double* K, int64_t n, double xlow, const noa_dcs_element* e
         const Outs<double> od{shift(D.brems), shift(D.pair), shift(D.photo), shift(D.ion)};
         const Outs<double> oc{shift(C.brems), shift(C.pair), shift(C.photo), shift(C.ion)};
         const int32_t group = recoil_group(nK, g.nodes);
-        hipLaunchKernelGGL(kernel, dim3(unsigned((nK + group - 1) / group)), dim3(WG), 0, stream, K + k0, nK, c, g,
-                           group, od, oc);
+        const unsigned blocks = unsigned((nK + group - 1) / group);
+        const bool in_blocks = g.nodes > RECOIL_TILE;
+        // up to 512 workgroups leave half of the chip's wave slots empty at 256
+        // lanes each, and their length is the call's. Measured (us, 256 / 512 /
+        // 1024 lanes; min_points 180): 146 K 27.9 / 20.3 / 20.4, 512 K 33.7 /
+        // 28.3 / 37.7, 700 K 39.1 / 43.9 / 54.1; 1000 points, 146 K 96 / 67 / 60
+        const bool wide = blocks <= 512;
+        const auto kernel = wide ? (in_blocks ? &recoil_kernel<RECOIL_TILE, true, 2 * WG>
+                                              : &recoil_kernel<RECOIL_TILE, false, 2 * WG>)
+                                 : (in_blocks ? &recoil_kernel<RECOIL_TILE, true, WG>
+                                              : &recoil_kernel<RECOIL_TILE, false, WG>);
+        const unsigned lanes = wide ? 2 * WG : WG;
+        hipLaunchKernelGGL(kernel, dim3(blocks), dim3(lanes), 0, stream, K + k0, nK, c, g, group, od, oc);
         if (int rc = check_hip(hipGetLastError(), "recoil_kernel")) return rc;
     }
     return ok();
