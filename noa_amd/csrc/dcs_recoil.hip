@@ -80,6 +80,17 @@ struct RecoilLds {
     uint32_t n_photo, n_pair;
 };
 
+// (SPLIT) the shared values and node terms of up to this many open integrals of
+// either kind at a time.
+constexpr int RECOIL_SPLIT = 192;
+struct RecoilSplitLds {
+    double x8[8], w8[8], x9[9], w9[9];
+    double beta[RECOIL_SPLIT], tmin[RECOIL_SPLIT], a[8 * RECOIL_SPLIT], b[8 * RECOIL_SPLIT];
+    F64::PhotoPre photo[RECOIL_SPLIT];
+    double f[9 * RECOIL_SPLIT];
+};
+struct NoSplitLds {};
+
 // Sum over the wave's lanes, in a fixed order, valid in lane 0.
 __device__ __forceinline__ double wave_sum(double v) {
 #pragma unroll
@@ -102,21 +113,32 @@ constexpr int RECOIL_TILE = 512;
 // memory instead (a kernel that wrote (K, q) pairs, the map in tiles of 2048,
 // and a sum per thread) took, at min_points 180, 444 us for 146 K values and
 // 1790 us for 65,536, of which 296 and 320 us were the serial sums; this
-// kernel takes 20 and 1567. At 30 points 189 -> 20 and 354 -> 336, at 6
-// points 81 -> 24 and 167 -> 127.
+// kernel takes 19 and 1567. At 30 points 189 -> 12 and 354 -> 336, at 6
+// points 81 -> 15 and 167 -> 127.
 // The nodes-in-blocks form is an instantiation of its own: its loop carries
 // values that made the common one spill 28 registers.
-template <int TILE, bool BLOCKS, int LANES>
+template <int TILE, bool BLOCKS, int LANES, bool SPLIT = false>
 __global__ __launch_bounds__(LANES) __attribute__((amdgpu_waves_per_eu(4))) void recoil_kernel(
     const double* __restrict__ K, int64_t n, DcsConsts, RecoilGrid g, int32_t group, Outs<double> del,
     Outs<double> cel) {
     __shared__ RecoilLds<TILE> s;
     __shared__ __attribute__((aligned(fm::TABLE_LDS_ALIGN))) double fm_block[fm::TABLE_DOUBLES];
+    __shared__ typename std::conditional<SPLIT, RecoilSplitLds, NoSplitLds>::type x;
     const ConstsPtr cp = vector_kernarg_consts();
     const int tid = threadIdx.x;
     const int lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     for (int i = tid; i < fm::TABLE_DOUBLES; i += LANES) fm_block[i] = fm::table_entry(i);
+    if constexpr (SPLIT) {  // the node tables in LDS: the node index varies by lane
+        if (tid < 9) {
+            x.x9[tid] = GL9_X[tid];
+            x.w9[tid] = GL9_W[tid];
+            if (tid < 8) {
+                x.x8[tid] = GL8_X[tid];
+                x.w8[tid] = GL8_W[tid];
+            }
+        }
+    }
     const fm::Tab t = fm::tab_from_block(fm_block);
     const bool want_b = del.b || cel.b, want_p = del.p || cel.p, want_ph = del.ph || cel.ph, want_i = del.i || cel.i;
     const int64_t k0 = int64_t(blockIdx.x) * group;
@@ -169,20 +191,103 @@ __global__ __launch_bounds__(LANES) __attribute__((amdgpu_waves_per_eu(4))) void
             if (want_p) wave_append(pa, &s.n_pair, s.pair_list, uint32_t(i));
         }
         __syncthreads();
-        // the integrals, whole waves of one kind, photonuclear (heavier) first
-        const uint32_t nph = s.n_photo;
-        const uint32_t pair0 = (nph + 63u) & ~63u;
-        const uint32_t total = pair0 + s.n_pair;
+        if constexpr (SPLIT) {
+            // the integrals by quadrature node: a chain is a set-up, a node or
+            // three and a sum, where an integral's own lane runs 8 or 9 in a row
+            // (the sums are those of that loop, bit for bit)
+            const uint32_t all_ph = s.n_photo, all_pa = s.n_pair;
 #pragma unroll 1
-        for (uint32_t v = tid; v < total; v += LANES) {
-            const DcsConsts& c = item_consts(cp);
-            if (v < pair0) {
-                if (v >= nph) continue;
-                const uint32_t i = s.photo_list[v];
-                s.dcs[2][i] = F64::photo(s.K[i / uint32_t(nb)], s.q[i], c, t);
-            } else {
-                const uint32_t i = s.pair_list[v - pair0];
-                s.dcs[1][i] = F64::pair_at(s.K[i / uint32_t(nb)], s.q[i], s.dcs[1][i], c, t);
+            for (uint32_t e0 = 0; e0 < max(all_ph, all_pa); e0 += RECOIL_SPLIT) {
+                const uint32_t nph = min(uint32_t(RECOIL_SPLIT), all_ph - min(e0, all_ph));
+                const uint32_t npa = min(uint32_t(RECOIL_SPLIT), all_pa - min(e0, all_pa));
+                const uint32_t pair0 = (nph + 63u) & ~63u, node0 = (9 * nph + 63u) & ~63u;
+                const auto is_fast = [&](uint32_t i, const DcsConsts& c) {
+                    return c.fast_ok && s.K[i / uint32_t(nb)] + c.mass <= F64::FAST_E_MAX;
+                };
+#pragma unroll 1
+                for (uint32_t v = tid; v < pair0 + npa; v += LANES) {
+                    const DcsConsts& c = item_consts(cp);
+                    if (v < pair0) {
+                        if (v >= nph) continue;
+                        const uint32_t i = s.photo_list[e0 + v];
+                        const double k = s.K[i / uint32_t(nb)];
+                        if (is_fast(i, c))
+                            x.photo[v] = F64::photo_setup<false, true>(k, s.q[i], c, t);
+                        else
+                            s.dcs[2][i] = F64::photo(k, s.q[i], c, t);
+                    } else {
+                        const uint32_t e = v - pair0, i = s.pair_list[e0 + e];
+                        const double k = s.K[i / uint32_t(nb)];
+                        if (is_fast(i, c)) {
+                            double gamma;
+                            const F64::PairPre p =
+                                F64::pair_setup<false, true, true>(k, s.q[i], c, t, s.dcs[1][i], gamma);
+                            x.beta[e] = p.beta;
+                            x.tmin[e] = p.tmin;
+                        } else {
+                            s.dcs[1][i] = F64::pair_at(k, s.q[i], s.dcs[1][i], c, t);
+                        }
+                    }
+                }
+                __syncthreads();
+#pragma unroll 1
+                for (uint32_t v = tid; v < node0 + 8 * npa; v += LANES) {
+                    const DcsConsts& c = item_consts(cp);
+                    if (v < node0) {
+                        if (v >= 9 * nph) continue;
+                        const uint32_t e = v / 9, i = s.photo_list[e0 + e];
+                        if (!is_fast(i, c)) continue;
+                        const F64::PhotoPre p = x.photo[e];
+                        x.f[v] = F64::photo_node<false, true>(p, x.x9[v - 9 * e], c, t);
+                    } else {
+                        const uint32_t u = v - node0, e = u / 8, j = u % 8, i = s.pair_list[e0 + e];
+                        if (!is_fast(i, c)) continue;
+                        const F64::PairPre p = F64::pair_pre(s.q[i], x.beta[e], x.tmin[e], c);
+                        double a, b;
+                        F64::pair_node<false, true>(p, x.x8[j], x.w8[j], c, t, a, b);
+                        x.a[u] = a;
+                        x.b[u] = b;
+                    }
+                }
+                __syncthreads();
+#pragma unroll 1
+                for (uint32_t v = tid; v < pair0 + npa; v += LANES) {
+                    const DcsConsts& c = item_consts(cp);
+                    if (v < pair0) {
+                        if (v >= nph) continue;
+                        const uint32_t i = s.photo_list[e0 + v];
+                        if (!is_fast(i, c)) continue;
+                        double ds = 0.;
+                        for (int j = 0; j < 9; j++) ds = F64::photo_add<false>(x.f[9 * v + j], x.w9[j], ds);
+                        s.dcs[2][i] = F64::photo_finish<false, true>(s.K[i / uint32_t(nb)], x.photo[v], ds, c);
+                    } else {
+                        const uint32_t e = v - pair0, i = s.pair_list[e0 + e];
+                        if (!is_fast(i, c)) continue;
+                        double I = 0.;
+                        for (int j = 0; j < 8; j++) I = F64::pair_add<false>(x.a[8 * e + j], x.b[8 * e + j], I);
+                        const double k = s.K[i / uint32_t(nb)];
+                        s.dcs[1][i] = F64::pair_finish<false, true>(k, s.q[i], F64::pair_gamma<true>(k, c), x.tmin[e],
+                                                                    I, c, t);
+                    }
+                }
+                __syncthreads();
+            }
+        } else {
+            // the integrals, whole waves of one kind, photonuclear (heavier) first
+            const uint32_t nph = s.n_photo;
+            const uint32_t pair0 = (nph + 63u) & ~63u;
+            const uint32_t total = pair0 + s.n_pair;
+#pragma unroll 1
+            for (uint32_t v = tid; v < total; v += LANES) {
+                const DcsConsts& c = item_consts(cp);
+                if (v < pair0) {
+                    if (v >= nph) continue;
+                    const uint32_t i = s.photo_list[v];
+                    s.dcs[2][i] = F64::photo(s.K[i / uint32_t(nb)], s.q[i], c, t);
+                } else {
+                    const uint32_t i = s.pair_list[v - pair0];
+                    s.dcs[1][i] = F64::pair_at(s.K[i / uint32_t(nb)], s.q[i], s.dcs[1][i], c, t);
+                }
             }
         }
         __syncthreads();
@@ -280,11 +385,16 @@ int recoil_run(const double* K, int64_t n, double xlow, const noa_dcs_element* e
         // 1024 lanes; min_points 180): 146 K 27.9 / 20.3 / 20.4, 512 K 33.7 /
         // 28.3 / 37.7, 700 K 39.1 / 43.9 / 54.1; 1000 points, 146 K 96 / 67 / 60
         const bool wide = blocks <= 512;
-        const auto kernel = wide ? (in_blocks ? &recoil_kernel<RECOIL_TILE, true, 2 * WG>
-                                              : &recoil_kernel<RECOIL_TILE, false, 2 * WG>)
-                                 : (in_blocks ? &recoil_kernel<RECOIL_TILE, true, WG>
-                                              : &recoil_kernel<RECOIL_TILE, false, WG>);
-        const unsigned lanes = wide ? 2 * WG : WG;
+        // up to one per CU also spread their integrals by node (1024 lanes): 6, 30
+        // and 180 points 22.5 / 14.8, 20.0 / 12.4, 19.5 / 18.9 us for 146 K (a
+        // CU's issue rate bounds the last)
+        const bool by_node = blocks <= 256 && !in_blocks;
+        const auto kernel = by_node ? &recoil_kernel<RECOIL_TILE, false, 4 * WG, true>
+                            : wide  ? (in_blocks ? &recoil_kernel<RECOIL_TILE, true, 2 * WG>
+                                                 : &recoil_kernel<RECOIL_TILE, false, 2 * WG>)
+                                    : (in_blocks ? &recoil_kernel<RECOIL_TILE, true, WG>
+                                                 : &recoil_kernel<RECOIL_TILE, false, WG>);
+        const unsigned lanes = by_node ? 4 * WG : wide ? 2 * WG : WG;
         hipLaunchKernelGGL(kernel, dim3(blocks), dim3(lanes), 0, stream, K + k0, nK, c, g, group, od, oc);
         if (int rc = check_hip(hipGetLastError(), "recoil_kernel")) return rc;
     }
