@@ -75,8 +75,6 @@ inline RowOrder epoch_order(uint64_t seed, int64_t epoch, int64_t n) {
     return o;
 }
 
-constexpr int EPOCH_ROOM = 511;
-
 struct MlpWork {
     // the layered forward's buffers, [rows x H] row-major
     float* Z[4] = {};  // pre-activations of the 4 hidden layers
@@ -88,8 +86,8 @@ struct MlpWork {
     float* small = nullptr;         // [rows/32][NSMALL]
     float* loss_partial = nullptr;  // one per 32 rows
     float* ws = nullptr;  // STEP_SPLITS partial gradients [STEP_SPLITS x NPARAM], then STEP_SPLITS losses
-    double* loss = nullptr;  // the last step's loss, then the sums of up to EPOCH_ROOM epochs' losses
-    double* epoch_loss = nullptr;  // the sums of a call of more epochs
+    double* loss = nullptr;  // the last step's loss
+    double* epoch_loss = nullptr;  // the sum of each epoch's losses
     int64_t epoch_room = 0;
 };
 
@@ -139,7 +137,7 @@ inline int mlp_alloc(noa_dcs_mlp* net, int max_rows) {
     m(&net->work.small, size_t(rp / 32) * NSMALL * sizeof(float));
     m(&net->work.loss_partial, size_t(rp / 32) * sizeof(float));
     m(&net->work.ws, size_t(STEP_SPLITS) * (NPARAM + 1) * sizeof(float));
-    m(&net->work.loss, (1 + EPOCH_ROOM) * sizeof(double));
+    m(&net->work.loss, sizeof(double));
     m(&net->packed, FRAG_TOTAL * sizeof(uint16_t));
     m(&net->packedT, FRAGT_TOTAL * sizeof(uint16_t));
     return rc;

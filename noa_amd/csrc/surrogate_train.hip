@@ -271,9 +271,8 @@ int noa_dcs_mlp_train(noa_dcs_mlp* net, const float* X, const float* T, const fl
     const int64_t total_steps = steps_per_epoch * epochs;
     const float b1 = 0.9f, b2 = 0.999f;
     // kept with the network: allocated, filled and released around every call
-    // it cost a 16-step call 15 of 472 us; in an allocation of its own, 280 us
-    // when the network is created and destroyed
-    if (epochs > EPOCH_ROOM && net->work.epoch_room < epochs) {
+    // it cost a 16-step call 15 of 472 us
+    if (net->work.epoch_room < epochs) {
         if (net->work.epoch_loss) (void)hipFree(net->work.epoch_loss);
         net->work.epoch_loss = nullptr;
         net->work.epoch_room = 0;
@@ -281,7 +280,7 @@ int noa_dcs_mlp_train(noa_dcs_mlp* net, const float* X, const float* T, const fl
             return rc;
         net->work.epoch_room = epochs;
     }
-    double* d_loss = epochs <= EPOCH_ROOM ? net->work.loss + 1 : net->work.epoch_loss;
+    double* d_loss = net->work.epoch_loss;
     int rc = NOA_DCS_OK;
     for (int ep = 0; ep < epochs && !rc; ep++) {
         const RowOrder order = epoch_order(seed, ep, n);
