@@ -818,7 +818,7 @@ __device__ __forceinline__ double dcs_wave(int process, const ElementConsts& c, 
 //
 // What bounds it is the instructions of a row's chain of rounds (about 20, up
 // to 60 where every point needs the model, of ~500 to 2000 vector instructions
-// each), with three waves per SIMD to overlap: the vector units are busy 72% of
+// each), with three waves per SIMD to overlap: the vector units are busy 73% of
 // the launch. Measured for 48 elements x 146 energies, the whole table call:
 // one point per step for the whole wave 10,600 us; trees of one search per wave
 // 4113; two searches side by side with the table log / exp 2810; the rows'
