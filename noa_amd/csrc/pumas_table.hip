@@ -1581,10 +1581,11 @@ int noa_pumas_dcs_table(const double* Z, const double* A, int32_t n_elements, do
             for (int j = 0; j < args.n_blk; j++)
                 args.blk.e[j] = pumas::make_element(Z[args.e0 + j], A[args.e0 + j], mass, G);
             const unsigned rows = unsigned(3 * args.n_blk * n_K);
-            // three waves per SIMD (a few registers spilled) where the rows
-            // exceed the 2048 that two hold: 1963 against 2115 us for 48
-            // elements x 146 energies, 766 against 718 for 1 x 30
-            hipLaunchKernelGGL((rows > 2048 ? &pumas::pumas_envelope_kernel<3> : &pumas::pumas_envelope_kernel<2>),
+            // three waves per SIMD (40 registers spilled) where the rows are many;
+            // below, the longest rows decide. Measured (us, two / three waves,
+            // 146 energies): 7 elements 548 / 564, 16 575 / 595, 20 632 / 605,
+            // 48 1171 / 947
+            hipLaunchKernelGGL((rows > 8000 ? &pumas::pumas_envelope_kernel<3> : &pumas::pumas_envelope_kernel<2>),
                                dim3(rows), dim3(64), size_t(pumas::ENVELOPE_LDS) * g.n * sizeof(float), stream, args);
             if (int rc = check_hip(hipGetLastError(), "pumas_envelope_kernel")) return rc;
         }
