@@ -103,13 +103,15 @@ def build_extension(verbose: bool = False) -> str:
 
 def build_test_kernels() -> str:
     """tests/native/libfm_dev.so: the device log / exp / reciprocal of
-    csrc/fastmath.hh over arrays, for the GPU accuracy tests; and
-    tests/native/libclock_probe.so: the FP64 tile kernel with per-workgroup
-    clock counters, for the GPU measurement test (neither is part of the
-    product library)."""
+    csrc/fastmath.hh over arrays, for the GPU accuracy tests;
+    tests/native/liblog_sel_dev.so: its branch-free log next to the branching
+    one; and tests/native/libclock_probe.so: the FP64 tile kernel with
+    per-workgroup clock counters, for the GPU measurement test (none is part
+    of the product library)."""
     native = os.path.join(ROOT, "tests", "native")
     outs = []
-    for src, name in (("fastmath_dev.hip", "libfm_dev.so"), ("clock_probe.hip", "libclock_probe.so")):
+    for src, name in (("fastmath_dev.hip", "libfm_dev.so"), ("clock_probe.hip", "libclock_probe.so"),
+                      ("log_sel_dev.hip", "liblog_sel_dev.so")):
         out = os.path.join(native, name)
         _run([HIPCC, *HIP_FLAGS, "-shared", "-o", out + ".tmp", os.path.join(native, src)])
         os.replace(out + ".tmp", out)
