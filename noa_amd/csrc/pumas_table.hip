@@ -28,6 +28,7 @@
 
 #include "capi_util.hh"
 #include "fastmath.hh"
+#include "pumas_search.hh"
 
 namespace noa_hip {
 namespace pumas {
@@ -852,18 +853,6 @@ struct EnvRow {
     bool below;  // K below the grid (never the case for a row's own energy)
 };
 
-// The cell of the nodes t[0..n-1] that holds x (t[0] <= x < t[n - 1]), or 0 for
-// NaN: four parts a step, so that three loads are in flight.
-__device__ __forceinline__ int cell(const float* t, int n, float x) {
-    int i = 0;
-    for (int d = n - 1; d > 1;) {
-        d = (d + 3) / 4;
-        const float a = t[min(i + d, n - 1)], b = t[min(i + 2 * d, n - 1)], c = t[min(i + 3 * d, n - 1)];
-        i += d * (int(x >= a) + int(x >= b) + int(x >= c));
-    }
-    return i;
-}
-
 // table_index without a context (pumas.c:4249-4290, 4299-4306).
 __device__ __forceinline__ int table_index(const double* table, int n_K, double value) {
     const int imax = n_K - 1;
@@ -908,7 +897,7 @@ __device__ __forceinline__ double dcs_from_table(const EnvRow& a, double K, doub
     bool ok = in && !(q < a.qlow) && !((x < a.xt[0]) || (x >= a.xt[nx - 1])) && !a.below;
     float r = 0.f;
     if (__ballot(ok)) {
-        const int ix = cell(a.xt, nx, ok ? x : a.xt[0]);
+        const int ix = cell(a.xt, nx, x, ok);
         const float p00 = a.ra[2 * ix], p01 = a.ra[2 * ix + 2], p10 = a.rb[2 * ix], p11 = a.rb[2 * ix + 2];
         float m00 = a.ra[2 * ix + 1], m01 = a.ra[2 * ix + 3], m10 = a.rb[2 * ix + 1], m11 = a.rb[2 * ix + 3];
         ok = ok & !(((p00 == 0.f) & (m00 == 0.f)) | ((p01 == 0.f) & (m01 == 0.f)) | ((p10 == 0.f) & (m10 == 0.f)) |
