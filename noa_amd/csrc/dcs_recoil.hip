@@ -23,6 +23,7 @@
 #include "dcs_f64.hh"
 #include "dcs_tile.hh"
 #include "fastmath.hh"
+#include "launch_slices.hh"
 
 namespace noa_hip {
 
@@ -371,33 +372,33 @@ int recoil_run(const double* K, int64_t n, double xlow, const noa_dcs_element* e
                int32_t min_points, const noa_dcs_outputs_f64& D, const noa_dcs_outputs_f64& C, hipStream_t stream) {
     const RecoilGrid g{xlow, int32_t((uint32_t(min_points) + 5u) / 6u), int32_t(nodes_of(min_points))};
     const DcsConsts c = make_consts(element->A, element->I, element->Z, mass);
-    constexpr int64_t most = int64_t(1) << 30;  // K values per launch (a grid has at most 2^31 - 1 workgroups)
-    for (int64_t k0 = 0; k0 < n; k0 += most) {
-        const int64_t nK = std::min<int64_t>(most, n - k0);
+    const int32_t group = recoil_group(n, g.nodes);
+    const int64_t blocks = (n + group - 1) / group;
+    const bool in_blocks = g.nodes > RECOIL_TILE;
+    // up to 512 workgroups leave half of the chip's wave slots empty at 256
+    // lanes each, and their length is the call's. Measured (us, 256 / 512 /
+    // 1024 lanes; min_points 180): 146 K 27.9 / 20.3 / 20.4, 512 K 33.7 /
+    // 28.3 / 37.7, 700 K 39.1 / 43.9 / 54.1; 1000 points, 146 K 96 / 67 / 60
+    const bool wide = blocks <= 512;
+    // up to one per CU also spread their integrals by node (1024 lanes): 6, 30
+    // and 180 points 22.5 / 14.8, 20.0 / 12.4, 19.5 / 18.9 us for 146 K (a
+    // CU's issue rate bounds the last)
+    const bool by_node = blocks <= 256 && !in_blocks;
+    const auto kernel = by_node ? &recoil_kernel<RECOIL_TILE, false, 4 * WG, true>
+                        : wide  ? (in_blocks ? &recoil_kernel<RECOIL_TILE, true, 2 * WG>
+                                             : &recoil_kernel<RECOIL_TILE, false, 2 * WG>)
+                                : (in_blocks ? &recoil_kernel<RECOIL_TILE, true, WG>
+                                             : &recoil_kernel<RECOIL_TILE, false, WG>);
+    const int lanes = by_node ? 4 * WG : wide ? 2 * WG : WG;
+    const int rc = launch_slices(blocks, lanes, [&](int64_t first, uint32_t count) {
+        const int64_t k0 = first * group, nK = std::min<int64_t>(n - k0, int64_t(count) * group);
         auto shift = [k0](double* p) { return p ? p + k0 : nullptr; };
         const Outs<double> od{shift(D.brems), shift(D.pair), shift(D.photo), shift(D.ion)};
         const Outs<double> oc{shift(C.brems), shift(C.pair), shift(C.photo), shift(C.ion)};
-        const int32_t group = recoil_group(nK, g.nodes);
-        const unsigned blocks = unsigned((nK + group - 1) / group);
-        const bool in_blocks = g.nodes > RECOIL_TILE;
-        // up to 512 workgroups leave half of the chip's wave slots empty at 256
-        // lanes each, and their length is the call's. Measured (us, 256 / 512 /
-        // 1024 lanes; min_points 180): 146 K 27.9 / 20.3 / 20.4, 512 K 33.7 /
-        // 28.3 / 37.7, 700 K 39.1 / 43.9 / 54.1; 1000 points, 146 K 96 / 67 / 60
-        const bool wide = blocks <= 512;
-        // up to one per CU also spread their integrals by node (1024 lanes): 6, 30
-        // and 180 points 22.5 / 14.8, 20.0 / 12.4, 19.5 / 18.9 us for 146 K (a
-        // CU's issue rate bounds the last)
-        const bool by_node = blocks <= 256 && !in_blocks;
-        const auto kernel = by_node ? &recoil_kernel<RECOIL_TILE, false, 4 * WG, true>
-                            : wide  ? (in_blocks ? &recoil_kernel<RECOIL_TILE, true, 2 * WG>
-                                                 : &recoil_kernel<RECOIL_TILE, false, 2 * WG>)
-                                    : (in_blocks ? &recoil_kernel<RECOIL_TILE, true, WG>
-                                                 : &recoil_kernel<RECOIL_TILE, false, WG>);
-        const unsigned lanes = by_node ? 4 * WG : wide ? 2 * WG : WG;
-        hipLaunchKernelGGL(kernel, dim3(blocks), dim3(lanes), 0, stream, K + k0, nK, c, g, group, od, oc);
-        if (int rc = check_hip(hipGetLastError(), "recoil_kernel")) return rc;
-    }
+        hipLaunchKernelGGL(kernel, dim3(count), dim3(lanes), 0, stream, K + k0, nK, c, g, group, od, oc);
+        return check_hip(hipGetLastError(), "recoil_kernel");
+    });
+    if (rc) return rc;
     return ok();
 }
 
