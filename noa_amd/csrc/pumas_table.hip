@@ -28,6 +28,7 @@
 
 #include "capi_util.hh"
 #include "fastmath.hh"
+#include "launch_slices.hh"
 #include "pumas_search.hh"
 
 namespace noa_hip {
@@ -555,8 +556,9 @@ __global__ __launch_bounds__(256) void pumas_dcs_kernel(int process, ElementCons
 constexpr int TABLE_WG = 256;
 constexpr int TABLE_ROWS = TABLE_WG / N_REVERSE;  // a grid has at least N_REVERSE nodes
 
-__global__ __launch_bounds__(TABLE_WG) void pumas_table_kernel(Grid g, ElementBlock blk, Globals G, int32_t e0,
-                                                               int32_t n_blk, int32_t n_el, double mass,
+// A launch runs the call's workgroups from number `start` on.
+__global__ __launch_bounds__(TABLE_WG) void pumas_table_kernel(Grid g, ElementBlock blk, Globals G, int64_t start,
+                                                               int32_t e0, int32_t n_blk, int32_t n_el, double mass,
                                                                const double* __restrict__ Ks, int32_t n_K,
                                                                float* __restrict__ table, double* __restrict__ table64,
                                                                float* __restrict__ x_out, float* __restrict__ env,
@@ -569,7 +571,7 @@ __global__ __launch_bounds__(TABLE_WG) void pumas_table_kernel(Grid g, ElementBl
     const int n = g.n;
     const int room = TABLE_WG / n;
     const int groups = (n_K + room - 1) / room;
-    const int64_t b = blockIdx.x;
+    const int64_t b = start + blockIdx.x;
     const int p = int(b / (int64_t(n_blk) * groups) + 1) % 3;
     const int j = int((b / groups) % n_blk);
     const int row = int(threadIdx.x) / n, i = int(threadIdx.x) % n;
@@ -1316,6 +1318,7 @@ struct EnvelopeArgs {
     const float* table;
     const double* csn;
     float* env;
+    int64_t start;  // number of the launch's first workgroup among the call's
     int32_t n_K;
 };
 static_assert(sizeof(EnvelopeArgs) <= MAX_KERNARG, "48 elements and the grid in one launch");
@@ -1350,7 +1353,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(WAVES))) voi
     const float* __restrict__ table = args->table;
     const double* __restrict__ csn = args->csn;
     float* __restrict__ env = args->env;
-    int64_t b = blockIdx.x;
+    int64_t b = args->start + blockIdx.x;
     int p = 1, j = 0;
     if (b < int64_t(3) * n_K) {
         p += int(b / n_K);
@@ -1531,22 +1534,24 @@ int noa_pumas_dcs_table(const double* Z, const double* A, int32_t n_elements, do
     pumas::EnvelopeGrid eg{};
     pumas::make_grid(cutoff, g, eg);
     const pumas::Globals G = pumas::make_globals();
-    // launches of equal numbers of elements (a grid has at most 2^31 - 1 workgroups)
-    const int64_t most = int64_t(0x7fffffff) / (int64_t(3) * n_K);
-    const auto per_launch = [&](int64_t room) {
-        room = std::min(room, most);
-        const int64_t launches = (n_elements + room - 1) / room;
-        return int((n_elements + launches - 1) / launches);
+    // launches of equal numbers of elements
+    const auto per_launch = [&](int room) {
+        const int launches = (n_elements + room - 1) / room;
+        return (n_elements + launches - 1) / launches;
     };
     for (int e0 = 0, per = per_launch(pumas::MAX_EL); e0 < n_elements; e0 += per) {
         const int n_blk = std::min(n_elements - e0, per);
         pumas::ElementBlock blk{};
         for (int j = 0; j < n_blk; j++) blk.e[j] = pumas::make_element(Z[e0 + j], A[e0 + j], mass, G);
         const int room = pumas::TABLE_WG / g.n;
-        const unsigned grid = unsigned(3 * n_blk * ((n_K + room - 1) / room));
-        hipLaunchKernelGGL(pumas::pumas_table_kernel, dim3(grid), dim3(pumas::TABLE_WG), 0, stream, g, blk, G, e0, n_blk,
-                           n_elements, mass, K, n_K, table, table_f64, e0 == 0 ? x : nullptr, envelope, csn);
-        if (int rc = check_hip(hipGetLastError(), "pumas_table_kernel")) return rc;
+        const int64_t workgroups = int64_t(3) * n_blk * ((n_K + room - 1) / room);
+        const int rc = launch_slices(workgroups, pumas::TABLE_WG, [&](int64_t start, uint32_t count) {
+            hipLaunchKernelGGL(pumas::pumas_table_kernel, dim3(count), dim3(pumas::TABLE_WG), 0, stream, g, blk, G,
+                               start, e0, n_blk, n_elements, mass, K, n_K, table, table_f64, e0 == 0 ? x : nullptr,
+                               envelope, csn);
+            return check_hip(hipGetLastError(), "pumas_table_kernel");
+        });
+        if (rc) return rc;
     }
     if (envelope) {
         hipLaunchKernelGGL(pumas::pumas_alpha_fill_kernel, dim3(unsigned(3 * n_elements)), dim3(64), 0, stream,
@@ -1569,14 +1574,19 @@ int noa_pumas_dcs_table(const double* Z, const double* A, int32_t n_elements, do
             args.n_blk = std::min(n_elements - args.e0, per);
             for (int j = 0; j < args.n_blk; j++)
                 args.blk.e[j] = pumas::make_element(Z[args.e0 + j], A[args.e0 + j], mass, G);
-            const unsigned rows = unsigned(3 * args.n_blk * n_K);
+            const int64_t rows = int64_t(3) * args.n_blk * n_K;
             // three waves per SIMD (40 registers spilled) where the rows are many;
             // below, the longest rows decide. Measured (us, two / three waves,
             // 146 energies): 7 elements 548 / 564, 16 575 / 595, 20 632 / 605,
             // 48 1171 / 947
-            hipLaunchKernelGGL((rows > 8000 ? &pumas::pumas_envelope_kernel<3> : &pumas::pumas_envelope_kernel<2>),
-                               dim3(rows), dim3(64), size_t(pumas::ENVELOPE_LDS) * g.n * sizeof(float), stream, args);
-            if (int rc = check_hip(hipGetLastError(), "pumas_envelope_kernel")) return rc;
+            const auto kernel = rows > 8000 ? &pumas::pumas_envelope_kernel<3> : &pumas::pumas_envelope_kernel<2>;
+            const int rc = launch_slices(rows, 64, [&](int64_t start, uint32_t count) {
+                args.start = start;
+                hipLaunchKernelGGL(kernel, dim3(count), dim3(64), size_t(pumas::ENVELOPE_LDS) * g.n * sizeof(float),
+                                   stream, args);
+                return check_hip(hipGetLastError(), "pumas_envelope_kernel");
+            });
+            if (rc) return rc;
         }
     }
     return ok();

@@ -24,3 +24,30 @@ def test_recoil(device, n, min_points):
                              dels=(part, None, None, None))
         assert torch.equal(out[a:a + 70000], part), a
     assert not bool(out.isnan().any())
+
+
+def _csn(n_el, n_K, at, device):
+    csn = torch.zeros(3, n_el, n_K, dtype=torch.float64, device=device)
+    csn[:, :, at] = 1.
+    return csn
+
+
+@pytest.mark.parametrize("n_el, n_K, cutoff", [(48, 466_100, 0.05), (30, 186_500, 3e-8)])
+def test_pumas_table(device, n_el, n_K, cutoff):
+    """2^26 rows and more of the envelope's 64-lane workgroups, and 2^24 and more of the table's of 256 lanes (one row
+    each where the grid has more than 128 nodes). A row depends on its own element's only, but for the first
+    element, whose envelope search takes the model everywhere."""
+    print(f"pumas table {n_el} x {n_K}, {pumas.n_table_dcs(cutoff)} nodes", flush=True)
+    Z = np.arange(1., n_el + 1.)
+    A = np.where(Z == 1., 1.008, 2.1 * Z)
+    K = torch.logspace(-2, 8, n_K, dtype=torch.float64, device=device)
+    at = torch.tensor([0, 1, n_K // 3, n_K // 2, n_K - 240, n_K - 204, n_K - 203, n_K - 202, n_K - 90, n_K - 2, n_K - 1],
+                      device=device)
+    table, x, env = pumas.dcs_table(Z, A, MUON_MASS, cutoff, K, csn=_csn(n_el, n_K, at, device))
+    some = [0, 1, n_el // 2, n_el - 1]
+    part, x_p, env_p = pumas.dcs_table(Z[some], A[some], MUON_MASS, cutoff, K, csn=_csn(4, n_K, at, device))
+    assert torch.equal(x, x_p)
+    for i, e in enumerate(some):
+        for a, b in ((table, part), (env, env_p)):
+            assert torch.equal(a[:, e].nan_to_num(nan=-7.0), b[:, i].nan_to_num(nan=-7.0)), e
+    assert bool((table[:, :, -1] != 0).any()) and bool((env[:, :, -1, 1] != 0).any())
