@@ -36,6 +36,7 @@
 #include "dcs_f64.hh"
 #include "dcs_small.hh"
 #include "dcs_tile.hh"
+#include "launch_slices.hh"
 
 namespace noa_hip {
 
@@ -170,9 +171,12 @@ static_assert(sizeof(Outs<double>) == sizeof(Outs<float>) && sizeof(Outs<double>
               "noa_dcs_batch::outs stands for either");
 
 hipError_t launch_direct(noa_dcs_batch* b, hipStream_t stream) {
-    if (b->n_items == 0) return hipSuccess;
-    void* args[] = {&b->K, &b->q, &b->d_consts, &b->d_items, &b->outs};
-    return hipLaunchKernel(b->kernel, dim3(b->n_items), dim3(WG), args, b->lds_pad, stream);
+    const int rc = launch_slices(b->n_items, WG, [&](int64_t first, uint32_t count) {
+        const WorkItem* items = b->d_items + first;
+        void* args[] = {&b->K, &b->q, &b->d_consts, &items, &b->outs};
+        return int(hipLaunchKernel(b->kernel, dim3(count), dim3(WG), args, b->lds_pad, stream));
+    });
+    return hipError_t(rc);
 }
 
 // Work items, longest first. Tiles are `tile` pairs while much is left, then
@@ -209,7 +213,7 @@ std::vector<WorkItem> make_items(const noa_dcs_batch* b) {
 int upload_items(noa_dcs_batch* b) {
     if (int rc = choose_kernel(b)) return rc;
     const std::vector<WorkItem> items = make_items(b);
-    if (items.size() > 0x7fffffffull) return fail(NOA_DCS_ERANGE, "too many work items");
+    if (items.size() > 0xffffffffull) return fail(NOA_DCS_ERANGE, "too many work items");
     if (b->d_items) (void)hipFree(b->d_items);
     b->d_items = nullptr;
     b->n_items = uint32_t(items.size());

@@ -1,11 +1,13 @@
 """Calls whose workgroups make 2^32 work items and more, the most that HIP takes in one launch, so that they go in
 several: against the same rows or energies in calls that one launch holds, bit for bit (a value does not depend on
 its place in a call). Most of the work is kept out of them: one closed-form process, or rows without a cross section."""
+import ctypes
+
 import numpy as np
 import pytest
 import torch
 
-from noa_amd import dcs, pumas
+from noa_amd import _lib, dcs, pumas, workload
 from noa_amd.physics import MUON_MASS, STANDARD_ROCK
 
 pytestmark = pytest.mark.gpu
@@ -51,3 +53,31 @@ def test_pumas_table(device, n_el, n_K, cutoff):
         for a, b in ((table, part), (env, env_p)):
             assert torch.equal(a[:, e].nan_to_num(nan=-7.0), b[:, i].nan_to_num(nan=-7.0)), e
     assert bool((table[:, :, -1] != 0).any()) and bool((env[:, :, -1, 1] != 0).any())
+
+
+def test_batch(device):
+    """2^24 work items and more, of one pair each: a captured graph of two launches, replayed, against the map."""
+    n = 2 ** 24 + 5
+    els = np.zeros(n, dtype=np.dtype([("A", "f8"), ("I", "f8"), ("Z", "i4")], align=True))
+    assert els.itemsize == ctypes.sizeof(_lib.Element)
+    els["A"], els["I"], els["Z"] = STANDARD_ROCK.A, STANDARD_ROCK.I, STANDARD_ROCK.Z
+    off = np.arange(n + 1, dtype=np.int64)
+    K = torch.empty(n, dtype=torch.float64, device=device)
+    q = torch.empty_like(K)
+    workload.fill_device(K, q, seed=1)
+    outs = [torch.empty_like(K) for _ in range(4)]
+    want = dcs.hip.map_all(K, q, STANDARD_ROCK, MUON_MASS)
+    config = _lib.BatchConfig(_lib.PREC_F64, 2048, 0, 1, None, 1)
+    plan = ctypes.c_void_p()
+    print("batch of 2^24 + 5 elements", flush=True)
+    _lib.check(_lib.lib().noa_dcs_batch_create(
+        els.ctypes.data_as(ctypes.POINTER(_lib.Element)), off.ctypes.data_as(ctypes.POINTER(ctypes.c_int64)), n,
+        MUON_MASS, K.data_ptr(), q.data_ptr(), *[o.data_ptr() for o in outs], ctypes.byref(config),
+        _lib.raw_stream(0), ctypes.byref(plan)))
+    for _ in range(3):
+        for o in outs:
+            o.fill_(-1.)
+        _lib.launch(_lib.lib().noa_dcs_batch_launch, 0, plan)
+        for g, w in zip(outs, want):
+            assert torch.equal(g, w)
+    _lib.check(_lib.lib().noa_dcs_batch_destroy(plan))
