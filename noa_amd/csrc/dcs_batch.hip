@@ -223,6 +223,9 @@ int upload_items(noa_dcs_batch* b) {
                      "hipMemcpy(items)");
 }
 
+// What a cache line is for. A batch that runs in small items has a line of its
+// own: nothing of it is timed, and batches of the same size bucket on the
+// other side of SMALL_BATCH must not take its values.
 std::string tune_key(const noa_dcs_batch* b) {
     hipDeviceProp_t prop;
     (void)hipGetDeviceProperties(&prop, b->device);
@@ -230,14 +233,15 @@ std::string tune_key(const noa_dcs_batch* b) {
     int lg = 0;
     while ((int64_t(1) << (lg + 1)) <= total) lg++;
     char buf[256];
-    snprintf(buf, sizeof(buf), "%s|cu%d|prec%d|el%zu|log2n%d|item-grid|tile-wpc-unroll", prop.gcnArchName, b->n_cu,
-             b->precision, b->elements.size(), lg);
+    snprintf(buf, sizeof(buf), "%s|cu%d|prec%d|el%zu|log2n%d|%s|tile-wpc-unroll", prop.gcnArchName, b->n_cu,
+             b->precision, b->elements.size(), lg, b->small ? "small-items" : "tiles");
     for (char* p = buf; *p; p++)
         if (*p == ' ') *p = '_';
     return buf;
 }
 
-// One line per tuned configuration: key, tile, workgroups per CU, unroll.
+// One line per configuration: key, tile, workgroups per CU (which the kernel
+// decides; for the reader), unroll.
 bool cache_lookup(const char* path, const std::string& key, int* tile, int* wpc, int* unroll) {
     if (!path) return false;
     FILE* f = fopen(path, "r");
@@ -389,6 +393,7 @@ int noa_dcs_batch_create(const noa_dcs_element* elements, const int64_t* offsets
         b->limit_wpc = cfg.waves_per_cu != 0;
         b->unroll = cfg.unroll ? cfg.unroll : 1;
         const bool all = cfg.tile == 0 && cfg.waves_per_cu == 0 && cfg.unroll == 0;
+        b->small = all && offsets[n_elements] - offsets[0] <= SMALL_BATCH;
         std::lock_guard<std::mutex> lock(g_tune_mutex);
         const std::string key = tune_key(b);
         int t = 0, w = 0, u = 0;
@@ -398,7 +403,6 @@ int noa_dcs_batch_create(const noa_dcs_element* elements, const int64_t* offsets
             b->tile = t;
             b->unroll = u;
         }
-        b->small = all && offsets[n_elements] - offsets[0] <= SMALL_BATCH;
         rc = cfg.tile == 0 && !cached && !b->small ? autotune(b, stream, cfg.unroll == 0) : upload_items(b);
         if (!rc && all && !cached) cache_store(cfg.tune_cache, key, b->tile, b->wpc, b->unroll);
     }
