@@ -269,17 +269,23 @@ void cache_store(const char* path, const std::string& key, int tile, int wpc, in
     fclose(f);
 }
 
-// Times the candidate tiles and node-loop unrolls on the real batch and keeps
-// the fastest. The outputs are overwritten with correct values by each run.
+// Times the candidate tiles and node-loop unrolls, those that are not given, on
+// the real batch and keeps the fastest. The outputs are overwritten with
+// correct values by each run.
 // Candidates are timed in turn, since the clock falls over the first
 // milliseconds of load: one after the other, the first looked up to 6% faster
 // than it was. Not among them, as never the fastest: tiles of 4096 (their LDS
 // leaves 2 or 3 workgroups per CU: 6.8e6 pairs FP64 648 us against 492 in
 // 2048) and the unrolled FP64 form (its registers leave one: 1111 us).
-int autotune(noa_dcs_batch* b, hipStream_t stream, bool tune_unroll) {
+// A given tile leaves the mixed form's unroll to be timed: unrolled by two it
+// is ahead where waves wait for each other and behind where the chip is full
+// (us, unroll 1 / 2: 7.9e6 pairs in tiles of 2048 423 / 445, 5.9e5 70.8 / 70.0,
+// 7.2e4 40.9 / 39.1).
+int autotune(noa_dcs_batch* b, hipStream_t stream, bool tune_tile, bool tune_unroll) {
     std::vector<noa_dcs_batch> cand;
-    for (const int t : {1024, 2048})
+    for (const int t : {1024, 2048, 4096})
         for (const int u : {1, 2}) {
+            if (tune_tile ? t == 4096 : t != b->tile) continue;
             if (tune_unroll ? u == 2 && b->precision == NOA_DCS_PREC_F64 : u != b->unroll) continue;
             cand.push_back(*b);
             cand.back().tile = t;
@@ -403,7 +409,8 @@ int noa_dcs_batch_create(const noa_dcs_element* elements, const int64_t* offsets
             b->tile = t;
             b->unroll = u;
         }
-        rc = cfg.tile == 0 && !cached && !b->small ? autotune(b, stream, cfg.unroll == 0) : upload_items(b);
+        const bool choice = cfg.tile == 0 || (cfg.unroll == 0 && cfg.precision == NOA_DCS_PREC_F32MIXED);
+        rc = choice && !cached && !b->small ? autotune(b, stream, cfg.tile == 0, cfg.unroll == 0) : upload_items(b);
         if (!rc && all && !cached) cache_store(cfg.tune_cache, key, b->tile, b->wpc, b->unroll);
     }
     if (!rc && b->use_graph && b->n_items) rc = capture_graph(b, stream);

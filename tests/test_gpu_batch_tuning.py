@@ -91,3 +91,26 @@ def test_tuned_plan_parity(device, precision, tol):
             for p in range(4):
                 r = compare(plan.outputs[p][a:b].double().cpu().numpy(), exp[p])
                 assert r["finite"] and r["zero_mismatch"] == 0 and r["max_rel"] <= tol, (e, p, r)
+
+
+@pytest.mark.parametrize("config, timed", [({"tile": 2048}, True), ({"tile": 4096, "waves_per_cu": 3}, True),
+                                           ({"waves_per_cu": 4}, True), ({"unroll": 2}, True),
+                                           ({"tile": 2048, "unroll": 1}, False)])
+@pytest.mark.parametrize("precision", ["f64", "f32mixed"])
+def test_what_is_not_given_is_timed(device, precision, config, timed):
+    """A given tile leaves the unroll open, which has a choice in the mixed form only."""
+    if precision == "f64" and "tile" in config:
+        timed = False
+    batch = _batch(70_001, device)
+    plan, was_timed = _plan(batch, precision=precision, **config)
+    assert was_timed == timed
+    info = plan.info()
+    assert {k: info[k] for k in config} == config and info["unroll"] in (1, 2)
+    if precision == "f64":
+        assert info["unroll"] == config.get("unroll", 1)
+    plan.launch()
+    both = [_plan(batch, precision=precision, tile=2048, unroll=u)[0] for u in (1, 2)]
+    for p in both:
+        p.launch()
+        for a, b in zip(plan.outputs, p.outputs):
+            assert torch.equal(a, b)
