@@ -3,6 +3,7 @@
 #pragma once
 
 #include <cmath>
+#include <cstdint>
 
 #if defined(__HIPCC__)
 #include <hip/hip_runtime.h>
@@ -32,6 +33,13 @@ NOA_SEARCH_HD int cell(const float* t, int n, float x, bool in) {
         i += d * (int(x >= a) + int(x >= b) + int(x >= c));
     }
     return i;
+}
+
+// The nodes of the first `levels` levels of a decision tree of 31 nodes, which
+// are numbered by level, as a mask. (The lane beside a tree's 31 asks for one
+// level more than there are.)
+NOA_SEARCH_HD constexpr uint32_t tree_levels(int levels) {
+    return (uint32_t(1) << ((1 << (levels < 5 ? levels : 5)) - 1)) - 1;
 }
 
 }  // namespace pumas

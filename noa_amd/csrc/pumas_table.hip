@@ -1154,9 +1154,8 @@ __device__ __forceinline__ float envelope_max(const EnvRow& a, ElementPtr cp, co
             if (m) {
                 // the model's points in the order of their levels, half 1 before
                 // half 0, as many as one batch takes
-                const auto levels = [](int l) { return (1u << ((1 << l) - 1)) - 1; };
                 const uint32_t own = uint32_t(m >> (32 * half)), other = uint32_t(m >> (32 * (half ^ 1)));
-                const int before = __popc(own & ((1u << node) - 1)) + __popc(other & levels(depth + 1 - half));
+                const int before = __popc(own & ((1u << node) - 1)) + __popc(other & tree_levels(depth + 1 - half));
                 need = need && before < batch;
             }
         }

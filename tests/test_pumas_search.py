@@ -15,6 +15,7 @@ def lib(tmp_path_factory):
     subprocess.run(["g++", "-O2", "-std=c++17", "-shared", "-fPIC",
                     os.path.join(HERE, "native", "pumas_search_host.cc"), "-o", so], check=True)
     handle = ctypes.CDLL(so)
+    handle.pumas_tree_levels.restype = ctypes.c_uint32
     handle.pumas_cell.argtypes = [ctypes.c_void_p, ctypes.c_int, ctypes.c_float, ctypes.c_int]
     return handle
 
@@ -33,3 +34,8 @@ def test_cell(lib, n):
         assert lib.pumas_cell(nodes.ctypes.data, n, np.nan, 1) == 0
         for x in (nodes[0], nodes[-1], 0.0, -1.0, 1.0, np.inf, -np.inf, np.nan):
             assert lib.pumas_cell(nodes.ctypes.data, n, x, 0) == 0
+
+
+def test_tree_levels(lib):
+    """The masks of 0 to 5 levels of a 31-node tree, and the whole tree for a level beyond its last."""
+    assert [lib.pumas_tree_levels(n) for n in range(7)] == [0, 1, 7, 127, 0x7fff, 0x7fffffff, 0x7fffffff]
