@@ -316,13 +316,9 @@ inline void soft_scattering(const Calculation& ms1, const Energies& kinetic_ener
     detail::check_output(ms1, kinetic_energies, torch::kFloat64);
     const c10::DeviceGuard guard(kinetic_energies.device());
     const int64_t n = kinetic_energies.numel();
-    const int64_t bytes = noa_dcs_soft_scattering_workspace_bytes(n);
-    const auto ws = torch::empty({std::max<int64_t>(bytes, 8)},
-                                 torch::TensorOptions().dtype(torch::kUInt8).device(kinetic_energies.device()));
     const noa_dcs_element e{element.A, element.I, element.Z};
-    detail::raise(noa_dcs_soft_scattering_f64(kinetic_energies.data_ptr<double>(), n, &e, mass,
-                                              ms1.data_ptr<double>(), ws.data_ptr(), bytes,
-                                              detail::stream_of(kinetic_energies)));
+    detail::raise(noa_dcs_soft_scattering_f64_noalloc(kinetic_energies.data_ptr<double>(), n, &e, mass,
+                                                      ms1.data_ptr<double>(), detail::stream_of(kinetic_energies)));
 }
 
 namespace hip {

@@ -202,10 +202,14 @@ int noa_dcs_hard_scattering_f64(int64_t nel, int64_t nkin, const double* G, cons
 /* Replaces dcs::soft_scattering (dcs.hh:940-950): the first transverse
  * transport coefficient of soft ionisation and photonuclear interactions.
  * workspace is a device buffer of noa_dcs_soft_scattering_workspace_bytes(n),
- * as the interface has always asked for; the kernel does not touch it. */
+ * as the interface has always asked for; the kernel does not touch it. A
+ * caller who would allocate it for this call alone takes the entry point
+ * below, which holds no device memory and gives the same results. */
 int64_t noa_dcs_soft_scattering_workspace_bytes(int64_t n);
 int noa_dcs_soft_scattering_f64(const double* K, int64_t n, const noa_dcs_element* element, double mass,
                                 double* result, void* workspace, int64_t workspace_bytes, hipStream_t stream);
+int noa_dcs_soft_scattering_f64_noalloc(const double* K, int64_t n, const noa_dcs_element* element, double mass,
+                                        double* result, hipStream_t stream);
 
 /* ---- batched uneven elements: one launch, captured in a hipGraph ----
  * Element e owns pairs [offsets[e], offsets[e+1]) of the concatenated K, q

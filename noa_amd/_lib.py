@@ -85,6 +85,7 @@ SIGNATURES = {
     "noa_dcs_hard_scattering_f64": (ctypes.c_int, [_I64, _I64, _P, _P, _P, _P, _P, _P, _P, _P]),
     "noa_dcs_soft_scattering_workspace_bytes": (ctypes.c_int64, [_I64]),
     "noa_dcs_soft_scattering_f64": (ctypes.c_int, [_P, _I64, ctypes.POINTER(Element), _D, _P, _P, _I64, _P]),
+    "noa_dcs_soft_scattering_f64_noalloc": (ctypes.c_int, [_P, _I64, ctypes.POINTER(Element), _D, _P, _P]),
     "noa_dcs_recoil_workspace_bytes": (ctypes.c_int64, [_I64, _I32]),
     "noa_dcs_recoil_integrals_f64": (ctypes.c_int, [_P, _I64, _D, ctypes.POINTER(Element), _D, _I32,
                                                     ctypes.POINTER(OutputsF64), ctypes.POINTER(OutputsF64), _P,

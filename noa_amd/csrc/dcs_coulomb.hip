@@ -731,19 +731,19 @@ int noa_dcs_hard_scattering_f64(int64_t nel, int64_t nkin, const double* G, cons
     return ok();
 }
 
-int64_t noa_dcs_soft_scattering_workspace_bytes(int64_t n) {
-    if (n <= 0) return 0;
-    return std::min<int64_t>(n, SOFT_CHUNK) * SOFT_NODES * int64_t(3 * sizeof(double));
-}
+}  // extern "C"
 
-int noa_dcs_soft_scattering_f64(const double* K, int64_t n, const noa_dcs_element* element, double mass,
-                                double* result, void* workspace, int64_t workspace_bytes, hipStream_t stream) {
+namespace {
+
+int check_soft_args(const double* K, int64_t n, const noa_dcs_element* element, double mass, const double* result) {
     if (int rc = check_element(element, mass)) return rc;
     if (n < 0) return fail(NOA_DCS_EINVAL, "n must be >= 0");
-    if (n == 0) return ok();
-    if (!K || !result) return fail(NOA_DCS_EINVAL, "K and result must be non-NULL");
-    if (!workspace || workspace_bytes < noa_dcs_soft_scattering_workspace_bytes(n))
-        return fail(NOA_DCS_EINVAL, "workspace must hold noa_dcs_soft_scattering_workspace_bytes(n) bytes");
+    if (n > 0 && (!K || !result)) return fail(NOA_DCS_EINVAL, "K and result must be non-NULL");
+    return NOA_DCS_OK;
+}
+
+int soft_run(const double* K, int64_t n, const noa_dcs_element* element, double mass, double* result,
+             hipStream_t stream) {
     // numerics.hh:72-108 on [ln 1e-6, 0] with min_points = 100 (dcs.hh:905-936)
     SoftNodes sn{};
     const double lb = std::log(1E-06);
@@ -767,6 +767,31 @@ int noa_dcs_soft_scattering_f64(const double* K, int64_t n, const noa_dcs_elemen
         if (int rc = check_hip(hipGetLastError(), "soft_kernel")) return rc;
     }
     return ok();
+}
+
+}  // namespace
+
+extern "C" {
+
+int64_t noa_dcs_soft_scattering_workspace_bytes(int64_t n) {
+    if (n <= 0) return 0;
+    return std::min<int64_t>(n, SOFT_CHUNK) * SOFT_NODES * int64_t(3 * sizeof(double));
+}
+
+int noa_dcs_soft_scattering_f64(const double* K, int64_t n, const noa_dcs_element* element, double mass,
+                                double* result, void* workspace, int64_t workspace_bytes, hipStream_t stream) {
+    if (int rc = check_soft_args(K, n, element, mass, result)) return rc;
+    if (n == 0) return ok();
+    if (!workspace || workspace_bytes < noa_dcs_soft_scattering_workspace_bytes(n))
+        return fail(NOA_DCS_EINVAL, "workspace must hold noa_dcs_soft_scattering_workspace_bytes(n) bytes");
+    return soft_run(K, n, element, mass, result, stream);
+}
+
+int noa_dcs_soft_scattering_f64_noalloc(const double* K, int64_t n, const noa_dcs_element* element, double mass,
+                                        double* result, hipStream_t stream) {
+    if (int rc = check_soft_args(K, n, element, mass, result)) return rc;
+    if (n == 0) return ok();
+    return soft_run(K, n, element, mass, result, stream);
 }
 
 }  // extern "C"

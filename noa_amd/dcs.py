@@ -394,11 +394,9 @@ def soft_scattering(ms1: torch.Tensor, kinetic_energies: torch.Tensor, element: 
     K = kinetic_energies
     _check_inputs(K, K)
     _check_output(ms1, K, torch.float64)
-    nbytes = _lib.lib().noa_dcs_soft_scattering_workspace_bytes(K.numel())
-    ws = torch.empty(max(nbytes, 8), dtype=torch.uint8, device=K.device)
     el = _element(element)
-    _launch(_lib.lib().noa_dcs_soft_scattering_f64, K, _ptr(K), K.numel(), ctypes.byref(el), float(mass), _ptr(ms1),
-            _ptr(ws), nbytes)
+    _launch(_lib.lib().noa_dcs_soft_scattering_f64_noalloc, K, _ptr(K), K.numel(), ctypes.byref(el), float(mass),
+            _ptr(ms1))
 
 
 def relative_error(computed: torch.Tensor, expected: torch.Tensor) -> torch.Tensor:
