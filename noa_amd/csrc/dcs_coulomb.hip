@@ -542,9 +542,9 @@ __device__ double soft_all_nodes(double k, const SoftNodes& sn, double mass, con
 // The photonuclear DCS is zero below nu = 2e-3 (and q = 1 GeV), so of an
 // ordinary K's 102 nodes only the last SOFT_NODES - first (23) can count and
 // the others' transport ratios need not be formed; those of K above ~500 GeV
-// all do. K outside [1e-20, 1e30] GeV and NaN, where a ratio might overflow
-// and carry its NaN into the sum, take all nodes in the reference's order
-// (soft_all_nodes).
+// all do. K outside [1e-20, 1e30] GeV and NaN, and masses outside it, where a
+// ratio might overflow and carry its NaN into the sum, take all nodes in the
+// reference's order (soft_all_nodes).
 //
 // Bound: FP64 VALU issue, ~4500 instructions per open node. Open nodes are
 // compacted in LDS and drained by whole waves; SPLIT spreads each over 9
@@ -626,7 +626,7 @@ __global__ __launch_bounds__(WG) __attribute__((amdgpu_waves_per_eu(SPLIT ? 3 : 
         if ((v & 7) == 0) {
             const DcsConsts& c = item_consts(cp);
             const double k = s.K[kk];
-            if (!(k >= 1e-20 && k <= 1e30)) acc = soft_all_nodes(k, sn, ce.mass, c, tab);
+            if (!(k >= 1e-20 && k <= 1e30 && ce.mass >= 1e-20 && ce.mass <= 1e30)) acc = soft_all_nodes(k, sn, ce.mass, c, tab);
             out[k0 + kk] = transverse_ionisation(k, ce, tab) + 2. * acc;
         }
     }
