@@ -500,6 +500,8 @@ struct SoftNodes {
     double nu[SOFT_NODES];  // X_FRACTION exp(t_j), host libm
     double h;               // subinterval width in t
     int32_t first;          // the nodes before this one have nu below the photonuclear model's 2e-3
+    double q_pole;          // sqrt(m0^2), the q whose square is m0^2: photo_ratio is 0 / 0 there
+    float pole_at, per_ln;  // K's subinterval that holds it: pole_at - per_ln ln K
 };
 
 // numerics.hh:91-108 weights.
@@ -544,7 +546,8 @@ __device__ double soft_all_nodes(double k, const SoftNodes& sn, double mass, con
 // the others' transport ratios need not be formed; those of K above ~500 GeV
 // all do. K outside [1e-20, 1e30] GeV and NaN, and masses outside it, where a
 // ratio might overflow and carry its NaN into the sum, take all nodes in the
-// reference's order (soft_all_nodes).
+// reference's order (soft_all_nodes), and so does a K one of whose nodes falls
+// on the pole of the ratio.
 //
 // Bound: FP64 VALU issue, ~4500 instructions per open node. Open nodes are
 // compacted in LDS and drained by whole waves; SPLIT spreads each over 9
@@ -623,10 +626,15 @@ __global__ __launch_bounds__(WG) __attribute__((amdgpu_waves_per_eu(SPLIT ? 3 : 
         acc += __shfl_xor(acc, 4, 8);
         acc += __shfl_xor(acc, 2, 8);
         acc += __shfl_xor(acc, 1, 8);
+        const double k = s.K[kk];
+        // (in range also where K is NaN)
+        const int itv = int(fminf(fmaxf(sn.pole_at - sn.per_ln * __logf(float(k)), 0.f), float(SOFT_ITV - 1)));
+        const bool on_pole = (v & 7) < 6 && s.nu[6 * itv + min(v & 7, 5)] * k == sn.q_pole;
+        const bool pole = (__ballot(on_pole) >> (tid & 56) & 0xff) != 0;
         if ((v & 7) == 0) {
             const DcsConsts& c = item_consts(cp);
-            const double k = s.K[kk];
-            if (!(k >= 1e-20 && k <= 1e30 && ce.mass >= 1e-20 && ce.mass <= 1e30)) acc = soft_all_nodes(k, sn, ce.mass, c, tab);
+            if (pole || !(k >= 1e-20 && k <= 1e30 && ce.mass >= 1e-20 && ce.mass <= 1e30))
+                acc = soft_all_nodes(k, sn, ce.mass, c, tab);
             out[k0 + kk] = transverse_ionisation(k, ce, tab) + 2. * acc;
         }
     }
@@ -751,6 +759,9 @@ int soft_run(const double* K, int64_t n, const noa_dcs_element* element, double 
     const double x6[6] = {0.03376524, 0.16939531, 0.38069041, 0.61930959, 0.83060469, 0.96623476};
     for (int j = 0; j < SOFT_NODES; j++)
         sn.nu[j] = X_FRACTION * std::exp(lb + sn.h * (double(uint32_t(j / 6)) + x6[j % 6]));
+    sn.q_pole = std::sqrt(0.4);
+    sn.per_ln = float(1. / sn.h);
+    sn.pole_at = float((std::log(sn.q_pole / X_FRACTION) - lb) / sn.h);
     sn.first = 0;
     while (sn.first < SOFT_NODES && sn.nu[sn.first] < 2E-03 * (1. - 1E-09)) sn.first++;
     const CoulombElement ce = make_coulomb_element(element->A, element->I, element->Z, mass);
