@@ -521,6 +521,7 @@ struct SoftLds {
     double K[TILE];
     double term[TILE];
     uint16_t list[TILE];
+    uint8_t whole[TILE];  // K slots whose nodes are all summed
     uint32_t n_open;
     // (SPLIT) the open integrals' shared values and node terms, by list entry
     double x9[9];
@@ -571,6 +572,15 @@ __global__ __launch_bounds__(WG) __attribute__((amdgpu_waves_per_eu(SPLIT ? 3 : 
     if (SPLIT && tid < 9) s.x9[tid] = GL9_X[tid];
     if (tid == 0) s.n_open = 0;
     __syncthreads();
+    for (int kk = tid; kk < nk; kk += WG) {
+        const double k = s.K[kk];
+        // (in range also where K is NaN)
+        const int itv = int(fminf(fmaxf(sn.pole_at - sn.per_ln * __logf(float(k)), 0.f), float(SOFT_ITV - 1)));
+        bool whole = !(k >= 1e-20 && k <= 1e30 && ce.mass >= 1e-20 && ce.mass <= 1e30);
+#pragma unroll
+        for (int m = 0; m < 6; m++) whole |= s.nu[6 * itv + m] * k == sn.q_pole;
+        s.whole[kk] = whole;
+    }
 #pragma unroll 1
     for (int i0 = 0; i0 < nk * nb; i0 += WG) {
         const DcsConsts& c = item_consts(cp);
@@ -626,15 +636,10 @@ __global__ __launch_bounds__(WG) __attribute__((amdgpu_waves_per_eu(SPLIT ? 3 : 
         acc += __shfl_xor(acc, 4, 8);
         acc += __shfl_xor(acc, 2, 8);
         acc += __shfl_xor(acc, 1, 8);
-        const double k = s.K[kk];
-        // (in range also where K is NaN)
-        const int itv = int(fminf(fmaxf(sn.pole_at - sn.per_ln * __logf(float(k)), 0.f), float(SOFT_ITV - 1)));
-        const bool on_pole = (v & 7) < 6 && s.nu[6 * itv + min(v & 7, 5)] * k == sn.q_pole;
-        const bool pole = (__ballot(on_pole) >> (tid & 56) & 0xff) != 0;
         if ((v & 7) == 0) {
             const DcsConsts& c = item_consts(cp);
-            if (pole || !(k >= 1e-20 && k <= 1e30 && ce.mass >= 1e-20 && ce.mass <= 1e30))
-                acc = soft_all_nodes(k, sn, ce.mass, c, tab);
+            const double k = s.K[kk];
+            if (s.whole[kk]) acc = soft_all_nodes(k, sn, ce.mass, c, tab);
             out[k0 + kk] = transverse_ionisation(k, ce, tab) + 2. * acc;
         }
     }
