@@ -6,7 +6,7 @@ A step is one fused FP64 evaluation of bremsstrahlung, pair production,
 photonuclear and ionisation over N = 2^24 (K, q) pairs of standard rock (muon),
 inputs resident in HBM. `value` is pairs evaluated per second (each pair = 4
 DCS values). The same JSON line also reports the mixed-precision FP32 form,
-the batched 48-element persistent launch and (when trained) the surrogate,
+the batched 48-element launch and (when trained) the surrogate,
 each with its max relative error against the FP64 GPU result over every pair,
 the roofline of the FP64 kernel against the FP64 vector peak, and the CPU
 baseline (the restated oracle, the reference's OpenMP path, on this host's

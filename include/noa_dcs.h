@@ -224,12 +224,17 @@ typedef struct noa_dcs_batch noa_dcs_batch;
 
 typedef struct noa_dcs_batch_config {
     int32_t precision;      /* NOA_DCS_PREC_F64 or NOA_DCS_PREC_F32MIXED */
-    int32_t tile;           /* most pairs per work item; 0 = autotuned */
+    int32_t tile;           /* most pairs per work item: 1024, 2048 or 4096; 0 = autotuned */
     int32_t waves_per_cu;   /* most workgroups resident per CU; 0 = what the kernel's registers and LDS allow */
     int32_t use_graph;      /* 1 = capture the launch in a hipGraph */
-    const char* tune_cache; /* autotune cache file, NULL = none */
+    const char* tune_cache; /* autotune cache file, NULL = none; read and written where all three are 0 */
     int32_t unroll;         /* unroll of the integrals' node loops, 1 or 2; 0 = autotuned */
 } noa_dcs_batch_config;
+
+/* Autotuning times tiles of 1024 and 2048 and, in the mixed form, either
+ * unroll, as far as they are not given. Batches of up to 200,000 pairs with
+ * tile, waves_per_cu and unroll all 0 run in work items of 64 pairs instead,
+ * with nothing to time. */
 
 /* elements and offsets are HOST arrays (n_elements and n_elements + 1
  * entries); K, q and the outputs are device arrays of offsets[n_elements]
@@ -240,7 +245,8 @@ int noa_dcs_batch_create(const noa_dcs_element* elements, const int64_t* offsets
                          hipStream_t stream, noa_dcs_batch** plan);
 int noa_dcs_batch_launch(noa_dcs_batch* plan, hipStream_t stream);
 /* Chosen tile, workgroups per CU and node-loop unroll, and the number of
- * work items; any output pointer may be NULL. */
+ * work items; any output pointer may be NULL. A plan that runs in items of 64
+ * pairs reports the defaults 2048 and 1, and the number of those items. */
 int noa_dcs_batch_info(const noa_dcs_batch* plan, int32_t* tile, int32_t* waves_per_cu, int32_t* unroll,
                        int64_t* n_items);
 int noa_dcs_batch_destroy(noa_dcs_batch* plan);
