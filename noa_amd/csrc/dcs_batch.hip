@@ -400,18 +400,22 @@ int noa_dcs_batch_create(const noa_dcs_element* elements, const int64_t* offsets
         b->unroll = cfg.unroll ? cfg.unroll : 1;
         const bool all = cfg.tile == 0 && cfg.waves_per_cu == 0 && cfg.unroll == 0;
         b->small = all && offsets[n_elements] - offsets[0] <= SMALL_BATCH;
-        std::lock_guard<std::mutex> lock(g_tune_mutex);
-        const std::string key = tune_key(b);
-        int t = 0, w = 0, u = 0;
-        const bool cached = all && cache_lookup(cfg.tune_cache, key, &t, &w, &u) &&
-                            (t == 1024 || t == 2048 || t == 4096) && w >= 1 && w <= 32 && (u == 1 || u == 2);
-        if (cached) {
-            b->tile = t;
-            b->unroll = u;
-        }
         const bool choice = cfg.tile == 0 || (cfg.unroll == 0 && cfg.precision == NOA_DCS_PREC_F32MIXED);
-        rc = choice && !cached && !b->small ? autotune(b, stream, cfg.tile == 0, cfg.unroll == 0) : upload_items(b);
-        if (!rc && all && !cached) cache_store(cfg.tune_cache, key, b->tile, b->wpc, b->unroll);
+        if (!choice && !all) {  // nothing to time, to look up or to store: nothing to wait for
+            rc = upload_items(b);
+        } else {
+            std::lock_guard<std::mutex> lock(g_tune_mutex);
+            const std::string key = tune_key(b);
+            int t = 0, w = 0, u = 0;
+            const bool cached = all && cache_lookup(cfg.tune_cache, key, &t, &w, &u) &&
+                                (t == 1024 || t == 2048 || t == 4096) && w >= 1 && w <= 32 && (u == 1 || u == 2);
+            if (cached) {
+                b->tile = t;
+                b->unroll = u;
+            }
+            rc = cached || b->small ? upload_items(b) : autotune(b, stream, cfg.tile == 0, cfg.unroll == 0);
+            if (!rc && all && !cached) cache_store(cfg.tune_cache, key, b->tile, b->wpc, b->unroll);
+        }
     }
     if (!rc && b->use_graph && b->n_items) rc = capture_graph(b, stream);
     if (rc) {

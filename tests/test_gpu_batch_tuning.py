@@ -1,6 +1,9 @@
 """The batch's autotuner and its cache file: which plans are timed, and which lines of the file they take. A timed
 plan leaves its results in the outputs before it is launched, which is how these tests see it. Batches of up to
 200,000 pairs with nothing pinned run in groups of 64 and have nothing to time."""
+import threading
+import time
+
 import numpy as np
 import pytest
 import torch
@@ -114,3 +117,36 @@ def test_what_is_not_given_is_timed(device, precision, config, timed):
         p.launch()
         for a, b in zip(plan.outputs, p.outputs):
             assert torch.equal(a, b)
+
+
+def test_given_plans_do_not_wait_for_timing(device):
+    """A plan with nothing to choose is created while another thread's is being timed (on a stream of its own). Each
+    creation takes a fraction of a millisecond, the timing ten passes over 2^26 pairs."""
+    big, small = _batch(1 << 26, device), _batch(5000, device)
+    given = dict(tile=2048, waves_per_cu=4, unroll=1, use_graph=False)
+    _plan(small, **given)[0].close()
+    torch.cuda.synchronize()
+    span = []
+
+    def timed():
+        with torch.cuda.stream(torch.cuda.Stream(device)):
+            t = time.perf_counter()
+            plan, _ = _plan(big, use_graph=False)
+            span.append(time.perf_counter() - t)
+            torch.cuda.synchronize()
+            plan.close()
+
+    outs = tuple(torch.empty(5000, dtype=torch.float64, device=device) for _ in range(4))
+    torch.cuda.synchronize()
+    thread = threading.Thread(target=timed)
+    thread.start()
+    waits, plans = [], []
+    while not span and len(plans) < 4000:
+        t = time.perf_counter()
+        plans.append(BatchPlan(*small, outputs=outs, **given))
+        waits.append(time.perf_counter() - t)
+    thread.join()
+    for p in plans:
+        p.close()
+    print(f"timing {span[0] * 1e3:.1f} ms; {len(waits)} creations beside it, the longest {max(waits) * 1e3:.2f} ms")
+    assert max(waits) < 0.5 * span[0]
